@@ -270,3 +270,23 @@ def test_lambert_shading(dev, ib):
     m = magnitude(O.lambert_backward, g, dirs, ints, nrm, diff)
     for a, b, mm, nm in zip((gdir, gint, gn, gd), r, m, ("dir", "int", "normal", "diffuse")):
         assert_close(a.cpu().numpy(), b, RTOL, "lambert grad " + nm, mag=mm)
+
+
+@pytest.mark.parametrize("W,H,L", [(1, 1, 1), (7, 37, 4), (300, 230, 5), (33, 16, 9)])
+def test_shading_backward_sums(dev, W, H, L):
+    """The light gradients are register sums of a grid-stride loop over a view's
+    pixels, lamps four at a time: one pixel, less than a workgroup, more pixels
+    than the grid has threads, and lamp counts at and past a multiple of four."""
+    from cudaExtensions import shading
+    rng = np.random.default_rng(W + L)
+    bn = 2
+    draw = lambda *s: rng.normal(size=s).astype(np.float32)
+    nrm, g, diff = draw(bn, W, H, 3), draw(bn, W, H, 3), rng.uniform(size=(bn, W, H, 3)).astype(np.float32)
+    dirs, ints, coef = draw(bn, L, 3), rng.uniform(size=(1, L, 3)).astype(np.float32), draw(bn, 3, 9)
+    for dt, rtol, eps, ops in ((np.float32, RTOL, 2.0 ** -24, 64), (np.float64, 1e-10, 2.0 ** -53, 1024)):
+        x = [t(a.astype(dt), dev) for a in (g, dirs, ints, nrm, diff, coef)]
+        got = [*shading.backward(*x[:5]), *shading.backwardSh(x[0], x[5], x[3], x[4])]
+        ref = [*O.lambert_backward(g, dirs, ints, nrm, diff), *O.sh_backward(g, coef, nrm, diff)]
+        mag = [*magnitude(O.lambert_backward, g, dirs, ints, nrm, diff), *magnitude(O.sh_backward, g, coef, nrm, diff)]
+        for q, (a, b, m) in enumerate(zip(got, ref, mag)):
+            assert_close(a.cpu().numpy(), b, rtol, "shading grad %d %s" % (q, dt.__name__), mag=m, eps=eps, ops=ops)
