@@ -156,3 +156,32 @@ def test_fused_backface_equals_torch_where(dev):
             assert a is None and b is None
             continue
         assert torch.allclose(a, b, rtol=1e-5, atol=1e-5 * float(b.abs().max()))
+
+
+def test_host_indices_of_consecutive_frames(dev):
+    """keepIndicesOnHost: each frame leaves its own complete host copy, which the
+    next frame (other samples, the same pool of page-locked blocks) leaves alone,
+    also when the shading raises."""
+    from splatting_amd import render, scenes
+    sc = scenes.config(0)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).to(dev)
+    opts = render.Options(numSamples=16, precision=0.01, shadingMode="None", device=dev)
+    r = render.Splatting(opts, None, sc.width, sc.height, sc.focal, 0.1, 10.0, 0.0)
+    zero = t(np.zeros((1, 1, 3)))
+    args = (None, None, t(sc.positions)[None], t(sc.normals)[None], t(sc.stddevs)[None], t(sc.albedo)[None], zero,
+            zero, zero)
+    kept = []
+    for seed in range(4):
+        r.seed = seed
+        _, indices, _ = r.forward(*args, transformMatrix=t(sc.view)[None])
+        assert r.indices.device.type == "cpu" and r.indices.dtype == indices.dtype
+        kept.append((r.indices, indices))
+        del indices
+    for host, device in kept:
+        assert torch.equal(host, device.cpu())
+    assert not torch.equal(kept[0][0], kept[1][0])
+    r.shadingMode = "unknown"
+    r.seed = 0
+    with pytest.raises(ValueError):
+        r.forward(*args, transformMatrix=t(sc.view)[None])
+    assert torch.equal(r.indices, kept[0][0])
