@@ -151,3 +151,20 @@ def test_sample_golden_fixture(dev):
                           t(g["sd"][None], dev), k, 0.0, float(g["precision"]), seed=seed)
     sampling.check_errors()
     assert np.array_equal(out[0].cpu().numpy(), g["idx"])
+
+
+@pytest.mark.parametrize("k", [1, 5, 63, 64, 65, 128, 129, 256])
+def test_sample_counts_at_row_edges(dev, k):
+    """The drawing kernel holds a pixel's selected keys in 1, 2 or 4 rows of 64
+    (k <= 64, 128, 256): the smallest count and both sides of every row edge, on
+    an image whose sides are no multiples of the 8x8 tile, 4,096 splats dense
+    enough that most pixels have more candidates than a row holds."""
+    from cudaExtensions import sampling
+    sc, p, n, nb, sd = scene_inputs(0, sd_scale=4.0)
+    W, H, f = 45, 31, 1.2 * 45
+    got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), t(sd[None], dev), t(sd[None], dev), k, 0.0,
+                          0.01, seed=k)
+    sampling.check_errors()
+    ref = O.sample_view(W, H, f, p, nb, sd, k, 0.0, 0.01, seed=k)
+    assert (ref >= 0).mean() > 0.2
+    assert np.array_equal(got[0].cpu().numpy(), ref)

@@ -19,8 +19,8 @@
 //   8 k_moments       Hermite moments per node over its contiguous leaf range,
 //                     accumulated in FP64 in leaf order
 //   9 k_sample_walk   per pixel tile: union FGT walk, capacity descents
-//  10 k_sample_draw   per pixel: sequential Poisson keys u/p from
-//                     Philox4x32-10, top-k in LDS
+//  10 k_sample_draw   wavefront per pixel: sequential Poisson keys u/p from
+//                     Philox4x32-10, the k smallest in order
 // The fixed-order and Poisson-rate paths share stages 1-6 and add expansion
 // selection and moments per band (k_fixed_*), walk records (k_fmm_records,
 // k_walk_records), the density walk (k_fmm_eval) and the thinning pass
@@ -1346,10 +1346,7 @@ __global__ __launch_bounds__(256) void k_samp_records(const ViewState* __restric
 // read weights and capacities from the trie and evaluate the few remaining
 // weights (below clusters that were not walked) on demand.  The reference
 // keeps the k smallest keys in a sorted insertion list (ties keep insertion
-// order, sequentialPoissonRadixTree.cuh:15-41); the same set and order are the
-// k smallest (key, draw number) words, kept here in a per-lane max-heap in LDS
-// (slot-major) and heap-sorted once at the end: O(log k) LDS steps per
-// accepted key instead of a lane-divergent O(k) shift.
+// order, sequentialPoissonRadixTree.cuh:15-41), which k_sample_draw selects.
 // Accumulators of the current DFS path, one per depth and lane, kept only for
 // the depths a descent compares (the leading nodes with more than k sources and
 // the first one below them): the first kDepthLds depths in LDS ([depth][lane],
@@ -1398,32 +1395,14 @@ struct TrieRef {
     __device__ void initCaps(int e) const { set(e, 0, 1.0f); setKids(e, 0); set(e, 4, 1.0f); }
 };
 
-// Replace the top of a per-lane max-heap of n words (LDS, slot-major
-// [slot][lane]) by x and restore the heap order.
-__device__ __forceinline__ void heap_replace_top(unsigned long long* list, int lane, int n, unsigned long long x)
-{
-    int i = 0;
-    while (true) {
-        int c = 2 * i + 1;
-        if (c >= n) break;
-        unsigned long long vc = list[c * 64 + lane];
-        if (c + 1 < n) {
-            unsigned long long vr = list[(c + 1) * 64 + lane];
-            if (vr > vc) { vc = vr; c = c + 1; }
-        }
-        if (vc <= x) break;
-        list[i * 64 + lane] = vc;
-        i = c;
-    }
-    list[i * 64 + lane] = x;
-}
-
 __global__ __launch_bounds__(64) void k_sample_walk(int W, int H, int k, int L, const ViewState* __restrict__ vs,
                                                     const NodeGeo* geo, const NodeLnk* lnk, const NodeAux* aux,
                                                     const float* coef, const SampRec* __restrict__ srec,
                                                     float* trieWs, int tcap,
-                                                    int2* __restrict__ reach, int* __restrict__ errOut)
+                                                    int2* __restrict__ reach, int* __restrict__ tieQueue,
+                                                    int* __restrict__ errOut)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) tieQueue[0] = 0;      // for k_sample_draw
     TreeView T;
     T.geo = (const NodeGeo UD_GLOBAL*)geo;
     T.lnk = (const NodeLnk UD_GLOBAL*)lnk;
@@ -1637,11 +1616,12 @@ __global__ __launch_bounds__(64) void k_sample_walk(int W, int H, int k, int L, 
     for (int la = drawn; la < L; la++) rch[(long)la * 64] = make_int2(0, 0);
 }
 
-// The key word of one candidate: (u / E(leaf) bits, draw number (launch << 16 |
-// ordinal)); false where the key is not finite (E = 0: never inserted).  Keys are
-// >= 0, so their bit patterns order like the floats.
-__device__ __forceinline__ bool draw_word(float qx, float qy, float2 xy, float is2h, uint32_t x, int la, int ord,
-                                          unsigned long long& ent)
+// The key u / E(leaf) of one candidate as its bit pattern (keys are positive, so
+// the patterns order like the floats); kNoKey where the key is not finite (E = 0:
+// never inserted).
+constexpr uint32_t kNoKey = 0xffffffffu;
+constexpr uint32_t kInfKey = 0x7f800000u;
+__device__ __forceinline__ uint32_t draw_key(float qx, float qy, float2 xy, float is2h, uint32_t x)
 {
     float tx = (qx - xy.x) * is2h;
     float ty = (qy - xy.y) * is2h;
@@ -1650,121 +1630,219 @@ __device__ __forceinline__ bool draw_word(float qx, float qy, float2 xy, float i
     wgt = wgt + (1.0f * ex) * ey;
     float p = fmaxf(0.0f, wgt);
     float key = u01(x) / p;
-    if (!(key < __builtin_huge_valf())) return false;
-    ent = ((unsigned long long)__float_as_uint(key) << 32) | (uint32_t)((la << 16) | ord);
+    return key < __builtin_huge_valf() ? __float_as_uint(key) : kNoKey;
+}
+
+// draw_key and the draw number (launch << 16 | ordinal) as one word (replay)
+__device__ __forceinline__ bool draw_word(float qx, float qy, float2 xy, float is2h, uint32_t x, int la, int ord,
+                                          unsigned long long& ent)
+{
+    const uint32_t key = draw_key(qx, qy, xy, is2h, x);
+    if (key == kNoKey) return false;
+    ent = ((unsigned long long)key << 32) | (uint32_t)((la << 16) | ord);
     return true;
+}
+
+// orders the wavefront's LDS accesses (its LDS operations execute in order)
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // Sequential Poisson keys over the leaves each launch reached (the walk's
 // capacity descents do not depend on the keys, so they run first, in
-// k_sample_walk, at the occupancy their long dependent loads need): in a Karras
-// tree the leaves of a subtree are the contiguous sorted range [first, first +
-// count), in the left-to-right order nextLeaf visits
+// k_sample_walk): in a Karras tree the leaves of a subtree are the contiguous
+// sorted range [first, first + count), in the left-to-right order nextLeaf visits
 // (sequentialPoissonDynamicTree.cuh:16-53), and every leaf carries the single
 // Hermite coefficient 1, so E(leaf) = e^{-tx^2} e^{-ty^2}.  Key u / E with u the
 // Philox word of (leaf ordinal, launch, pixel, view).  The reference keeps the
 // keys in a sorted list of k slots, inserting with a strict < and carrying each
-// displaced entry down (insertSample, sequentialPoissonRadixTree.cuh:15-41).
-// With distinct keys that list is the k smallest (key, draw number) words in
-// order, and they are kept here in a per-lane bounded max-heap in LDS,
-// heap-sorted at the end.  Equal keys are where the two differ: a carried entry
+// displaced entry down (insertSample, sequentialPoissonRadixTree.cuh:15-41); with
+// distinct keys that list is the k smallest keys in order.
+//
+// One wavefront per pixel.  A lane keys one Philox block (four leaves of one
+// launch) per iteration: at most L ceil(k / 4) blocks, since a descent stops at a
+// subtree of at most k leaves, so all keys of a pixel stay in 4 IT registers.  A
+// threshold that between k and 64 ROWS keys meet is found by galloping and
+// bisection on the key bits (ballots and scalar counts, a few steps); the keys
+// below it are compacted into LDS, ranked by comparison with LDS broadcasts, and
+// written in rank order as one coalesced row.  A lane per pixel with its k best
+// keys in an LDS heap ran the pixel's about 210 candidates and 120 heap
+// replacements as one serial chain at 2 wavefronts per SIMD (the heap's 20 KB):
+// 673 us at 1M splats, 512x512, k = 40 (now 261 us) and 226 us at 128x128, where
+// 256 wavefronts left most of the chip idle (now 19 us).
+//
+// Equal keys are where the reference's list differs from a sort: a carried entry
 // passes over entries equal to it, so an insertion ahead of a run of equal keys
 // moves the run's first entry to the run's end, and a full list drops the front
-// of its last run.  That matters exactly when two equal keys are in the heap at
-// once: the sorted heap holds two equal neighbours, or an entry it dropped ties
-// with the final maximum -- dropped keys never increase, so it is enough that
-// the last one dropped equals the final maximum (a run dropped whole leaves the
-// sample as the heap has it).  Such a lane (rare: none in 16,384 pixels of the
-// 1M-splat frame) queues itself, and k_sample_replay redraws it through the
-// reference's insertion.  (A replay path inside this kernel, never
-// taken, cost 45 % of its time in code generation.)
-__global__ __launch_bounds__(64) void k_sample_draw(int W, int H, int k, int L, uint32_t seedLo, uint32_t seedHi,
-                                                    uint32_t view, const ViewState* __restrict__ vs,
-                                                    const float2* __restrict__ leafXY,
-                                                    const int32_t* __restrict__ leafId,
-                                                    const int2* __restrict__ reach, int32_t* __restrict__ out,
-                                                    int* __restrict__ tieQueue)
+// of its last run.  A pixel with two equal keys among those at or below the
+// threshold queues itself (tieQueue: its sampler lane and its k-th smallest key,
+// infinite with fewer than k keys), and k_sample_replay redraws it through the
+// reference's insertion.
+constexpr int kDrawWaves = 4;
+template <int ROWS, int IT>
+__global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw(int W, int H, int k, int L, int tiles,
+                                                                 uint32_t seedLo, uint32_t seedHi, uint32_t view,
+                                                                 const ViewState* __restrict__ vs,
+                                                                 const float2* __restrict__ leafXY,
+                                                                 const int32_t* __restrict__ leafId,
+                                                                 const int2* __restrict__ reach,
+                                                                 int32_t* __restrict__ out, int* __restrict__ tieQueue)
 {
-    extern __shared__ unsigned long long list[];
-    const int lane = threadIdx.x;
+    constexpr int CAP = 64 * ROWS;
+    __shared__ __align__(16) uint32_t sKey[kDrawWaves][CAP];
+    __shared__ int sPos[kDrawWaves][CAP];
+    __shared__ int sOwner[kDrawWaves][CAP];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    // the blocks of a sampler tile run on the XCD its walk ran on (tile t was
+    // workgroup t of the walk: XCD t mod 8), whose L2 holds its reached ranges and
+    // most of its leaves
+    constexpr int per = 64 / kDrawWaves;                // workgroups per tile
+    const int full = tiles & ~7, d = blockIdx.x;
+    const int blk = d < full * per ? (d >> 3) / per * 8 + (d & 7) : d / per;
+    const int pl = (d < full * per ? (d >> 3) % per : d % per) * kDrawWaves + wv;
     const int tilesY = (H + 7) >> 3;
-    const uint32_t tile = xcd_chunk_remap<kSampTileRun>(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
     const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
-    const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
-    const bool valid = (i < W) && (j < H);
-    if (!valid) return;
-    // the padding word (key +inf, draw 0xffffffff) is larger than any real entry
-    const unsigned long long empty = ((unsigned long long)0x7f800000u << 32) | 0xffffffffull;
-    for (int s = 0; s < k; s++) list[s * 64 + lane] = empty;
+    const int i = ti * 8 + (pl >> 3), j = tj * 8 + (pl & 7);
+    if (i >= W || j >= H) return;                       // wave-uniform
     const float is2h = vs->is2h;
     const float qx = (float)i, qy = (float)j;
     const uint32_t pixel = (uint32_t)(j + H * i);
-    const int2* rch = reach + (long)blockIdx.x * L * 64 + lane;
-    int firstPos[16];                                   // per launch: first leaf position drawn
-    unsigned long long lastDrop = empty;               // the last word the heap dropped
-    // The lane's groups of 4 leaves, launch after launch, in one loop: the
-    // wavefront runs as many iterations as its busiest lane has groups (a loop
-    // per launch would run the busiest lane of each launch).  Each lane keys
-    // the same leaves in the same order as a loop per launch.
-    int la = 0, kk0 = 0;
-    int2 fc = rch[0];
-    firstPos[0] = fc.x;
-    while (la < L && fc.y == 0) {
-        if (++la < L) { fc = rch[(long)la * 64]; firstPos[la] = fc.x; }
-    }
-    while (la < L) {
-        const int first = fc.x, cnt = fc.y;
-        u32x4 c4 = { (uint32_t)(kk0 >> 2), (uint32_t)la, pixel, view };
-        u32x4 rnd = philox4x32_10(c4, seedLo, seedHi);
+    const int2 fc = lane < L ? reach[((long)blk * L + lane) * 64 + pl] : make_int2(0, 0);
+    uint32_t key[4 * IT];
+    int pos[IT];
+    int blocks = 0;                                     // Philox blocks of the pixel
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        if (it > 0 && blocks <= 64 * it) {              // wave-uniform
+#pragma unroll
+            for (int q = 0; q < 4; q++) key[4 * it + q] = kNoKey;
+            pos[it] = 0;
+            continue;
+        }
+        const int t = it * 64 + lane;
+        int la = 0, kk0 = 0, first = 0, cnt = 0;
+        blocks = 0;
+        for (int l = 0; l < L; l++) {
+            const int f = __builtin_amdgcn_readlane(fc.x, l), c = __builtin_amdgcn_readlane(fc.y, l);
+            const int nb = (c + 3) >> 2;
+            if (t >= blocks && t < blocks + nb) { la = l; kk0 = 4 * (t - blocks); first = f; cnt = c; }
+            blocks += nb;
+        }
+        const u32x4 rnd = philox4x32_10(u32x4{ (uint32_t)(kk0 >> 2), (uint32_t)la, pixel, view }, seedLo, seedHi);
+        pos[it] = first + kk0;
         float2 xy[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            int pos = first + kk0 + q;
-            bool ok = kk0 + q < cnt;
-            xy[q] = ok ? leafXY[pos] : make_float2(0.0f, 0.0f);
-        }
+        for (int q = 0; q < 4; q++) xy[q] = kk0 + q < cnt ? leafXY[pos[it] + q] : make_float2(0.0f, 0.0f);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            if (kk0 + q >= cnt) break;
-            unsigned long long ent;
-            if (!draw_word(qx, qy, xy[q], is2h, (q == 0) ? rnd.x : (q == 1) ? rnd.y : (q == 2) ? rnd.z : rnd.w,
-                           la, kk0 + q, ent))
-                continue;
-            const unsigned long long top = list[lane];
-            if (ent < top) {
-                lastDrop = top;
-                heap_replace_top(list, lane, k, ent);
+            const uint32_t kb = draw_key(qx, qy, xy[q], is2h,
+                                         (q == 0) ? rnd.x : (q == 1) ? rnd.y : (q == 2) ? rnd.z : rnd.w);
+            key[4 * it + q] = kk0 + q < cnt ? kb : kNoKey;
+        }
+    }
+    auto count = [&](uint32_t x) {
+        int c = 0;
+#pragma unroll
+        for (int e = 0; e < 4 * IT; e++) c += __popcll(__ballot(key[e] <= x));
+        return c;
+    };
+    // threshold: every finite key if at most CAP, else one that k .. CAP keys meet
+    uint32_t thr = kInfKey - 1;
+    int m = count(thr);
+    bool tie = false;
+    uint32_t kth = kInfKey;                             // the k-th smallest key
+    if (m > CAP) {
+        uint32_t lo = 0, hi = kInfKey - 1, step = 1u << 23;   // count(lo) < k, count(hi) > CAP
+        uint32_t mid = 0x3f800000u;                     // keys lie around 1: gallop by octaves from there
+        while (true) {
+            m = count(mid);
+            if (m >= k && m <= CAP) { thr = mid; break; }
+            const bool up = m < k;
+            if (up) lo = mid; else hi = mid;
+            if (hi - lo <= 1) { tie = true; kth = hi; break; }    // more than CAP - k keys equal hi
+            if (up && hi == kInfKey - 1) mid = hi - mid > step ? mid + step : lo + ((hi - lo) >> 1);
+            else if (!up && lo == 0) mid = mid > step ? mid - step : hi >> 1;
+            else mid = lo + ((hi - lo) >> 1);
+            step <<= 1;
+        }
+    }
+    if (!tie) {
+        uint32_t* sk = sKey[wv];
+        int base = 0;
+#pragma unroll
+        for (int e = 0; e < 4 * IT; e++) {
+            const bool in = key[e] <= thr;
+            const unsigned long long mk = __ballot(in);
+            const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0));
+            if (in) { sk[at] = key[e]; sPos[wv][at] = pos[e >> 2] + (e & 3); }
+            base += __popcll(mk);
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+            if (r * 64 + lane >= m) sk[r * 64 + lane] = kNoKey;
+        wave_lds_fence();
+        uint32_t mine[ROWS];
+        int id[ROWS], rank[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int e = r * 64 + lane;
+            mine[r] = sk[e];
+            id[r] = e < m ? leafId[sPos[wv][e]] : -1;
+            rank[r] = 0;
+        }
+        for (int q0 = 0; q0 < CAP; q0 += 16) {
+            if (q0 >= m) break;                         // wave-uniform
+            uint32_t o[16];
+#pragma unroll
+            for (int q = 0; q < 16; q += 4) {
+                const uint4 v = *(const uint4*)(sk + q0 + q);
+                o[q] = v.x; o[q + 1] = v.y; o[q + 2] = v.z; o[q + 3] = v.w;
             }
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+#pragma unroll
+                for (int r = 0; r < ROWS; r++) rank[r] += o[q] < mine[r];
         }
-        kk0 += 4;
-        if (kk0 >= cnt) {
-            kk0 = 0;
-            do {
-                if (++la < L) { fc = rch[(long)la * 64]; firstPos[la] = fc.x; }
-            } while (la < L && fc.y == 0);
+        // equal keys share a rank: of the lanes writing one place, one reads its own entry back
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+            if (r * 64 + lane < m) sOwner[wv][rank[r]] = r * 64 + lane;
+        wave_lds_fence();
+        bool dup = false;
+        uint32_t top = 0;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            if (r * 64 + lane >= m) continue;
+            dup |= sOwner[wv][rank[r]] != r * 64 + lane;
+            if (rank[r] < k && mine[r] > top) top = mine[r];
+        }
+        tie = __ballot(dup) != 0ull;
+        if (tie && m >= k) {
+            for (int o = 32; o > 0; o >>= 1) {
+                const uint32_t x = (uint32_t)__shfl_xor((int)top, o, 64);
+                top = x > top ? x : top;
+            }
+            kth = top;
+        }
+        wave_lds_fence();
+        int32_t* o = out + (long)pixel * k;
+        if (!tie) {
+            int* so = sOwner[wv];                       // ids in rank order
+#pragma unroll
+            for (int r = 0; r < ROWS; r++)
+                if (r * 64 + lane < m) so[rank[r]] = id[r];
+            wave_lds_fence();
+            for (int s = lane; s < k; s += 64) o[s] = s < m ? so[s] : -1;
         }
     }
-    // heap -> ascending order (heapsort)
-    for (int end = k - 1; end > 0; end--) {
-        unsigned long long x = list[end * 64 + lane];
-        list[end * 64 + lane] = list[lane];
-        heap_replace_top(list, lane, end, x);
-    }
-    bool tie = lastDrop != empty && key_of(lastDrop) == key_of(list[(k - 1) * 64 + lane]);
-    for (int s = 1; s < k && !tie; s++) {
-        const unsigned long long b = list[s * 64 + lane];
-        tie = b != empty && key_of(b) == key_of(list[(s - 1) * 64 + lane]);
-    }
-    if (tie) {
+    if (tie && lane == 0) {
         const int e = atomicAdd(tieQueue, 1);
-        tieQueue[1 + 2 * e] = (int)blockIdx.x * 64 + lane;
-        tieQueue[2 + 2 * e] = (int)(uint32_t)(list[(k - 1) * 64 + lane] >> 32);   // the final maximum key
-    }
-    // draw numbers -> splat ids
-    int32_t* o = out + ((long)j + (long)H * i) * k;
-    for (int s = 0; s < k; s++) {
-        uint32_t dn = (uint32_t)(list[s * 64 + lane] & 0xffffffffull);
-        o[s] = dn == 0xffffffffu ? -1 : leafId[firstPos[dn >> 16] + (int)(dn & 0xffffu)];
+        tieQueue[1 + 2 * e] = blk * 64 + pl;
+        tieQueue[2 + 2 * e] = (int)kth;
     }
 }
 
@@ -1899,12 +1977,6 @@ __global__ __launch_bounds__(64) void k_sample_replay(int W, int H, int k, int L
             }
         }
     }
-}
-
-__global__ void k_fill_i32(int* p, long n, int v)
-{
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = v;
 }
 
 __global__ void k_fill_f32(float* p, long n, float v)
@@ -2923,16 +2995,21 @@ void launch_sample(int N, int W, int H, int k, uint32_t seedLo, uint32_t seedHi,
 {
     k_samp_records<<<grid1(N, 256), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, w.srec);
     unsigned tiles = (unsigned)(((W + 7) / 8) * ((H + 7) / 8));
-    size_t lds = (size_t)k * 64 * sizeof(unsigned long long);
     const int L = num_launches(k);
     hipEvent_t e0, e1;
     bool timed = timing_pair(0, &e0, &e1);
     if (timed) (void)hipEventRecord(e0, st);
     k_sample_walk<<<tiles, 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
-                                        trie_entries(k), w.reach, err);
-    k_fill_i32<<<1, 64, 0, st>>>(w.tieQueue, 1, 0);
-    k_sample_draw<<<tiles, 64, lds, st>>>(W, H, k, L, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out,
-                                          w.tieQueue);
+                                        trie_entries(k), w.reach, w.tieQueue, err);
+    const dim3 dg(tiles * (64 / kDrawWaves));
+    // a pixel has at most L ceil(k / 4) Philox blocks, 64 per iteration: 8 x 16, 12 x 32
+    // and 16 x 64 at k = 64, 128 and 256
+#define UD_DRAW(R, I) k_sample_draw<R, I><<<dg, 64 * kDrawWaves, 0, st>>>(                                            \
+        W, H, k, L, (int)tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out, w.tieQueue)
+    if (k <= 64) UD_DRAW(1, 2);
+    else if (k <= 128) UD_DRAW(2, 6);
+    else UD_DRAW(4, 16);
+#undef UD_DRAW
     k_sample_replay<<<64, 64, 0, st>>>(W, H, k, L, tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach,
                                        w.tieQueue, out);
     if (timed) (void)hipEventRecord(e1, st);
