@@ -168,3 +168,20 @@ def test_sample_counts_at_row_edges(dev, k):
     ref = O.sample_view(W, H, f, p, nb, sd, k, 0.0, 0.01, seed=k)
     assert (ref >= 0).mean() > 0.2
     assert np.array_equal(got[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("W,H,precision,k", [(24, 24, 1e-7, 40), (20, 13, 1e-6, 16), (16, 16, 1e-8, 3)])
+def test_sample_walk_beyond_the_tile_lists(dev, W, H, precision, k):
+    """A tile's walk keeps up to 448 walked and 448 evaluated nodes in LDS; tiles
+    with more go to the depth-first form.  8,192 small splats over a few tiles at a
+    small precision: 300 to 960 evaluated nodes per tile (so both forms run, on
+    ragged tiles too), with a count of samples whose trie rows are the fewest."""
+    from cudaExtensions import sampling
+    sc, p, n, nb, sd = scene_inputs(0, 8192, sd_scale=4.0 if W == 16 else 2.0)
+    f = 1.2 * W
+    got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), t(sd[None], dev), t(sd[None], dev), k, 0.0,
+                          precision, seed=k)
+    sampling.check_errors()
+    ref = O.sample_view(W, H, f, p, nb, sd, k, 0.0, precision, seed=k)
+    assert (ref >= 0).mean() > 0.5
+    assert np.array_equal(got[0].cpu().numpy(), ref)

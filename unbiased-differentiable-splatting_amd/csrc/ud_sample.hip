@@ -18,7 +18,8 @@
 //                     nodes, device-wide exclusive scan
 //   8 k_moments       Hermite moments per node over its contiguous leaf range,
 //                     accumulated in FP64 in leaf order
-//   9 k_sample_walk   per pixel tile: union FGT walk, capacity descents
+//   9 k_sample_walk   per pixel tile: union FGT walk (k_sample_descend: the capacity
+//                     descents)
 //  10 k_sample_draw   wavefront per pixel: sequential Poisson keys u/p from
 //                     Philox4x32-10, the k smallest in order
 // The fixed-order and Poisson-rate paths share stages 1-6 and add expansion
@@ -31,6 +32,7 @@
 #include "ud_device.h"
 #include "../../include/udsplat.h"
 
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -46,6 +48,13 @@ constexpr int kMaxDepth = 64;        // descent trace bound (reference STACKSIZE
 // at 1M splats, 512x512, against one contiguous block of tiles per XCD)
 constexpr uint32_t kSampTileRun = 4;
 constexpr int kTrieFields = 5;       // 4-byte fields per descent-trie entry (TrieRef)
+constexpr int kWalkEntries = 320;    // trie entries the walk may create
+// per tile, for the descents: entries of the walk (-1: left to the serial form), error
+// flag; the pixels' totals from 64 on; the entries' info and node from 128 on
+constexpr int kTileInfo = 128 + 2 * kWalkEntries;
+// entries the descents may add: 32 per launch, and at least 96, since the walk keeps
+// its up to 5 x 96 rows of values there
+__host__ __device__ constexpr int walk_extra(int L) { return 32 * (L > 3 ? L : 3); }
 constexpr int kCullTile = 1024;      // elements per workgroup in the cull pass
 constexpr int kSortTile = 2048;      // elements per workgroup in a sort pass
 constexpr int kFixedDegree = 6;      // default expansion order of the fixed-order densities (hermitefmm.cuh:11)
@@ -91,7 +100,7 @@ struct SampChild {
     float lox, loy, hix, hiy;    // box
     float cx, cy, r2;            // expansion centre, squared truncation radius
     int deg;                     // Hermite degree, -1 when the walk goes below
-    int off, count, id, pad;     // coefficient offset, leaves under it, node index
+    int off, count, id, first;   // coefficient offset, leaves under it, node index, its first leaf
 };
 struct SampRec {
     SampChild l, r;
@@ -142,6 +151,8 @@ struct TreeWs {
     float* trie;
     SampRec* srec;        // per internal node: children records of the sampler's walk
     int2* reach;          // per launch and pixel lane: leaf range the capacity descent reached
+    int* tileInfo;        // per sampler tile: what the descents need of its walk (kTileInfo words)
+    int* walkQueue;       // [0]: count, then the tiles k_sample_walk left to its serial form
     int* tieQueue;                    // [0]: count, then (sampler lane, final key bits) per lane that met equal keys
     float2* leafXY;       // sorted position -> screen position of the leaf
     float* coef;
@@ -200,6 +211,8 @@ size_t carve(void* ws, int N, int W, int H, int k, int mode, TreeWs* t)
     w.trie = fixedOrder ? nullptr : (float*)take(4L * kTrieFields * trie_entries(k) * lanes);
     w.srec = fixedOrder ? nullptr : (SampRec*)take(sizeof(SampRec) * n);
     w.reach = fixedOrder ? nullptr : (int2*)take(8L * 16 * lanes);
+    w.tileInfo = fixedOrder ? nullptr : (int*)take(4L * kTileInfo * (lanes / 64));
+    w.walkQueue = fixedOrder ? nullptr : (int*)take(4 * (lanes / 64 + 1));
     w.tieQueue = fixedOrder ? nullptr : (int*)take(4 * (2 * lanes + 1));
     w.leafXY = (float2*)take(8 * n);
     w.coef = fixedOrder ? nullptr : (float*)take(4 * coefCap);
@@ -1181,18 +1194,25 @@ __device__ __forceinline__ float eval_node(const TreeView& T, const NodeGeo& g, 
 #pragma unroll
     for (int n = 2; n <= kMaxDegree; n++)
         hy[n] = (n <= p) ? __builtin_fmaf(2.0f * ty, hy[n - 1], -((2.0f * (float)(n - 1)) * hy[n - 2])) : 0.0f;
+    // a row's loads are issued together, past its end with the last element again
+    // (predicated loads would wait for each other)
     float w = 0.0f;
     float hprev = 0.0f, ha = ex;
     for (int a = 0; a <= p; a++) {
+        const float UD_GLOBAL* at = c + a * (p + 1);
+        float row[kMaxDegree + 1];
+#pragma unroll
+        for (int b = 0; b <= kMaxDegree; b++) row[b] = at[b < p ? b : p];
         if (a == 1) { hprev = ex; ha = (2.0f * tx) * ex; }
         else if (a >= 2) {
             float hn = __builtin_fmaf(2.0f * tx, ha, -((2.0f * (float)(a - 1)) * hprev));
             hprev = ha; ha = hn;
         }
-        const float UD_GLOBAL* row = c + a * (p + 1);
 #pragma unroll
-        for (int b = 0; b <= kMaxDegree; b++)
-            if (b <= p) w = __builtin_fmaf(row[b] * ha, hy[b], w);
+        for (int b = 0; b <= kMaxDegree; b++) {
+            const float t = __builtin_fmaf(row[b] * ha, hy[b], w);
+            w = b <= p ? t : w;
+        }
     }
     return w;
 }
@@ -1225,50 +1245,64 @@ __device__ __forceinline__ float hermite_series(const float* sc, float tx, float
     return w;
 }
 
+// hermite_series for the higher degrees: the rows in a loop (unrolling 100 and more
+// terms makes the compiler hoist their LDS reads into 256 registers), the terms of
+// a row unrolled exactly
+template <int P>
+__device__ __forceinline__ float hermite_rows(const float* sc, float tx, float ty, float ex, float ey)
+{
+    float hy[P + 1];
+    hy[0] = ey;
+    hy[1] = (2.0f * ty) * ey;
+#pragma unroll
+    for (int n = 2; n <= P; n++) hy[n] = __builtin_fmaf(2.0f * ty, hy[n - 1], -((2.0f * (float)(n - 1)) * hy[n - 2]));
+    float w = 0.0f, hprev = ex, ha = (2.0f * tx) * ex;
+#pragma unroll
+    for (int b = 0; b <= P; b++) w = __builtin_fmaf(sc[b] * ex, hy[b], w);
+#pragma unroll 1
+    for (int a = 1; a <= P; a++) {
+        const float* row = sc + a * (P + 1);
+#pragma unroll
+        for (int b = 0; b <= P; b++) w = __builtin_fmaf(row[b] * ha, hy[b], w);
+        const float hn = __builtin_fmaf(2.0f * tx, ha, -((2.0f * (float)a) * hprev));
+        hprev = ha; ha = hn;
+    }
+    return w;
+}
+
+// orders the wavefront's LDS accesses (its LDS operations execute in order)
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the degree-p expansion at scaled offset (tx, ty), its coefficients in LDS (read by
+// broadcast; p wave-uniform), the series unrolled for its degree
+__device__ __forceinline__ float hermite_at(const float* sc, int p, float tx, float ty)
+{
+    const float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
+    switch (p) {
+#define UD_SERIES(P) case P: return hermite_series<P>(sc, tx, ty, ex, ey);
+    UD_SERIES(0) UD_SERIES(1) UD_SERIES(2) UD_SERIES(3) UD_SERIES(4) UD_SERIES(5) UD_SERIES(6) UD_SERIES(7)
+#undef UD_SERIES
+#define UD_SERIES(P) case P: return hermite_rows<P>(sc, tx, ty, ex, ey);
+    UD_SERIES(8) UD_SERIES(9) UD_SERIES(10) UD_SERIES(11) UD_SERIES(12) UD_SERIES(13) UD_SERIES(14) UD_SERIES(15)
+#undef UD_SERIES
+    default: return hermite_rows<kMaxDegree>(sc, tx, ty, ex, ey);
+    }
+}
+
 // eval_node for a wave-uniform node: the coefficient block is staged in LDS
-// (read by broadcast) and the series is unrolled for the node's degree
 __device__ __forceinline__ float eval_node_staged(const TreeView& T, const NodeGeo& g, int off, float qx, float qy,
                                                   bool act, float* sc, int lane)
 {
-    const int p = g.deg;
-    const int np = (p + 1) * (p + 1);
+    const int np = (g.deg + 1) * (g.deg + 1);
     const float UD_GLOBAL* c = T.coef + off;
     for (int q = lane; q < np; q += 64) sc[q] = c[q];
-    __builtin_amdgcn_wave_barrier();
-    float w = 0.0f;
-    if (act) {
-        float tx = (qx - g.cx) * T.is2h;
-        float ty = (qy - g.cy) * T.is2h;
-        float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
-        switch (p) {
-#define UD_SERIES(P) case P: w = hermite_series<P>(sc, tx, ty, ex, ey); break;
-        UD_SERIES(0) UD_SERIES(1) UD_SERIES(2) UD_SERIES(3) UD_SERIES(4) UD_SERIES(5) UD_SERIES(6)
-        UD_SERIES(7) UD_SERIES(8)
-#undef UD_SERIES
-        default: {
-            // degrees 9 .. 16 (few nodes): loops to the maximum degree, predicated
-            float hy[kMaxDegree + 1];
-            hy[0] = ey;
-            hy[1] = (2.0f * ty) * ey;
-#pragma unroll
-            for (int n = 2; n <= kMaxDegree; n++)
-                hy[n] = (n <= p) ? __builtin_fmaf(2.0f * ty, hy[n - 1], -((2.0f * (float)(n - 1)) * hy[n - 2])) : 0.0f;
-            float hprev = 0.0f, ha = ex;
-            for (int a = 0; a <= p; a++) {
-                if (a == 1) { hprev = ex; ha = (2.0f * tx) * ex; }
-                else if (a >= 2) {
-                    float hn = __builtin_fmaf(2.0f * tx, ha, -((2.0f * (float)(a - 1)) * hprev));
-                    hprev = ha; ha = hn;
-                }
-                const float* row = sc + a * (p + 1);
-#pragma unroll
-                for (int b = 0; b <= kMaxDegree; b++)
-                    if (b <= p) w = __builtin_fmaf(row[b] * ha, hy[b], w);
-            }
-        }
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_fence();
+    const float w = act ? hermite_at(sc, g.deg, (qx - g.cx) * T.is2h, (qy - g.cy) * T.is2h) : 0.0f;
+    wave_lds_fence();
     return w;
 }
 
@@ -1282,7 +1316,7 @@ __device__ __forceinline__ bool truncated(const NodeGeo& g, float qx, float qy)
     return !(d2 < g.r2);
 }
 
-__device__ __noinline__ float tree_weight(const TreeView& T, int entry, float qx, float qy)
+__device__ __forceinline__ float tree_weight(const TreeView& T, int entry, float qx, float qy)
 {
     NodeGeo g = ld_geo(T, entry);
     if (g.deg >= 0) return eval_node(T, g, entry, qx, qy);
@@ -1312,16 +1346,25 @@ __device__ __forceinline__ SampChild samp_child(int c, const NodeGeo* __restrict
     SampChild r;
     r.lox = g.lox; r.loy = g.loy; r.hix = g.hix; r.hiy = g.hiy;
     r.cx = g.cx; r.cy = g.cy; r.r2 = g.r2; r.deg = g.deg;
-    r.off = aux[c].off; r.count = lnk[c].count; r.id = c; r.pad = 0;
+    const NodeAux a = aux[c];
+    r.off = a.off; r.count = lnk[c].count; r.id = c; r.first = a.first;
     return r;
 }
 
 __global__ __launch_bounds__(256) void k_samp_records(const ViewState* __restrict__ vs,
                                                       const NodeGeo* __restrict__ geo,
                                                       const NodeLnk* __restrict__ lnk,
-                                                      const NodeAux* __restrict__ aux, SampRec* __restrict__ rec)
+                                                      const NodeAux* __restrict__ aux, SampRec* __restrict__ rec,
+                                                      int* __restrict__ walkQueue, int* __restrict__ tieQueue,
+                                                      VStride vsd)
 {
+    vs = vw(vs, vsd.ws);
+    geo = vw(geo, vsd.ws);
+    lnk = vw(lnk, vsd.ws);
+    aux = vw(aux, vsd.ws);
+    rec = vw(rec, vsd.ws);
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == 0) { *vw(walkQueue, vsd.ws) = 0; *vw(tieQueue, vsd.ws) = 0; }      // filled by the next passes
     const int nc = vs->nc;
     if (nc <= 1 || p >= nc - 1) return;
     const NodeLnk lk = lnk[p];
@@ -1337,17 +1380,16 @@ __global__ __launch_bounds__(256) void k_samp_records(const ViewState* __restric
 // frontier of the root's walk (nodes with degree >= 0, or truncated ones that
 // contribute 0): the walk from any node n stops exactly where the root's walk
 // stops inside n's subtree, because the stop rule depends only on the node and
-// the pixel.  So one depth-first pass over the root's walk, adding each
-// frontier value to the accumulators of its ancestors in traversal order,
-// produces W(n) for every node on it bit for bit as the reference's
-// per-call walks (evaluateDynamicRadixTree.cuh:128-174) would.  The pass
+// the pixel.  So the frontier values of the root's walk, added up for each
+// ancestor in traversal order, give W(n) for every node on it bit for bit as the
+// reference's per-call walks (evaluateDynamicRadixTree.cuh:128-174) would.  The pass
 // records, for each walked node with more than k sources, the weights of its
 // two children in a trie of descent states; the ceil(sqrt(k)) descents then
 // read weights and capacities from the trie and evaluate the few remaining
 // weights (below clusters that were not walked) on demand.  The reference
 // keeps the k smallest keys in a sorted insertion list (ties keep insertion
 // order, sequentialPoissonRadixTree.cuh:15-41), which k_sample_draw selects.
-// Accumulators of the current DFS path, one per depth and lane, kept only for
+// Accumulators of k_sample_walk_serial's path, one per depth and lane, kept only for
 // the depths a descent compares (the leading nodes with more than k sources and
 // the first one below them): the first kDepthLds depths in LDS ([depth][lane],
 // indices are wave-uniform), deeper ones (rare: about 20 levels cover k = 40 at
@@ -1395,44 +1437,317 @@ struct TrieRef {
     __device__ void initCaps(int e) const { set(e, 0, 1.0f); setKids(e, 0); set(e, 4, 1.0f); }
 };
 
-__global__ __launch_bounds__(64) void k_sample_walk(int W, int H, int k, int L, const ViewState* __restrict__ vs,
-                                                    const NodeGeo* geo, const NodeLnk* lnk, const NodeAux* aux,
-                                                    const float* coef, const SampRec* __restrict__ srec,
-                                                    float* trieWs, int tcap,
-                                                    int2* __restrict__ reach, int* __restrict__ tieQueue,
-                                                    int* __restrict__ errOut)
+// The ceil(sqrt(k)) capacity descents of one pixel over its trie (nt entries so
+// far), recording each launch's reached leaf range; returns the launches recorded
+// (bad: a path or the trie grew past its bound).
+__device__ __forceinline__ int capacity_descents(const TreeView& T, const TrieRef& tr, int nt, int TMAX, int k, int L,
+                                                 int L0, float qx, float qy, int2* rch, bool& bad)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) tieQueue[0] = 0;      // for k_sample_draw
+    const float unset = __builtin_nanf("");              // weight not computed yet
+    int drawn = 0;
+    int pe[kMaxDepth];
+    float pp[kMaxDepth], pc[kMaxDepth];
+    for (int la = 0; la < L && !bad; la++) {
+        int e = 0, nd = 0, depth = 0;
+        uint64_t sideBits = 0;         // bit d: the step to depth d went right
+        pe[0] = 0;
+        NodeLnk lk = ld_lnk(T, nd);
+        while (lk.count > k) {
+            // one round of loads: the node's link (issued at the end of the last
+            // step) and the entry's weights, children and capacities
+            float wl = tr.get(e, 1), wr = tr.get(e, 2);
+            const int kids = tr.kids(e);
+            const float cl = tr.get(e, 0), cr = tr.get(e, 4);
+            if (wl != wl) {
+#pragma unroll 1
+                for (int c = 0; c < 2; c++) {              // one copy of the inlined walk
+                    const float w = tree_weight(T, c ? lk.right : lk.left, qx, qy);
+                    tr.set(e, 1 + c, w);
+                    if (c) wr = w; else wl = w;
+                }
+            }
+            wl = fmaxf(0.0f, wl); wr = fmaxf(0.0f, wr);
+            float sum = wl + wr;
+            wl = wl / sum; wr = wr / sum;
+            int el = (kids & 0xffff) - 1, er = (kids >> 16) - 1;
+            float sl = wl * cl, sr = wr * cr;
+            bool goRight = sl < sr;
+            int ce = goRight ? er : el;
+            int cnode = goRight ? lk.right : lk.left;
+            if (ce < 0) {
+                if (nt >= TMAX) { bad = true; break; }
+                ce = nt++;
+                tr.init(ce, unset);
+                tr.setKidHalf(e, goRight, ce + 1);
+            }
+            depth++;
+            if (depth >= kMaxDepth) { bad = true; break; }
+            pe[depth] = ce;
+            pp[depth] = goRight ? wr : wl;
+            pc[depth] = goRight ? cr : cl;     // its capacity, unchanged until the update below
+            if (goRight) sideBits |= 1ull << depth;
+            e = ce;
+            nd = cnode;
+            lk = ld_lnk(T, nd);
+        }
+        if (bad) break;
+        // capacities: an entry's lives in its parent's entry (field 4 if it is
+        // the right child, else 0); the path's were read on the way down
+        float prob = 1.0f;
+        for (int dd = depth; dd >= 1; dd--) {
+            const int par = pe[dd - 1];
+            const int fld = ((sideBits >> dd) & 1ull) ? 4 : 0;
+            tr.set(par, fld, fmaxf(0.0f, pc[dd] - prob));
+            prob = prob * pp[dd];
+        }
+        // the reached subtree's leaves are the contiguous sorted range
+        // [first, first + count); k_sample_draw keys them
+        const int cnt = lk.count;
+        const int first = (nd >= L0) ? nd - L0 : T.aux[nd].first;
+        rch[(long)la * 64] = make_int2(first, cnt);
+        drawn = la + 1;
+    }
+    return drawn;
+}
+
+// The path of a descent: entry << 1 | side (-1: no capacity to update), probability of
+// the step, capacity before it.  The first kPathLds steps in LDS ([step][lane]; a
+// descent has about 4 at 1M splats), the rest in private memory.
+constexpr int kPathLds = 8;
+struct PathStep {
+    int at;
+    float prob, cap;
+};
+struct DescentPath {
+    int* lds;                       // [3][kPathLds][64], offset by the lane
+    int at[kMaxDepth - kPathLds];
+    float prob[kMaxDepth - kPathLds], cap[kMaxDepth - kPathLds];
+    __device__ void set(int q, int a, float p, float c)
+    {
+        if (q < kPathLds) {
+            lds[q * 64] = a;
+            lds[(kPathLds + q) * 64] = __float_as_int(p);
+            lds[(2 * kPathLds + q) * 64] = __float_as_int(c);
+        } else {
+            at[q - kPathLds] = a; prob[q - kPathLds] = p; cap[q - kPathLds] = c;
+        }
+    }
+    __device__ PathStep get(int q) const
+    {
+        if (q < kPathLds)
+            return PathStep{ lds[q * 64], __int_as_float(lds[(kPathLds + q) * 64]),
+                             __int_as_float(lds[(2 * kPathLds + q) * 64]) };
+        return PathStep{ at[q - kPathLds], prob[q - kPathLds], cap[q - kPathLds] };
+    }
+};
+
+// capacity_descents for a tile whose trie k_sample_walk built, with the tile's
+// entries described in LDS: info[e] holds the entries + 1 of its children (left |
+// right << 10) and which of them hold rows of the walk (bit 20 left, 21 right),
+// node[e] its tree node.
+//
+// Where only one child of an entry holds rows, its sibling weighs exactly 0 for
+// every pixel that reaches the entry, so that child has its parent's weight W, the
+// step to it has probability W / W = 1, and the capacities along a run of such
+// entries are all the same number: 1 less the probabilities below the run of the
+// launches that took it.  A pixel with W > 0 therefore crosses the run in LDS with
+// the capacity of its first child (rootCap, or the one in the entry that branches
+// above it) and no memory access: a left step always goes left (1 cap < 0 cr never
+// holds), a right step goes right while cap > 0 and otherwise left, into a child of
+// weight 0, where the general descent goes on.  Entries where both children hold rows
+// are stepped as ever; at 1M splats, 512x512 they are 3.6 of the 14.6 steps of a
+// descent.  A pixel that steps into a child of weight <= 0 stays with the general
+// descent there, in this launch and every other (its weight is fixed), so the
+// capacities of a run are kept in one place.  A general part whose steps all find
+// weights 0 / 0 goes left at each of them whatever the capacities are, and ends at the
+// same leaves with probability NaN each time: it is remembered (memo*).
+__device__ __forceinline__ int tile_descents(const TreeView& T, const SampRec UD_GLOBAL* srec, const TrieRef& tr,
+                                             int tileEnts, int nt, int TMAX, int k, int L, int L0, float qx, float qy,
+                                             float total, const uint32_t* info, const int* node, int* ldsPath,
+                                             int2* rch, bool& bad)
+{
+    const float unset = __builtin_nanf("");              // weight not computed yet
+    const float inf = __builtin_huge_valf();
+    DescentPath path;
+    path.lds = ldsPath;
+    float rootCap = 1.0f;
+    int memoKey = -1, memoFirst = 0, memoCnt = 0;
+    const bool inTile = tileEnts > 0 && total > 0.0f && total < inf;
+    int drawn = 0;
+    for (int la = 0; la < L; la++) {
+        int np = 0, depth = 0, e = 0, side = 0;
+        float cap = rootCap, own = total;                // own: clamped weight of the node reached
+        i4v ref = { 0, L0 + 1, 0, 0 };                   // the root: all leaves from the first
+        while (inTile) {
+            const uint32_t inf_ = info[e];
+            const uint32_t type = (inf_ >> 20) & 3u;
+            depth++;
+            if (type == 3u) {
+                float wl = fmaxf(0.0f, tr.get(e, 1)), wr = fmaxf(0.0f, tr.get(e, 2));
+                const float cl = tr.get(e, 0), cr = tr.get(e, 4);
+                const float l0 = wl, r0 = wr, sum = wl + wr;
+                wl = wl / sum; wr = wr / sum;
+                side = wl * cl < wr * cr ? 1 : 0;
+                own = side ? r0 : l0;
+                cap = side ? cr : cl;
+                path.set(np++, e << 1 | side, side ? wr : wl, cap);
+            } else if (type == 2u && !(cap > 0.0f)) {
+                path.set(np++, -1, 0.0f, 0.0f);
+                side = 0;
+                own = 0.0f;
+                break;
+            } else {
+                side = type == 2u ? 1 : 0;
+            }
+            const int kid = (int)((inf_ >> (10 * side)) & 1023u);
+            if (kid == 0 || !(own > 0.0f && own < inf)) break;
+            e = kid - 1;
+        }
+        // child `side` of entry e (or the root): a subtree of at most k leaves, or the
+        // general descent
+        if (inTile) ref = *((const i4v UD_GLOBAL*)(srec + node[e]) + 3 * side + 2);
+        int first = ref.w, cnt = ref.y;
+        float prob = 1.0f;
+        if (cnt > k && memoKey == (e << 1 | side)) {
+            first = memoFirst; cnt = memoCnt; prob = unset;
+        } else if (cnt > k) {
+            const int key = e << 1 | side;
+            int ge = 0, nd = ref.z;
+            bool fresh = false;                           // an entry of this step: nothing to load
+            if (inTile) {
+                const int kids = tr.kids(e);
+                ge = (side ? kids >> 16 : kids & 0xffff) - 1;
+                if (ge < 0) {
+                    if (nt >= TMAX) { bad = true; break; }
+                    ge = nt++;
+                    fresh = true;
+                    tr.setKidHalf(e, side, ge + 1);
+                }
+            }
+            bool still = true;                            // every step so far found 0 / 0
+            while (cnt > k) {
+                // one round of loads: the children's records and, of an entry that is
+                // there already, its weights, children and capacities
+                const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + nd);
+                const i4v lref = *(const i4v UD_GLOBAL*)(rec + 2), rref = *(const i4v UD_GLOBAL*)(rec + 5);
+                float wl = unset, wr = unset, cl = 1.0f, cr = 1.0f;
+                int gk = 0;
+                if (!fresh) {
+                    wl = tr.get(ge, 1); wr = tr.get(ge, 2);
+                    cl = tr.get(ge, 0); cr = tr.get(ge, 4);
+                    gk = tr.kids(ge);
+                }
+                if (wl != wl) {
+                    // a child truncated for this pixel weighs 0; others are walked
+                    f4v box[2], mid[2];
+#pragma unroll
+                    for (int c = 0; c < 2; c++) { box[c] = rec[3 * c]; mid[c] = rec[3 * c + 1]; }
+                    bool zero[2];
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        NodeGeo g;
+                        g.lox = box[c].x; g.loy = box[c].y; g.hix = box[c].z; g.hiy = box[c].w;
+                        g.r2 = mid[c].z;
+                        zero[c] = __float_as_int(mid[c].w) < 0 && truncated(g, qx, qy);
+                    }
+#pragma unroll 1
+                    for (int c = 0; c < 2; c++) {              // one copy of the inlined walk
+                        float w = 0.0f;
+                        if (!(c ? zero[1] : zero[0])) w = tree_weight(T, c ? rref.z : lref.z, qx, qy);
+                        tr.set(ge, 1 + c, w);
+                        if (c) wr = w; else wl = w;
+                    }
+                    if (fresh) { tr.set(ge, 0, 1.0f); tr.set(ge, 4, 1.0f); }
+                }
+                wl = fmaxf(0.0f, wl); wr = fmaxf(0.0f, wr);
+                if (ge < tileEnts && wl == 0.0f && wr == 0.0f) {
+                    // an entry of the tile whose rows one child holds is stored as 0, 0
+                    // (the pixel reached it): that child's weight is the entry's own
+                    const uint32_t type = (info[ge] >> 20) & 3u;
+                    if (type == 1u) wl = own;
+                    if (type == 2u) wr = own;
+                }
+                const float l0 = wl, r0 = wr, sum = wl + wr;
+                wl = wl / sum; wr = wr / sum;
+                still = still && wl != wl && wr != wr;
+                const bool right = wl * cl < wr * cr;
+                own = right ? r0 : l0;
+                const i4v to = right ? rref : lref;
+                nd = to.z; cnt = to.y; first = to.w;
+                int ce = (right ? gk >> 16 : gk & 0xffff) - 1;
+                const bool was = fresh;
+                fresh = false;
+                if (ce < 0) {
+                    if (nt >= TMAX) { bad = true; break; }
+                    ce = nt++;
+                    fresh = true;
+                    if (was) tr.setKids(ge, right ? (ce + 1) << 16 : ce + 1);
+                    else tr.setKidHalf(ge, right, ce + 1);
+                }
+                depth++;
+                if (depth >= kMaxDepth) { bad = true; break; }
+                path.set(np++, ge << 1 | (right ? 1 : 0), right ? wr : wl, right ? cr : cl);
+                ge = ce;
+            }
+            if (bad) break;
+            if (still) { memoKey = key; memoFirst = first; memoCnt = cnt; }
+        }
+        for (int q = np - 1; q >= 0; q--) {
+            const PathStep st = path.get(q);
+            if (st.at >= 0) tr.set(st.at >> 1, (st.at & 1) ? 4 : 0, fmaxf(0.0f, st.cap - prob));
+            prob = prob * st.prob;
+        }
+        rootCap = fmaxf(0.0f, rootCap - prob);
+        rch[(long)la * 64] = make_int2(first, cnt);
+        drawn = la + 1;
+    }
+    return drawn;
+}
+
+// k_sample_walk's pass for the tiles whose walk outgrows its LDS lists (queued
+// there): the same weights by one depth-first walk per wavefront, a persistent grid
+// over the queue.
+__global__ __launch_bounds__(64) void k_sample_walk_serial(int W, int H, int k, int L, int tiles,
+                                                           const ViewState* __restrict__ vs, const NodeGeo* geo,
+                                                           const NodeLnk* lnk, const NodeAux* aux, const float* coef,
+                                                           const SampRec* __restrict__ srec, float* trieWs, int tcap,
+                                                           int2* __restrict__ reach,
+                                                           const int* __restrict__ walkQueue,
+                                                           int* __restrict__ errOut, VStride vsd)
+{
+    walkQueue = vw(walkQueue, vsd.ws);
+    const int queued = walkQueue[0];
+    if ((int)blockIdx.x >= queued) return;
+    vs = vw(vs, vsd.ws);
+    srec = vw(srec, vsd.ws);
+    trieWs = vw(trieWs, vsd.ws);
+    reach = vw(reach, vsd.ws);
     TreeView T;
-    T.geo = (const NodeGeo UD_GLOBAL*)geo;
-    T.lnk = (const NodeLnk UD_GLOBAL*)lnk;
-    T.aux = (const NodeAux UD_GLOBAL*)aux;
-    T.coef = (const float UD_GLOBAL*)coef;
+    T.geo = (const NodeGeo UD_GLOBAL*)vw(geo, vsd.ws);
+    T.lnk = (const NodeLnk UD_GLOBAL*)vw(lnk, vsd.ws);
+    T.aux = (const NodeAux UD_GLOBAL*)vw(aux, vsd.ws);
+    T.coef = (const float UD_GLOBAL*)vw(coef, vsd.ws);
     T.s2h = vs->s2h;
     T.is2h = vs->is2h;
-    const int TMAX = tcap;
-    const int DFSMAX = tcap - L * 32;                 // entries the walk may create
+    const int DFSMAX = tcap - walk_extra(L);             // entries the walk may create
     const int lane = threadIdx.x;
-    TrieRef tr;
-    tr.base = (float UD_GLOBAL*)trieWs + (long)blockIdx.x * kTrieFields * tcap * 64 + lane;
     const int tilesY = (H + 7) >> 3;
-    const uint32_t tile = xcd_chunk_remap<kSampTileRun>(blockIdx.x, gridDim.x);
-    const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
-    const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
-    const bool valid = (i < W) && (j < H);
-    int2* rch = reach + (long)blockIdx.x * L * 64 + lane;   // [launch][lane] of this tile
-    int drawn = 0;                                      // launches whose leaf range is recorded
-    const int n = vs->nc;
+    const int L0 = vs->nc - 1;
     const float prec = vs->prec;
-    const bool runTree = n > 0 && vs->err == 0;          // wave-uniform
-    const int L0 = n - 1;
-    const float qx = (float)i, qy = (float)j;
     const float unset = __builtin_nanf("");              // weight not computed yet
-    // trie fields: cap, wl, wr, kids = (left entry + 1) | (right entry + 1) << 16
-    int nt = 1;
-    bool bad = false;
-    float total = 0.0f;
-    if (runTree) {
+    for (int qe = blockIdx.x; qe < queued; qe += gridDim.x) {
+        const int blk = walkQueue[1 + qe];
+        TrieRef tr;
+        tr.base = (float UD_GLOBAL*)trieWs + (long)blk * kTrieFields * tcap * 64 + lane;
+        const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
+        const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
+        const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
+        const bool valid = (i < W) && (j < H);
+        int2* rch = reach + (long)blk * L * 64 + lane;   // [launch][lane] of this tile
+        const float qx = (float)i, qy = (float)j;
+        int nt = 1;
+        bool bad = false;
+        float total = 0.0f;
         tr.init(0, unset);                                // entry 0: the root
         // ---- one depth-first pass over the union of the 64 lanes' FGT walks ----
         // The wavefront visits nodes in the reference's left-to-right order; a lane
@@ -1461,7 +1776,7 @@ __global__ __launch_bounds__(64) void k_sample_walk(int W, int H, int k, int L, 
             const NodeGeo g0 = ld_geo(T, 0);
             cur.lox = g0.lox; cur.loy = g0.loy; cur.hix = g0.hix; cur.hiy = g0.hiy;
             cur.cx = g0.cx; cur.cy = g0.cy; cur.r2 = g0.r2; cur.deg = g0.deg;
-            cur.off = T.aux[0].off; cur.count = T.lnk[0].count; cur.id = 0; cur.pad = 0;
+            cur.off = T.aux[0].off; cur.count = T.lnk[0].count; cur.id = 0; cur.first = 0;
         }
         // a node's weight into its parent's entry (the root's: the total)
         // a completed node's weight into its parent's entry, for every lane: the
@@ -1546,71 +1861,457 @@ __global__ __launch_bounds__(64) void k_sample_walk(int W, int H, int k, int L, 
             if (done) break;
         }
         if (overflow) bad = true;
-    }
-    if (valid && runTree) {
         total = fmaxf(0.0f, total);
-        if (!bad && total >= prec) {
-            int pe[kMaxDepth];
-            float pp[kMaxDepth], pc[kMaxDepth];
-            for (int la = 0; la < L && !bad; la++) {
-                int e = 0, nd = 0, depth = 0;
-                uint64_t sideBits = 0;         // bit d: the step to depth d went right
-                pe[0] = 0;
-                NodeLnk lk = ld_lnk(T, nd);
-                while (lk.count > k) {
-                    // one round of loads: the node's link (issued at the end of the last
-                    // step) and the entry's weights, children and capacities
-                    float wl = tr.get(e, 1), wr = tr.get(e, 2);
-                    const int kids = tr.kids(e);
-                    const float cl = tr.get(e, 0), cr = tr.get(e, 4);
-                    if (wl != wl) {
-                        wl = tree_weight(T, lk.left, qx, qy);
-                        wr = tree_weight(T, lk.right, qx, qy);
-                        tr.set(e, 1, wl);
-                        tr.set(e, 2, wr);
-                    }
-                    wl = fmaxf(0.0f, wl); wr = fmaxf(0.0f, wr);
-                    float sum = wl + wr;
-                    wl = wl / sum; wr = wr / sum;
-                    int el = (kids & 0xffff) - 1, er = (kids >> 16) - 1;
-                    float sl = wl * cl, sr = wr * cr;
-                    bool goRight = sl < sr;
-                    int ce = goRight ? er : el;
-                    int cnode = goRight ? lk.right : lk.left;
-                    if (ce < 0) {
-                        if (nt >= TMAX) { bad = true; break; }
-                        ce = nt++;
-                        tr.init(ce, unset);
-                        tr.setKidHalf(e, goRight, ce + 1);
-                    }
-                    depth++;
-                    if (depth >= kMaxDepth) { bad = true; break; }
-                    pe[depth] = ce;
-                    pp[depth] = goRight ? wr : wl;
-                    pc[depth] = goRight ? cr : cl;     // its capacity, unchanged until the update below
-                    if (goRight) sideBits |= 1ull << depth;
-                    e = ce;
-                    nd = cnode;
-                    lk = ld_lnk(T, nd);
+        int drawn = 0;
+        if (valid && !bad && total >= prec)
+            drawn = capacity_descents(T, tr, nt, tcap, k, L, L0, qx, qy, rch, bad);
+        if (valid && bad) atomicOr(errOut, 1);
+        for (int la = drawn; la < L; la++) rch[(long)la * 64] = make_int2(0, 0);
+    }
+}
+
+// Sampler walk: one workgroup of four wavefronts per 8x8 pixel tile, one lane per
+// pixel for the weights and the descents.
+//
+// The union of the 64 pixels' FGT walks is traversed level by level, eight walked
+// nodes per wavefront and step: eight lanes take a node, four of them each of its
+// children (one 48 B SampChild load), and test the child against 16 pixels each, so a
+// step settles 64 children with one round of loads.  A child is evaluated (it carries
+// an expansion or is a leaf), walked (some pixel's walk goes below it) or dropped
+// (truncated for every pixel that reaches it: it adds nothing).  Both kinds go to LDS
+// lists.  The evaluated ones are shared out over the wavefronts (records and
+// coefficients fetched ahead); their values for the pixels that reach them are
+// stored as rows of 64 floats, 0 for the other pixels.  What the reference asks for
+// are sums of those rows in depth-first order: with every node's count of evaluated
+// nodes below its left and right child (bottom-up over the levels) and its first
+// place in that order (top-down), W of a child is the sum of a contiguous run of rows,
+// in order, from 0.  Walked nodes with more than k sources get a trie entry with
+// both children's weights, for the descents (k_sample_descend).
+//
+// The depth-first form of this pass (k_sample_walk_serial, still used where the
+// lists overflow) waits for a record or a coefficient block at nearly every one of
+// its steps, 250 of them per tile on average at 1M splats, 512x512 (555 in the densest
+// tile, which set the kernel's time), and its descents load every node of a path:
+// walk and descents 1912 us against 464 + 394 us (128x128, 4096 splats: 235 us against
+// 47 + 46 us).  Four wavefronts share a tile because a dense tile's own time ends the
+// kernel and a small image has fewer tiles than the chip has SIMDs (one wavefront per
+// tile, its descents in the same kernel: 1173 us and 118 us).
+constexpr int kWalkWaves = 4;
+constexpr int kWalkNodes = 448;      // walked nodes a tile's lists hold (277 in that densest tile)
+constexpr int kWalkRows = 448;       // evaluated nodes (220); the trie has rows for as many (walk_extra)
+constexpr int kWalkTake = 8;         // evaluated nodes a wavefront takes at a time
+
+// OR over the four lanes of a quad
+__device__ __forceinline__ uint32_t quad_or(uint32_t v)
+{
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false);   // lane ^ 1
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false);   // lane ^ 2
+    return v;
+}
+
+// a Hermite coefficient block on its way from memory to LDS (up to 289 floats)
+struct CoefFetch {
+    float c[5];
+    int np;
+    __device__ void load(const float UD_GLOBAL* p, int np_, int lane)
+    {
+        np = np_;
+        // every lane loads (the last element past the end), so no lane waits for a branch
+        c[0] = p[lane < np ? lane : np - 1];
+        c[1] = p[lane + 64 < np ? lane + 64 : np - 1];
+        if (np > 128) {
+#pragma unroll
+            for (int q = 2; q < 5; q++) c[q] = p[lane + 64 * q < np ? lane + 64 * q : np - 1];
+        }
+    }
+    __device__ void store(float* sc, int lane) const
+    {
+        if (lane < np) sc[lane] = c[0];
+        if (lane + 64 < np) sc[lane + 64] = c[1];
+        if (np > 128) {
+#pragma unroll
+            for (int q = 2; q < 5; q++)
+                if (lane + 64 * q < np) sc[lane + 64 * q] = c[q];
+        }
+    }
+};
+
+__global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H, int k, int L,
+                                                                 const ViewState* __restrict__ vs, const NodeGeo* geo,
+                                                                 const NodeLnk* lnk, const NodeAux* aux,
+                                                                 const float* coef, const SampRec* __restrict__ srec_,
+                                                                 float* trieWs, int tcap,
+                                                                 int* __restrict__ tileInfo,
+                                                                 int* __restrict__ walkQueue, VStride vsd)
+{
+    // walked nodes in level order: the pixels walking below it; its index; parent place
+    // | side << 9 | (trie entry + 1) << 10 | first place in depth-first order << 19; its
+    // evaluated nodes below the left | right << 16 child
+    __shared__ unsigned long long sMask[kWalkNodes];
+    __shared__ int sNode[kWalkNodes];
+    __shared__ uint32_t sLink[kWalkNodes];
+    __shared__ uint32_t sBelow[kWalkNodes];
+    __shared__ unsigned short sRowLink[kWalkRows];         // evaluated: parent place | side << 9
+    __shared__ unsigned short sRowAt[kWalkRows];           // row at each depth-first place
+    __shared__ uint32_t sInfo[kWalkEntries];               // trie entries: children, which hold rows (tile_descents)
+    __shared__ int sEntNode[kWalkEntries];                 // their tree nodes
+    __shared__ unsigned short sEntAt[kWalkEntries];        // their places among the walked nodes
+    __shared__ unsigned short sLevel[kMaxDepth + 1];       // first walked node of each level
+    __shared__ float sCoef[kWalkWaves][(kMaxDegree + 1) * (kMaxDegree + 1)];
+    __shared__ unsigned long long sCount;                  // walked | evaluated << 20 | entries << 40
+    __shared__ int sTicket;
+    vs = vw(vs, vsd.ws);
+    trieWs = vw(trieWs, vsd.ws);
+    const SampRec UD_GLOBAL* srec = (const SampRec UD_GLOBAL*)vw(srec_, vsd.ws);
+    TreeView T;
+    T.geo = (const NodeGeo UD_GLOBAL*)vw(geo, vsd.ws);
+    T.lnk = (const NodeLnk UD_GLOBAL*)vw(lnk, vsd.ws);
+    T.aux = (const NodeAux UD_GLOBAL*)vw(aux, vsd.ws);
+    T.coef = (const float UD_GLOBAL*)vw(coef, vsd.ws);
+    T.s2h = vs->s2h;
+    T.is2h = vs->is2h;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int entMax = tcap - walk_extra(L);              // entries the walk may create
+    TrieRef tr;
+    tr.base = (float UD_GLOBAL*)trieWs + (long)blockIdx.x * kTrieFields * tcap * 64 + lane;
+    float UD_GLOBAL* rows = tr.base + (long)kTrieFields * entMax * 64;     // entries only the descents create
+    const int tilesY = (H + 7) >> 3;
+    const uint32_t tile = xcd_chunk_remap<kSampTileRun>(blockIdx.x, gridDim.x);
+    const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
+    const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
+    const bool valid = (i < W) && (j < H);
+    if (vs->nc <= 0 || vs->err != 0) return;               // uniform over the launch
+    const float qx = (float)i, qy = (float)j;
+    const float unset = __builtin_nanf("");              // weight not computed yet
+    const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    bool bad = false;
+    float total = 0.0f;
+    // value of an expansion or leaf for the pixels of mask, the coefficients in f
+    auto eval = [&](const CoefFetch& f, int p, float cx, float cy, unsigned long long mask) {
+        f.store(sCoef[wv], lane);
+        wave_lds_fence();
+        float w = 0.0f;
+        if ((mask >> lane) & 1ull) w = hermite_at(sCoef[wv], p, (qx - cx) * T.is2h, (qy - cy) * T.is2h);
+        wave_lds_fence();
+        return w;
+    };
+    // ---- the root ----
+    const NodeGeo g0 = ld_geo(T, 0);
+    const unsigned long long wm0 = __ballot(valid && g0.deg < 0 && !truncated(g0, qx, qy));
+    if (threadIdx.x == 0) {
+        sMask[0] = wm0; sNode[0] = 0; sLink[0] = 1u << 10;
+        sInfo[0] = 0u; sEntNode[0] = 0; sEntAt[0] = 0;
+        sCount = (wm0 ? 1ull : 0ull) | (1ull << 40);
+        sTicket = 0;
+    }
+    __syncthreads();
+    int levels = 0, nodes = wm0 ? 1 : 0, evals = 0, nt = 1;
+    // ---- traversal ----
+    {
+        const int slot = lane >> 3, side = (lane >> 2) & 1, quad = lane & 3;
+        const float x0 = (float)(ti * 8), y0 = (float)(tj * 8 + 2 * quad);
+        int lo = 0, hi = nodes;                           // the level's walked nodes
+        while (lo < hi) {
+            if (levels >= kMaxDepth - 1) { bad = true; break; }       // a walk below the depth bound
+            if (threadIdx.x == 0) sLevel[levels] = (unsigned short)lo;
+            levels++;
+            for (int b0 = lo + 8 * wv; b0 < hi; b0 += 8 * kWalkWaves) {
+                const int at = b0 + slot;
+                const bool on = at < hi;
+                const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + (on ? sNode[at] : 0)) + 3 * side;
+                const f4v box = rec[0], mid = rec[1];
+                const i4v ref = *(const i4v UD_GLOBAL*)(rec + 2);
+                const unsigned long long act = on ? sMask[at] : 0ull;
+                const int parentEnt = on ? (int)((sLink[at] >> 10) & 511u) - 1 : -1;
+                const int deg = __float_as_int(mid.w);
+                // !truncated for the 8 x 2 pixels of this lane (same operations per pixel)
+                float dx2[8];
+#pragma unroll
+                for (int x = 0; x < 8; x++) {
+                    const float px = x0 + (float)x;
+                    const float dx = px - fminf(fmaxf(px, box.x), box.z);
+                    dx2[x] = dx * dx;
                 }
-                if (bad) break;
-                // capacities: an entry's lives in its parent's entry (field 4 if it is
-                // the right child, else 0); the path's were read on the way down
-                float prob = 1.0f;
-                for (int dd = depth; dd >= 1; dd--) {
-                    const int par = pe[dd - 1];
-                    const int fld = ((sideBits >> dd) & 1ull) ? 4 : 0;
-                    tr.set(par, fld, fmaxf(0.0f, pc[dd] - prob));
-                    prob = prob * pp[dd];
+                uint32_t in[2] = { 0u, 0u };
+#pragma unroll
+                for (int y = 0; y < 2; y++) {
+                    const float py = y0 + (float)y;
+                    const float dy = py - fminf(fmaxf(py, box.y), box.w);
+                    const float dy2 = dy * dy;
+#pragma unroll
+                    for (int x = 0; x < 8; x++) in[x >> 2] |= dx2[x] + dy2 < mid.z ? 1u << (8 * (x & 3) + y) : 0u;
                 }
-                // the reached subtree's leaves are the contiguous sorted range
-                // [first, first + count); k_sample_draw keys them
-                const int cnt = lk.count;
-                const int first = (nd >= L0) ? nd - L0 : T.aux[nd].first;
-                rch[(long)la * 64] = make_int2(first, cnt);
-                drawn = la + 1;
+                const uint32_t inLo = quad_or(in[0] << (2 * quad)), inHi = quad_or(in[1] << (2 * quad));
+                const unsigned long long walk = act & (((unsigned long long)inHi << 32) | inLo);
+                const bool lead = on && quad == 0;
+                const bool isEval = lead && deg >= 0;
+                const bool isWalk = lead && deg < 0 && walk != 0ull;
+                const bool wantEnt = isWalk && ref.y > k && parentEnt >= 0;
+                const unsigned long long bw = __ballot(isWalk), be = __ballot(isEval), bt = __ballot(wantEnt);
+                unsigned long long base = 0;
+                if (lane == 0)
+                    base = atomicAdd(&sCount, (unsigned long long)__popcll(bw) | ((unsigned long long)__popcll(be) << 20) |
+                                                  ((unsigned long long)__popcll(bt) << 40));
+                base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(base >> 32)) << 32) |
+                       (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                const int to = (int)(base & 0xfffffu) + __popcll(bw & lt);
+                const int row = (int)((base >> 20) & 0xfffffu) + __popcll(be & lt);
+                int ent = wantEnt ? (int)(base >> 40) + __popcll(bt & lt) : -1;
+                if (ent >= entMax) ent = -1;
+                if (isWalk && to < kWalkNodes) {
+                    sMask[to] = walk;
+                    sNode[to] = ref.z;
+                    sLink[to] = (uint32_t)at | ((uint32_t)side << 9) | ((uint32_t)(ent + 1) << 10);
+                    if (ent >= 0) {
+                        sInfo[ent] = 0u;
+                        sEntNode[ent] = ref.z;
+                        sEntAt[ent] = (unsigned short)to;
+                        atomicOr(&sInfo[parentEnt], (uint32_t)(ent + 1) << (10 * side));
+                    }
+                }
+                if (isEval && row < kWalkRows) sRowLink[row] = (unsigned short)(at | (side << 9));
+            }
+            __syncthreads();
+            const unsigned long long c = sCount;
+            nodes = (int)(c & 0xfffffu);
+            evals = (int)((c >> 20) & 0xfffffu);
+            nt = (int)(c >> 40);
+            if (nodes > kWalkNodes || evals > kWalkRows) {            // left to the serial form
+                if (threadIdx.x == 0) {
+                    int* q = vw(walkQueue, vsd.ws);
+                    q[1 + atomicAdd(q, 1)] = (int)blockIdx.x;
+                    vw(tileInfo, vsd.ws)[(long)blockIdx.x * kTileInfo] = -1;
+                }
+                return;
+            }
+            lo = hi;
+            hi = nodes;
+            __syncthreads();                               // sCount is read before the next level adds to it
+        }
+        if (nt > entMax) nt = entMax;
+    }
+    if (nodes > 0 && !bad) {
+        // ---- places (first wavefront) ----
+        if (wv == 0) {
+            if (lane == 0) sLevel[levels] = (unsigned short)nodes;
+            for (int x = lane; x < nodes; x += 64) sBelow[x] = 0u;
+            wave_lds_fence();
+            // evaluated nodes below each side, bottom-up
+            for (int e = lane; e < evals; e += 64) {
+                const uint32_t l = sRowLink[e];
+                atomicAdd(&sBelow[l & 511u], 1u << (16 * (l >> 9)));
+            }
+            wave_lds_fence();
+            for (int d = levels - 1; d > 0; d--) {
+                for (int x = sLevel[d] + lane; x < sLevel[d + 1]; x += 64) {
+                    const uint32_t l = sLink[x], c = sBelow[x];
+                    atomicAdd(&sBelow[l & 511u], ((c & 0xffffu) + (c >> 16)) << (16 * ((l >> 9) & 1u)));
+                }
+                wave_lds_fence();
+            }
+            // first places in depth-first order, top-down (the root's is 0)
+            for (int d = 1; d < levels; d++) {
+                for (int x = sLevel[d] + lane; x < sLevel[d + 1]; x += 64) {
+                    const uint32_t l = sLink[x], up = l & 511u;
+                    const uint32_t first = (sLink[up] >> 19) + (((l >> 9) & 1u) ? sBelow[up] & 0xffffu : 0u);
+                    sLink[x] = l | (first << 19);
+                }
+                wave_lds_fence();
+            }
+            for (int e = lane; e < evals; e += 64) {
+                const uint32_t l = sRowLink[e], up = l & 511u;
+                sRowAt[(sLink[up] >> 19) + ((l >> 9) ? sBelow[up] & 0xffffu : 0u)] = (unsigned short)e;
+            }
+            for (int t = lane; t < nt; t += 64) {
+                const uint32_t c = sBelow[sEntAt[t]];
+                sInfo[t] |= ((c & 0xffffu) ? 1u << 20 : 0u) | ((c >> 16) ? 1u << 21 : 0u);
             }
         }
+        // ---- values: kWalkTake nodes at a time, the next ones' records in flight ----
+        {
+            struct Take {
+                f4v mid;
+                int off, first, num;
+                unsigned long long mask;
+            };
+            auto take = [&]() {
+                Take t;
+                int b = 0;
+                if (lane == 0) b = atomicAdd(&sTicket, kWalkTake);
+                t.first = __builtin_amdgcn_readfirstlane(b);
+                t.num = evals - t.first < kWalkTake ? evals - t.first : kWalkTake;
+                const uint32_t l = lane < t.num ? sRowLink[t.first + lane] : 0u;
+                const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + sNode[l & 511u]) + 3 * (l >> 9);
+                t.mid = rec[1];
+                t.off = ((const i4v UD_GLOBAL*)(rec + 2))->x;
+                t.mask = sMask[l & 511u];
+                return t;
+            };
+            Take next = take();
+            while (next.num > 0) {                         // wave-uniform
+                const Take t = next;
+                next = take();
+                auto coefs = [&](int q, CoefFetch& f) {
+                    const int p = __builtin_amdgcn_readlane(__float_as_int(t.mid.w), q);
+                    f.load(T.coef + __builtin_amdgcn_readlane(t.off, q), (p + 1) * (p + 1), lane);
+                };
+                CoefFetch f;
+                coefs(0, f);
+                for (int q = 0; q < t.num; q++) {
+                    const CoefFetch cur = f;
+                    if (q + 1 < t.num) coefs(q + 1, f);
+                    const unsigned long long m =
+                        ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(t.mask >> 32), q) << 32) |
+                        (uint32_t)__builtin_amdgcn_readlane((int)t.mask, q);
+                    rows[(long)(t.first + q) * 64] =
+                        eval(cur, __builtin_amdgcn_readlane(__float_as_int(t.mid.w), q),
+                             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.mid.x), q)),
+                             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.mid.y), q)), m);
+                }
+            }
+        }
+        __syncthreads();
+        // ---- sums ----
+        // N sums of rows at once, num[q] of them from place at[q] on, each in order
+        auto sums = [&](auto count, const int* at, const int* num, float* out) {
+            constexpr int N = decltype(count)::value;
+            int m = 0;
+#pragma unroll
+            for (int q = 0; q < N; q++) m = num[q] > m ? num[q] : m;
+            for (int r = 0; r < m; r += 16 / N) {
+                float v[N][16 / N];
+#pragma unroll
+                for (int u = 0; u < 16 / N; u++)
+#pragma unroll
+                    for (int q = 0; q < N; q++)
+                        v[q][u] = r + u < num[q] ? rows[(long)sRowAt[at[q] + r + u] * 64] : 0.0f;
+#pragma unroll
+                for (int u = 0; u < 16 / N; u++)           // adding 0 past the end changes nothing
+#pragma unroll
+                    for (int q = 0; q < N; q++) out[q] = out[q] + v[q][u];
+            }
+        };
+        if (wv == 0) {
+            const int at0 = 0;
+            sums(std::integral_constant<int, 1>{}, &at0, &evals, &total);
+        } else {
+            // trie entries.  Where one child holds all rows, only pixels of weight <= 0
+            // there read the weights (tile_descents): 0 and 0 for a pixel that reached it
+            auto put = [&](int ent, bool mine, float wl, float wr) {
+                const uint32_t kids = sInfo[ent];
+                tr.set(ent, 0, 1.0f);
+                tr.set(ent, 1, mine ? wl : unset);
+                tr.set(ent, 2, mine ? wr : unset);
+                tr.setKids(ent, (int)((kids & 1023u) | (((kids >> 10) & 1023u) << 16)));
+                tr.set(ent, 4, 1.0f);
+            };
+            for (int c0 = 0; c0 < nt; c0 += 64 * (kWalkWaves - 1)) {
+                const int mine = c0 + lane * (kWalkWaves - 1) + wv - 1;       // this lane's entry
+                const bool has = mine < nt;
+                const bool both = has && (sInfo[has ? mine : 0] >> 20) == 3u;
+                unsigned long long plain = __ballot(has && !both), branch = __ballot(both);
+                auto entry = [&](int q) { return c0 + q * (kWalkWaves - 1) + wv - 1; };
+                while (plain) {
+                    const int ent = entry(__builtin_ctzll(plain));
+                    plain &= plain - 1;
+                    put(ent, (sMask[sEntAt[ent]] >> lane) & 1ull, 0.0f, 0.0f);
+                }
+                while (branch) {                                // two at a time: 16 row loads in flight
+                    int ent[2], at[4], num[4];
+                    float w[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+                    ent[0] = entry(__builtin_ctzll(branch));
+                    branch &= branch - 1;
+                    const bool two = branch != 0ull;
+                    ent[1] = two ? entry(__builtin_ctzll(branch)) : ent[0];
+                    branch &= branch - 1;
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        const int x = __builtin_amdgcn_readfirstlane((int)sEntAt[ent[q]]);
+                        const uint32_t below = __builtin_amdgcn_readfirstlane(sBelow[x]);
+                        at[2 * q] = (int)(__builtin_amdgcn_readfirstlane(sLink[x]) >> 19);
+                        num[2 * q] = q == 0 || two ? (int)(below & 0xffffu) : 0;
+                        at[2 * q + 1] = at[2 * q] + num[2 * q];
+                        num[2 * q + 1] = q == 0 || two ? (int)(below >> 16) : 0;
+                    }
+                    sums(std::integral_constant<int, 4>{}, at, num, w);
+                    put(ent[0], (sMask[sEntAt[ent[0]]] >> lane) & 1ull, w[0], w[1]);
+                    if (two) put(ent[1], (sMask[sEntAt[ent[1]]] >> lane) & 1ull, w[2], w[3]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // ---- for k_sample_descend: the pixels' totals, the entries of the trie ----
+    int* tileOut = vw(tileInfo, vsd.ws) + (long)blockIdx.x * kTileInfo;
+    const int tileEnts = nodes > 0 ? nt : 0;
+    for (int t = threadIdx.x; t < tileEnts; t += 64 * kWalkWaves) {
+        tileOut[128 + t] = (int)sInfo[t];
+        tileOut[128 + kWalkEntries + t] = sEntNode[t];
+    }
+    if (wv > 0) return;
+    if (nodes == 0) {
+        if (g0.deg >= 0) {
+            CoefFetch f;
+            f.load(T.coef + T.aux[0].off, (g0.deg + 1) * (g0.deg + 1), lane);
+            total = eval(f, g0.deg, g0.cx, g0.cy, __ballot(valid));
+        }
+        tr.init(0, unset);
+    }
+    if (lane == 0) { tileOut[0] = tileEnts; tileOut[1] = bad ? 1 : 0; }
+    tileOut[64 + lane] = __float_as_int(total);
+}
+
+// The capacity descents of every tile k_sample_walk finished, one lane per pixel.  A
+// pass of its own: a tile's descents take one wavefront where its walk takes four,
+// and as long as both together (the slowest tile, whose pixels weigh subtrees on
+// demand, sets this pass's time: all tiles are in flight at once at 512x512).
+__global__ __launch_bounds__(64, 4) void k_sample_descend(int W, int H, int k, int L, const ViewState* __restrict__ vs,
+                                                       const NodeGeo* geo, const NodeLnk* lnk, const NodeAux* aux,
+                                                       const float* coef, const SampRec* __restrict__ srec,
+                                                       float* trieWs, int tcap, const int* __restrict__ tileInfo,
+                                                       int2* __restrict__ reach, int* __restrict__ errOut,
+                                                       VStride vsd)
+{
+    __shared__ uint32_t sInfo[kWalkEntries];
+    __shared__ int sEntNode[kWalkEntries];
+    __shared__ int sPath[3 * kPathLds * 64];
+    vs = vw(vs, vsd.ws);
+    trieWs = vw(trieWs, vsd.ws);
+    reach = vw(reach, vsd.ws);
+    const int* tile_ = vw(tileInfo, vsd.ws) + (long)blockIdx.x * kTileInfo;
+    TreeView T;
+    T.geo = (const NodeGeo UD_GLOBAL*)vw(geo, vsd.ws);
+    T.lnk = (const NodeLnk UD_GLOBAL*)vw(lnk, vsd.ws);
+    T.aux = (const NodeAux UD_GLOBAL*)vw(aux, vsd.ws);
+    T.coef = (const float UD_GLOBAL*)vw(coef, vsd.ws);
+    T.s2h = vs->s2h;
+    T.is2h = vs->is2h;
+    const int lane = threadIdx.x;
+    const int n = vs->nc;
+    const bool runTree = n > 0 && vs->err == 0;
+    const int ents = runTree ? tile_[0] : 0;
+    if (ents < 0) return;                                // left to k_sample_walk_serial
+    for (int t = lane; t < ents; t += 64) {
+        sInfo[t] = (uint32_t)tile_[128 + t];
+        sEntNode[t] = tile_[128 + kWalkEntries + t];
+    }
+    wave_lds_fence();
+    TrieRef tr;
+    tr.base = (float UD_GLOBAL*)trieWs + (long)blockIdx.x * kTrieFields * tcap * 64 + lane;
+    const int tilesY = (H + 7) >> 3;
+    const uint32_t tile = xcd_chunk_remap<kSampTileRun>(blockIdx.x, gridDim.x);
+    const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
+    const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
+    const bool valid = (i < W) && (j < H);
+    int2* rch = reach + (long)blockIdx.x * L * 64 + lane;   // [launch][lane] of this tile
+    int drawn = 0;                                      // launches whose leaf range is recorded
+    if (valid && runTree) {
+        const float total = fmaxf(0.0f, __int_as_float(tile_[64 + lane]));
+        bool bad = tile_[1] != 0;
+        if (!bad && total >= vs->prec)
+            drawn = tile_descents(T, (const SampRec UD_GLOBAL*)vw(srec, vsd.ws), tr, ents, ents > 0 ? ents : 1, tcap, k, L,
+                                  n - 1, (float)i, (float)j, total, sInfo, sEntNode, sPath + lane, rch, bad);
         if (bad) atomicOr(errOut, 1);
     }
     for (int la = drawn; la < L; la++) rch[(long)la * 64] = make_int2(0, 0);
@@ -1641,13 +2342,6 @@ __device__ __forceinline__ bool draw_word(float qx, float qy, float2 xy, float i
     if (key == kNoKey) return false;
     ent = ((unsigned long long)key << 32) | (uint32_t)((la << 16) | ord);
     return true;
-}
-
-// orders the wavefront's LDS accesses (its LDS operations execute in order)
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // Sequential Poisson keys over the leaves each launch reached (the walk's
@@ -1688,8 +2382,16 @@ __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw(int W, int H, i
                                                                  const float2* __restrict__ leafXY,
                                                                  const int32_t* __restrict__ leafId,
                                                                  const int2* __restrict__ reach,
-                                                                 int32_t* __restrict__ out, int* __restrict__ tieQueue)
+                                                                 int32_t* __restrict__ out, int* __restrict__ tieQueue,
+                                                                 VStride vsd)
 {
+    vs = vw(vs, vsd.ws);
+    leafXY = vw(leafXY, vsd.ws);
+    leafId = vw(leafId, vsd.ws);
+    reach = vw(reach, vsd.ws);
+    tieQueue = vw(tieQueue, vsd.ws);
+    view += blockIdx.y;
+    out += (long)blockIdx.y * W * H * k;
     constexpr int CAP = 64 * ROWS;
     __shared__ __align__(16) uint32_t sKey[kDrawWaves][CAP];
     __shared__ int sPos[kDrawWaves][CAP];
@@ -1866,10 +2568,17 @@ __global__ __launch_bounds__(64) void k_sample_replay(int W, int H, int k, int L
                                                       const float2* __restrict__ leafXY,
                                                       const int32_t* __restrict__ leafId,
                                                       const int2* __restrict__ reach, const int* __restrict__ tieQueue,
-                                                      int32_t* __restrict__ out)
+                                                      int32_t* __restrict__ out, VStride vsd)
 {
+    tieQueue = vw(tieQueue, vsd.ws);
     const int lane = threadIdx.x;
     const int count = tieQueue[0];
+    vs = vw(vs, vsd.ws);
+    leafXY = vw(leafXY, vsd.ws);
+    leafId = vw(leafId, vsd.ws);
+    reach = vw(reach, vsd.ws);
+    view += blockIdx.y;
+    out += (long)blockIdx.y * W * H * k;
     const unsigned long long empty = ((unsigned long long)0x7f800000u << 32) | 0xffffffffull;
     const int R = (k + 63) >> 6;
     for (int e = blockIdx.x; e < count; e += gridDim.x) {
@@ -2960,8 +3669,8 @@ int num_launches(int k)
     return L;
 }
 
-// trie entries per lane: room for the walk plus 32 new entries per descent
-int trie_entries(int k) { return 384 + 32 * num_launches(k); }
+// trie entries per lane: room for the walk plus what the descents may add
+int trie_entries(int k) { return kWalkEntries + walk_extra(num_launches(k)); }
 
 // Optional timing of one sampling kernel (0 the walk + draw pair of
 // sampling.sample, 1 k_fmm_eval, 2 k_poisson): while enabled, its launches are
@@ -2990,28 +3699,36 @@ bool timing_pair(int kernel, hipEvent_t* a, hipEvent_t* b)
     return true;
 }
 
+// The sampler's per-pixel passes over `views` views (workspaces vsd.ws bytes apart).
 void launch_sample(int N, int W, int H, int k, uint32_t seedLo, uint32_t seedHi, uint32_t view, const TreeWs& w,
-                   int32_t* out, int* err, hipStream_t st)
+                   int32_t* out, int* err, hipStream_t st, int views, VStride vsd)
 {
-    k_samp_records<<<grid1(N, 256), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, w.srec);
-    unsigned tiles = (unsigned)(((W + 7) / 8) * ((H + 7) / 8));
+    k_samp_records<<<dim3(grid1(N, 256), views), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, w.srec, w.walkQueue,
+                                                               w.tieQueue, vsd);
+    const unsigned tiles = (unsigned)(((W + 7) / 8) * ((H + 7) / 8));
     const int L = num_launches(k);
     hipEvent_t e0, e1;
     bool timed = timing_pair(0, &e0, &e1);
     if (timed) (void)hipEventRecord(e0, st);
-    k_sample_walk<<<tiles, 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
-                                        trie_entries(k), w.reach, w.tieQueue, err);
-    const dim3 dg(tiles * (64 / kDrawWaves));
+    k_sample_walk<<<dim3(tiles, views), 64 * kWalkWaves, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec,
+                                                                  w.trie, trie_entries(k), w.tileInfo, w.walkQueue,
+                                                                  vsd);
+    k_sample_descend<<<dim3(tiles, views), 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
+                                                        trie_entries(k), w.tileInfo, w.reach, err, vsd);
+    k_sample_walk_serial<<<dim3(tiles < 64u ? tiles : 64u, views), 64, 0, st>>>(
+        W, H, k, L, (int)tiles, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie, trie_entries(k), w.reach,
+        w.walkQueue, err, vsd);
+    const dim3 dg(tiles * (64 / kDrawWaves), views);
     // a pixel has at most L ceil(k / 4) Philox blocks, 64 per iteration: 8 x 16, 12 x 32
     // and 16 x 64 at k = 64, 128 and 256
 #define UD_DRAW(R, I) k_sample_draw<R, I><<<dg, 64 * kDrawWaves, 0, st>>>(                                            \
-        W, H, k, L, (int)tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out, w.tieQueue)
+        W, H, k, L, (int)tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out, w.tieQueue, vsd)
     if (k <= 64) UD_DRAW(1, 2);
     else if (k <= 128) UD_DRAW(2, 6);
     else UD_DRAW(4, 16);
 #undef UD_DRAW
-    k_sample_replay<<<64, 64, 0, st>>>(W, H, k, L, tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach,
-                                       w.tieQueue, out);
+    k_sample_replay<<<dim3(64, views), 64, 0, st>>>(W, H, k, L, tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA,
+                                                    w.reach, w.tieQueue, out, vsd);
     if (timed) (void)hipEventRecord(e1, st);
 }
 
@@ -3106,7 +3823,7 @@ int ude_sample(int bn, int N, int W, int H, int k, double f, double smoothing, d
         if (rc == UDE_OK) rc = build_moments(N, k, w, st);
         if (rc != UDE_OK) return rc;
         int32_t* ob = out + perView * b;
-        launch_sample(N, W, H, k, sLo, sHi, (uint32_t)b, w, ob, errFlag, st);
+        launch_sample(N, W, H, k, sLo, sHi, (uint32_t)b, w, ob, errFlag, st, 1, VStride{});
         k_copy_err<<<1, 64, 0, st>>>(w.vs, errFlag);
     }
     hipError_t e = hipGetLastError();
