@@ -163,6 +163,15 @@ int ude_mlp_forward(int T, const float* X, const float* params, float* y, void* 
 int ude_mlp_loss_grad(int T, const float* X, const float* params, const float* target, const float* weight,
                       float* grad, float* loss, void* ws, size_t wsBytes, ude_stream_t stream);
 
+/* Rate multipliers of T tiles: y = network((feats - mean) / std) (non-finite: 0, 20,
+ * -20), less its count-weighted mean, s = exp(y) with y kept in [-20, 20], then three
+ * times s = clamp(s sum(counts) / sum(s counts), lo, hi); FP64 after the network.
+ * feats (T, 32), mean / std (32), counts (T) doubles, out (T) floats. */
+size_t ude_rate_scale_workspace_bytes(int T);
+int ude_rate_scale(int T, const float* feats, const float* mean, const float* std, const float* params,
+                   const double* counts, double lo, double hi, float* out, void* ws, size_t wsBytes,
+                   ude_stream_t stream);
+
 /* One Adam step (bias-corrected, step >= 1) on n FP32 parameters. */
 int ude_adam_step(int n, float* params, const float* grad, float* m, float* v, float lr, float beta1, float beta2,
                   float eps, int step, ude_stream_t stream);

@@ -64,3 +64,46 @@ def test_training_fits_a_known_network(dev):
     net = RateNet.init(dev, seed=1)
     hist = net.fit(t(X, dev), t(y, dev), steps=1500, lr=3e-3, log_every=500)
     assert hist[-1][1] < 0.05 * hist[0][1], hist
+
+
+@pytest.mark.parametrize("T,weighted", [(16, True), (64, False), (65, True), (8193, False), (20011, True)])
+def test_mlp_grad_over_row_blocks(dev, T, weighted):
+    """16 rows per wavefront, 64 per workgroup, 8,192 per pass of the grid: both sides
+    of each, against the FP64 oracle with the same rounding points (bounds as above:
+    occasional one-ulp bfloat16 flips of hidden units)."""
+    from splatting_amd.learned import RateNet
+    rng = np.random.default_rng(T)
+    X = rng.normal(size=(T, M.N_IN)).astype(np.float32)
+    P = (rng.normal(size=M.N_PARAMS) * 0.2).astype(np.float32)
+    tgt = rng.normal(size=T).astype(np.float32)
+    w = rng.uniform(0.5, 2.0, size=T).astype(np.float32) if weighted else None
+    net = RateNet(t(P, dev), t(np.zeros(M.N_IN), dev), t(np.ones(M.N_IN), dev))
+    loss, g = net.loss_grad(t(X, dev), t(tgt, dev), None if w is None else t(w, dev))
+    lr, gr = M.loss_grad(X, P, tgt, w, quant=True)
+    assert abs(float(loss.item()) - lr) <= 1e-2 * lr
+    assert rel(g.cpu().numpy(), gr) < 2e-2
+    assert rel(net.forward(t(X, dev)).cpu().numpy(), M.forward(X, P, quant=True)[0]) < 5e-3
+
+
+@pytest.mark.parametrize("shape", [(1,), (2, 5, 7), (1, 1500)])
+def test_tile_scale_formula(dev, shape):
+    """RateNet.tile_scale equals its formula in float64 on the network's own
+    predictions (non-finite ones included) to float32 rounding."""
+    from splatting_amd.learned import RateNet
+    rng = np.random.default_rng(len(shape))
+    T = int(np.prod(shape))
+    F = t(rng.normal(size=shape + (M.N_IN,)), dev)
+    if T > 1:
+        F.view(-1, M.N_IN)[1, 3] = float("nan")
+    c = t(rng.uniform(0.0, 3000.0, size=shape), dev)
+    net = RateNet(t(rng.normal(size=M.N_PARAMS) * 0.3, dev), t(rng.normal(size=M.N_IN), dev),
+                  t(rng.uniform(0.5, 2.0, size=M.N_IN), dev))
+    y = torch.nan_to_num(net.forward(F.reshape(-1, M.N_IN)).double(), nan=0.0, posinf=20.0, neginf=-20.0)
+    cd = c.reshape(-1).double()
+    tot = cd.sum().clamp(min=1e-30)
+    s = torch.exp((y - (y * cd).sum() / tot).clamp(-20.0, 20.0))
+    for _ in range(3):
+        s = (s * (tot / (s * cd).sum().clamp(min=1e-30))).clamp(0.75, 4.0)
+    got = net.tile_scale(F, c)
+    assert got.shape == c.shape
+    assert rel(got.reshape(-1).cpu().numpy(), s.cpu().numpy()) < 2.0 ** -23

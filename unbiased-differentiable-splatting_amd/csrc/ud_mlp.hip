@@ -7,6 +7,14 @@
 // loss and the optimiser run in FP32.  Forward, backward and Adam are all
 // kernels here, so the network trains on the GPU with no library GEMM.
 //
+// A wavefront takes 16 rows (tiles) through the whole network: the weights sit in
+// LDS as bfloat16, the activations pass from one layer's accumulator layout to the
+// next one's operand layout through 2 KB of LDS, and the weight gradients of all its
+// rows accumulate in registers (the accumulator layout of H1 and dZ2 is the operand
+// layout of H1^T dZ2).  One kernel per layer and direction took 15 launches per
+// training evaluation, and its weight-gradient products walked all T rows in one
+// wavefront per 16x16 weights: 1310 us at T = 20480 (now 48 us).
+//
 // Parameter block (FP32, 6337 floats): W1 [32][64], b1 [64], W2 [64][64],
 // b2 [64], W3 [64], b3 [1] (row-major, input index first).
 #include "ud_device.h"
@@ -34,138 +42,331 @@ __device__ __forceinline__ uint16_t f2bf(float x)
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
-__global__ void k_to_bf16(long n, const float* __restrict__ src, uint16_t* __restrict__ dst)
+__device__ __forceinline__ float bfr(float x) { return bf2f(f2bf(x)); }
+
+constexpr int kWaves = 4;                    // wavefronts per workgroup
+constexpr int kPad1 = kIn + 4, kPad2 = kHid + 4;      // LDS row strides (8-byte fragments, spread over the banks)
+constexpr int kTrainBlocks = 128;            // workgroups of the training pass (partial gradients)
+constexpr int kPartial = kParams + 1;        // gradient and loss
+
+struct Weights {
+    uint16_t w1t[kHid * kPad1];              // W1 transposed: [out][in]
+    uint16_t w2t[kHid * kPad2];              // W2 transposed: [out][in]
+    uint16_t w2[kHid * kPad2];               // W2: [in][out]
+    float b1[kHid], b2[kHid], w3[kHid], b3;  // w3 rounded to bfloat16
+};
+
+__device__ __forceinline__ void load_weights(const float* __restrict__ P, Weights& w, bool back)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[t] = f2bf(src[t]);
+    for (int e = threadIdx.x; e < kIn * kHid; e += blockDim.x)
+        w.w1t[(e % kHid) * kPad1 + e / kHid] = f2bf(P[kOffW1 + e]);
+    for (int e = threadIdx.x; e < kHid * kHid; e += blockDim.x) {
+        const uint16_t x = f2bf(P[kOffW2 + e]);
+        w.w2t[(e % kHid) * kPad2 + e / kHid] = x;
+        if (back) w.w2[(e / kHid) * kPad2 + e % kHid] = x;
+    }
+    if (threadIdx.x < kHid) {
+        w.b1[threadIdx.x] = P[kOffB1 + threadIdx.x];
+        w.b2[threadIdx.x] = P[kOffB2 + threadIdx.x];
+        w.w3[threadIdx.x] = bfr(P[kOffW3 + threadIdx.x]);
+    }
+    if (threadIdx.x == 0) w.b3 = P[kOffB3];
 }
 
-// C (M x N) = A (M x K) * B (K x N) on the matrix cores: one wavefront per
-// 16 x 16 output tile, K in steps of 16.  A(i, k) = A[i * sai + k * sak],
-// B(k, j) = B[k * sbk + j * sbj] (bf16), so transposed operands are strides.
-// Lane l holds A(i0 + l % 16, k0 + 4 (l / 16) + v), B(k0 + 4 (l / 16) + v,
-// j0 + l % 16) and gets D(i0 + 4 (l / 16) + v, j0 + l % 16), v = 0..3.
-// Epilogue: + bias[j] (optional), ReLU (optional), FP32 and/or bf16 store.
-__global__ __launch_bounds__(64) void k_gemm_bf16(int M, int N, int K, const uint16_t* __restrict__ A, long sai,
-                                                  long sak, const uint16_t* __restrict__ B, long sbk, long sbj,
-                                                  const float* __restrict__ bias, int relu, float* __restrict__ C,
-                                                  uint16_t* __restrict__ Cb, long ldc)
+__device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c)
 {
-    const int lane = threadIdx.x;
-    const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
-    const int r = lane & 15, g = lane >> 4;
-    const int ia = i0 + r, jb = j0 + r;
-    f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        bf16x4 a, b;
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+
+// four consecutive bfloat16 of an LDS row (8-byte aligned)
+__device__ __forceinline__ bf16x4 frag(const uint16_t* p) { return *(const bf16x4*)p; }
+
+__device__ __forceinline__ void lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// an accumulator tile set (rows 4g + v, columns 16c + r) as operand rows (row r,
+// columns 16s + 4g ...), through the wavefront's 16 x kPad2 LDS buffer
+__device__ __forceinline__ void to_rows(uint16_t* buf, const bf16x4 (&x)[4], bf16x4 (&out)[4], int r, int g)
+{
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) buf[(4 * g + v) * kPad2 + 16 * c + r] = (uint16_t)x[c][v];
+    lds_fence();
+#pragma unroll
+    for (int s = 0; s < 4; s++) out[s] = frag(buf + r * kPad2 + 16 * s + 4 * g);
+    lds_fence();
+}
+
+// H1, H2 (bfloat16, accumulator layout) and y (rows 4g + v, in every lane of a row
+// group) of the 16 rows from t0 on; feature k is (X[k] - mean[k]) / std[k], or X[k]
+__device__ __forceinline__ void forward16(int T, const float* __restrict__ X, const float* __restrict__ mean,
+                                          const float* __restrict__ std, long t0, const Weights& w, uint16_t* buf,
+                                          int r, int g, bf16x4 (&h1)[4], bf16x4 (&h2)[4], float (&y)[4])
+{
+    const long row = t0 + r;
+    bf16x4 a[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++)
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            int k = k0 + 4 * g + v;
-            a[v] = (ia < M && k < K) ? (short)A[(long)ia * sai + (long)k * sak] : (short)0;
-            b[v] = (jb < N && k < K) ? (short)B[(long)k * sbk + (long)jb * sbj] : (short)0;
+            const int k = 16 * s + 4 * g + v;
+            float x = row < T ? X[row * kIn + k] : 0.0f;
+            if (mean) x = (x - mean[k]) / std[k];
+            a[s][v] = (short)f2bf(x);
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int s = 0; s < 2; s++) z = mfma(a[s], frag(w.w1t + (16 * c + r) * kPad1 + 16 * s + 4 * g), z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) h1[c][v] = (short)f2bf(fmaxf(z[v] + w.b1[16 * c + r], 0.0f));
+    }
+    bf16x4 rows[4];
+    to_rows(buf, h1, rows, r, g);
+#pragma unroll
+    for (int v = 0; v < 4; v++) y[v] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int s = 0; s < 4; s++) z = mfma(rows[s], frag(w.w2t + (16 * c + r) * kPad2 + 16 * s + 4 * g), z);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const uint16_t h = f2bf(fmaxf(z[v] + w.b2[16 * c + r], 0.0f));
+            h2[c][v] = (short)h;
+            y[v] += bf2f(h) * w.w3[16 * c + r];
+        }
     }
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-        int i = i0 + 4 * g + v, j = j0 + r;
-        if (i >= M || j >= N) continue;
-        float x = acc[v];
-        if (bias) x = x + bias[j];
-        if (relu) x = fmaxf(x, 0.0f);
-        if (C) C[(long)i * ldc + j] = x;
-        if (Cb) Cb[(long)i * ldc + j] = f2bf(x);
+        for (int o = 1; o < 16; o <<= 1) y[v] += __shfl_xor(y[v], o, 64);
+        y[v] += w.b3;
     }
 }
 
-// output layer: y[t] = sum_k H2[t][k] W3[k] (bf16 products, FP32 sum in k order) + b3
-__global__ __launch_bounds__(256) void k_out_layer(int T, const uint16_t* __restrict__ H2b,
-                                                   const uint16_t* __restrict__ W3b, const float* __restrict__ b3,
-                                                   float* __restrict__ y)
+__global__ __launch_bounds__(64 * kWaves) void k_mlp_forward(int T, const float* __restrict__ X,
+                                                             const float* __restrict__ mean,
+                                                             const float* __restrict__ std,
+                                                             const float* __restrict__ P, float* __restrict__ y)
 {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    float s = 0.0f;
-    for (int k = 0; k < kHid; k++) s = s + bf2f(H2b[(long)t * kHid + k]) * bf2f(W3b[k]);
-    y[t] = s + b3[0];
-}
-
-// weighted mean-square loss and its gradient dy = 2 w (y - target) / sum(w);
-// one workgroup, fixed-order tree reduction (deterministic)
-__global__ __launch_bounds__(1024) void k_loss(int T, const float* __restrict__ y, const float* __restrict__ target,
-                                               const float* __restrict__ weight, float* __restrict__ dy,
-                                               float* __restrict__ lossOut)
-{
-    __shared__ float sw[1024], sl[1024];
-    float w = 0.0f, l = 0.0f;
-    for (int t = threadIdx.x; t < T; t += 1024) {
-        float wt = weight ? weight[t] : 1.0f;
-        float e = y[t] - target[t];
-        w = w + wt;
-        l = l + wt * (e * e);
-    }
-    sw[threadIdx.x] = w;
-    sl[threadIdx.x] = l;
+    __shared__ __align__(16) Weights w;
+    __shared__ __align__(16) uint16_t buf[kWaves][16 * kPad2];
+    load_weights(P, w, false);
     __syncthreads();
-    for (int s = 512; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            sw[threadIdx.x] = sw[threadIdx.x] + sw[threadIdx.x + s];
-            sl[threadIdx.x] = sl[threadIdx.x] + sl[threadIdx.x + s];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    for (long t0 = ((long)blockIdx.x * kWaves + wv) * 16; t0 < T; t0 += (long)gridDim.x * kWaves * 16) {
+        bf16x4 h1[4], h2[4];
+        float o[4];
+        forward16(T, X, mean, std, t0, w, buf[wv], r, g, h1, h2, o);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (r == v && t0 + 4 * g + v < T) y[t0 + 4 * g + v] = o[v];
+    }
+}
+
+// sum of the loss weights (T without weights), fixed order; its inverse, 0 for no weight
+__global__ __launch_bounds__(1024) void k_weight_sum(int T, const float* __restrict__ weight, float* __restrict__ inv)
+{
+    __shared__ float sw[16];
+    float s = 0.0f;
+    for (int t = threadIdx.x; t < T; t += 1024) s = s + (weight ? weight[t] : 1.0f);
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float W = sw[0];
+        for (int q = 1; q < 16; q++) W = W + sw[q];
+        inv[0] = W > 0.0f ? 1.0f / W : 0.0f;
+    }
+}
+
+// Forward and backward of the weighted mean-square loss, dy = 2 w (y - target) / sum(w):
+// the gradient and loss of this workgroup's rows to part[blockIdx.x].
+__global__ __launch_bounds__(64 * kWaves) void k_mlp_train(int T, const float* __restrict__ X,
+                                                           const float* __restrict__ P,
+                                                           const float* __restrict__ target,
+                                                           const float* __restrict__ weight,
+                                                           const float* __restrict__ inv, float* __restrict__ part)
+{
+    // the weights, then (after the last row) the workgroup's gradient
+    __shared__ __align__(16) union { Weights w; float sum[kPartial]; } u;
+    __shared__ __align__(16) uint16_t buf[kWaves][16 * kPad2];
+    load_weights(P, u.w, true);
+    __syncthreads();
+    const Weights& w = u.w;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const float iw = inv[0];
+    f32x4 gW1[2][4], gW2[4][4];
+    float gb1[4], gb2[4], gw3[4], gb3 = 0.0f, loss = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        gb1[c] = gb2[c] = gw3[c] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) gW2[q][c] = f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int q = 0; q < 2; q++) gW1[q][c] = f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+    }
+    for (long t0 = ((long)blockIdx.x * kWaves + wv) * 16; t0 < T; t0 += (long)gridDim.x * kWaves * 16) {
+        bf16x4 h1[4], h2[4], z[4], rows[4];
+        float y[4], dy[4];
+        forward16(T, X, nullptr, nullptr, t0, w, buf[wv], r, g, h1, h2, y);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const long t = t0 + 4 * g + v;
+            const float wt = t < T ? (weight ? weight[t] : 1.0f) : 0.0f;
+            const float e = t < T ? y[v] - target[t] : 0.0f;
+            dy[v] = (2.0f * wt) * e * iw;
+            if (r == 0) { loss += wt * (e * e); gb3 += dy[v]; }
+        }
+        // dZ2 = dy W3^T where H2 > 0
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float h = bf2f((uint16_t)h2[c][v]);
+                const float x = h > 0.0f ? dy[v] * w.w3[16 * c + r] : 0.0f;
+                gw3[c] += dy[v] * h;
+                gb2[c] += x;
+                z[c][v] = (short)f2bf(x);
+            }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) gW2[q][c] = mfma(h1[q], z[c], gW2[q][c]);
+        // dZ1 = dZ2 W2^T where H1 > 0
+        to_rows(buf[wv], z, rows, r, g);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            f32x4 d = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+            for (int s = 0; s < 4; s++) d = mfma(rows[s], frag(w.w2 + (16 * c + r) * kPad2 + 16 * s + 4 * g), d);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float x = bf2f((uint16_t)h1[c][v]) > 0.0f ? d[v] : 0.0f;
+                gb1[c] += x;
+                z[c][v] = (short)f2bf(x);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            bf16x4 xt;                                   // X^T: row 16 q + r of the features, rows 4g + v
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const long t = t0 + 4 * g + v;
+                xt[v] = (short)f2bf(t < T ? X[t * kIn + 16 * q + r] : 0.0f);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++) gW1[q][c] = mfma(xt, z[c], gW1[q][c]);
+        }
+    }
+    // column sums over the row groups (lanes of equal r), the loss over all lanes
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        for (int o = 16; o < 64; o <<= 1) {
+            gb1[c] += __shfl_xor(gb1[c], o, 64);
+            gb2[c] += __shfl_xor(gb2[c], o, 64);
+            gw3[c] += __shfl_xor(gw3[c], o, 64);
+        }
+    gb3 = wave_sum(gb3);
+    loss = wave_sum(loss);
+    __syncthreads();                                     // the weights are no longer read
+    for (int q = 0; q < kWaves; q++) {                   // the wavefronts' sums, in order
+        if (wv == q) {
+            auto add = [&](int at, float x) { u.sum[at] = q ? u.sum[at] + x : x; };
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+#pragma unroll
+                    for (int i = 0; i < 2; i++) add(kOffW1 + (16 * i + 4 * g + v) * kHid + 16 * c + r, gW1[i][c][v]);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) add(kOffW2 + (16 * i + 4 * g + v) * kHid + 16 * c + r, gW2[i][c][v]);
+                }
+                if (g == 0) {
+                    add(kOffB1 + 16 * c + r, gb1[c]);
+                    add(kOffB2 + 16 * c + r, gb2[c]);
+                    add(kOffW3 + 16 * c + r, gw3[c]);
+                }
+            }
+            if (lane == 0) { add(kOffB3, gb3); add(kParams, loss); }
         }
         __syncthreads();
     }
-    const float W = sw[0];
-    const float inv = W > 0.0f ? 1.0f / W : 0.0f;
-    if (threadIdx.x == 0 && lossOut) lossOut[0] = sl[0] * inv;
-    for (int t = threadIdx.x; t < T; t += 1024) {
-        float wt = weight ? weight[t] : 1.0f;
-        dy[t] = (2.0f * wt) * (y[t] - target[t]) * inv;
-    }
+    for (int e = threadIdx.x; e < kPartial; e += blockDim.x) part[(long)blockIdx.x * kPartial + e] = u.sum[e];
 }
 
-// dZ2[t][k] = dy[t] W3[k] where H2[t][k] > 0 (ReLU), FP32 and bf16
-__global__ __launch_bounds__(256) void k_back_out(int T, const float* __restrict__ dy, const uint16_t* __restrict__ H2b,
-                                                  const uint16_t* __restrict__ W3b, float* __restrict__ dZ,
-                                                  uint16_t* __restrict__ dZb)
+// grad = the workgroups' partial gradients added in order, loss = their losses / sum(w)
+__global__ __launch_bounds__(256) void k_mlp_reduce(int blocks, const float* __restrict__ part,
+                                                    const float* __restrict__ inv, float* __restrict__ grad,
+                                                    float* __restrict__ loss)
 {
-    long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long)T * kHid) return;
-    int k = (int)(e % kHid);
-    float x = bf2f(H2b[e]) > 0.0f ? dy[e / kHid] * bf2f(W3b[k]) : 0.0f;
-    dZ[e] = x;
-    dZb[e] = f2bf(x);
-}
-
-// apply the ReLU mask of H (bf16) to dH in place; bf16 copy
-__global__ __launch_bounds__(256) void k_relu_back(long n, const uint16_t* __restrict__ Hb, float* __restrict__ dH,
-                                                   uint16_t* __restrict__ dHb)
-{
-    long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    float x = bf2f(Hb[e]) > 0.0f ? dH[e] : 0.0f;
-    dH[e] = x;
-    dHb[e] = f2bf(x);
-}
-
-// out[c] = sum_t M[t][c] (or, with V, sum_t M[t] V[t][c]) in fixed order: one
-// workgroup per column, strided partial sums then a tree
-__global__ __launch_bounds__(256) void k_colsum(int T, int C, const float* __restrict__ Mx, const uint16_t* __restrict__ Vb,
-                                                float* __restrict__ out)
-{
-    __shared__ float sh[256];
-    const int c = blockIdx.x;
+    __shared__ float sh[4][64];
+    const int e = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
     float s = 0.0f;
-    for (int t = threadIdx.x; t < T; t += 256) {
-        float x = Vb ? Mx[t] * bf2f(Vb[(long)t * C + c]) : Mx[(long)t * C + c];
-        s = s + x;
+    if (e < kPartial) {
+#pragma unroll 8
+        for (int b = q; b < blocks; b += 4) s += part[(long)b * kPartial + e];
     }
-    sh[threadIdx.x] = s;
+    sh[q][threadIdx.x & 63] = s;
     __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (threadIdx.x < st) sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + st];
-        __syncthreads();
+    if (q == 0 && e < kPartial) {
+        s = ((sh[0][threadIdx.x] + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
+        if (e < kParams) grad[e] = s;
+        else if (loss) loss[0] = s * inv[0];
     }
-    if (threadIdx.x == 0) out[c] = sh[0];
+}
+
+// Rate multipliers from the predictions (ude_rate_scale), one workgroup: about 30
+// elementwise and reduction kernels of a tensor library otherwise (8 us here at 1024
+// tiles, about 100 us of launches there).
+__device__ __forceinline__ double block_sum(double x, double* sh)
+{
+    x = wave_sum_d(x);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
+    __syncthreads();
+    double s = sh[0];
+    for (int q = 1; q < 16; q++) s += sh[q];
+    __syncthreads();
+    return s;
+}
+
+// a NaN stays a NaN
+__device__ __forceinline__ double clamp_d(double x, double lo, double hi)
+{
+    x = x < lo ? lo : x;
+    return x > hi ? hi : x;
+}
+
+__global__ __launch_bounds__(1024) void k_rate_scale(int T, const float* __restrict__ y, const double* __restrict__ count,
+                                                     double lo, double hi, double* __restrict__ s,
+                                                     float* __restrict__ out)
+{
+    __shared__ double sh[16];
+    const double inf = __builtin_huge_val();
+    auto at = [&](int t) {
+        const double v = (double)y[t];
+        return v != v ? 0.0 : v == inf ? 20.0 : v == -inf ? -20.0 : v;
+    };
+    double c = 0.0, yc = 0.0;
+    for (int t = threadIdx.x; t < T; t += 1024) c += count[t];
+    const double sum = block_sum(c, sh);
+    const double tot = sum < 1e-30 ? 1e-30 : sum;
+    for (int t = threadIdx.x; t < T; t += 1024) yc += at(t) * count[t];
+    const double mean = block_sum(yc, sh) / tot;
+    for (int t = threadIdx.x; t < T; t += 1024) s[t] = exp(clamp_d(at(t) - mean, -20.0, 20.0));
+    for (int it = 0; it < 3; it++) {
+        double a = 0.0;
+        for (int t = threadIdx.x; t < T; t += 1024) a += s[t] * count[t];
+        const double b = block_sum(a, sh);
+        const double f = tot / (b < 1e-30 ? 1e-30 : b);
+        for (int t = threadIdx.x; t < T; t += 1024) s[t] = clamp_d(s[t] * f, lo, hi);
+    }
+    for (int t = threadIdx.x; t < T; t += 1024) out[t] = (float)s[t];
 }
 
 // Adam (Kingma & Ba 2015) with bias correction, FP32 master parameters
@@ -183,47 +384,20 @@ __global__ __launch_bounds__(256) void k_adam(int n, float* __restrict__ p, cons
     p[t] = p[t] - lr * (mt / c1) / (sqrtf(vt / c2) + eps);
 }
 
-struct MlpWs {
-    uint16_t *Xb, *Pb, *H1b, *H2b, *dZ2b, *dZ1b;
-    float *y, *dy, *dZ2, *dZ1;
-};
-
 inline size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-size_t mlp_carve(void* ws, int T, MlpWs* w)
-{
-    size_t off = 0;
-    char* base = (char*)ws;
-    auto take = [&](size_t bytes) { size_t o = off; off = a256(off + bytes); return base ? (void*)(base + o) : nullptr; };
-    MlpWs m;
-    long t = T > 0 ? T : 1;
-    m.Xb = (uint16_t*)take(2 * t * kIn);
-    m.Pb = (uint16_t*)take(2 * kParams);
-    m.H1b = (uint16_t*)take(2 * t * kHid);
-    m.H2b = (uint16_t*)take(2 * t * kHid);
-    m.dZ2b = (uint16_t*)take(2 * t * kHid);
-    m.dZ1b = (uint16_t*)take(2 * t * kHid);
-    m.y = (float*)take(4 * t);
-    m.dy = (float*)take(4 * t);
-    m.dZ2 = (float*)take(4 * t * kHid);
-    m.dZ1 = (float*)take(4 * t * kHid);
-    if (w) *w = m;
-    return off;
-}
-
 inline unsigned g256(long n) { return (unsigned)((n + 255) / 256); }
 
-void mlp_forward(int T, const float* X, const float* P, const MlpWs& w, float* y, hipStream_t st)
+// workgroups for T rows, 16 per wavefront and pass
+inline unsigned row_blocks(int T, unsigned most)
 {
-    k_to_bf16<<<g256((long)T * kIn), 256, 0, st>>>((long)T * kIn, X, w.Xb);
-    k_to_bf16<<<g256(kParams), 256, 0, st>>>(kParams, P, w.Pb);
-    dim3 grid(kHid / 16, (T + 15) / 16);
-    // H1 = relu(X W1 + b1), H2 = relu(H1 W2 + b2)
-    k_gemm_bf16<<<grid, 64, 0, st>>>(T, kHid, kIn, w.Xb, kIn, 1, w.Pb + kOffW1, kHid, 1, P + kOffB1, 1, nullptr,
-                                     w.H1b, kHid);
-    k_gemm_bf16<<<grid, 64, 0, st>>>(T, kHid, kHid, w.H1b, kHid, 1, w.Pb + kOffW2, kHid, 1, P + kOffB2, 1, nullptr,
-                                     w.H2b, kHid);
-    k_out_layer<<<g256(T), 256, 0, st>>>(T, w.H2b, w.Pb + kOffW3, P + kOffB3, y);
+    const unsigned b = (unsigned)((T + 16 * kWaves - 1) / (16 * kWaves));
+    return b < most ? b : most;
+}
+
+inline int launch_status()
+{
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
 }
 
 } // namespace
@@ -232,17 +406,18 @@ extern "C" {
 
 int ude_mlp_param_count(void) { return kParams; }
 
-size_t ude_mlp_workspace_bytes(int T) { return mlp_carve(nullptr, T, nullptr) + 256; }
+// training: the inverse weight sum, the partial gradients
+size_t ude_mlp_workspace_bytes(int T)
+{
+    return 256 + a256(sizeof(float) * (size_t)kPartial * row_blocks(T > 0 ? T : 1, kTrainBlocks)) + 256;
+}
 
 int ude_mlp_forward(int T, const float* X, const float* params, float* y, void* ws, size_t wsBytes, hipStream_t st)
 {
     if (T <= 0) return UDE_OK;
     if (wsBytes < ude_mlp_workspace_bytes(T)) return UDE_ERR_WORKSPACE;
-    MlpWs w;
-    mlp_carve(ws, T, &w);
-    mlp_forward(T, X, params, w, y, st);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
+    k_mlp_forward<<<row_blocks(T, 1024), 64 * kWaves, 0, st>>>(T, X, nullptr, nullptr, params, y);
+    return launch_status();
 }
 
 int ude_mlp_loss_grad(int T, const float* X, const float* params, const float* target, const float* weight,
@@ -250,30 +425,28 @@ int ude_mlp_loss_grad(int T, const float* X, const float* params, const float* t
 {
     if (T <= 0) return UDE_ERR_ARG;
     if (wsBytes < ude_mlp_workspace_bytes(T)) return UDE_ERR_WORKSPACE;
-    MlpWs w;
-    mlp_carve(ws, T, &w);
-    mlp_forward(T, X, params, w, w.y, st);
-    k_loss<<<1, 1024, 0, st>>>(T, w.y, target, weight, w.dy, loss);
-    // output layer: dW3 = H2^T dy, db3 = sum dy, dZ2 = dy W3^T masked by ReLU
-    k_colsum<<<kHid, 256, 0, st>>>(T, kHid, w.dy, w.H2b, grad + kOffW3);
-    k_colsum<<<1, 256, 0, st>>>(T, 1, w.dy, nullptr, grad + kOffB3);
-    k_back_out<<<g256((long)T * kHid), 256, 0, st>>>(T, w.dy, w.H2b, w.Pb + kOffW3, w.dZ2, w.dZ2b);
-    // layer 2: dW2 = H1^T dZ2 (64 x T x 64), db2 = colsum dZ2, dH1 = dZ2 W2^T
-    dim3 gw(kHid / 16, kHid / 16);
-    k_gemm_bf16<<<gw, 64, 0, st>>>(kHid, kHid, T, w.H1b, 1, kHid, w.dZ2b, kHid, 1, nullptr, 0, grad + kOffW2, nullptr,
-                                   kHid);
-    k_colsum<<<kHid, 256, 0, st>>>(T, kHid, w.dZ2, nullptr, grad + kOffB2);
-    dim3 gh(kHid / 16, (T + 15) / 16);
-    k_gemm_bf16<<<gh, 64, 0, st>>>(T, kHid, kHid, w.dZ2b, kHid, 1, w.Pb + kOffW2, 1, kHid, nullptr, 0, w.dZ1, nullptr,
-                                   kHid);
-    k_relu_back<<<g256((long)T * kHid), 256, 0, st>>>((long)T * kHid, w.H1b, w.dZ1, w.dZ1b);
-    // layer 1: dW1 = X^T dZ1 (32 x T x 64), db1 = colsum dZ1
-    dim3 g1(kHid / 16, kIn / 16);
-    k_gemm_bf16<<<g1, 64, 0, st>>>(kIn, kHid, T, w.Xb, 1, kIn, w.dZ1b, kHid, 1, nullptr, 0, grad + kOffW1, nullptr,
-                                   kHid);
-    k_colsum<<<kHid, 256, 0, st>>>(T, kHid, w.dZ1, nullptr, grad + kOffB1);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
+    float* inv = (float*)ws;
+    float* part = (float*)((char*)ws + 256);
+    const unsigned blocks = row_blocks(T, kTrainBlocks);
+    k_weight_sum<<<1, 1024, 0, st>>>(T, weight, inv);
+    k_mlp_train<<<blocks, 64 * kWaves, 0, st>>>(T, X, params, target, weight, inv, part);
+    k_mlp_reduce<<<(kPartial + 63) / 64, 256, 0, st>>>((int)blocks, part, inv, grad, loss);
+    return launch_status();
+}
+
+size_t ude_rate_scale_workspace_bytes(int T) { return 12 * (size_t)(T > 0 ? T : 0) + 512; }
+
+int ude_rate_scale(int T, const float* feats, const float* mean, const float* std, const float* params,
+                   const double* counts, double lo, double hi, float* out, void* ws, size_t wsBytes, hipStream_t st)
+{
+    if (T < 0 || !mean || !std) return UDE_ERR_ARG;
+    if (T == 0) return UDE_OK;
+    if (wsBytes < ude_rate_scale_workspace_bytes(T)) return UDE_ERR_WORKSPACE;
+    double* s = (double*)ws;
+    float* y = (float*)(s + T);
+    k_mlp_forward<<<row_blocks(T, 1024), 64 * kWaves, 0, st>>>(T, feats, mean, std, params, y);
+    k_rate_scale<<<1, 1024, 0, st>>>(T, y, counts, lo, hi, s, out);
+    return launch_status();
 }
 
 int ude_adam_step(int n, float* params, const float* grad, float* m, float* v, float lr, float beta1, float beta2,

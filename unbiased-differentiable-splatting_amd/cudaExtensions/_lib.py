@@ -37,6 +37,8 @@ _SIGS = {
     "ude_mlp_workspace_bytes": (c_size, [c_int]),
     "ude_mlp_forward": (c_int, [c_int] + [c_ptr] * 4 + [c_size, c_ptr]),
     "ude_mlp_loss_grad": (c_int, [c_int] + [c_ptr] * 7 + [c_size, c_ptr]),
+    "ude_rate_scale_workspace_bytes": (c_size, [c_int]),
+    "ude_rate_scale": (c_int, [c_int] + [c_ptr] * 5 + [c_dbl] * 2 + [c_ptr] * 2 + [c_size, c_ptr]),
     "ude_adam_step": (c_int, [c_int] + [c_ptr] * 4 + [ctypes.c_float] * 4 + [c_int, c_ptr]),
     "ude_set_poisson_proposal": (c_int, [c_int, c_dbl]),
     "ude_get_poisson_proposal": (c_int, [c_ptr]),

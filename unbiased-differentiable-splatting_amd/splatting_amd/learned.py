@@ -92,16 +92,18 @@ class RateNet:
         """Rate multipliers for tiles with features (..., 32) and plain-rate sample
         counts (...): exp(prediction), rescaled so that the expected sample count
         sum(scale * counts) is unchanged, and kept within [lo, hi]."""
-        shape = counts.shape
-        y = self.forward(feats.reshape(-1, N_IN)).reshape(shape).double()
-        y = torch.nan_to_num(y, nan=0.0, posinf=20.0, neginf=-20.0)     # a non-finite feature: plain rate
-        c = counts.double()
-        tot = c.sum().clamp(min=1e-30)
-        y = y - (y * c).sum() / tot
-        s = torch.exp(y.clamp(-20.0, 20.0))
-        for _ in range(3):
-            s = (s * (tot / (s * c).sum().clamp(min=1e-30))).clamp(lo, hi)
-        return s.float().contiguous()
+        F = _lib.f32(feats.reshape(-1, N_IN), "features")
+        c = counts.reshape(-1).double().contiguous()
+        T = F.shape[0]
+        if c.shape[0] != T:
+            raise ValueError("tile_scale: %d counts for %d tiles" % (c.shape[0], T))
+        mean, std = (_lib.f32(torch.broadcast_to(x, (1, N_IN)), q) for x, q in ((self.mean, "mean"), (self.std, "std")))
+        _lib.require_gpu(F, c, mean, std, self.params)
+        out = torch.empty(T, dtype=torch.float32, device=F.device)
+        ws = _lib.workspace(_lib.lib().ude_rate_scale_workspace_bytes(T), F.device)
+        _call("ude_rate_scale", T, _lib.ptr(F), _lib.ptr(mean), _lib.ptr(std), _lib.ptr(self.params), _lib.ptr(c),
+              float(lo), float(hi), _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream(F.device))
+        return out.reshape(counts.shape)
 
     def save(self, path):
         np.savez(path, params=self.params.cpu().numpy(), mean=self.mean.cpu().numpy(), std=self.std.cpu().numpy())
