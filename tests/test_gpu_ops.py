@@ -181,6 +181,35 @@ def test_filter_equal_depths(dev, k):
     assert np.abs(wrong - ref).max() > 1e-2
 
 
+@pytest.mark.parametrize("splats", [3, 400])
+@pytest.mark.parametrize("k", [65, 127, 128, 129, 250, 256, 257, 319, 1024])
+def test_filter_wide(dev, k, splats):
+    """More than 64 slots: around the lane-row, wavefront and workgroup sizes, with many
+    equal depths (three splats) and few (400); both batch entries, every slot filled in some
+    pixels and none in others.  A product of k factors 1 - w carries up to 2 k float32
+    roundings (2^-24 each), a suffix sum over it twice as many."""
+    from cudaExtensions import filtering
+    sc, p, n, nb, sd = scene_inputs(2, sd_scale=8.0)[:5]
+    W, H = 5, 3                                         # 15 pixels: a partial group of wavefronts
+    rng = np.random.default_rng(177 + k)
+    idx = rng.integers(0, min(splats, p.shape[0]), size=(2, W, H, k)).astype(np.int32)
+    idx[rng.uniform(size=idx.shape) < 0.3] = -1
+    idx[0, 0, 0] = 1
+    idx[1, 2, 1] = -1
+    w = (rng.uniform(0.0, 1.0, size=idx.shape) * min(1.0, 24.0 / k)).astype(np.float32)
+    g = rng.normal(size=idx.shape).astype(np.float32)
+    a = (W, H, sc.focal)
+    dv = (t(idx, dev), t(w, dev))
+    out = filtering.forward(*dv, *a, t(p[None], dev), t(n[None], dev))
+    rtol = max(RTOL, 2 * k * 2.0 ** -24)
+    assert_close(out.cpu().numpy(), O.filter_forward(idx, w, *a, p[None], n[None]), rtol, "wide filter forward")
+    for exact in (False, True):
+        gw = filtering.backward(*dv, t(g, dev), *a, t(p[None], dev), t(n[None], dev), exact=exact)
+        rg = O.filter_backward(idx, w, g, *a, p[None], n[None], exact=exact)
+        mg = magnitude(O.filter_backward, idx, w, g, *a, p[None], n[None], exact=exact)
+        assert_close(gw.cpu().numpy(), rg, RTOL, "wide filter backward", mag=mg, ops=max(64, 4 * k))
+
+
 @pytest.mark.parametrize("affine", [True, False])
 @pytest.mark.parametrize("bn,vb", [(1, 1), (3, 1), (3, 3)])
 def test_transform(dev, affine, bn, vb):

@@ -749,6 +749,13 @@ __device__ __forceinline__ void wave_affine_incl(C& A, C& B)
     affine_step<0x143, 0xc>(A, B);
 }
 
+// orders the wavefront's LDS accesses (its LDS operations execute in order)
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ float quiet_nan(float) { return __int_as_float(0x7fc00000); }
 __device__ __forceinline__ double quiet_nan(double) { return __longlong_as_double(0x7ff8000000000000ll); }
 
@@ -853,7 +860,147 @@ __global__ __launch_bounds__(256) void k_filter_wave(long npix, int N, int W, in
     if (act) st_c(out, base + s, g);
 }
 
-// General k (64 < k <= 1024): one workgroup per pixel, ranks from LDS, serial scans.
+// 64 < k <= 256: one wavefront per pixel, ROWS = 2 or 4 slots per lane (slot
+// 64 r + lane).  A lane counts, for each of its depths, the smaller ones over LDS
+// broadcasts of all of them.  Slots of equal depth (empty slots, splats drawn twice) get
+// equal counts; each sets its bit in the word of its count and row, and the bits below its
+// own are its rank among them, as in k_filter_wave.  The scans run over
+// 64 lanes with ROWS consecutive ranks each.  Bound by the instructions of the counting
+// loop.  At 256x192, k = 100 forward / backward take 50 / 52 us; a workgroup per pixel with
+// the prefix and suffix run by its first thread took 154 / 227 us, and this kernel with a
+// second pass over the depths for ties 98 / 98 us.
+template <bool BACKWARD, int ROWS, class S>
+__global__ __launch_bounds__(256) void k_filter_rows(long npix, int N, int W, int H, int k,
+                                                     typename CompOf<S>::type ff, typename CompOf<S>::type gate,
+                                                     const int32_t* __restrict__ idx, const S* __restrict__ wts,
+                                                     const S* __restrict__ gin,
+                                                     const S* __restrict__ pts, const S* __restrict__ nrm, int pb,
+                                                     S* __restrict__ out)
+{
+    using C = typename CompOf<S>::type;
+    constexpr int CAP = 64 * ROWS;
+    __shared__ __align__(16) C sa_[4][CAP];             // depths by slot; gin w, then S, by rank
+    __shared__ __align__(16) C sb_[4][CAP];             // 1 - w, then the transmittance, by rank
+    __shared__ unsigned long long sg_[4][CAP][ROWS];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const long pix = (long)blockIdx.x * 4 + wv;
+    if (pix >= npix) return;   // whole wave exits together
+    C* sa = sa_[wv];
+    C* sb = sb_[wv];
+    unsigned long long (*sg)[ROWS] = sg_[wv];
+    const long b = pix / ((long)W * H);
+    const int rp = (int)(pix - b * (long)W * H);
+    const int i = rp / H, j = rp - (rp / H) * H;
+    const long base = pix * k;
+    C w[ROWS], gi[ROWS], d[ROWS];
+    bool act[ROWS];
+    int rank[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        const int s = 64 * r + lane;
+        act[r] = s < k;
+        const int id = act[r] ? idx[base + s] : -1;
+        w[r] = act[r] ? ld_c(wts, base + s) : C(0);
+        gi[r] = (BACKWARD && act[r]) ? ld_c(gin, base + s) : C(0);
+        d[r] = C(10000);
+        if (id >= 0) {
+            const long po = 3 * ((pb > 1 ? b * N : 0) + id);
+            C p[3] = { ld_c(pts, po), ld_c(pts, po + 1), ld_c(pts, po + 2) };
+            C n[3] = { ld_c(nrm, po), ld_c(nrm, po + 1), ld_c(nrm, po + 2) };
+            d[r] = ray_depth<C>(i, j, (C)W, (C)H, ff, p, n);
+        }
+        sa[s] = act[r] ? d[r] : quiet_nan(C(0));        // compares false
+        rank[r] = 0;
+#pragma unroll
+        for (int q = 0; q < ROWS; q++) sg[s][q] = 0ull;
+    }
+    wave_order();
+    const int k16 = (k + 15) & ~15;                     // <= CAP
+    for (int q0 = 0; q0 < k16; q0 += 16) {
+        C kq[16];
+#pragma unroll
+        for (int q = 0; q < 16; q++) kq[q] = sa[q0 + q];
+#pragma unroll
+        for (int q = 0; q < 16; q++)
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) rank[r] += kq[q] < d[r];
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; r++)
+        if (act[r]) atomicOr(&sg[rank[r]][r], 1ull << lane);
+    wave_order();
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        const int lt = rank[r] < CAP ? rank[r] : 0;     // an inactive slot counts nothing of use
+#pragma unroll
+        for (int q = 0; q < r; q++) rank[r] += __popcll(sg[lt][q]);
+        const unsigned long long m = sg[lt][r];
+        rank[r] = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, rank[r]));
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) { sb[64 * r + lane] = C(1); if (BACKWARD) sa[64 * r + lane] = C(0); }
+    wave_order();
+#pragma unroll
+    for (int r = 0; r < ROWS; r++)
+        if (act[r]) {
+            sb[rank[r]] = C(1) - w[r];
+            if (BACKWARD) sa[rank[r]] = gi[r] * w[r];
+        }
+    wave_order();
+    // lane l holds ranks ROWS l ...: exclusive products in rank order
+    C one[ROWS], inc = C(1);
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) { one[r] = sb[ROWS * lane + r]; inc = inc * one[r]; }
+    inc = wave_prod_incl(inc);
+    C front = __shfl_up(inc, 1, 64);
+    if (lane == 0) front = C(1);
+    C after[ROWS];
+    if (BACKWARD) {
+        // S_r = a_{r+1} + b_{r+1} S_{r+1} (k_filter_wave): lane l composes the maps x ->
+        // a + b x of the ranks ROWS (63 - l) ..., the later ones applied first
+        C A = C(0), B = C(1), a_[ROWS], b_[ROWS];
+#pragma unroll
+        for (int r = ROWS - 1; r >= 0; r--) {
+            a_[r] = sa[ROWS * (63 - lane) + r];
+            b_[r] = sb[ROWS * (63 - lane) + r];
+            A = a_[r] + b_[r] * A;
+            B = b_[r] * B;
+        }
+        wave_affine_incl(A, B);
+        C acc = __shfl_up(A, 1, 64);                    // S of the lane's last rank
+        if (lane == 0) acc = C(0);
+#pragma unroll
+        for (int r = ROWS - 1; r >= 0; r--) {
+            after[r] = acc;
+            acc = a_[r] + b_[r] * acc;
+        }
+    }
+    wave_order();
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        sb[ROWS * lane + r] = front;
+        front = front * one[r];
+        if (BACKWARD) sa[ROWS * (63 - lane) + r] = after[r];
+    }
+    wave_order();
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        if (!act[r]) continue;
+        const C rem = sb[rank[r]];
+        C g = rem * w[r];
+        if (BACKWARD) {
+            g = C(0);
+            if (fabs(w[r]) > gate) g += gi[r] * rem;
+            if (fabs(C(1) - w[r]) > gate) g -= rem * sa[rank[r]];
+        }
+        st_c(out, base + 64 * r + lane, g);
+    }
+}
+
+// 256 < k <= 1024: one workgroup per pixel, a thread per slot, ranks from LDS; the
+// scans over the ranks run per wavefront and then over the wavefronts' totals (128x96,
+// k = 512: 392 / 526 -> 347 / 353 us against scans by the first thread).  The line lies at
+// 256: there four rows take 58 / 59 us, the workgroup 108 / 150 us as it was.
 template <bool BACKWARD, class S>
 __global__ __launch_bounds__(1024) void k_filter_block(long npix, int N, int W, int H, int k,
                                                        typename CompOf<S>::type ff, typename CompOf<S>::type gate,
@@ -863,17 +1010,19 @@ __global__ __launch_bounds__(1024) void k_filter_block(long npix, int N, int W, 
                                                        S* __restrict__ out)
 {
     using C = typename CompOf<S>::type;
-    __shared__ C sd_[1024], sw[1024], sx[1024];
-    __shared__ int srank[1024];
+    __shared__ C sd_[1024], sb[1024];
+    __shared__ C tot[16][2];
     long pix = blockIdx.x;
     long b = pix / ((long)W * H);
     int r = (int)(pix - b * (long)W * H);
     int i = r / H, j = r - (r / H) * H;
     long base = pix * k;
     int s = threadIdx.x;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     bool act = s < k;
     int id = act ? idx[base + s] : -1;
     C w = act ? ld_c(wts, base + s) : C(0);
+    C gi = (BACKWARD && act) ? ld_c(gin, base + s) : C(0);
     C d = C(10000);
     if (id >= 0) {
         long po = 3 * ((pb > 1 ? b * N : 0) + id);
@@ -881,36 +1030,49 @@ __global__ __launch_bounds__(1024) void k_filter_block(long npix, int N, int W, 
         C n[3] = { ld_c(nrm, po), ld_c(nrm, po + 1), ld_c(nrm, po + 2) };
         d = ray_depth<C>(i, j, (C)W, (C)H, ff, p, n);
     }
-    if (act) { sd_[s] = d; sw[s] = w; }
+    if (act) sd_[s] = d;
     __syncthreads();
     int rank = 0;
-    if (act) {
+    if (act)
         for (int q = 0; q < k; q++) { C dq = sd_[q]; rank += (dq < d) || (dq == d && q < s); }
-        srank[rank] = s;
+    __syncthreads();
+    sb[s] = C(1);                                       // thread t: rank t
+    sd_[s] = C(0);
+    __syncthreads();
+    if (act) { sb[rank] = C(1) - w; sd_[rank] = gi * w; }
+    __syncthreads();
+    // transmittance in front of rank t: exclusive product of (1 - w)
+    const C one = sb[s];
+    C inc = wave_prod_incl(one);
+    if (lane == 63) tot[wv][0] = inc;
+    __syncthreads();
+    C front = __shfl_up(inc, 1, 64);
+    if (lane == 0) front = C(1);
+    C before = C(1);
+    for (int q = 0; q < wv; q++) before = before * tot[q][0];
+    front = before * front;
+    C after = C(0);
+    if (BACKWARD) {
+        // the division-free form of the wave kernel: the map of rank n - 1 - t, composed
+        // from the last rank on
+        const int m = (int)blockDim.x - 1 - s;
+        C A = sd_[m], B = sb[m];
+        wave_affine_incl(A, B);
+        __syncthreads();
+        if (lane == 63) { tot[wv][0] = A; tot[wv][1] = B; }
+        __syncthreads();
+        C acc = C(0);                                   // S at the end of this wavefront's ranks
+        for (int q = 0; q < wv; q++) acc = tot[q][0] + tot[q][1] * acc;
+        C pa = __shfl_up(A, 1, 64), pbm = __shfl_up(B, 1, 64);
+        after = lane == 0 ? acc : pa + pbm * acc;       // S of rank m
     }
     __syncthreads();
-    if (s == 0) {   // sx[rank] = exclusive product of (1 - w) in rank order
-        C rem = C(1);
-        for (int q = 0; q < k; q++) { sx[q] = rem; rem *= (C(1) - sw[srank[q]]); }
-    }
-    __syncthreads();
-    C rem = act ? sx[rank] : C(0);
-    if (!BACKWARD) { if (act) st_c(out, base + s, rem * w); return; }
-    // backward: the division-free form of the wave kernel, S in a serial suffix pass
-    C gi = act ? ld_c(gin, base + s) : C(0);
-    __syncthreads();
-    if (act) sd_[rank] = gi * w;
-    __syncthreads();
-    if (s == 0) {   // sd_[rank] = S_rank = sum over later ranks, recurrence from the back
-        C acc = C(0);
-        for (int q = k - 1; q >= 0; q--) {
-            C a = sd_[q];
-            sd_[q] = acc;
-            acc = a + (C(1) - sw[srank[q]]) * acc;
-        }
-    }
+    sb[s] = front;
+    if (BACKWARD) sd_[(int)blockDim.x - 1 - s] = after;
     __syncthreads();
     if (!act) return;
+    const C rem = sb[rank];
+    if (!BACKWARD) { st_c(out, base + s, rem * w); return; }
     C g = C(0);
     if (fabs(w) > gate) g += gi * rem;
     if (fabs(C(1) - w) > gate) g -= rem * sd_[rank];
@@ -1598,6 +1760,12 @@ int filter_t(int bn, int N, int W, int H, int k, double f, const int32_t* idx, c
     if (k <= 64)
         k_filter_wave<BWD, S><<<grid1(npix, 4), 256, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx, wts, gin, pts, nrm,
                                                                pb, out);
+    else if (k <= 128)
+        k_filter_rows<BWD, 2, S><<<grid1(npix, 4), 256, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx, wts, gin, pts, nrm,
+                                                                 pb, out);
+    else if (k <= 256)
+        k_filter_rows<BWD, 4, S><<<grid1(npix, 4), 256, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx, wts, gin, pts, nrm,
+                                                                 pb, out);
     else
         k_filter_block<BWD, S><<<(unsigned)npix, ((k + 63) / 64) * 64, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx,
                                                                                  wts, gin, pts, nrm, pb, out);
