@@ -56,6 +56,29 @@ def test_nearest_independent_of_pixel_order(dev):
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("k,K,N", [(1, 3, 9), (2, 2, 9), (5, 40, 30), (16, 10, 60), (17, 3, 200), (64, 12, 90),
+                                   (65, 7, 2000), (130, 64, 150)])
+def test_nearest_of_shared_rows(dev, k, K, N):
+    """Few splats under many pixels: rows that many wavefronts enter at once, splats drawn
+    twice at a pixel, equal points (ties by index), equal and NaN weights, empty slots, and
+    slot counts around the lane groups.  The rows are whole numbers and equal the oracle's."""
+    from cudaExtensions import nearestsamples
+    rng = np.random.default_rng(100 * k + K)
+    idx = rng.integers(-1, N, size=(2, 37, 11, k)).astype(np.int32)
+    idx[0, 0, 0] = -1
+    w = (rng.integers(0, 6, size=idx.shape) / 4).astype(np.float32)
+    w[rng.uniform(size=idx.shape) < 0.05] = np.nan
+    p = (rng.integers(0, 8, size=(1, N, 3)) / 8).astype(np.float32)
+    # slots are compared in order by w > largest: a NaN in slot 0 stays, one elsewhere never
+    # wins (the oracle's argmax orders NaN first wherever it stands)
+    wo = np.where(np.isnan(w), np.float32(-1.0), w)
+    wo[..., 0] = np.where(np.isnan(w[..., 0]), np.float32(9.0), w[..., 0])
+    ref = O.nearest_samples(idx, wo, p, K)
+    for dt in (torch.float32, torch.float64):
+        got = nearestsamples.nearest(t(idx, dev), t(w, dev).to(dt), t(p, dev).to(dt), K)
+        assert np.array_equal(got.cpu().numpy(), ref), dt
+
+
 def test_nearest_empty(dev):
     from cudaExtensions import nearestsamples
     idx = torch.full((1, 4, 4, 5), -1, dtype=torch.int32, device=dev)

@@ -42,6 +42,24 @@ def test_scatter_gather_against_oracle(dev, C):
     assert_close(g64.cpu().numpy(), ref, 1e-12, "gather f64", mag=mag, ops=256, eps=EPS64)
 
 
+@pytest.mark.parametrize("C", [2, 15, 16, 30, 31])
+@pytest.mark.parametrize("W,H,k,N", [(16, 16, 1, 3), (17, 15, 9, 40), (1, 50, 64, 3000), (64, 3, 33, 100_000)])
+def test_gather_tiles(dev, W, H, k, N, C):
+    """Partial tiles, fewer and more splats than a tile's table holds, and row widths on
+    both sides of what its sums take; entries that cancel and zeros.  Bounds as above."""
+    from cudaExtensions import pixelgather
+    rng = np.random.default_rng(W + C)
+    idx = random_slots(rng, 2, W, H, k, N)
+    u = rng.normal(size=idx.shape + (C,)).astype(np.float32)
+    u[rng.uniform(size=u.shape) < 0.1] = 0.0
+    mag = O.pixel_gather(idx, np.abs(u.astype(np.float64)), N)
+    ref = O.pixel_gather(idx, u.astype(np.float64), N)
+    g32 = pixelgather.gather(t(idx, dev), t(u, dev), N)
+    assert_close(g32.cpu().numpy(), ref, 1e-5, "gather f32", mag=mag, ops=max(64, idx[0].size // N))
+    g64 = pixelgather.gather(t(idx, dev), t(u, dev, torch.float64), N)
+    assert_close(g64.cpu().numpy(), ref, 1e-12, "gather f64", mag=mag, ops=256, eps=EPS64)
+
+
 def test_autograd_adjoint(dev):
     from splatting_amd.extensions import PixelScatterGather
     rng = np.random.default_rng(5)
