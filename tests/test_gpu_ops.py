@@ -210,6 +210,26 @@ def test_filter_wide(dev, k, splats):
         assert_close(gw.cpu().numpy(), rg, RTOL, "wide filter backward", mag=mg, ops=max(64, 4 * k))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("bn,N", [(2, 1), (2, 4095), (3, 4097), (65, 1030), (130, 64)])
+def test_transform_backward_shared_vectors(dev, bn, N, dtype):
+    """One vector set under all views, around the workgroup's points and its views in LDS;
+    each sum has N or bn terms, so its bound takes that many roundoffs."""
+    from cudaExtensions import transform
+    rng = np.random.default_rng(bn + N)
+    M, v, g = rng.normal(size=(bn, 4, 4)), rng.normal(size=(1, N, 3)), rng.normal(size=(bn, N, 3))
+    if dtype == torch.float32:
+        M, v, g = (x.astype(np.float32) for x in (M, v, g))
+    eps = float(np.finfo(M.dtype).eps) / 2
+    for affine in (True, False):
+        bw = transform.affineBackward if affine else transform.linearBackward
+        got = bw(t(g, dev), t(M, dev), t(v, dev))
+        ref = O.transform_backward(affine, g, M, v)
+        mag = magnitude(O.transform_backward, affine, g, M, v)
+        for a, r, m in zip(got, ref, mag):
+            assert_close(a.cpu().numpy(), r, 8 * eps, "shared transform backward", mag=m, ops=max(64, bn), eps=eps)
+
+
 @pytest.mark.parametrize("affine", [True, False])
 @pytest.mark.parametrize("bn,vb", [(1, 1), (3, 1), (3, 3)])
 def test_transform(dev, affine, bn, vb):

@@ -749,6 +749,18 @@ __device__ __forceinline__ void wave_affine_incl(C& A, C& B)
     affine_step<0x143, 0xc>(A, B);
 }
 
+// Sum over the lanes, in lane 63 (zeros come in at the ends of the shifts).
+template <class C>
+__device__ __forceinline__ C wave_sum_last(C v)
+{
+    v = v + dpp_from<0x111, 0xf>(C(0), v);
+    v = v + dpp_from<0x112, 0xf>(C(0), v);
+    v = v + dpp_from<0x114, 0xf>(C(0), v);
+    v = v + dpp_from<0x118, 0xf>(C(0), v);
+    v = v + dpp_from<0x142, 0xa>(C(0), v);
+    return v + dpp_from<0x143, 0xc>(C(0), v);
+}
+
 // orders the wavefront's LDS accesses (its LDS operations execute in order)
 __device__ __forceinline__ void wave_order()
 {
@@ -1259,7 +1271,7 @@ __device__ __forceinline__ double wave_sum_t(double v) { return wave_sum_d(v); }
 // atomics (1M points: 11.7 us, where 512 x 256 threads took 15.5 us and
 // 2048 x 256 33.5 us).
 template <class T>
-__global__ __launch_bounds__(1024) void k_transform_backward(int affine, int bn, int vb, int N, const T* __restrict__ g,
+__global__ __launch_bounds__(1024) void k_transform_backward(int affine, int vb, int N, const T* __restrict__ g,
                                                             const T* __restrict__ M, const T* __restrict__ v,
                                                             T* __restrict__ gM, T* __restrict__ gV)
 {
@@ -1282,8 +1294,7 @@ __global__ __launch_bounds__(1024) void k_transform_backward(int affine, int bn,
         }
         T gv[3];
         for (int c = 0; c < 3; c++) gv[c] = m[c] * g0 + m[4 + c] * g1 + m[8 + c] * g2;
-        if (vb > 1 || bn == 1) { for (int c = 0; c < 3; c++) gV[vo + c] = gv[c]; }
-        else { for (int c = 0; c < 3; c++) atomicAdd(gV + vo + c, gv[c]); }
+        for (int c = 0; c < 3; c++) gV[vo + c] = gv[c];
     }
     for (int q = 0; q < 12; q++) acc[q] = wave_sum_t(acc[q]);
     int wv = threadIdx.x >> 6;
@@ -1293,6 +1304,81 @@ __global__ __launch_bounds__(1024) void k_transform_backward(int affine, int bn,
         T s = red[0][threadIdx.x];
         for (int w = 1; w < 16; w++) s += red[w][threadIdx.x];
         atomicAdd(gM + 16 * b + threadIdx.x, s);
+    }
+}
+
+// The same with one vector set for all views (vb == 1 < bn).  A thread keeps its points
+// and their gradients in registers while it runs over the views, so the points' sums need
+// no atomics; the matrix sums of up to 64 views wait in LDS until the workgroup has seen
+// all its points.  Bound by reading g (the next view's values are loaded ahead): 2M points
+// and 16 views 124 us (81 at the rate of a copy), where a workgroup per view and a global atomic per point and
+// component took 890 us.
+constexpr int kSharedViews = 64;
+template <class T>
+constexpr int shared_points() { return sizeof(T) == 8 ? 2 : 4; }   // four doubles would not fit the registers
+
+template <class T>
+__global__ __launch_bounds__(1024) void k_transform_backward_shared(int affine, int bn, int N,
+                                                                   const T* __restrict__ g, const T* __restrict__ M,
+                                                                   const T* __restrict__ v, T* __restrict__ gM,
+                                                                   T* __restrict__ gV)
+{
+    constexpr int P = shared_points<T>();
+    __shared__ T red[kSharedViews][12];
+    for (int b0 = 0; b0 < bn; b0 += kSharedViews) {
+        const int nb = min(kSharedViews, bn - b0);
+        for (int t = threadIdx.x; t < nb * 12; t += 1024) ((T*)red)[t] = T(0);
+        __syncthreads();
+        for (long x0 = (long)blockIdx.x * (1024 * P); x0 < N; x0 += (long)gridDim.x * (1024 * P)) {
+            T a[P][3], gv[P][3], gg[P][3];
+            long at[P];
+            bool in[P];
+#pragma unroll
+            for (int p = 0; p < P; p++) {
+                const long x = x0 + p * 1024 + threadIdx.x;
+                in[p] = x < N;
+                at[p] = 3 * (in[p] ? x : 0);
+                for (int c = 0; c < 3; c++) {
+                    a[p][c] = v[at[p] + c];
+                    gv[p][c] = T(0);
+                    gg[p][c] = in[p] ? g[3 * (long)b0 * N + at[p] + c] : T(0);
+                }
+            }
+            for (int b = 0; b < nb; b++) {
+                const T* m = M + 16 * (long)(b0 + b);
+                T acc[12], nx[P][3];
+                for (int q = 0; q < 12; q++) acc[q] = T(0);
+                const long next = 3 * (long)(b0 + min(b + 1, nb - 1)) * N;
+#pragma unroll
+                for (int p = 0; p < P; p++)
+                    for (int c = 0; c < 3; c++) nx[p][c] = in[p] ? g[next + at[p] + c] : T(0);
+#pragma unroll
+                for (int p = 0; p < P; p++) {
+                    if (in[p])
+                        for (int r = 0; r < 3; r++) {
+                            for (int c = 0; c < 3; c++) acc[4 * r + c] += gg[p][r] * a[p][c];
+                            if (affine) acc[4 * r + 3] += gg[p][r];
+                        }
+                    for (int c = 0; c < 3; c++)
+                        gv[p][c] += m[c] * gg[p][0] + m[4 + c] * gg[p][1] + m[8 + c] * gg[p][2];
+                }
+                for (int q = 0; q < 12; q++) {
+                    if ((q & 3) == 3 && !affine) continue;
+                    const T s = wave_sum_last(acc[q]);
+                    if ((threadIdx.x & 63) == 63) atomicAdd(&red[b][q], s);
+                }
+#pragma unroll
+                for (int p = 0; p < P; p++)
+                    for (int c = 0; c < 3; c++) gg[p][c] = nx[p][c];
+            }
+#pragma unroll
+            for (int p = 0; p < P; p++)
+                if (in[p])
+                    for (int c = 0; c < 3; c++) gV[at[p] + c] += gv[p][c];
+        }
+        __syncthreads();
+        for (int t = threadIdx.x; t < nb * 12; t += 1024) atomicAdd(gM + 16 * (long)(b0 + t / 12) + t % 12, ((T*)red)[t]);
+        __syncthreads();
     }
 }
 
@@ -1788,9 +1874,14 @@ int transform_backward_t(int affine, int bn, int vb, int N, const T* g, const T*
 {
     if (bn <= 0 || bn > 65535 || N < 0 || (vb != 1 && vb != bn)) return UDE_ERR_ARG;
     if (N == 0) return UDE_OK;
+    if (vb == 1 && bn > 1) {
+        const unsigned blocks = grid1(N, 1024 * shared_points<T>());
+        k_transform_backward_shared<T><<<blocks < 256u ? blocks : 256u, 1024, 0, st>>>(affine, bn, N, g, M, v, gM, gV);
+        return launch_status();
+    }
     const unsigned blocks = grid1(N, 1024) < 256u ? grid1(N, 1024) : 256u;
     dim3 grid(blocks, bn);
-    k_transform_backward<T><<<grid, 1024, 0, st>>>(affine, bn, vb, N, g, M, v, gM, gV);
+    k_transform_backward<T><<<grid, 1024, 0, st>>>(affine, vb, N, g, M, v, gM, gV);
     return launch_status();
 }
 
