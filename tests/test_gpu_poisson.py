@@ -40,6 +40,28 @@ def test_poisson_bit_exact(dev, cfg, sds, kcap, rate, prec):
     assert np.array_equal(ipi[0], ripi)
 
 
+@pytest.mark.parametrize("proposal", ["bands", "footprint"])
+@pytest.mark.parametrize("m,rate", [(1, 5.0), (2, 0.05), (3, 1e30), (65, 300.0), (4096, 0.05), (4096, 40.0)])
+def test_poisson_range_queue(dev, m, rate, proposal):
+    """Lanes whose lists of ranges stay empty, hold one, and run full, side by side in a
+    partial tile: trees of one to a few leaves, rates at which nearly nothing or every
+    candidate is kept.  Equal to the oracle bit for bit, the overflow flag too."""
+    from cudaExtensions import sampling
+    sc, p, n, nb, sd = scene_inputs(0, sd_scale=2.0)
+    p, nb, sd = (np.ascontiguousarray(x[:: max(1, len(x) // m)][:m]) for x in (p, nb, sd))
+    W, H, kcap = 37, 23, 96
+    f = sc.focal * W / sc.width
+    ids, ipi = sampling.samplePoisson(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), kcap, 0.0, 0.01,
+                                      seed=11, rate=rate, proposal=proposal)
+    rid, ripi, dens, over = O.poisson_view(W, H, f, p, nb, sd, kcap, rate, 0.0, 0.01, seed=11, proposal=proposal)
+    assert np.array_equal(ids[0].cpu().numpy(), rid) and np.array_equal(ipi[0].cpu().numpy(), ripi)
+    if over:
+        with pytest.raises(RuntimeError, match="more than numSamples"):
+            sampling.check_errors()
+    else:
+        sampling.check_errors()
+
+
 def test_poisson_tile_scale_batch_and_edges(dev):
     from cudaExtensions import sampling
     sc, p, n, nb, sd = scene_inputs(2, sd_scale=8.0)

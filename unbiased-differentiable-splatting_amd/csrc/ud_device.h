@@ -25,9 +25,6 @@ constexpr int kWave = 64;
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float pexpf(float x)
 {
-    if (x != x) return x;
-    if (x > 88.0f) return __builtin_huge_valf();
-    if (x < -87.0f) return 0.0f;
     const float log2e = 1.44269504088896341f;
     const float ln2hi = 0.693145751953125f;
     const float ln2lo = 1.428606765330187045e-06f;
@@ -44,22 +41,22 @@ __device__ __forceinline__ float pexpf(float x)
     p = fmaf(p, r, 1.0f);
     int k = (int)kf;
     float sc = __uint_as_float((uint32_t)(k + 127) << 23);
-    return p * sc;
+    float e = p * sc;                        // selects, not branches: lanes differ
+    e = x < -87.0f ? 0.0f : e;
+    e = x > 88.0f ? __builtin_huge_valf() : e;
+    return x != x ? x : e;
 }
 
-// log: x = m 2^e, m in [sqrt(1/2), sqrt(2)), log m = 2 atanh((m-1)/(m+1)).
-__device__ __forceinline__ float plogf(float x)
+// log of a positive normal number: x = m 2^e, m in [sqrt(1/2), sqrt(2)),
+// log m = 2 atanh((m-1)/(m+1)); times 2^e of the argument
+__device__ __forceinline__ float plogf_normal(float x, int e = 0)
 {
-    if (x != x) return x;
-    if (x < 0.0f) return __builtin_nanf("");
-    if (x == 0.0f) return -__builtin_huge_valf();
-    if (x == __builtin_huge_valf()) return x;
-    uint32_t u = __float_as_uint(x);
-    int e = 0;
-    if (u < 0x00800000u) { u = __float_as_uint(x * 16777216.0f); e = -24; }
-    e += (int)((u >> 23) & 0xffu) - 127;
+    const uint32_t u = __float_as_uint(x);
+    e += (int)(u >> 23) - 127;
     float m = __uint_as_float((u & 0x007fffffu) | 0x3f800000u);
-    if (m > 1.41421356f) { m = m * 0.5f; e += 1; }
+    const bool high = m > 1.41421356f;
+    m = high ? m * 0.5f : m;
+    e += high;
     float s = (m - 1.0f) / (m + 1.0f);
     float s2 = s * s;
     float p = 1.0f / 9.0f;
@@ -72,6 +69,15 @@ __device__ __forceinline__ float plogf(float x)
     const float ln2lo = 1.428606765330187045e-06f;
     float ef = (float)e;
     return fmaf(ef, ln2hi, fmaf(ef, ln2lo, lm));
+}
+
+__device__ __forceinline__ float plogf(float x)
+{
+    if (x != x) return x;
+    if (x < 0.0f) return __builtin_nanf("");
+    if (x == 0.0f) return -__builtin_huge_valf();
+    if (x == __builtin_huge_valf()) return x;
+    return x < 1.17549435e-38f ? plogf_normal(x * 16777216.0f, -24) : plogf_normal(x);
 }
 
 // log(1 - u) for u in [0, 1]: the log1p series -(u + u^2/2 + ... + u^8/8) for
@@ -90,7 +96,7 @@ __device__ __forceinline__ float plog1mf(float u)
         p = p * u + 1.0f;
         return -(p * u);
     }
-    return plogf(1.0f - u);
+    return plogf_normal(1.0f - u);                          // 1 - u >= 2^-24
 }
 
 // ---------------------------------------------------------------------------

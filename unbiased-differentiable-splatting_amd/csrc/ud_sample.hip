@@ -3298,12 +3298,24 @@ __global__ void k_zero_f64(double* p, size_t stride, int views)
 // (step, 0x80000000, pixel, view), one block per geometric-skip step of the
 // pixel (word x the skip, word y the acceptance test).  A skipped or thinned
 // subtree is left through its escape pointer.
+// Walking and thinning alternate: a lane queues its ranges in registers and thins them
+// in the order found, and each turn of the wavefront takes the step that more lanes can
+// take.  A pixel at 512x512 under 1M splats visits 109 nodes and takes 59 thinning steps
+// (tile maxima 130 and 75), but the pixels find their ranges at different nodes: thinned
+// on the spot, every visit waited for some lane's steps.  Bound by instruction issue (a
+// thinning step is a Philox block, a logarithm and a mixture).  16 views of 640x480 under
+// 2M splats: 5.85 -> 3.91 ms (512x512, 1M: 578 -> 368 us); queues of 2, 3, 6 ranges take
+// 4.37, 4.21, 4.21 against 4.15 ms here (before the branch-free exponential), walking
+// at twice as many thinning lanes 4.48, thinning at twice as many walking ones 4.47.  One
+// walk over the union of the tile's nodes with scalar loads visits 392 nodes: 7.24 ms.
 // The first kPoissonStage samples of each lane are staged in LDS (slot-major,
-// [slot][lane], so the walk's stores hit 64 distinct banks) and written out at
+// [slot][lane], so the stores hit 64 distinct banks) and written out at
 // the end together with the empty slots, one tile row (2^lth contiguous pixels
 // x kcap slots) per coalesced pass of the wavefront; only samples past the
 // staged ones are stored directly.  A lane's scattered 4-byte stores would
 // otherwise leave partly written lines in L2 for the length of the walk.
+constexpr int kPoissonQueue = 4;
+
 constexpr int kPoissonStage = 16;
 constexpr size_t kPoissonStageBytes = (size_t)kPoissonStage * 64 * 8;    // per wavefront
 
@@ -3356,16 +3368,16 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_poisson(TileCfg cfg,
     bool over = false;
     const int n = vs->nc;
     const float D0 = (n > 0 && valid) ? dens0[pix] : 0.0f;
-    if (valid && n > 0 && D0 >= vs->prec) {
-        const int L0 = n - 1;
+    const bool draws = valid && n > 0 && D0 >= vs->prec;
+    if (__ballot(draws)) {
         const Band B0 = vs->band[0], B1 = vs->band[1];
         float lam = rate;
-        if (tscale) lam = lam * tscale[(long)(i >> 4) * tsH + (j >> 4)];
+        if (tscale && draws) lam = lam * tscale[(long)(i >> 4) * tsH + (j >> 4)];
         // a negative or non-finite multiplier would make every candidate's pi 1
         // (fminf drops a NaN): draw nothing there and say so
-        if (!(lam >= 0.0f && lam <= 3.0e38f)) { atomicOr(err, 16); lam = 0.0f; }
+        if (draws && !(lam >= 0.0f && lam <= 3.0e38f)) { atomicOr(err, 16); lam = 0.0f; }
         const float t0 = 0.5f / fmaxf(D0, B0.c);
-        const float t1 = 0.5f / fmaxf(dens1[pix], B1.c);
+        const float t1 = 0.5f / fmaxf(draws ? dens1[pix] : 0.0f, B1.c);
         const float k0 = t0 * B0.c, k1 = t1 * B1.c;
         const float a0 = B0.is2h * B0.is2h, a1 = B1.is2h * B1.is2h;
         // footprint mode: the wide band's half as above, and in place of band 0
@@ -3384,61 +3396,79 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_poisson(TileCfg cfg,
         const float qx = (float)i, qy = (float)j;
         const uint32_t pixel = (uint32_t)pix;
         uint32_t step = 0;                            // geometric-skip steps of this pixel
-        int nd = 0;
+        // the ranges still to be thinned, the current one (from its last candidate on) in slot 0
+        int qpos[kPoissonQueue], qlast[kPoissonQueue];
+        float qU[kPoissonQueue], il1 = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kPoissonQueue; q++) { qpos[q] = qlast[q] = 0; qU[q] = 0.5f; }
+        int cnt = 0;
+        bool fresh = true;                            // il1 is not slot 0's yet
+        int nd = draws ? 0 : -1;
         int visits = 0;                               // a preorder walk visits each node at most once
+        PNode pn = pnode[0];
         while (true) {
-            if (++visits > 2 * n) { atomicOr(err, 8); break; }
-            const PNode pn = pnode[nd];
-            float cx = fminf(fmaxf(qx, pn.lox), pn.hix);
-            float cy = fminf(fmaxf(qy, pn.loy), pn.hiy);
-            const float d2b = dist2(qx, qy, cx, cy);
-            // proposal bound over the node
-            float pB = fmode ? foot_mix(k1, a1, kf, d2b, foot_bound(a1, d2b)) : mix_d2(k0, a0, k1, a1, d2b);
-            float U = fminf(1.0f, lam * pB);
-            const int last = pn.last;
-            int next = pn.esc;                        // past the subtree
-            if (pB >= kProposalPMin && U > 0.0f) {
-                const bool leaf = nd >= L0;
-                if (!leaf && (float)(last - pn.first + 1) * U > 1.0f) next = pn.left;
-                else {
-                    const float il1 = 1.0f / plog1mf(U);
-                    int pos = pn.first - 1;
-                    while (true) {
-                        // one Philox block per step, computed by every lane of the
-                        // wavefront in the same iteration: word x draws the skip,
-                        // word y the acceptance test
-                        const u32x4 blk = philox4x32_10(u32x4{ step, 0x80000000u, pixel, view }, seedLo, seedHi);
-                        step++;
-                        float u = u01(blk.x);
-                        float r = plogf(u) * il1;         // failures before the next candidate
-                        if (!(r < (float)(last - pos))) break;
-                        pos += (int)r + 1;
-                        float pl;
-                        if (fmode) {
-                            const FootLeaf L = footLeaf[pos];
-                            const float d2 = dist2(qx, qy, L.x, L.y);
-                            pl = foot_mix(k1, a1, kf, d2, foot_leaf(L, a1, qx, qy, d2));
-                        } else {
-                            const float2 lp = leafXY[pos];
-                            pl = mix_d2(k0, a0, k1, a1, dist2(qx, qy, lp.x, lp.y));
-                        }
-                        if (!(pl >= kProposalPMin)) continue;     // outside the support
-                        float pi = fminf(1.0f, lam * pl);
-                        float a = u01(blk.y);
-                        if (a * U <= pi) {            // P = pi / U, exactly 1 when pi = U
-                            if (ns < kcap) {
-                                const int32_t id = leafId[pos];
-                                const float ip = 1.0f / pi;
-                                if (ns < kPoissonStage) { sid[ns * 64 + lane] = id; sip[ns * 64 + lane] = ip; }
-                                else { oid[ns] = id; oip[ns] = ip; }
-                                ns++;
-                            } else over = true;
-                        }
+            const bool walks = nd >= 0 && cnt < kPoissonQueue, thins = cnt > 0;
+            const unsigned long long mw = __ballot(walks), mt = __ballot(thins);
+            if (!(mw | mt)) break;
+            if (__popcll(mw) >= __popcll(mt)) {
+                if (!walks) continue;
+                float cx = fminf(fmaxf(qx, pn.lox), pn.hix);
+                float cy = fminf(fmaxf(qy, pn.loy), pn.hiy);
+                const float d2b = dist2(qx, qy, cx, cy);
+                // proposal bound over the node
+                float pB = fmode ? foot_mix(k1, a1, kf, d2b, foot_bound(a1, d2b)) : mix_d2(k0, a0, k1, a1, d2b);
+                float U = fminf(1.0f, lam * pB);
+                nd = pn.left;
+                if (!(pB >= kProposalPMin && U > 0.0f)) nd = pn.esc;      // past the subtree
+                else if (nd < 0 || !((float)(pn.last - pn.first + 1) * U > 1.0f)) {
+                    nd = pn.esc;
+#pragma unroll
+                    for (int q = 0; q < kPoissonQueue; q++)
+                        if (cnt == q) { qpos[q] = pn.first - 1; qlast[q] = pn.last; qU[q] = U; }
+                    cnt++;
+                }
+                if (++visits > 2 * n) { atomicOr(err, 8); nd = -1; }
+                if (nd >= 0) pn = pnode[nd];          // on its way while others thin
+            } else if (thins) {
+                // one Philox block per step: word x draws the skip, word y the acceptance test
+                if (fresh) { il1 = 1.0f / plog1mf(qU[0]); fresh = false; }
+                const u32x4 blk = philox4x32_10(u32x4{ step, 0x80000000u, pixel, view }, seedLo, seedHi);
+                step++;
+                float u = u01(blk.x);
+                float r = plogf_normal(u) * il1;      // failures before the next candidate
+                if (!(r < (float)(qlast[0] - qpos[0]))) {
+#pragma unroll
+                    for (int q = 0; q + 1 < kPoissonQueue; q++) {
+                        qpos[q] = qpos[q + 1]; qlast[q] = qlast[q + 1]; qU[q] = qU[q + 1];
                     }
+                    cnt--;
+                    fresh = true;
+                    continue;
+                }
+                const int pos = qpos[0] + (int)r + 1;
+                qpos[0] = pos;
+                float pl;
+                if (fmode) {
+                    const FootLeaf L = footLeaf[pos];
+                    const float d2 = dist2(qx, qy, L.x, L.y);
+                    pl = foot_mix(k1, a1, kf, d2, foot_leaf(L, a1, qx, qy, d2));
+                } else {
+                    const float2 lp = leafXY[pos];
+                    pl = mix_d2(k0, a0, k1, a1, dist2(qx, qy, lp.x, lp.y));
+                }
+                float pi = fminf(1.0f, lam * pl);
+                float a = u01(blk.y);
+                // in the support, and P = pi / U, exactly 1 when pi = U
+                if (pl >= kProposalPMin && a * qU[0] <= pi) {
+                    if (ns < kcap) {
+                        const int32_t id = leafId[pos];
+                        const float ip = 1.0f / pi;
+                        if (ns < kPoissonStage) { sid[ns * 64 + lane] = id; sip[ns * 64 + lane] = ip; }
+                        else { oid[ns] = id; oip[ns] = ip; }
+                        ns++;
+                    } else over = true;
                 }
             }
-            nd = next;
-            if (nd < 0) break;
         }
     }
     // staged samples and empty slots: a row of the tile (2^lth pixels) is contiguous
