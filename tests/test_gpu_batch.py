@@ -53,6 +53,31 @@ def test_tile_shapes_bit_exact(dev, restore_tiles):
         assert np.array_equal(fmm[0].cpu().numpy(), rfmm), tag
 
 
+@pytest.mark.parametrize("N,cell,wpb", [(1, 1.0, 4), (3, 1.0, 8), (3000, 1.0, 4), (12000, 1.0, 4), (12000, 1.0, 8),
+                                        (60000, 1.0, 8), (60000, 0.25, 2), (60000, 0.0, 1)])
+def test_density_lists_of_any_length(dev, restore_tiles, N, cell, wpb):
+    """Splats far smaller than a pixel, so that the density's terms are single leaves: tiles
+    whose term lists are empty, longer than the list (put off in segments) and longer than
+    the segments hold (walked with a stack), spread over the image (cell 1), over a quarter
+    of each side, and at one point.  Bit for bit the oracle's densities."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng(N)
+    W, H, f = 40, 33, 48.0
+    z = -np.float32(2.0) - rng.uniform(size=N).astype(np.float32)
+    x = (0.5 + (rng.uniform(size=N) - 0.5) * cell) * W - W / 2
+    y = (0.5 + (rng.uniform(size=N) - 0.5) * cell) * H - H / 2
+    p = np.stack([-x * z / f, y * z / f, z], -1).astype(np.float32)
+    nb = np.tile(np.float32([0.0, 0.0, -1.0]), (N, 1))
+    sd = np.full((N, 2), 2e-4, np.float32)
+    sampling.set_tile_config("fmm_eval", 8, 8, wpb, 0)
+    dens = torch.zeros((1, 2, W, H), dtype=torch.float32, device=dev)
+    sampling.samplePoisson(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), 8, 0.0, 0.01, seed=5,
+                           rate=0.5, densities=dens)
+    rdens = O.poisson_view(W, H, f, p, nb, sd, 8, 0.5, 0.0, 0.01, seed=5)[2]
+    assert np.array_equal(dens[0].cpu().numpy(), rdens)
+    assert (rdens > 0).any()
+
+
 def test_tile_config_rejects_bad_shapes():
     from cudaExtensions import sampling
     for args in [("poisson", 8, 4, 4), ("poisson", 3, 21, 4), ("fmm_eval", 8, 8, 3), ("fmm_eval", 8, 8, 16)]:

@@ -2927,32 +2927,57 @@ __device__ __forceinline__ bool box4_meets_disc(const float* bx, float qx, float
     return d2 < rad * rad;
 }
 
-// One lane per pixel, one pixel tile per wavefront (TileCfg), bands on
+// Densities: one lane per pixel, one pixel tile per wavefront (TileCfg), bands on
 // blockIdx.y (nbands per view).
 // The reference walks each pixel with an explicit stack: pop a node; evaluate
 // it if it is a leaf or carries an expansion, else push its left child and then
 // its right child, each only if its box meets the query disc
-// (transformRadixTree.cuh:15-69).  Here the wavefront runs that walk once for
-// the union of its 64 pixels: stack entries carry the mask of lanes for which
-// the node was pushed, so each lane sees its own nodes in its own order (the
-// shared stack is its stack with other lanes' entries interleaved, in the same
-// last-in-first-out order) and sums bit for bit like the reference.  A pushed
-// entry also carries the child's centre and expansion offset from its parent's
-// FmmRec, so leaves and expansions need no node load and a descent needs one
-// wave-uniform record load.  An internal entry just below the top is handled
-// in the same step as the top entry (two record loads in flight, or a record
-// load under a leaf's or expansion's term), its children pushed in the order
-// that popping one after the other leaves, so the accumulation order is
-// unchanged.  Karras trees on 64-bit keys are at most 64 levels deep; a level
-// keeps at most two entries pending, so the stack stays within 2 * 64 + 4.
+// (transformRadixTree.cuh:15-69).  The terms of a pixel are therefore the leaves and
+// expansions whose boxes meet its disc, rightmost first (a child's box lies in its
+// parent's, and rounding keeps that order: a pixel that meets the child meets the parent).
+// A workgroup finds the terms of its tiles level by level: a list of nodes in walk order,
+// each node without a term replaced by its children that meet some pixel's disc, one
+// thread per node, so a level's record loads are in flight together.  A level that would
+// overflow the list is taken again for its first half, the rest waits in segments.  Then
+// kFmmTerms terms at a time come to LDS, each wavefront evaluates the (term, pixel) pairs
+// that meet, 64 at a time, and each pixel adds its values in order: bit for bit the
+// reference's sums.  (A term meets 9 of a tile's 64 pixels in the narrow band, 28 to 49 in
+// the wide one: a lane per pixel left most lanes idle.)
+// Bound by the latency of the levels' and terms' loads (62 % miss L2 in the larger case),
+// then by instruction issue.  Both bands of 512x512 under 1M splats 676 -> 490 us against
+// one wavefront's walk with a stack; 16 views of 640x480 under 2M splats 3.53 -> 3.24 ms.
+// Lists of 2048 take 555 us and 4.03 ms, two wavefronts per workgroup 554 us and 4.63 ms,
+// 32 terms at a time 672 us and 3.12 ms, one lane per pixel over its own terms 1023 us and
+// 3.34 ms.
+constexpr int kFmmTerms = 64, kFmmList = 1024, kFmmPairs = 384, kFmmSegments = 16;
+
+// each active lane's word goes to LDS at the wavefront's base plus its lane's word
+__device__ __forceinline__ void load_to_lds(const float UD_GLOBAL* from, float* base)
+{
+    __builtin_amdgcn_global_load_lds((const void UD_GLOBAL*)from, (void __attribute__((address_space(3)))*)(base), 4, 0, 0);
+}
+// those loads have arrived (a barrier alone does not wait for them)
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long m)
+{
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32 |
+           (unsigned)__builtin_amdgcn_readfirstlane((int)m);
+}
+
+// bits of m below this lane's
+__device__ __forceinline__ int wave_rank(unsigned long long m)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+}
+
 // A fixed-order expansion at scaled offset t = (q - c) / sqrt(2 h^2):
 // sum_a h_a(tx) sum_b C_ab h_b(ty), Hermite functions by their three-term
-// recurrence, every product-sum one fused multiply-add (the oracle uses fmaf in
-// the same order).
+// recurrence from ex = e^{-tx^2}, ey = e^{-ty^2}, every product-sum one fused multiply-add
+// (the oracle uses fmaf in the same order).
 template <int P>
-__device__ __forceinline__ float fixed_series(const float* co, float tx, float ty)
+__device__ __forceinline__ float fixed_series(const float4* co, float tx, float ty, float ex, float ey)
 {
-    const float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
     float hx[P + 1], hy[P + 1];
     hx[0] = ex; hy[0] = ey;
     hx[1] = (2.0f * tx) * ex; hy[1] = (2.0f * ty) * ey;
@@ -2961,15 +2986,142 @@ __device__ __forceinline__ float fixed_series(const float* co, float tx, float t
         hx[q] = __builtin_fmaf(2.0f * tx, hx[q - 1], -((2.0f * (float)(q - 1)) * hx[q - 2]));
         hy[q] = __builtin_fmaf(2.0f * ty, hy[q - 1], -((2.0f * (float)(q - 1)) * hy[q - 2]));
     }
-    float val = 0.0f;
+    float val = 0.0f, sa = 0.0f;
 #pragma unroll
+    for (int q4 = 0; q4 < ((P + 1) * (P + 1) + 3) / 4; q4++) {
+        const float4 c4 = co[q4];
+        const float c[4] = { c4.x, c4.y, c4.z, c4.w };
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int q = 4 * q4 + e, a = q / (P + 1), b = q - a * (P + 1);
+            if (a > P) break;
+            sa = __builtin_fmaf(c[e], hy[b], b == 0 ? 0.0f : sa);
+            if (b == P) val = __builtin_fmaf(hx[a], sa, val);
+        }
+    }
+    return val;
+}
+
+// the same a row at a time from memory (few registers)
+template <int P>
+__device__ __forceinline__ float fixed_series_rows(const float UD_GLOBAL* co, float tx, float ty)
+{
+    const float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
+    float hy[P + 1];
+    hy[0] = ey;
+    hy[1] = (2.0f * ty) * ey;
+#pragma unroll
+    for (int q = 2; q <= P; q++) hy[q] = __builtin_fmaf(2.0f * ty, hy[q - 1], -((2.0f * (float)(q - 1)) * hy[q - 2]));
+    float val = 0.0f, h = ex, hm = 0.0f;
+#pragma unroll 1
     for (int a = 0; a <= P; a++) {
         float sa = 0.0f;
 #pragma unroll
         for (int b = 0; b <= P; b++) sa = __builtin_fmaf(co[a * (P + 1) + b], hy[b], sa);
-        val = __builtin_fmaf(hx[a], sa, val);
+        val = __builtin_fmaf(h, sa, val);
+        const float hn = a == 0 ? (2.0f * tx) * ex : __builtin_fmaf(2.0f * tx, h, -((2.0f * (float)a) * hm));
+        hm = h;
+        h = hn;
     }
     return val;
+}
+
+// words of an expansion's block in LDS: whole float4 words, an odd number of them, so
+// that lanes reading different blocks meet different banks
+constexpr int fmm_block(int p)
+{
+    const int q = ((p + 1) * (p + 1) + 3) / 4;
+    return 4 * (q | 1);
+}
+// LDS bytes of a workgroup of wpb wavefronts: the terms' blocks, boxes, centres, block
+// offsets and each wavefront's masks of them, two lists of nodes and the segments put
+// off; or the serial walk's stacks.  The list that is free while terms are added holds
+// the wavefronts' pairs.
+constexpr size_t fmm_lds(int p, int wpb)
+{
+    const size_t lists = (size_t)kFmmTerms * (4 * fmm_block(p) + 28 + 8 * wpb) + 3 * kFmmList * 4 +
+                         (size_t)kFmmPairs * 6 * wpb;
+    const size_t stacks = (size_t)kFmmStack * 24 * wpb;
+    return lists > stacks ? lists : stacks;
+}
+
+// |q - closest point of [lo, hi]| for the closest whole q in [a, b]
+__device__ __forceinline__ float pixel_gap(float lo, float hi, float a, float b)
+{
+    const float p = fminf(fmaxf(ceilf(lo), a), b), q = fminf(fmaxf(floorf(hi), a), b);
+    const float dp = p - fminf(fmaxf(p, lo), hi), dq = q - fminf(fmaxf(q, lo), hi);
+    return fminf(fabsf(dp), fabsf(dq));
+}
+
+// some pixel of the tile (x, y the first and last i, z, w of j) meets the box within rad
+__device__ __forceinline__ bool box4_meets_tile(const float4& bx, const float4& tile, float rad)
+{
+    const float dx = pixel_gap(bx.x, bx.z, tile.x, tile.y), dy = pixel_gap(bx.y, bx.w, tile.z, tile.w);
+    float d2 = 0.0f;
+    d2 = d2 + dx * dx;
+    d2 = d2 + dy * dy;
+    return d2 < rad * rad;
+}
+
+// The walk of one tile with an explicit stack, for tiles whose lists run over: the
+// wavefront runs it once for the union of its 64 pixels, each entry with the mask of the
+// lanes it was pushed for, so each lane sees its own nodes in its own order.  Karras trees
+// on 64-bit keys are at most 64 levels deep; a level keeps at most two entries pending, so
+// the stack stays within 2 * 64 + 4.
+template <int P>
+__device__ float fmm_serial(unsigned char* lds, int lane, bool valid, float qx, float qy, const Band& B, int L0, int b,
+                            const NodeGeo* geo, const FmmRec* frec, const int* fixOff, const float UD_GLOBAL* cf)
+{
+    unsigned long long* sM = (unsigned long long*)lds;
+    float2* sC = (float2*)(sM + kFmmStack);
+    int* sN = (int*)(sC + kFmmStack);
+    int* sF = sN + kFmmStack;
+    float w = 0.0f;
+    const unsigned long long all = __ballot(valid);
+    if (lane == 0) {
+        sN[0] = 0;
+        sF[0] = L0 > 0 ? fixOff[0] : -1;
+        sC[0] = make_float2(geo[0].cx, geo[0].cy);
+        sM[0] = all;
+    }
+    int sp = 1;
+    while (sp > 0) {
+        sp--;
+        wave_lds_fence();
+        const int nd = __builtin_amdgcn_readfirstlane(sN[sp]);
+        const int off = __builtin_amdgcn_readfirstlane(sF[sp]);
+        const float2 c = sC[sp];
+        const unsigned long long mask = sM[sp];
+        wave_lds_fence();
+        const bool act = (mask >> lane) & 1ull;
+        if (nd >= L0) {
+            if (act) w = w + band_point(B, qx, qy, c.x, c.y);
+            continue;
+        }
+        if (off >= 0) {
+            if (act) w = w + fixed_series_rows<P>(cf + off, (qx - c.x) * B.is2h, (qy - c.y) * B.is2h);
+            continue;
+        }
+        const FmmRec r = frec[nd];
+        const unsigned long long ml = __ballot(act && box4_meets_disc(r.lbox, qx, qy, B.radius));
+        const unsigned long long mr = __ballot(act && box4_meets_disc(r.rbox, qx, qy, B.radius));
+        if (sp + 2 > kFmmStack) break;                       // unreachable for trees of depth <= 64
+        if (ml) {
+            if (lane == 0) {
+                sN[sp] = r.left; sF[sp] = b ? r.lfix[1] : r.lfix[0];
+                sC[sp] = make_float2(r.lc[0], r.lc[1]); sM[sp] = ml;
+            }
+            sp++;
+        }
+        if (mr) {
+            if (lane == 0) {
+                sN[sp] = r.right; sF[sp] = b ? r.rfix[1] : r.rfix[0];
+                sC[sp] = make_float2(r.rc[0], r.rc[1]); sM[sp] = mr;
+            }
+            sp++;
+        }
+    }
+    return w;
 }
 
 template <int P>
@@ -2983,14 +3135,23 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
                                                                     float* __restrict__ out, size_t outStride,
                                                                     size_t bandStride)
 {
-    __shared__ int stkN[kMaxWavesPerBlock][kFmmStack];
-    __shared__ int stkF[kMaxWavesPerBlock][kFmmStack];
-    __shared__ float2 stkC[kMaxWavesPerBlock][kFmmStack];
-    __shared__ unsigned long long stkM[kMaxWavesPerBlock][kFmmStack];
-    const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
-    int i, j;
-    if (!tile_lane(cfg, W, H, lane, i, j)) return;           // wave-uniform
+    constexpr int NC = (P + 1) * (P + 1), BLK = fmm_block(P), T = kFmmTerms;
+    extern __shared__ __align__(16) unsigned char fmmLds[];
+    float* tB = (float*)fmmLds;                              // [T][BLK]
+    float4* tBox = (float4*)(tB + T * BLK);
+    float2* tC = (float2*)(tBox + T);
+    unsigned long long* tMask = (unsigned long long*)(tC + T);   // [wpb][T]
+    int* tOff = (int*)(tMask + T * cfg.wpb);                 // -1: a leaf
+    int* list = tOff + T;                                    // three of kFmmList
+    __shared__ float4 area[kMaxWavesPerBlock];               // the tiles, joined down a column
+    __shared__ int areas;
+    __shared__ int total[2][kMaxWavesPerBlock];
+    __shared__ int seg[kFmmSegments];
+    const int tid = threadIdx.x, lane = tid & 63, wpb = cfg.wpb;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int i = W, j = H;
+    const bool has = tile_lane(cfg, W, H, lane, i, j);       // wave-uniform
+    const bool valid = has && i < W && j < H;
     const int b = (int)blockIdx.y % nbands;                  // band
     const size_t v = blockIdx.y / nbands;                    // view
     vs = (const ViewState*)((const char*)vs + v * vstride);
@@ -2999,7 +3160,6 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
     const int* fixOff = (const int*)((const char*)(b ? fixOff1 : fixOff0) + v * vstride);
     const float* coef = (const float*)((const char*)(b ? coef1 : coef0) + v * vstride);
     out = (float*)((char*)out + v * outStride + (size_t)b * bandStride);
-    const bool valid = i < W && j < H;
     const int n = vs->nc;
     float w = 0.0f;
     if (n > 0) {
@@ -3007,97 +3167,195 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
         const Band B = vs->band[b];
         const int L0 = n - 1;
         const float qx = (float)i, qy = (float)j;
-        int* sN = stkN[wid];
-        int* sF = stkF[wid];
-        float2* sC = stkC[wid];
-        unsigned long long* sM = stkM[wid];
-        const unsigned long long all = __ballot(valid);
-        if (lane == 0) {
-            sN[0] = 0;
-            sF[0] = L0 > 0 ? fixOff[0] : -1;
-            sC[0] = make_float2(geo[0].cx, geo[0].cy);
-            sM[0] = all;
+        const int i0 = __builtin_amdgcn_readfirstlane(i), j0 = __builtin_amdgcn_readfirstlane(j);
+        const int i1 = min(i0 + cfg.tw, W) - 1, j1 = min(j0 + (1 << cfg.lth), H) - 1;
+        const float4 own = make_float4((float)i0, (float)i1, (float)j0, (float)j1);   // if has
+        if (lane == 0) total[0][wid] = has ? 1 : 0;
+        if (lane == 0) area[wid] = own;
+        __syncthreads();
+        if (tid == 0) {
+            int m = 0;                                       // the wavefronts with a tile come first
+            for (int q = 0; q < wpb && total[0][q]; q++) {
+                const float4 t = area[q];
+                if (m > 0 && area[m - 1].x == t.x) area[m - 1].w = t.w;
+                else area[m++] = t;
+            }
+            areas = m;
         }
-        int sp = 1;
-        while (sp > 0) {
-            sp--;
-            __builtin_amdgcn_wave_barrier();
-            const int nd = __builtin_amdgcn_readfirstlane(sN[sp]);
-            const int off = __builtin_amdgcn_readfirstlane(sF[sp]);
-            const int sp2 = sp > 0 ? sp - 1 : 0;
-            const int nd2 = __builtin_amdgcn_readfirstlane(sN[sp2]);
-            const int off2 = __builtin_amdgcn_readfirstlane(sF[sp2]);
-            const float2 c = sC[sp];
-            const unsigned long long mask = sM[sp];
-            const unsigned long long mask2 = sM[sp2];
-            __builtin_amdgcn_wave_barrier();
-            const bool act = (mask >> lane) & 1ull;
-            // the term of a leaf or an expansion on top of the stack
-            auto add_top = [&]() {
-                if (nd >= L0) {
-                    if (act) w = w + band_point(B, qx, qy, c.x, c.y);
+        // entries: a node to be replaced by its children, or ~(2 parent + side) of a term
+        const int rootOff = L0 > 0 ? fixOff[0] : -1;
+        const bool rootTerm = L0 == 0 || rootOff >= 0;
+        int* A = list;
+        int* O = list + kFmmList;
+        int* S = list + 2 * kFmmList;
+        float* val = (float*)(list + 3 * kFmmList) + kFmmPairs * wid;        // this wavefront's pairs
+        uint16_t* pair = (uint16_t*)((float*)(list + 3 * kFmmList) + kFmmPairs * wpb) + kFmmPairs * wid;
+        if (tid == 0) A[0] = 0;
+        int F = 1, put = 0, segs = 0;                        // entries, entries and segments put off
+        bool more = !rootTerm, serial = false;
+        int turn = 1;
+        __syncthreads();
+        while (true) {
+            while (more) {
+                more = false;
+                int kept = 0;
+                for (int c0 = 0; c0 < F; c0 += 64 * wpb) {
+                    const int at = c0 + tid;
+                    const int e = at < F ? A[at] : -1;
+                    bool f1 = at < F, f2 = false;
+                    int o1 = e, o2 = 0;
+                    if (at < F && e >= 0) {
+                        const FmmRec UD_GLOBAL* r = (const FmmRec UD_GLOBAL*)(frec + e);
+                        const float4 lb = make_float4(r->lbox[0], r->lbox[1], r->lbox[2], r->lbox[3]);
+                        const float4 rb = make_float4(r->rbox[0], r->rbox[1], r->rbox[2], r->rbox[3]);
+                        const int cl = r->left, cr = r->right, fl = r->lfix[b], fr = r->rfix[b];
+                        f1 = false;
+                        for (int t = 0; t < areas; t++) {
+                            f1 |= box4_meets_tile(rb, area[t], B.radius);
+                            f2 |= box4_meets_tile(lb, area[t], B.radius);
+                        }
+                        o1 = cr >= L0 || fr >= 0 ? ~(2 * e + 1) : cr;
+                        o2 = cl >= L0 || fl >= 0 ? ~(2 * e) : cl;
+                    }
+                    const unsigned long long m1 = __ballot(f1), m2 = __ballot(f2);
+                    const int inner = __ballot((f1 && o1 >= 0) || (f2 && o2 >= 0)) ? 1 << 16 : 0;
+                    if (lane == 0) total[turn][wid] = (__popcll(m1) + __popcll(m2)) | inner;
+                    __syncthreads();
+                    int base = kept;
+                    for (int q = 0; q < wpb; q++) {
+                        const int x = total[turn][q];
+                        more |= (x >> 16) != 0;
+                        if (q < wid) base += x & 0xffff;
+                        kept += x & 0xffff;
+                    }
+                    turn ^= 1;
+                    if (kept > kFmmList) break;              // nothing of this chunk is written
+                    const int p = base + wave_rank(m1) + wave_rank(m2);
+                    if (f1) O[p] = o1;
+                    if (f2) O[p + (f1 ? 1 : 0)] = o2;
+                }
+                if (kept > kFmmList) {
+                    // put the later half of this level's list off and take the level again
+                    const int half = F / 2;
+                    if (put + F - half > kFmmList || segs == kFmmSegments) { serial = true; break; }
+                    for (int t = tid; t < F - half; t += 64 * wpb) S[put + t] = A[half + t];
+                    if (tid == 0) seg[segs] = F - half;
+                    put += F - half;
+                    segs++;
+                    F = half;
+                    more = true;
                 } else {
-                    // wave-uniform block, fetched by broadcast vector loads issued
-                    // together (faster here than scalar loads or staging in LDS)
-                    float co[(P + 1) * (P + 1)];
-                    const float UD_GLOBAL* cc = cf + off;
+                    F = kept;
+                    int* t = A; A = O; O = t;
+                }
+                __syncthreads();
+            }
+            if (serial) break;
+            for (int t0 = 0; t0 < F; t0 += T) {
+                const int nt = min(T, F - t0);
+                for (int t = tid; t < nt; t += 64 * wpb) {
+                    if (rootTerm) {
+                        tC[0] = make_float2(geo[0].cx, geo[0].cy);
+                        tOff[0] = rootOff;
+                        tBox[0] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    } else {
+                        const int e = ~A[t0 + t];
+                        const FmmRec UD_GLOBAL* r = (const FmmRec UD_GLOBAL*)(frec + (e >> 1));
+                        const float UD_GLOBAL* bx = e & 1 ? r->rbox : r->lbox;
+                        const float UD_GLOBAL* cc = e & 1 ? r->rc : r->lc;
+                        tBox[t] = make_float4(bx[0], bx[1], bx[2], bx[3]);
+                        tC[t] = make_float2(cc[0], cc[1]);
+                        tOff[t] = (e & 1 ? r->right : r->left) >= L0 ? -1 : (e & 1 ? r->rfix[b] : r->lfix[b]);
+                    }
+                }
+                __syncthreads();
+                // the blocks, a wavefront per term, straight to LDS
+                for (int t = wid; t < nt; t += wpb) {
+                    const int off = __builtin_amdgcn_readfirstlane(tOff[t]);
+                    if (off < 0) continue;
 #pragma unroll
-                    for (int q = 0; q < (P + 1) * (P + 1); q++) co[q] = cc[q];
-                    if (act) w = w + fixed_series<P>(co, (qx - c.x) * B.is2h, (qy - c.y) * B.is2h);
+                    for (int q = 0; q < NC; q += 64)
+                        if (lane + q < NC) load_to_lds(cf + off + q + lane, tB + t * BLK + q);
                 }
-            };
-            // An internal entry without an expansion just below the top is taken
-            // along: its record loads with the top's record (two internal entries)
-            // or while the top's term is evaluated (a leaf or expansion on top,
-            // whose term is added first).  The lower entry's children are pushed
-            // below the upper entry's: the stack a pop of each in turn leaves.
-            const bool topInt = nd < L0 && off < 0;
-            const bool lowInt = sp > 0 && nd2 < L0 && off2 < 0;
-            if (!topInt && !lowInt) {
-                add_top();
-                continue;
-            }
-            if (lowInt) sp--;
-            const bool two = topInt && lowInt;
-            const int ndA = topInt ? nd : nd2;               // the upper internal entry
-            const FmmRec r = frec[ndA];
-            const FmmRec r2 = frec[two ? nd2 : ndA];
-            if (!topInt) add_top();
-            const bool actA = topInt ? act : (bool)((mask2 >> lane) & 1ull);
-            const bool act2 = two && ((mask2 >> lane) & 1ull);
-            const unsigned long long ml = __ballot(actA && box4_meets_disc(r.lbox, qx, qy, B.radius));
-            const unsigned long long mr = __ballot(actA && box4_meets_disc(r.rbox, qx, qy, B.radius));
-            const unsigned long long ml2 = __ballot(act2 && box4_meets_disc(r2.lbox, qx, qy, B.radius));
-            const unsigned long long mr2 = __ballot(act2 && box4_meets_disc(r2.rbox, qx, qy, B.radius));
-            if (sp + 4 > kFmmStack) break;                   // unreachable for trees of depth <= 64
-            if (ml2) {
-                if (lane == 0) {
-                    sN[sp] = r2.left; sF[sp] = b ? r2.lfix[1] : r2.lfix[0];
-                    sC[sp] = make_float2(r2.lc[0], r2.lc[1]); sM[sp] = ml2;
+                wait_loads();
+                // the terms that some pixel of this tile meets
+                unsigned long long todo =
+                    __ballot(has && lane < nt && (rootTerm || box4_meets_tile(tBox[lane], own, B.radius)));
+                __syncthreads();
+                while (todo) {
+                    // (term, pixel) pairs of the next terms, as many as there is room for
+                    int pairs = 0, nm = 0;
+                    while (todo && pairs <= kFmmPairs - 256) {
+                        // four terms at a time, their box reads in flight together
+                        unsigned long long m[4];
+                        int t[4];
+                        bool mine[4];
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+                            t[u] = todo ? __builtin_amdgcn_readfirstlane(__ffsll(todo) - 1) : -1;
+                            todo &= todo - 1ull;
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+                            const float4 bx = tBox[t[u] < 0 ? 0 : t[u]];
+                            const float q[4] = { bx.x, bx.y, bx.z, bx.w };
+                            mine[u] = t[u] >= 0 && valid && (rootTerm || box4_meets_disc(q, qx, qy, B.radius));
+                            m[u] = __ballot(mine[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+                            if (!m[u]) continue;
+                            if (mine[u]) pair[pairs + wave_rank(m[u])] = (uint16_t)(t[u] << 6 | lane);
+                            if (lane == 0) tMask[wid * T + nm] = m[u];
+                            pairs += __popcll(m[u]);
+                            nm++;
+                        }
+                    }
+                    wave_lds_fence();
+                    for (int k0 = 0; k0 < pairs; k0 += 64) {
+                        const int k = k0 + lane;
+                        if (k < pairs) {
+                            const int e = pair[k], t = e >> 6, px = e & 63;
+                            const float2 c = tC[t];
+                            const float x = (float)(i0 + (px >> cfg.lth)), y = (float)(j0 + (px & ((1 << cfg.lth) - 1)));
+                            const float tx = (x - c.x) * B.is2h, ty = (y - c.y) * B.is2h;
+                            const float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
+                            if (tOff[t] < 0) val[k] = 0.0f + (B.c * ex) * ey;       // band_point
+                            else val[k] = fixed_series<P>((const float4*)(tB + t * BLK), tx, ty, ex, ey);
+                        }
+                    }
+                    wave_lds_fence();
+                    // each pixel adds its terms in order
+                    for (int k0 = 0, at = 0; k0 < nm; k0 += 4) {
+                        float x[4];
+                        unsigned long long m[4];
+#pragma unroll
+                        for (int u = 0; u < 4; u++) m[u] = k0 + u < nm ? tMask[wid * T + k0 + u] : 0ull;
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+                            m[u] = uniform64(m[u]);
+                            x[u] = (m[u] >> lane) & 1ull ? val[at + wave_rank(m[u])] : 0.0f;
+                            at += __popcll(m[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; u++)
+                            if ((m[u] >> lane) & 1ull) w = w + x[u];
+                    }
+                    wave_lds_fence();
                 }
-                sp++;
+                __syncthreads();
             }
-            if (mr2) {
-                if (lane == 0) {
-                    sN[sp] = r2.right; sF[sp] = b ? r2.rfix[1] : r2.rfix[0];
-                    sC[sp] = make_float2(r2.rc[0], r2.rc[1]); sM[sp] = mr2;
-                }
-                sp++;
-            }
-            if (ml) {
-                if (lane == 0) {
-                    sN[sp] = r.left; sF[sp] = b ? r.lfix[1] : r.lfix[0];
-                    sC[sp] = make_float2(r.lc[0], r.lc[1]); sM[sp] = ml;
-                }
-                sp++;
-            }
-            if (mr) {
-                if (lane == 0) {
-                    sN[sp] = r.right; sF[sp] = b ? r.rfix[1] : r.rfix[0];
-                    sC[sp] = make_float2(r.rc[0], r.rc[1]); sM[sp] = mr;
-                }
-                sp++;
-            }
+            if (segs == 0) break;
+            segs--;
+            F = seg[segs];
+            put -= F;
+            for (int t = tid; t < F; t += 64 * wpb) A[t] = S[put + t];
+            more = true;
+            __syncthreads();
+        }
+        if (serial) {
+            __syncthreads();
+            w = fmm_serial<P>(fmmLds + (size_t)wid * (kFmmStack * 24), lane, valid, qx, qy, B, L0, b, geo, frec, fixOff, cf);
         }
     }
     if (valid) out[(long)j + (long)H * i] = w;
@@ -3808,7 +4066,7 @@ void fmm_eval(int W, int H, int views, int nbands, int p, const TreeWs& w, size_
     if (timed) (void)hipEventRecord(e0, st);
     const dim3 grid = tile_grid(c, W, H, views * nbands);
     switch (p) {
-#define UD_EVAL(P) case P: k_fmm_eval<P><<<grid, 64 * c.wpb, 0, st>>>(                                             \
+#define UD_EVAL(P) case P: k_fmm_eval<P><<<grid, 64 * c.wpb, fmm_lds(P, c.wpb), st>>>(                             \
         c, W, H, w.vs, vstride, nbands, w.geo, w.frec, w.fixOff[0], nbands > 1 ? w.fixOff[1] : nullptr,            \
         w.fixCoef[0], nbands > 1 ? w.fixCoef[1] : nullptr, out, outStride, bandStride); break;
     UD_EVAL(4) UD_EVAL(5) UD_EVAL(6) UD_EVAL(7) UD_EVAL(8)
