@@ -38,7 +38,8 @@ typedef struct ihipStream_t* ude_stream_t;
 
 /* ---- sampling ---------------------------------------------------------- */
 
-/* Workspace for ude_sample (one view's tree, reused across views). */
+/* Workspace for ude_sample (one view's tree, reused across views; v times as much lets v
+ * views run in each launch). */
 size_t ude_sample_workspace_bytes(int N, int W, int H, int k);
 
 /* sampling.sample -- replaces cudaSample / batchSample

@@ -185,3 +185,31 @@ def test_sample_walk_beyond_the_tile_lists(dev, W, H, precision, k):
     ref = O.sample_view(W, H, f, p, nb, sd, k, 0.0, precision, seed=k)
     assert (ref >= 0).mean() > 0.5
     assert np.array_equal(got[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("perViewSd", [False, True])
+def test_sample_views_in_groups(dev, monkeypatch, perViewSd):
+    """Five views with different counts of visible splats (one sees none): in one group, in
+    groups of two with a last one of one, one by one, and where the memory for a group is
+    not there: the same indices bit for bit (the batch above is equal to the oracle's)."""
+    from cudaExtensions import _lib, sampling
+    sc, p, n, nb, sd = scene_inputs(2, sd_scale=8.0)
+    W, H, f = 52, 36, sc.focal * 52 / sc.width
+    shift = np.float32([[0, 0, 0], [1.5, 0, 0], [0, 0, 2000.0], [0, -2.0, 0], [0, 0, -3.0]])
+    P = t(np.stack([p + s for s in shift]), dev)
+    NB = t(np.stack([nb] * 5), dev)
+    SD = t(np.stack([sd * (1 + 0.2 * b) for b in range(5)]) if perViewSd else sd[None], dev)
+    run = lambda: sampling.sample(W, H, f, P, NB, None, SD, 16, 0.0, 0.01, seed=9).cpu().numpy()  # noqa: E731
+    ref = run()
+    for views in (1, 2, 5):
+        monkeypatch.setattr(sampling, "_views_at_once", lambda *a, v=views: v)
+        assert np.array_equal(run(), ref), views
+    full = _lib.workspace
+
+    def small(nbytes, device):
+        if nbytes > _lib.lib().ude_sample_workspace_bytes(P.shape[1], W, H, 16):
+            raise torch.OutOfMemoryError("not for several trees")
+        return full(nbytes, device)
+    monkeypatch.setattr(_lib, "workspace", small)
+    assert np.array_equal(run(), ref)
+    assert (ref[0] >= 0).any() and (ref[2] == -1).all()

@@ -60,7 +60,6 @@ constexpr int kSortTile = 2048;      // elements per workgroup in a sort pass
 constexpr int kFixedDegree = 6;      // default expansion order of the fixed-order densities (hermitefmm.cuh:11)
 constexpr int kFixedPMin = 4, kFixedPMax = 8;              // orders ude_set_fixed_degree accepts
 constexpr int kFixedCoefsMax = (kFixedPMax + 1) * (kFixedPMax + 1);
-constexpr int kScanTile = 1024;      // elements per workgroup in a scan pass
 
 // Gaussian bandwidth of a fixed-order density: h, 1 / sqrt(2 h^2), the leaf
 // coefficient 1 / (2 pi sqrt(h)) and the query radius
@@ -73,8 +72,8 @@ struct ViewState {
     unsigned int hcnt;
     int nc;
     float h, radius, lo, hix, hiy, s2h, prec, is2h;
-    int err;
-    int ncoef;
+    int ncoef;        // coefficients of the internal nodes' blocks
+    int spare;
     int nseeds;       // block-spanning fan-in starts (bottom-up, second level)
     int nmom;         // internal nodes with a Hermite expansion
     int pad;
@@ -141,7 +140,7 @@ struct TreeWs {
     ViewState* vs;
     uint32_t *keysA, *keysB;
     int32_t *idsA, *idsB;
-    int *cullCounts, *sortHist, *scanTmp, *scanBlocks;
+    int *cullCounts, *sortHist, *scanBlocks;
     NodeGeo* geo;
     NodeLnk* lnk;
     NodeAux* aux;
@@ -156,7 +155,6 @@ struct TreeWs {
     int* tieQueue;                    // [0]: count, then (sampler lane, final key bits) per lane that met equal keys
     float2* leafXY;       // sorted position -> screen position of the leaf
     float* coef;
-    long coefCap;
     // fixed-order densities (approximateFMMWeights, Poisson-rate sampling)
     int* fixOff[2];       // per internal node and band: coefficient offset, -1 = no expansion
     int* fixList[2];      // per band: accepted internal nodes
@@ -185,7 +183,6 @@ size_t carve(void* ws, int N, int W, int H, int k, int mode, TreeWs* t)
     long nn = 2 * n;
     long nCull = (n + kCullTile - 1) / kCullTile;
     long nSort = (n + kSortTile - 1) / kSortTile;
-    long nScan = (nn + kScanTile - 1) / kScanTile;
     const bool fixedOrder = mode != kModeSample;
     long coefCap = (long)(kMaxDegree + 1) * (kMaxDegree + 1) * (n - 1 > 0 ? n - 1 : 1) + n;
     size_t off = 0;
@@ -199,8 +196,7 @@ size_t carve(void* ws, int N, int W, int H, int k, int mode, TreeWs* t)
     w.idsB = (int32_t*)take(4 * n);
     w.cullCounts = (int*)take(4 * (nCull + 1));
     w.sortHist = (int*)take(4 * 256 * (nSort + 1));
-    w.scanTmp = (int*)take(4 * nn);
-    w.scanBlocks = (int*)take(4 * (nScan + 1) > 4 * (256 * (nSort + 1)) ? 4 * (nScan + 1) : 4 * 256 * (nSort + 1));
+    w.scanBlocks = (int*)take(4 * 256 * (nSort + 1));
     w.geo = (NodeGeo*)take(sizeof(NodeGeo) * nn);
     w.lnk = (NodeLnk*)take(sizeof(NodeLnk) * nn);
     w.aux = (NodeAux*)take(sizeof(NodeAux) * nn);
@@ -216,7 +212,6 @@ size_t carve(void* ws, int N, int W, int H, int k, int mode, TreeWs* t)
     w.tieQueue = fixedOrder ? nullptr : (int*)take(4 * (2 * lanes + 1));
     w.leafXY = (float2*)take(8 * n);
     w.coef = fixedOrder ? nullptr : (float*)take(4 * coefCap);
-    w.coefCap = fixedOrder ? 0 : coefCap;
     w.hraw = nullptr;
     w.pnode = nullptr;
     w.footLeaf = nullptr;
@@ -387,7 +382,7 @@ __global__ void k_zero_state(ViewState* vs, VStride vsd)
 {
     vs = vw(vs, vsd.ws);
     if (threadIdx.x == 0) {
-        vs->hsum = 0; vs->hcnt = 0; vs->nc = 0; vs->err = 0; vs->ncoef = 0; vs->nseeds = 0; vs->nmom = 0;
+        vs->hsum = 0; vs->hcnt = 0; vs->nc = 0; vs->ncoef = 0; vs->nseeds = 0; vs->nmom = 0;
         vs->nfix[0] = 0; vs->nfix[1] = 0;
     }
     for (int b = threadIdx.x; b < 256; b += blockDim.x) vs->hhist[b] = 0;
@@ -998,19 +993,27 @@ __global__ __launch_bounds__(256) void k_bottom_up_global(const ViewState* __res
     }
 }
 
-// Coefficient block sizes.  FGT walks start at the root and at the children of
+// Coefficient blocks.  FGT walks start at the root and at the children of
 // nodes with more than k sources (the capacity descent asks for their weights);
 // a walk stops at the first node with an expansion.  An internal node below an
 // expanded node, with no start in between, is therefore never evaluated and
-// gets no block.
-__global__ __launch_bounds__(256) void k_coef_sizes(ViewState* vs, const NodeGeo* __restrict__ geo,
-                                                    const NodeLnk* __restrict__ lnk, int k, int* sizes, int* momList)
+// gets no block.  The leaves' single coefficients lie first, in leaf order; a workgroup
+// reserves its nodes' blocks behind them with one atomic (where a block lies changes no
+// value), which takes the place of a scan over all nodes in three launches.
+__global__ __launch_bounds__(256) void k_coef_blocks(ViewState* vs, const NodeGeo* __restrict__ geo,
+                                                     const NodeLnk* __restrict__ lnk, NodeAux* __restrict__ aux, int k,
+                                                     int* momList, VStride vsd)
 {
-    int n = vs->nc;
-    int nn = 2 * n - 1;
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int d = t < nn ? geo[t].deg : -1;
-    if (d >= 0 && t < n - 1) {
+    vs = vw(vs, vsd.ws);
+    geo = vw(geo, vsd.ws);
+    lnk = vw(lnk, vsd.ws);
+    aux = vw(aux, vsd.ws);
+    momList = vw(momList, vsd.ws);
+    const int n = vs->nc;
+    const int nn = 2 * n - 1;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    int d = t < n - 1 ? geo[t].deg : -1;
+    if (d >= 0) {
         int x = t;
         while (true) {
             const int p = lnk[x].parent;
@@ -1019,60 +1022,54 @@ __global__ __launch_bounds__(256) void k_coef_sizes(ViewState* vs, const NodeGeo
             x = p;
         }
     }
-    if (t < nn) sizes[t] = d >= 0 ? (d + 1) * (d + 1) : 0;
     // list the internal nodes that need moments: one slot reservation per workgroup
-    __shared__ int wcnt[4];
-    __shared__ int bbase;
-    const bool want = d >= 0 && t < n - 1;
+    __shared__ int wcnt[4], sh[4];
+    __shared__ int bbase, cbase;
+    const bool want = d >= 0;
     const unsigned long long m = __ballot(want);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) wcnt[wid] = __popcll(m);
-    __syncthreads();
+    int coefs;
+    const int at = block_excl_scan(want ? (d + 1) * (d + 1) : 0, sh, coefs);
     if (threadIdx.x == 0) {
         const int tot = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
         bbase = tot ? atomicAdd(&vs->nmom, tot) : 0;
+        cbase = tot ? atomicAdd(&vs->ncoef, coefs) : 0;
     }
     __syncthreads();
     int base = bbase;
     for (int q = 0; q < wid; q++) base += wcnt[q];
     if (want) momList[base + __popcll(m & ((1ull << lane) - 1ull))] = t;
+    if (t < nn) aux[t].off = t >= n - 1 ? t - (n - 1) : want ? n + cbase + at : 0;
 }
 
-// device-wide exclusive scan, phase 1: per-tile scan + tile totals
-__global__ __launch_bounds__(256) void k_scan_tiles(const ViewState* __restrict__ vs, int* data, int* tileSums)
+// Children records of the sampler's walk, one per internal node (after the tree's
+// degrees and coefficient offsets are final).
+__device__ __forceinline__ SampChild samp_child(int c, const NodeGeo* __restrict__ geo,
+                                                const NodeLnk* __restrict__ lnk, const NodeAux* __restrict__ aux)
 {
-    __shared__ int sh[4];
-    int nn = 2 * vs->nc - 1;
-    int base = blockIdx.x * kScanTile;
-    if (base >= nn) { if (threadIdx.x == 0) tileSums[blockIdx.x] = 0; return; }
-    int v[4], s = 0;
-    for (int q = 0; q < 4; q++) {
-        int e = base + 4 * threadIdx.x + q;
-        v[q] = e < nn ? data[e] : 0;
-        s += v[q];
-    }
-    int total;
-    int ex = block_excl_scan(s, sh, total);
-    for (int q = 0; q < 4; q++) {
-        int e = base + 4 * threadIdx.x + q;
-        if (e < nn) data[e] = ex;
-        ex += v[q];
-    }
-    if (threadIdx.x == 0) tileSums[blockIdx.x] = total;
+    const NodeGeo g = geo[c];
+    SampChild r;
+    r.lox = g.lox; r.loy = g.loy; r.hix = g.hix; r.hiy = g.hiy;
+    r.cx = g.cx; r.cy = g.cy; r.r2 = g.r2; r.deg = g.deg;
+    const NodeAux a = aux[c];
+    r.off = a.off; r.count = lnk[c].count; r.id = c; r.first = a.first;
+    return r;
 }
 
-__global__ __launch_bounds__(256) void k_scan_apply(const ViewState* __restrict__ vs, const int* data,
-                                                    const int* tileOffs, NodeAux* aux)
+__device__ __forceinline__ SampRec samp_record(int p, const NodeGeo* __restrict__ geo, const NodeLnk* __restrict__ lnk,
+                                               const NodeAux* __restrict__ aux)
 {
-    int nn = 2 * vs->nc - 1;
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nn) return;
-    aux[t].off = data[t] + tileOffs[t / kScanTile];
+    const NodeLnk lk = lnk[p];
+    SampRec r;
+    r.l = samp_child(lk.left, geo, lnk, aux);
+    r.r = samp_child(lk.right, geo, lnk, aux);
+    return r;
 }
 
 // Hermite moments A[a][b] = sum_leaves tx^a ty^b / (a! b!), t = (x - c) / sqrt(2 h^2)
 // (hermitefmm.cuh:119-138).  Leaves carry the single coefficient 1.  Internal
-// nodes with an expansion are listed by k_coef_sizes; thread (node, row a)
+// nodes with an expansion are listed by k_coef_blocks; thread (node, row a)
 // computes row a of one node, accumulating in FP64 in leaf order.  A workgroup
 // of 255 threads covers 15 nodes x 17 rows.
 constexpr int kMomNodes = 15;
@@ -1084,16 +1081,25 @@ __constant__ double kInvFact[kMaxDegree + 1] = {
     ifact_c(9), ifact_c(10), ifact_c(11), ifact_c(12), ifact_c(13), ifact_c(14), ifact_c(15), ifact_c(16) };
 __global__ __launch_bounds__(256) void k_moments(const ViewState* __restrict__ vs, const NodeGeo* __restrict__ geo,
                                                  const NodeAux* __restrict__ aux, const int* __restrict__ momList,
-                                                 float* __restrict__ coef, long coefCap)
+                                                 float* __restrict__ coef, const NodeLnk* __restrict__ lnk,
+                                                 SampRec* __restrict__ rec, int* __restrict__ walkQueue,
+                                                 int* __restrict__ tieQueue, VStride vsd)
 {
+    vs = vw(vs, vsd.ws);
+    geo = vw(geo, vsd.ws);
+    aux = vw(aux, vsd.ws);
+    momList = vw(momList, vsd.ws);
+    coef = vw(coef, vsd.ws);
     const int n = vs->nc;
-    if (vs->ncoef > coefCap) return;
     const int L0 = n - 1;
     const int t = threadIdx.x;
     // leaves: 256 per workgroup
     {
         long lf = (long)blockIdx.x * 256 + t;
         if (lf < n) coef[aux[L0 + lf].off] = 1.0f;
+        // and the children's record of an internal node for the walks, with empty queues
+        if (lf < L0) vw(rec, vsd.ws)[lf] = samp_record((int)lf, geo, vw(lnk, vsd.ws), aux);
+        if (lf == 0) { *vw(walkQueue, vsd.ws) = 0; *vw(tieQueue, vsd.ws) = 0; }
     }
     if (t >= kMomNodes * (kMaxDegree + 1)) return;
     const long slot = (long)blockIdx.x * kMomNodes + t / (kMaxDegree + 1);
@@ -1129,11 +1135,6 @@ __global__ __launch_bounds__(256) void k_moments(const ViewState* __restrict__ v
 #pragma unroll
     for (int bb = 0; bb <= kMaxDegree; bb++)
         if (bb <= p) coef[a.off + ax * P1 + bb] = (float)acc[bb];
-}
-
-__global__ void k_check_coef(ViewState* vs, long coefCap)
-{
-    if (threadIdx.x == 0 && (long)vs->ncoef > coefCap) vs->err |= 2;
 }
 
 // ---------------------------------------------------------------------------
@@ -1336,43 +1337,6 @@ __device__ __forceinline__ float tree_weight(const TreeView& T, int entry, float
 
 
 __device__ __forceinline__ float key_of(unsigned long long v) { return __uint_as_float((uint32_t)(v >> 32)); }
-
-// Children records of the sampler's walk, one per internal node (after the tree's
-// degrees and coefficient offsets are final).
-__device__ __forceinline__ SampChild samp_child(int c, const NodeGeo* __restrict__ geo,
-                                                const NodeLnk* __restrict__ lnk, const NodeAux* __restrict__ aux)
-{
-    const NodeGeo g = geo[c];
-    SampChild r;
-    r.lox = g.lox; r.loy = g.loy; r.hix = g.hix; r.hiy = g.hiy;
-    r.cx = g.cx; r.cy = g.cy; r.r2 = g.r2; r.deg = g.deg;
-    const NodeAux a = aux[c];
-    r.off = a.off; r.count = lnk[c].count; r.id = c; r.first = a.first;
-    return r;
-}
-
-__global__ __launch_bounds__(256) void k_samp_records(const ViewState* __restrict__ vs,
-                                                      const NodeGeo* __restrict__ geo,
-                                                      const NodeLnk* __restrict__ lnk,
-                                                      const NodeAux* __restrict__ aux, SampRec* __restrict__ rec,
-                                                      int* __restrict__ walkQueue, int* __restrict__ tieQueue,
-                                                      VStride vsd)
-{
-    vs = vw(vs, vsd.ws);
-    geo = vw(geo, vsd.ws);
-    lnk = vw(lnk, vsd.ws);
-    aux = vw(aux, vsd.ws);
-    rec = vw(rec, vsd.ws);
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == 0) { *vw(walkQueue, vsd.ws) = 0; *vw(tieQueue, vsd.ws) = 0; }      // filled by the next passes
-    const int nc = vs->nc;
-    if (nc <= 1 || p >= nc - 1) return;
-    const NodeLnk lk = lnk[p];
-    SampRec r;
-    r.l = samp_child(lk.left, geo, lnk, aux);
-    r.r = samp_child(lk.right, geo, lnk, aux);
-    rec[p] = r;
-}
 
 // Sampler: one lane per pixel, 8x8 pixel tile per wavefront.
 //
@@ -1981,7 +1945,7 @@ __global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H
     const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
     const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
     const bool valid = (i < W) && (j < H);
-    if (vs->nc <= 0 || vs->err != 0) return;               // uniform over the launch
+    if (vs->nc <= 0) return;                               // uniform over the launch
     const float qx = (float)i, qy = (float)j;
     const float unset = __builtin_nanf("");              // weight not computed yet
     const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -2289,7 +2253,7 @@ __global__ __launch_bounds__(64, 4) void k_sample_descend(int W, int H, int k, i
     T.is2h = vs->is2h;
     const int lane = threadIdx.x;
     const int n = vs->nc;
-    const bool runTree = n > 0 && vs->err == 0;
+    const bool runTree = n > 0;
     const int ents = runTree ? tile_[0] : 0;
     if (ents < 0) return;                                // left to k_sample_walk_serial
     for (int t = lane; t < ents; t += 64) {
@@ -2698,11 +2662,6 @@ __global__ void k_fill_idx(int32_t* p, long n)
 {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) p[t] = -1;
-}
-
-__global__ void k_copy_err(const ViewState* vs, int* err)
-{
-    if (threadIdx.x == 0 && vs->err) atomicOr(err, vs->err);
 }
 
 // ---------------------------------------------------------------------------
@@ -3936,16 +3895,12 @@ int build_structure(int N, int W, int H, double f, double smoothing, double prec
 }
 
 // Dynamic-degree Hermite moments of the sampler's tree.
-int build_moments(int N, int k, const TreeWs& w, hipStream_t st)
+int build_moments(int N, int k, const TreeWs& w, hipStream_t st, int views, VStride vsd)
 {
-    long nScan = (2L * N + kScanTile - 1) / kScanTile;
-    k_coef_sizes<<<grid1(2L * N, 256), 256, 0, st>>>(w.vs, w.geo, w.lnk, k, w.scanTmp, w.momList);
-    k_scan_tiles<<<(unsigned)nScan, 256, 0, st>>>(w.vs, w.scanTmp, w.scanBlocks);
-    k_scan_small<<<1, 1024, 0, st>>>(w.scanBlocks, (int)nScan, &w.vs->ncoef, VStride{});
-    k_scan_apply<<<grid1(2L * N, 256), 256, 0, st>>>(w.vs, w.scanTmp, w.scanBlocks, w.aux);
-    k_check_coef<<<1, 64, 0, st>>>(w.vs, w.coefCap);
+    k_coef_blocks<<<dim3(grid1(2L * N, 256), views), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, k, w.momList, vsd);
     // enough workgroups for max(N leaves / 256, N nodes / 15)
-    k_moments<<<grid1(N, kMomNodes), 256, 0, st>>>(w.vs, w.geo, w.aux, w.momList, w.coef, w.coefCap);
+    k_moments<<<dim3(grid1(N, kMomNodes), views), 256, 0, st>>>(w.vs, w.geo, w.aux, w.momList, w.coef, w.lnk, w.srec,
+                                                                w.walkQueue, w.tieQueue, vsd);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
 }
@@ -3991,8 +3946,6 @@ bool timing_pair(int kernel, hipEvent_t* a, hipEvent_t* b)
 void launch_sample(int N, int W, int H, int k, uint32_t seedLo, uint32_t seedHi, uint32_t view, const TreeWs& w,
                    int32_t* out, int* err, hipStream_t st, int views, VStride vsd)
 {
-    k_samp_records<<<dim3(grid1(N, 256), views), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, w.srec, w.walkQueue,
-                                                               w.tieQueue, vsd);
     const unsigned tiles = (unsigned)(((W + 7) / 8) * ((H + 7) / 8));
     const int L = num_launches(k);
     hipEvent_t e0, e1;
@@ -4100,19 +4053,22 @@ int ude_sample(int bn, int N, int W, int H, int k, double f, double smoothing, d
         return UDE_OK;
     }
     if (wsBytes < ude_sample_workspace_bytes(N, W, H, k)) return UDE_ERR_WORKSPACE;
+    // as many views at once as the workspace holds
     TreeWs w;
-    carve(ws, N, W, H, k, kModeSample, &w);
+    const size_t per = carve(ws, N, W, H, k, kModeSample, &w);
+    const size_t most = bn < 65535 ? bn : 65535;             // views are the grid's second dimension
+    const int span = (int)((wsBytes - 256) / per < most ? (wsBytes - 256) / per : most);
     uint32_t sLo = (uint32_t)seed, sHi = (uint32_t)(seed >> 32);
-    for (int b = 0; b < bn; b++) {
+    for (int b = 0; b < bn; b += span) {
+        const int views = span < bn - b ? span : bn - b;
+        const VStride vsd{per, sizeof(float) * 3 * (size_t)N, sdBatch > 1 ? sizeof(float) * 2 * (size_t)N : 0};
         const float* pb = pts + 3L * N * b;
         const float* nb = nrm + 3L * N * b;
         const float* sb = sd + (sdBatch > 1 ? 2L * N * b : 0);
-        int rc = build_structure(N, W, H, f, smoothing, prec, pb, nb, sb, w, st);
-        if (rc == UDE_OK) rc = build_moments(N, k, w, st);
+        int rc = build_structure(N, W, H, f, smoothing, prec, pb, nb, sb, w, st, views, vsd);
+        if (rc == UDE_OK) rc = build_moments(N, k, w, st, views, vsd);
         if (rc != UDE_OK) return rc;
-        int32_t* ob = out + perView * b;
-        launch_sample(N, W, H, k, sLo, sHi, (uint32_t)b, w, ob, errFlag, st, 1, VStride{});
-        k_copy_err<<<1, 64, 0, st>>>(w.vs, errFlag);
+        launch_sample(N, W, H, k, sLo, sHi, (uint32_t)b, w, out + perView * b, errFlag, st, views, vsd);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
