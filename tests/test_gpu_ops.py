@@ -280,6 +280,32 @@ def test_interpolation(dev, C, ab):
     assert_close(gA.cpu().numpy(), rA, RTOL, "interp grad attr", mag=mA)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("W,H,k,N,ab", [(8, 8, 1, 2, 1), (9, 7, 40, 30, 2), (3, 50, 130, 5000, 1), (300, 190, 9, 100_000, 2),
+                                        (257, 241, 16, 700, 1)])
+def test_interpolation_tiles(dev, W, H, k, N, ab, dtype):
+    """Three channels around the tiles of both sizes: partial tiles, slots that share their
+    rows and slots that share none, more rows in a tile than its table holds, zero weights.
+    An attribute row sums as many terms as slots name it."""
+    from cudaExtensions import interpolation
+    rng = np.random.default_rng(W + k)
+    idx = random_slots(rng, 2, W, H, k, N)
+    w = rng.uniform(size=idx.shape).astype(dtype)
+    w[rng.uniform(size=idx.shape) < 0.1] = 0.0
+    a = rng.normal(size=(ab, N, 3)).astype(dtype)
+    g = rng.normal(size=(2, W, H, 3)).astype(dtype)
+    eps = float(np.finfo(dtype).eps) / 2
+    most = int(np.bincount(idx[idx >= 0].ravel()).max())
+    out = interpolation.forward(t(idx, dev), t(w, dev), t(a, dev))
+    assert_close(out.cpu().numpy(), O.interp_forward(idx, w, a), 8 * eps, "interp forward",
+                 mag=magnitude(O.interp_forward, idx, w, a), ops=max(64, k), eps=eps)
+    gW, gA = interpolation.backward(t(g, dev), t(idx, dev), t(w, dev), t(a, dev))
+    rW, rA = O.interp_backward(g, idx, w, a)
+    mW, mA = magnitude(O.interp_backward, g, idx, w, a)
+    assert_close(gW.cpu().numpy(), rW, 8 * eps, "interp grad w", mag=mW, eps=eps)
+    assert_close(gA.cpu().numpy(), rA, 8 * eps, "interp grad attr", mag=mA, ops=max(64, most), eps=eps)
+
+
 @pytest.mark.parametrize("cb", [1, 2])
 def test_sh_shading(dev, cb):
     from cudaExtensions import shading
