@@ -72,13 +72,11 @@ struct ViewState {
     unsigned int hcnt;
     int nc;
     float h, radius, lo, hix, hiy, s2h, prec, is2h;
-    int ncoef;        // coefficients of the internal nodes' blocks
-    int spare;
+    unsigned long long blocks;   // internal nodes with a Hermite expansion, and above bit 32 their coefficients
     int nseeds;       // block-spanning fan-in starts (bottom-up, second level)
-    int nmom;         // internal nodes with a Hermite expansion
     int pad;
     Band band[2];     // fixed-order densities: tree bandwidth, wide proposal bandwidth
-    int nfix[2];      // accepted internal nodes per band
+    unsigned long long nfix;     // accepted internal nodes of band 0, and of band 1 above bit 32
     int hhist[256];   // visible splats' proposal bandwidths, 1/16 px bins over [0, 16)
 };
 
@@ -382,8 +380,8 @@ __global__ void k_zero_state(ViewState* vs, VStride vsd)
 {
     vs = vw(vs, vsd.ws);
     if (threadIdx.x == 0) {
-        vs->hsum = 0; vs->hcnt = 0; vs->nc = 0; vs->ncoef = 0; vs->nseeds = 0; vs->nmom = 0;
-        vs->nfix[0] = 0; vs->nfix[1] = 0;
+        vs->hsum = 0; vs->hcnt = 0; vs->nc = 0; vs->blocks = 0; vs->nseeds = 0;
+        vs->nfix = 0;
     }
     for (int b = threadIdx.x; b < 256; b += blockDim.x) vs->hhist[b] = 0;
 }
@@ -1033,9 +1031,12 @@ __global__ __launch_bounds__(256) void k_bottom_up_global(const ViewState* __res
 // a walk stops at the first node with an expansion.  An internal node below an
 // expanded node, with no start in between, is therefore never evaluated and
 // gets no block.  The leaves' single coefficients lie first, in leaf order; a workgroup
-// reserves its nodes' blocks behind them with one atomic (where a block lies changes no
-// value), which takes the place of a scan over all nodes in three launches.
-__global__ __launch_bounds__(256) void k_coef_blocks(ViewState* vs, const NodeGeo* __restrict__ geo,
+// reserves its nodes' list entries and blocks behind them with one atomic (where a block
+// lies changes no value), which takes the place of a scan over all nodes in three launches.
+// The atomics of one word follow one another: workgroups of 1024, 1M splats 81 -> 24 us
+// against 256 with an atomic for each of the two counts.
+constexpr int kCoefThreads = 1024;
+__global__ __launch_bounds__(kCoefThreads) void k_coef_blocks(ViewState* vs, const NodeGeo* __restrict__ geo,
                                                      const NodeLnk* __restrict__ lnk, NodeAux* __restrict__ aux, int k,
                                                      int* momList, VStride vsd)
 {
@@ -1058,24 +1059,24 @@ __global__ __launch_bounds__(256) void k_coef_blocks(ViewState* vs, const NodeGe
         }
     }
     // list the internal nodes that need moments: one slot reservation per workgroup
-    __shared__ int wcnt[4], sh[4];
-    __shared__ int bbase, cbase;
+    __shared__ unsigned long long sums[kCoefThreads / 64];
+    __shared__ unsigned long long base;
     const bool want = d >= 0;
     const unsigned long long m = __ballot(want);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) wcnt[wid] = __popcll(m);
-    int coefs;
-    const int at = block_excl_scan(want ? (d + 1) * (d + 1) : 0, sh, coefs);
+    const int incl = wave_incl_scan(want ? (d + 1) * (d + 1) : 0);
+    if (lane == 63) sums[wid] = (unsigned long long)incl << 32 | (unsigned)__popcll(m);
+    __syncthreads();
     if (threadIdx.x == 0) {
-        const int tot = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
-        bbase = tot ? atomicAdd(&vs->nmom, tot) : 0;
-        cbase = tot ? atomicAdd(&vs->ncoef, coefs) : 0;
+        unsigned long long tot = 0ull;
+        for (int q = 0; q < kCoefThreads / 64; q++) tot += sums[q];
+        base = tot ? atomicAdd(&vs->blocks, tot) : 0ull;
     }
     __syncthreads();
-    int base = bbase;
-    for (int q = 0; q < wid; q++) base += wcnt[q];
-    if (want) momList[base + __popcll(m & ((1ull << lane) - 1ull))] = t;
-    if (t < nn) aux[t].off = t >= n - 1 ? t - (n - 1) : want ? n + cbase + at : 0;
+    unsigned long long at = base;
+    for (int q = 0; q < wid; q++) at += sums[q];
+    if (want) momList[(int)(unsigned)at + __popcll(m & ((1ull << lane) - 1ull))] = t;
+    if (t < nn) aux[t].off = t >= n - 1 ? t - (n - 1) : want ? n + (int)(at >> 32) + incl - (d + 1) * (d + 1) : 0;
 }
 
 // Children records of the sampler's walk, one per internal node (after the tree's
@@ -1114,9 +1115,33 @@ constexpr double ifact_c(int a) { double f = 1.0; for (int q = 2; q <= a; q++) f
 __constant__ double kInvFact[kMaxDegree + 1] = {
     ifact_c(0), ifact_c(1), ifact_c(2), ifact_c(3), ifact_c(4), ifact_c(5), ifact_c(6), ifact_c(7), ifact_c(8),
     ifact_c(9), ifact_c(10), ifact_c(11), ifact_c(12), ifact_c(13), ifact_c(14), ifact_c(15), ifact_c(16) };
+// Row ax of kMomLeaves leaves from position pos on: x^ax / ax! and y.  The leaves' reads are
+// in flight together and their power chains interleave; a leaf at a time, each waited for
+// its read and then for its own chain (the two bands' degree-6 moments of 1M splats
+// 100 -> 63 us, with both bands in one launch).
+constexpr int kMomLeaves = 4;
+__device__ __forceinline__ void moment_leaves(const float2* __restrict__ leafXY, int pos, int last, const NodeGeo& g,
+                                              float is2h, int ax, double ifx, double* mx, double* ty)
+{
+    double tx[kMomLeaves];
+#pragma unroll
+    for (int u = 0; u < kMomLeaves; u++) {
+        const float2 q = leafXY[pos + u < last ? pos + u : last];
+        tx[u] = (double)((q.x - g.cx) * is2h);
+        ty[u] = (double)((q.y - g.cy) * is2h);
+        mx[u] = 1.0;
+    }
+    for (int q = 0; q < ax; q++)
+#pragma unroll
+        for (int u = 0; u < kMomLeaves; u++) mx[u] = mx[u] * tx[u];
+#pragma unroll
+    for (int u = 0; u < kMomLeaves; u++) mx[u] = mx[u] * ifx;
+}
+
 __global__ __launch_bounds__(256) void k_moments(const ViewState* __restrict__ vs, const NodeGeo* __restrict__ geo,
                                                  const NodeAux* __restrict__ aux, const int* __restrict__ momList,
-                                                 float* __restrict__ coef, const NodeLnk* __restrict__ lnk,
+                                                 float* __restrict__ coef, const float2* __restrict__ leafXY,
+                                                 const NodeLnk* __restrict__ lnk,
                                                  SampRec* __restrict__ rec, int* __restrict__ walkQueue,
                                                  int* __restrict__ tieQueue, VStride vsd)
 {
@@ -1125,6 +1150,7 @@ __global__ __launch_bounds__(256) void k_moments(const ViewState* __restrict__ v
     aux = vw(aux, vsd.ws);
     momList = vw(momList, vsd.ws);
     coef = vw(coef, vsd.ws);
+    leafXY = vw(leafXY, vsd.ws);
     const int n = vs->nc;
     const int L0 = n - 1;
     const int t = threadIdx.x;
@@ -1139,7 +1165,7 @@ __global__ __launch_bounds__(256) void k_moments(const ViewState* __restrict__ v
     if (t >= kMomNodes * (kMaxDegree + 1)) return;
     const long slot = (long)blockIdx.x * kMomNodes + t / (kMaxDegree + 1);
     const int ax = t % (kMaxDegree + 1);
-    if (slot >= vs->nmom) return;
+    if (slot >= (int)(unsigned)vs->blocks) return;
     const int nd = momList[slot];
     NodeGeo g = geo[nd];
     const int p = g.deg;
@@ -1151,19 +1177,19 @@ __global__ __launch_bounds__(256) void k_moments(const ViewState* __restrict__ v
     double acc[kMaxDegree + 1];
 #pragma unroll
     for (int bb = 0; bb <= kMaxDegree; bb++) acc[bb] = 0.0;
-    for (int pos = a.first; pos <= a.last; pos++) {
-        NodeGeo lf = geo[L0 + pos];
-        float tx = (lf.cx - g.cx) * is2h;
-        float ty = (lf.cy - g.cy) * is2h;
-        double px = 1.0;
-        for (int q = 0; q < ax; q++) px = px * (double)tx;
-        double mx = px * ifx;
-        double py = 1.0;
+    for (int pos = a.first; pos <= a.last; pos += kMomLeaves) {
+        double mx[kMomLeaves], ty[kMomLeaves];
+        moment_leaves(leafXY, pos, a.last, g, is2h, ax, ifx, mx, ty);
 #pragma unroll
-        for (int bb = 0; bb <= kMaxDegree; bb++) {
-            if (bb <= p) {
-                acc[bb] += mx * (py * ifact_c(bb));
-                py = py * (double)ty;
+        for (int u = 0; u < kMomLeaves; u++) {
+            if (pos + u > a.last) break;
+            double py = 1.0;
+#pragma unroll
+            for (int bb = 0; bb <= kMaxDegree; bb++) {
+                if (bb <= p) {
+                    acc[bb] += mx[u] * (py * ifact_c(bb));
+                    py = py * ty[u];
+                }
             }
         }
     }
@@ -2709,8 +2735,11 @@ __global__ void k_fill_idx(int32_t* p, long n)
 
 // Internal nodes whose degree-6 truncation bound at band b meets the
 // precision, and whose parent's does not, carry an expansion: a 49-float
-// block at fixOff[node].
-__global__ __launch_bounds__(256) void k_fixed_select(ViewState* vs, int nbands, int p, const NodeGeo* __restrict__ geo,
+// block at fixOff[node].  A workgroup reserves its slots of both bands with one atomic:
+// those of one word follow one another, and 1M splats took 45 us with one per band and 256
+// nodes (now 23).
+constexpr int kSelectThreads = 1024;
+__global__ __launch_bounds__(kSelectThreads) void k_fixed_select(ViewState* vs, int nbands, int p, const NodeGeo* __restrict__ geo,
                                                       const NodeLnk* __restrict__ lnk, int* fixOff0, int* fixOff1,
                                                       int* list0, int* list1, VStride vsd)
 {
@@ -2721,8 +2750,8 @@ __global__ __launch_bounds__(256) void k_fixed_select(ViewState* vs, int nbands,
     fixOff1 = vw(fixOff1, vsd.ws);
     list0 = vw(list0, vsd.ws);
     list1 = vw(list1, vsd.ws);
-    __shared__ int wcnt[2][4];
-    __shared__ int bbase[2];
+    __shared__ unsigned long long wcnt[kSelectThreads / 64];
+    __shared__ unsigned long long first;
     const int n = vs->nc;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -2743,21 +2772,20 @@ __global__ __launch_bounds__(256) void k_fixed_select(ViewState* vs, int nbands,
         // bound and skips its subtree, so only those nodes need an expansion
         if (t < n - 1) acc[b] = meets(t) && (t == 0 || !meets(lnk[t].parent));
         m[b] = __ballot(acc[b]);
-        if (lane == 0) wcnt[b][wid] = __popcll(m[b]);
+    }
+    if (lane == 0) wcnt[wid] = (unsigned long long)__popcll(m[1]) << 32 | (unsigned)__popcll(m[0]);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long tot = 0ull;
+        for (int q = 0; q < kSelectThreads / 64; q++) tot += wcnt[q];
+        first = tot ? atomicAdd(&vs->nfix, tot) : 0ull;
     }
     __syncthreads();
-    // one slot reservation per band and workgroup
-    if (threadIdx.x < nbands) {
-        const int b = threadIdx.x;
-        const int tot = wcnt[b][0] + wcnt[b][1] + wcnt[b][2] + wcnt[b][3];
-        bbase[b] = tot ? atomicAdd(&vs->nfix[b], tot) : 0;
-    }
-    __syncthreads();
+    unsigned long long at = first;
+    for (int q = 0; q < wid; q++) at += wcnt[q];
     if (t >= n - 1) return;
     for (int b = 0; b < nbands; b++) {
-        int base = bbase[b];
-        for (int q = 0; q < wid; q++) base += wcnt[b][q];
-        const int slot = base + __popcll(m[b] & ((1ull << lane) - 1ull));
+        const int slot = (int)(unsigned)(b ? at >> 32 : at) + __popcll(m[b] & ((1ull << lane) - 1ull));
         int* fixOff = b ? fixOff1 : fixOff0;
         int* list = b ? list1 : list0;
         fixOff[t] = acc[b] ? slot * (p + 1) * (p + 1) : -1;
@@ -2769,24 +2797,27 @@ __global__ __launch_bounds__(256) void k_fixed_select(ViewState* vs, int nbands,
 // (node, row a) sums row a over the node's leaf range in FP64 (leaf order).
 // 256 / (P + 1) nodes x (P + 1) rows per 256-thread workgroup.
 template <int P>
-__global__ __launch_bounds__(256) void k_fixed_moments(const ViewState* __restrict__ vs, int b,
+__global__ __launch_bounds__(256) void k_fixed_moments(const ViewState* __restrict__ vs,
                                                        const NodeGeo* __restrict__ geo, const NodeAux* __restrict__ aux,
-                                                       const int* __restrict__ list, const int* __restrict__ fixOff,
-                                                       float* __restrict__ coef, VStride vsd)
+                                                       const float2* __restrict__ leafXY,
+                                                       const int* __restrict__ list0, const int* __restrict__ list1,
+                                                       const int* __restrict__ fixOff0, const int* __restrict__ fixOff1,
+                                                       float* __restrict__ coef0, float* __restrict__ coef1, VStride vsd)
 {
+    const int b = blockIdx.z;
     vs = vw(vs, vsd.ws);
     geo = vw(geo, vsd.ws);
     aux = vw(aux, vsd.ws);
-    list = vw(list, vsd.ws);
-    fixOff = vw(fixOff, vsd.ws);
-    coef = vw(coef, vsd.ws);
+    leafXY = vw(leafXY, vsd.ws);
+    const int* list = vw(b ? list1 : list0, vsd.ws);
+    const int* fixOff = vw(b ? fixOff1 : fixOff0, vsd.ws);
+    float* coef = vw(b ? coef1 : coef0, vsd.ws);
     const int t = threadIdx.x;
     if (t >= (256 / (P + 1)) * (P + 1)) return;
     const long slot = (long)blockIdx.x * (256 / (P + 1)) + t / (P + 1);
     const int ax = t % (P + 1);
-    if (slot >= vs->nfix[b]) return;
+    if (slot >= (int)(unsigned)(b ? vs->nfix >> 32 : vs->nfix)) return;
     const int nd = list[slot];
-    const int L0 = vs->nc - 1;
     const float is2h = vs->band[b].is2h;
     const double c = (double)vs->band[b].c;
     NodeGeo g = geo[nd];
@@ -2796,18 +2827,18 @@ __global__ __launch_bounds__(256) void k_fixed_moments(const ViewState* __restri
     double acc[P + 1];
 #pragma unroll
     for (int bb = 0; bb <= P; bb++) acc[bb] = 0.0;
-    for (int pos = a.first; pos <= a.last; pos++) {
-        NodeGeo lf = geo[L0 + pos];
-        float tx = (lf.cx - g.cx) * is2h;
-        float ty = (lf.cy - g.cy) * is2h;
-        double px = 1.0;
-        for (int q = 0; q < ax; q++) px = px * (double)tx;
-        double mx = px * ifx;
-        double py = 1.0;
+    for (int pos = a.first; pos <= a.last; pos += kMomLeaves) {
+        double mx[kMomLeaves], ty[kMomLeaves];
+        moment_leaves(leafXY, pos, a.last, g, is2h, ax, ifx, mx, ty);
 #pragma unroll
-        for (int bb = 0; bb <= P; bb++) {
-            acc[bb] += mx * (py * ifact_c(bb));
-            py = py * (double)ty;
+        for (int u = 0; u < kMomLeaves; u++) {
+            if (pos + u > a.last) break;
+            double py = 1.0;
+#pragma unroll
+            for (int bb = 0; bb <= P; bb++) {
+                acc[bb] += mx[u] * (py * ifact_c(bb));
+                py = py * ty[u];
+            }
         }
     }
 #pragma unroll
@@ -3932,9 +3963,9 @@ int build_structure(int N, int W, int H, double f, double smoothing, double prec
 // Dynamic-degree Hermite moments of the sampler's tree.
 int build_moments(int N, int k, const TreeWs& w, hipStream_t st, int views, VStride vsd)
 {
-    k_coef_blocks<<<dim3(grid1(2L * N, 256), views), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, k, w.momList, vsd);
+    k_coef_blocks<<<dim3(grid1(2L * N, kCoefThreads), views), kCoefThreads, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, k, w.momList, vsd);
     // enough workgroups for max(N leaves / 256, N nodes / 15)
-    k_moments<<<dim3(grid1(N, kMomNodes), views), 256, 0, st>>>(w.vs, w.geo, w.aux, w.momList, w.coef, w.lnk, w.srec,
+    k_moments<<<dim3(grid1(N, kMomNodes), views), 256, 0, st>>>(w.vs, w.geo, w.aux, w.momList, w.coef, w.leafXY, w.lnk, w.srec,
                                                                 w.walkQueue, w.tieQueue, vsd);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
@@ -4027,18 +4058,17 @@ dim3 tile_grid(const TileCfg& c, int W, int H, int views)
 void fixed_expansions(int N, int nbands, int p, const TreeWs& w, hipStream_t st, int views = 1,
                       VStride vsd = VStride{})
 {
-    k_fixed_select<<<dim3(grid1(N, 256), views), 256, 0, st>>>(w.vs, nbands, p, w.geo, w.lnk, w.fixOff[0],
-                                                                nbands > 1 ? w.fixOff[1] : nullptr, w.fixList[0],
-                                                                nbands > 1 ? w.fixList[1] : nullptr, vsd);
-    for (int b = 0; b < nbands; b++) {
-        const dim3 grid(grid1(N, 256 / (p + 1)), views);
-        switch (p) {
-#define UD_MOMENTS(P) case P: k_fixed_moments<P><<<grid, 256, 0, st>>>(w.vs, b, w.geo, w.aux, w.fixList[b], \
-                                                                        w.fixOff[b], w.fixCoef[b], vsd); break;
-        UD_MOMENTS(4) UD_MOMENTS(5) UD_MOMENTS(6) UD_MOMENTS(7) UD_MOMENTS(8)
+    k_fixed_select<<<dim3(grid1(N, kSelectThreads), views), kSelectThreads, 0, st>>>(
+        w.vs, nbands, p, w.geo, w.lnk, w.fixOff[0], nbands > 1 ? w.fixOff[1] : nullptr, w.fixList[0],
+        nbands > 1 ? w.fixList[1] : nullptr, vsd);
+    const dim3 grid(grid1(N, 256 / (p + 1)), views, nbands);
+    switch (p) {
+#define UD_MOMENTS(P) case P: k_fixed_moments<P><<<grid, 256, 0, st>>>(w.vs, w.geo, w.aux, w.leafXY, w.fixList[0], \
+                                                                        w.fixList[1], w.fixOff[0], w.fixOff[1],    \
+                                                                        w.fixCoef[0], w.fixCoef[1], vsd); break;
+    UD_MOMENTS(4) UD_MOMENTS(5) UD_MOMENTS(6) UD_MOMENTS(7) UD_MOMENTS(8)
 #undef UD_MOMENTS
-        default: break;
-        }
+    default: break;
     }
 }
 
