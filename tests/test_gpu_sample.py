@@ -213,3 +213,17 @@ def test_sample_views_in_groups(dev, monkeypatch, perViewSd):
     monkeypatch.setattr(_lib, "workspace", small)
     assert np.array_equal(run(), ref)
     assert (ref[0] >= 0).any() and (ref[2] == -1).all()
+
+
+@pytest.mark.parametrize("N,k", [(2, 12), (3, 40), (5, 5), (11, 12), (12, 12), (13, 12), (40, 40)])
+def test_sample_fewer_splats_than_slots(dev, N, k):
+    """At most k visible splats, spread so far that many pixels see one or none: the root is
+    one subtree for every launch's descent, so a pixel draws each splat once per launch."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng(N)
+    W, H, f = 33, 26, 40.0
+    p = rng.uniform([-1.2, -1.0, -4.0], [1.2, 1.0, -2.0], size=(N, 3)).astype(np.float32)
+    nb = np.tile(np.float32([0.0, 0.0, -1.0]), (N, 1))
+    sd = rng.uniform(0.02, 0.2, size=(N, 2)).astype(np.float32)
+    got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), k, 0.0, 0.01, seed=3)
+    assert np.array_equal(got[0].cpu().numpy(), O.sample_view(W, H, f, p, nb, sd, k, 0.0, 0.01, seed=3))

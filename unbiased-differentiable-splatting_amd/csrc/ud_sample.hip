@@ -1597,7 +1597,8 @@ __device__ __forceinline__ int tile_descents(const TreeView& T, const SampRec UD
     path.lds = ldsPath;
     float rootCap = 1.0f;
     int memoKey = -1, memoFirst = 0, memoCnt = 0;
-    const bool inTile = tileEnts > 0 && total > 0.0f && total < inf;
+    // a tree of at most k leaves is one subtree: no step is taken in it
+    const bool inTile = tileEnts > 0 && L0 + 1 > k && total > 0.0f && total < inf;
     int drawn = 0;
     for (int la = 0; la < L; la++) {
         int np = 0, depth = 0, e = 0, side = 0;
