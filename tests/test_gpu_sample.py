@@ -227,3 +227,33 @@ def test_sample_fewer_splats_than_slots(dev, N, k):
     sd = rng.uniform(0.02, 0.2, size=(N, 2)).astype(np.float32)
     got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), k, 0.0, 0.01, seed=3)
     assert np.array_equal(got[0].cpu().numpy(), O.sample_view(W, H, f, p, nb, sd, k, 0.0, 0.01, seed=3))
+
+
+@pytest.mark.parametrize("case", [28, 70, 145, 216])
+def test_sample_keys_near_the_largest(dev, case):
+    """Random scenes in which a pixel has fewer than k draws of ordinary keys and more others
+    than its wavefront keeps, with keys near the largest float: the search for the pixel's
+    threshold ends there too."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng([1, case])
+    N = int(np.exp(rng.uniform(0, np.log(20000))))
+    bn, W, H = int(rng.integers(1, 4)), int(rng.integers(1, 90)), int(rng.integers(1, 90))
+    k = int(rng.choice([1, 2, 3, 5, 8, 12, 16, 24, 40, 64, 65, 100, 128, 200, 256]))
+    precision = float(10 ** rng.uniform(-3.5, -0.5))
+    f = float(max(W, H)) * rng.uniform(0.6, 2.5)
+    ext = rng.uniform(0.05, 1.5)
+    p = rng.uniform([-ext, -ext, -4], [ext, ext, -1.5], size=(bn, N, 3)).astype(np.float32)
+    if rng.uniform() < 0.3:
+        p[..., :2] = np.round(p[..., :2] * 8) / 8
+    if rng.uniform() < 0.3:
+        p[rng.uniform(size=(bn, N)) < 0.3, 2] *= -1
+    if rng.uniform() < 0.2:
+        p[:, :N // 2] = p[:, :1]
+    n = rng.normal(size=(bn, N, 3)).astype(np.float32)
+    n[..., 2] = -np.abs(n[..., 2]) - 0.2
+    n /= np.linalg.norm(n, axis=-1, keepdims=True)
+    sd = (10 ** rng.uniform(-3.5, -0.3) * rng.uniform(0.5, 2, size=(1 if rng.uniform() < .5 else bn, N, 2))).astype(np.float32)
+    smoothing = 0.0 if rng.uniform() < 0.6 else float(rng.uniform(0, 0.5))
+    got = sampling.sample(W, H, f, t(p, dev), t(n, dev), None, t(sd, dev), k, smoothing, precision, seed=case)
+    ref = O.sample(W, H, f, p, n, sd, k, smoothing, precision, seed=case)
+    assert np.array_equal(got.cpu().numpy(), ref)

@@ -2494,7 +2494,7 @@ __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw(int W, int H, i
             if (up && hi == kInfKey - 1) mid = hi - mid > step ? mid + step : lo + ((hi - lo) >> 1);
             else if (!up && lo == 0) mid = mid > step ? mid - step : hi >> 1;
             else mid = lo + ((hi - lo) >> 1);
-            step <<= 1;
+            if (step < 1u << 30) step <<= 1;            // 2^30 spans the keys above 1; past that, halve
         }
     }
     if (!tie) {
