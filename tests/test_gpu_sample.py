@@ -257,3 +257,26 @@ def test_sample_keys_near_the_largest(dev, case):
     got = sampling.sample(W, H, f, t(p, dev), t(n, dev), None, t(sd, dev), k, smoothing, precision, seed=case)
     ref = O.sample(W, H, f, p, n, sd, k, smoothing, precision, seed=case)
     assert np.array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 64, 65, 129, 1023, 1025, 4095, 4096, 4097])
+def test_sizes_around_one_workgroup(dev, N):
+    """The tree's front in one workgroup up to 4096 splats: counts around its wavefronts, its
+    rounds and its sorting network, with splats behind the camera among them, splats at the
+    same place (equal keys keep their order) and out of the frame; sampler and Poisson-rate
+    draws equal to the oracle bit for bit."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng(N)
+    W, H, f = 33, 26, 40.0
+    p = rng.uniform([-1.2, -1.0, -4.0], [1.2, 1.0, -2.0], size=(N, 3)).astype(np.float32)
+    if N > 3:
+        p[rng.uniform(size=N) < 0.1, 2] *= -1.0
+        p[N // 2:N // 2 + N // 8] = p[0]
+    nb = np.tile(np.float32([0.0, 0.0, -1.0]), (N, 1))
+    sd = rng.uniform(0.02, 0.2, size=(N, 2)).astype(np.float32)
+    got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), 12, 0.0, 0.01, seed=3)
+    assert np.array_equal(got[0].cpu().numpy(), O.sample_view(W, H, f, p, nb, sd, 12, 0.0, 0.01, seed=3))
+    ids, ipi = sampling.samplePoisson(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), 40, 0.0, 0.01,
+                                      seed=3, rate=3.0)
+    rid, ripi, _, over = O.poisson_view(W, H, f, p, nb, sd, 40, 3.0, 0.0, 0.01, seed=3)
+    assert not over and np.array_equal(ids[0].cpu().numpy(), rid) and np.array_equal(ipi[0].cpu().numpy(), ripi)

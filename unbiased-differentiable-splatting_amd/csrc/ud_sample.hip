@@ -376,15 +376,16 @@ __device__ __forceinline__ T* vw(T* p, size_t stride)
     return p ? (T*)((char*)p + (size_t)blockIdx.y * stride) : p;
 }
 
-__global__ void k_zero_state(ViewState* vs, VStride vsd)
+__device__ __forceinline__ void zero_state(ViewState* vs)
 {
-    vs = vw(vs, vsd.ws);
     if (threadIdx.x == 0) {
         vs->hsum = 0; vs->hcnt = 0; vs->nc = 0; vs->blocks = 0; vs->nseeds = 0;
         vs->nfix = 0;
     }
     for (int b = threadIdx.x; b < 256; b += blockDim.x) vs->hhist[b] = 0;
 }
+
+__global__ void k_zero_state(ViewState* vs, VStride vsd) { zero_state(vw(vs, vsd.ws)); }
 
 __global__ __launch_bounds__(1024) void k_bandwidth(int N, float Wf, float Hf, float ff, float smoothing,
                                                    const float* __restrict__ pts, const float* __restrict__ nrm,
@@ -439,10 +440,8 @@ __device__ Band make_band(float h, double prec)
     return b;
 }
 
-__global__ void k_view_params(ViewState* vs, float Wf, float Hf, double prec, VStride vsd)
+__device__ __forceinline__ void view_params(ViewState* vs, float Wf, float Hf, double prec)
 {
-    vs = vw(vs, vsd.ws);
-    if (threadIdx.x != 0) return;
     double hd = ((double)vs->hsum * (1.0 / 1099511627776.0)) / (double)vs->hcnt;
     float h = (float)hd;
     float radius = band_radius(h, prec);
@@ -456,6 +455,11 @@ __global__ void k_view_params(ViewState* vs, float Wf, float Hf, double prec, VS
     vs->prec = (float)prec;
     vs->nc = 0;
     vs->band[0] = make_band(h, prec);
+}
+
+__global__ void k_view_params(ViewState* vs, float Wf, float Hf, double prec, VStride vsd)
+{
+    if (threadIdx.x == 0) view_params(vw(vs, vsd.ws), Wf, Hf, prec);
 }
 
 __device__ __forceinline__ bool visible(const ViewState& v, float Wf, float Hf, float ff, const float* p, float& sx, float& sy)
@@ -487,6 +491,13 @@ __device__ __forceinline__ uint32_t morton2(float ux, float uy)
     float cx = fminf(fmaxf(ux * 1024.0f, 0.0f), 1023.0f);
     float cy = fminf(fmaxf(uy * 1024.0f, 0.0f), 1023.0f);
     return 2u * expand_bits2((uint32_t)cx) + expand_bits2((uint32_t)cy);
+}
+
+// orders the wavefront's LDS accesses (its LDS operations execute in order)
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // exclusive scan of one int per thread over a 256-thread workgroup
@@ -688,6 +699,104 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const ViewState* __restric
         run[threadIdx.x] += wc[0][threadIdx.x] + wc[1][threadIdx.x] + wc[2][threadIdx.x] + wc[3][threadIdx.x];
         __syncthreads();
     }
+}
+
+// ---------------------------------------------------------------------------
+// State, bandwidth, cull and sort of up to kFrontSplats splats in one workgroup and one
+// launch: at these sizes the 18 kernels above take 2 to 9 us each, most of it their own
+// start and end (4096 splats: 71 us in all, here 47; 256: 47, here 12).  The line lies
+// where a 20-bit key and a position fill a 32-bit word, which a bitonic network in LDS
+// sorts; the order is the stable radix sort's.
+// ---------------------------------------------------------------------------
+constexpr int kFrontSplats = 4096;
+
+__global__ __launch_bounds__(1024) void k_front_small(int N, float Wf, float Hf, float ff, float smoothing, double prec,
+                                                      const float* __restrict__ pts, const float* __restrict__ nrm,
+                                                      const float* __restrict__ sd, ViewState* vs, float* hraw,
+                                                      uint32_t* __restrict__ keys, int32_t* __restrict__ ids,
+                                                      VStride vsd)
+{
+    pts = vw(pts, vsd.pts);
+    nrm = vw(nrm, vsd.pts);
+    sd = vw(sd, vsd.sd);
+    vs = vw(vs, vsd.ws);
+    hraw = vw(hraw, vsd.ws);
+    keys = vw(keys, vsd.ws);
+    ids = vw(ids, vsd.ws);
+    __shared__ uint32_t word[kFrontSplats];
+    __shared__ int32_t idAt[kFrontSplats];
+    __shared__ ViewState v;
+    __shared__ unsigned long long ssum[16];
+    __shared__ unsigned int scnt[16];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    zero_state(vs);
+    unsigned long long q = 0;
+    unsigned int c = 0;
+    for (int t = tid; t < N; t += 1024) {
+        const float hk = iso_h(Wf, Hf, ff, pts + 3L * t, nrm + 3L * t, sd + 2L * t, smoothing);
+        if (hraw) hraw[t] = prop_h(Wf, Hf, ff, pts + 3L * t, nrm + 3L * t, sd + 2L * t, smoothing);
+        if (isfinite(hk)) { q += (unsigned long long)((double)hk * 1099511627776.0); c += 1; }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        q += __shfl_xor(q, o, 64);
+        c += __shfl_xor(c, o, 64);
+    }
+    if (lane == 0) { ssum[wid] = q; scnt[wid] = c; }
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < 16; w++) { ssum[0] += ssum[w]; scnt[0] += scnt[w]; }
+        vs->hsum = v.hsum = ssum[0];
+        vs->hcnt = v.hcnt = scnt[0];
+        view_params(vs, Wf, Hf, prec);
+        view_params(&v, Wf, Hf, prec);
+    }
+    __syncthreads();
+    // the visible splats in order: key, and the position in that order
+    int n = 0;
+    for (int r = 0; r < N; r += 1024) {
+        const int e = r + tid;
+        float sx = 0.0f, sy = 0.0f;
+        const bool vis = e < N && visible(v, Wf, Hf, ff, pts + 3L * e, sx, sy);
+        const unsigned long long m = __ballot(vis);
+        __syncthreads();
+        if (lane == 0) scnt[wid] = __popcll(m);
+        __syncthreads();
+        int at = n;
+        for (int w = 0; w < 16; w++) {
+            if (w < wid) at += scnt[w];
+            n += scnt[w];
+        }
+        if (vis) {
+            at += __popcll(m & ((1ull << lane) - 1ull));
+            const float ux = (sx - v.lo) / (v.hix - v.lo);
+            const float uy = (sy - v.lo) / (v.hiy - v.lo);
+            word[at] = morton2(ux, uy) << 12 | (uint32_t)at;
+            idAt[at] = e;
+        }
+    }
+    int n2 = 2;
+    while (n2 < n) n2 *= 2;
+    __syncthreads();
+    for (int t = n + tid; t < n2; t += 1024) word[t] = 0xffffffffu;     // positions stay below 4095 where n < n2
+    __syncthreads();
+    for (int k = 2; k <= n2; k *= 2)
+        for (int j = k / 2; j > 0; j /= 2) {
+            for (int x = tid; x < n2 / 2; x += 1024) {
+                const int i = 2 * x - (x & (j - 1));
+                const uint32_t a = word[i], b = word[i + j];
+                if ((a > b) == ((i & k) == 0)) { word[i] = b; word[i + j] = a; }
+            }
+            // 64 neighbouring pairs at a distance of up to 64 cover 128 words of one wavefront
+            const int next = j > 1 ? j / 2 : k;
+            if (j > 64 || next > 64) __syncthreads();
+            else wave_lds_fence();
+        }
+    __syncthreads();
+    for (int t = tid; t < n; t += 1024) {
+        keys[t] = word[t] >> 12;
+        ids[t] = idAt[word[t] & (kFrontSplats - 1)];
+    }
+    if (tid == 0) vs->nc = n;
 }
 
 // ---------------------------------------------------------------------------
@@ -1330,13 +1439,6 @@ __device__ __forceinline__ float hermite_rows(const float* sc, float tx, float t
         hprev = ha; ha = hn;
     }
     return w;
-}
-
-// orders the wavefront's LDS accesses (its LDS operations execute in order)
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // the degree-p expansion at scaled offset (tx, ty), its coefficients in LDS (read by
@@ -3929,31 +4031,36 @@ int build_structure(int N, int W, int H, double f, double smoothing, double prec
                     const float* sd, const TreeWs& w, hipStream_t st, int views = 1, VStride vsd = VStride{})
 {
     float Wf = (float)W, Hf = (float)H, ff = (float)f;
-    long nCull = (N + kCullTile - 1) / kCullTile;
-    long nSort = (N + kSortTile - 1) / kSortTile;
-    k_zero_state<<<dim3(1, views), 64, 0, st>>>(w.vs, vsd);
-    // 256 workgroups of 1024 threads per view: 16 waves per CU stream the splats,
-    // and the two sums take 512 device atomics (1M splats: 23.7 -> 17.2 us)
-    const unsigned bwBlocks = grid1(N, 1024) < 256u ? grid1(N, 1024) : 256u;
-    k_bandwidth<<<dim3(bwBlocks, views), 1024, 0, st>>>(N, Wf, Hf, ff, (float)smoothing, pts, nrm, sd, w.vs, w.hraw,
-                                                       vsd);
-    k_view_params<<<dim3(1, views), 64, 0, st>>>(w.vs, Wf, Hf, prec, vsd);
-    k_cull_count<<<dim3((unsigned)nCull, views), 256, 0, st>>>(N, Wf, Hf, ff, pts, w.vs, w.cullCounts, vsd);
-    k_scan_small<<<dim3(1, views), 1024, 0, st>>>(w.cullCounts, (int)nCull, &w.vs->nc, vsd);
-    k_cull_scatter<<<dim3((unsigned)nCull, views), 256, 0, st>>>(N, Wf, Hf, ff, pts, w.vs, w.cullCounts, w.keysB, w.idsB, vsd);
-    uint32_t* kin = w.keysB; uint32_t* kout = w.keysA;
-    int32_t* iin = w.idsB; int32_t* iout = w.idsA;
-    for (int shift = 0; shift < 24; shift += 8) {                  // 20-bit keys
-        k_sort_hist<<<dim3((unsigned)nSort, views), 256, 0, st>>>(w.vs, kin, shift, (int)nSort, w.sortHist, vsd);
-        k_sort_scan_digits<<<dim3(256, views), 256, 0, st>>>(w.sortHist, (int)nSort, w.scanBlocks, vsd);
-        k_sort_scan_top<<<dim3(1, views), 256, 0, st>>>(w.scanBlocks, vsd);
-        k_sort_scatter<<<dim3((unsigned)nSort, views), 256, 0, st>>>(w.vs, kin, iin, shift, (int)nSort, w.sortHist, w.scanBlocks,
-                                                        kout, iout, vsd);
-        uint32_t* tk = kin; kin = kout; kout = tk;
-        int32_t* ti = iin; iin = iout; iout = ti;
+    if (N <= kFrontSplats) {
+        k_front_small<<<dim3(1, views), 1024, 0, st>>>(N, Wf, Hf, ff, (float)smoothing, prec, pts, nrm, sd, w.vs, w.hraw,
+                                                       w.keysA, w.idsA, vsd);
+    } else {
+        long nCull = (N + kCullTile - 1) / kCullTile;
+        long nSort = (N + kSortTile - 1) / kSortTile;
+        k_zero_state<<<dim3(1, views), 64, 0, st>>>(w.vs, vsd);
+        // 256 workgroups of 1024 threads per view: 16 waves per CU stream the splats,
+        // and the two sums take 512 device atomics (1M splats: 23.7 -> 17.2 us)
+        const unsigned bwBlocks = grid1(N, 1024) < 256u ? grid1(N, 1024) : 256u;
+        k_bandwidth<<<dim3(bwBlocks, views), 1024, 0, st>>>(N, Wf, Hf, ff, (float)smoothing, pts, nrm, sd, w.vs, w.hraw,
+                                                           vsd);
+        k_view_params<<<dim3(1, views), 64, 0, st>>>(w.vs, Wf, Hf, prec, vsd);
+        k_cull_count<<<dim3((unsigned)nCull, views), 256, 0, st>>>(N, Wf, Hf, ff, pts, w.vs, w.cullCounts, vsd);
+        k_scan_small<<<dim3(1, views), 1024, 0, st>>>(w.cullCounts, (int)nCull, &w.vs->nc, vsd);
+        k_cull_scatter<<<dim3((unsigned)nCull, views), 256, 0, st>>>(N, Wf, Hf, ff, pts, w.vs, w.cullCounts, w.keysB, w.idsB, vsd);
+        uint32_t* kin = w.keysB; uint32_t* kout = w.keysA;
+        int32_t* iin = w.idsB; int32_t* iout = w.idsA;
+        for (int shift = 0; shift < 24; shift += 8) {                  // 20-bit keys
+            k_sort_hist<<<dim3((unsigned)nSort, views), 256, 0, st>>>(w.vs, kin, shift, (int)nSort, w.sortHist, vsd);
+            k_sort_scan_digits<<<dim3(256, views), 256, 0, st>>>(w.sortHist, (int)nSort, w.scanBlocks, vsd);
+            k_sort_scan_top<<<dim3(1, views), 256, 0, st>>>(w.scanBlocks, vsd);
+            k_sort_scatter<<<dim3((unsigned)nSort, views), 256, 0, st>>>(w.vs, kin, iin, shift, (int)nSort, w.sortHist, w.scanBlocks,
+                                                            kout, iout, vsd);
+            uint32_t* tk = kin; kin = kout; kout = tk;
+            int32_t* ti = iin; iin = iout; iout = ti;
+        }
     }
-    // after 3 passes the sorted data is in keysA / idsA
-    k_hierarchy<<<dim3(grid1(N, 256), views), 256, 0, st>>>(Wf, Hf, ff, pts, w.vs, kin, iin, w.geo, w.lnk, w.aux, w.leafXY,
+    // the sorted data is in keysA / idsA (three passes)
+    k_hierarchy<<<dim3(grid1(N, 256), views), 256, 0, st>>>(Wf, Hf, ff, pts, w.vs, w.keysA, w.idsA, w.geo, w.lnk, w.aux, w.leafXY,
                                                             w.flags, vsd);
     k_bottom_up_local<<<dim3(grid1(N, kFanBlock), views), kFanBlock, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, w.seeds, vsd);
     k_bottom_up_global<<<dim3(grid1(N, 256), views), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.aux, w.flags, w.seeds, vsd);
