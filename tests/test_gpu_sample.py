@@ -280,3 +280,23 @@ def test_sizes_around_one_workgroup(dev, N):
                                       seed=3, rate=3.0)
     rid, ripi, _, over = O.poisson_view(W, H, f, p, nb, sd, 40, 3.0, 0.0, 0.01, seed=3)
     assert not over and np.array_equal(ids[0].cpu().numpy(), rid) and np.array_equal(ipi[0].cpu().numpy(), ripi)
+
+
+@pytest.mark.parametrize("N", [4097, 5121, 65536, 131_071, 131_073, 262_144, 262_145, 300_000])
+def test_sort_and_cull_sizes(dev, N):
+    """Around the line between the sort's tiles, the counts that the cull's workgroups add up
+    themselves, and partial tiles, with most splats out of the frame in one view and all in
+    the other; a low precision keeps the trees shallow.  Density images equal to the
+    oracle's, which any splat lost or out of order changes."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng(N)
+    W, H, f = 24, 17, 30.0
+    p = rng.uniform([-1.0, -0.7, -4.0], [1.0, 0.7, -3.0], size=(2, N, 3)).astype(np.float32)
+    p[1, :, :2] *= 3.0
+    p[1, N // 3:N // 2, 2] *= -1.0
+    nb = np.tile(np.float32([0.0, 0.0, -1.0]), (2, N, 1))
+    sd = np.full((1, N, 2), 0.05, np.float32)
+    got = sampling.approximateFMMWeights(W, H, f, t(p, dev), t(nb, dev), None, t(sd, dev), 0.0, 0.05).cpu().numpy()
+    for b in range(2):
+        ref = O.fmm_weights_view(W, H, f, p[b], nb[b], sd[0], 0.0, 0.05)
+        assert np.array_equal(got[b], ref), b

@@ -56,7 +56,12 @@ constexpr int kTileInfo = 128 + 2 * kWalkEntries;
 // its up to 5 x 96 rows of values there
 __host__ __device__ constexpr int walk_extra(int L) { return 32 * (L > 3 ? L : 3); }
 constexpr int kCullTile = 1024;      // elements per workgroup in the cull pass
-constexpr int kSortTile = 2048;      // elements per workgroup in a sort pass
+// elements per workgroup in a sort pass: up to 128 workgroups of the smaller tile each add up
+// the others' histograms themselves, one launch less per pass and fewer rounds in each
+// (20 011 splats of two views: 12 sort launches of 55 us, here 6 of 34); beyond, the
+// histograms are scanned in a launch of their own
+constexpr int kSortTile = 2048, kSortTileSmall = 1024, kSortSelf = 128;
+inline int sort_tile(long n) { return n <= (long)kSortTileSmall * kSortSelf ? kSortTileSmall : kSortTile; }
 constexpr int kFixedDegree = 6;      // default expansion order of the fixed-order densities (hermitefmm.cuh:11)
 constexpr int kFixedPMin = 4, kFixedPMax = 8;              // orders ude_set_fixed_degree accepts
 constexpr int kFixedCoefsMax = (kFixedPMax + 1) * (kFixedPMax + 1);
@@ -180,7 +185,7 @@ size_t carve(void* ws, int N, int W, int H, int k, int mode, TreeWs* t)
     long n = N > 0 ? N : 1;
     long nn = 2 * n;
     long nCull = (n + kCullTile - 1) / kCullTile;
-    long nSort = (n + kSortTile - 1) / kSortTile;
+    long nSort = (n + sort_tile(n) - 1) / sort_tile(n);
     const bool fixedOrder = mode != kModeSample;
     long coefCap = (long)(kMaxDegree + 1) * (kMaxDegree + 1) * (n - 1 > 0 ? n - 1 : 1) + n;
     size_t off = 0;
@@ -565,7 +570,7 @@ __global__ __launch_bounds__(1024) void k_scan_small(int* data, int n, int* tota
 }
 
 __global__ __launch_bounds__(256) void k_cull_scatter(int N, float Wf, float Hf, float ff,
-                                                      const float* __restrict__ pts, const ViewState* __restrict__ vs,
+                                                      const float* __restrict__ pts, ViewState* vs,
                                                       const int* __restrict__ offs, uint32_t* __restrict__ keys,
                                                       int32_t* __restrict__ ids, VStride vsd)
 {
@@ -577,7 +582,13 @@ __global__ __launch_bounds__(256) void k_cull_scatter(int N, float Wf, float Hf,
     __shared__ int sh[4];
     ViewState v = *vs;
     int base = blockIdx.x * kCullTile;
-    int run = offs[blockIdx.x];
+    int run;
+    if (gridDim.x <= 256) {                                 // counts, not yet scanned: add those before
+        block_excl_scan((int)threadIdx.x < (int)blockIdx.x ? offs[threadIdx.x] : 0, sh, run);
+        if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) vs->nc = run + offs[blockIdx.x];
+    } else {
+        run = offs[blockIdx.x];
+    }
     for (int r = 0; r < kCullTile / 256; r++) {
         int e = base + r * 256 + threadIdx.x;
         float sx = 0.0f, sy = 0.0f;
@@ -597,6 +608,7 @@ __global__ __launch_bounds__(256) void k_cull_scatter(int N, float Wf, float Hf,
 // ---------------------------------------------------------------------------
 // LSD radix sort, 8-bit digits.  Histogram -> digit-major scan -> stable scatter.
 // ---------------------------------------------------------------------------
+template <int TILE>
 __global__ __launch_bounds__(256) void k_sort_hist(const ViewState* __restrict__ vs, const uint32_t* __restrict__ keys,
                                                    int shift, int nblk, int* __restrict__ hist, VStride vsd)
 {
@@ -607,13 +619,15 @@ __global__ __launch_bounds__(256) void k_sort_hist(const ViewState* __restrict__
     h[threadIdx.x] = 0;
     __syncthreads();
     int n = vs->nc;
-    int base = blockIdx.x * kSortTile;
-    for (int r = 0; r < kSortTile / 256; r++) {
+    int base = blockIdx.x * TILE;
+    for (int r = 0; r < TILE / 256; r++) {
         int e = base + r * 256 + threadIdx.x;
         if (e < n) atomicAdd(&h[(keys[e] >> shift) & 255u], 1);
     }
     __syncthreads();
-    hist[threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
+    // the smaller tile's histograms by workgroup, the larger's by digit for the scan
+    if (TILE == kSortTileSmall) hist[blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+    else hist[threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
 }
 
 // exclusive scan of hist[d][0..nblk) for each digit d (one workgroup per digit);
@@ -641,37 +655,42 @@ __global__ __launch_bounds__(256) void k_sort_scan_digits(int* hist, int nblk, i
     if (threadIdx.x == 0) tot[blockIdx.x] = carry;
 }
 
-// digit bases: exclusive scan of the 256 digit totals (in place)
-__global__ __launch_bounds__(256) void k_sort_scan_top(int* tot, VStride vsd)
-{
-    tot = vw(tot, vsd.ws);
-    __shared__ int sh[4];
-    int total;
-    int v = tot[threadIdx.x];
-    int ex = block_excl_scan(v, sh, total);
-    tot[threadIdx.x] = ex;
-}
-
+template <int TILE>
 __global__ __launch_bounds__(256) void k_sort_scatter(const ViewState* __restrict__ vs, const uint32_t* __restrict__ kin,
                                                       const int32_t* __restrict__ iin, int shift, int nblk,
-                                                      const int* __restrict__ hist, const int* __restrict__ digitBase,
+                                                      const int* __restrict__ hist, const int* __restrict__ digitTot,
                                                       uint32_t* __restrict__ kout, int32_t* __restrict__ iout, VStride vsd)
 {
     vs = vw(vs, vsd.ws);
     kin = vw(kin, vsd.ws);
     iin = vw(iin, vsd.ws);
     hist = vw(hist, vsd.ws);
-    digitBase = vw(digitBase, vsd.ws);
+    digitTot = vw(digitTot, vsd.ws);
     kout = vw(kout, vsd.ws);
     iout = vw(iout, vsd.ws);
     __shared__ int run[256];
     __shared__ int wc[4][256];
     int n = vs->nc;
-    int base = blockIdx.x * kSortTile;
-    run[threadIdx.x] = hist[threadIdx.x * nblk + blockIdx.x] + digitBase[threadIdx.x];
+    __shared__ int sh[4];
+    int base = blockIdx.x * TILE;
+    // this workgroup's place in each digit: those of the digits before, and of the same
+    // digit in the workgroups before
+    int tot = 0, pre = 0, all;
+    if (TILE == kSortTileSmall) {
+#pragma unroll 8
+        for (int q = 0; q < nblk; q++) {
+            const int v = hist[q * 256 + threadIdx.x];
+            tot += v;
+            pre += q < (int)blockIdx.x ? v : 0;
+        }
+    } else {
+        tot = digitTot[threadIdx.x];
+        pre = hist[threadIdx.x * nblk + blockIdx.x];
+    }
+    run[threadIdx.x] = block_excl_scan(tot, sh, all) + pre;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int r = 0; r < kSortTile / 256; r++) {
+    for (int r = 0; r < TILE / 256; r++) {
         for (int q = 0; q < 4; q++) wc[q][threadIdx.x] = 0;
         __syncthreads();
         int e = base + r * 256 + threadIdx.x;
@@ -4036,7 +4055,8 @@ int build_structure(int N, int W, int H, double f, double smoothing, double prec
                                                        w.keysA, w.idsA, vsd);
     } else {
         long nCull = (N + kCullTile - 1) / kCullTile;
-        long nSort = (N + kSortTile - 1) / kSortTile;
+        const bool small = sort_tile(N) == kSortTileSmall;
+        long nSort = (N + sort_tile(N) - 1) / sort_tile(N);
         k_zero_state<<<dim3(1, views), 64, 0, st>>>(w.vs, vsd);
         // 256 workgroups of 1024 threads per view: 16 waves per CU stream the splats,
         // and the two sums take 512 device atomics (1M splats: 23.7 -> 17.2 us)
@@ -4045,16 +4065,23 @@ int build_structure(int N, int W, int H, double f, double smoothing, double prec
                                                            vsd);
         k_view_params<<<dim3(1, views), 64, 0, st>>>(w.vs, Wf, Hf, prec, vsd);
         k_cull_count<<<dim3((unsigned)nCull, views), 256, 0, st>>>(N, Wf, Hf, ff, pts, w.vs, w.cullCounts, vsd);
-        k_scan_small<<<dim3(1, views), 1024, 0, st>>>(w.cullCounts, (int)nCull, &w.vs->nc, vsd);
+        // up to 256 counts the workgroups of the next launch add up themselves
+        if (nCull > 256) k_scan_small<<<dim3(1, views), 1024, 0, st>>>(w.cullCounts, (int)nCull, &w.vs->nc, vsd);
         k_cull_scatter<<<dim3((unsigned)nCull, views), 256, 0, st>>>(N, Wf, Hf, ff, pts, w.vs, w.cullCounts, w.keysB, w.idsB, vsd);
         uint32_t* kin = w.keysB; uint32_t* kout = w.keysA;
         int32_t* iin = w.idsB; int32_t* iout = w.idsA;
         for (int shift = 0; shift < 24; shift += 8) {                  // 20-bit keys
-            k_sort_hist<<<dim3((unsigned)nSort, views), 256, 0, st>>>(w.vs, kin, shift, (int)nSort, w.sortHist, vsd);
-            k_sort_scan_digits<<<dim3(256, views), 256, 0, st>>>(w.sortHist, (int)nSort, w.scanBlocks, vsd);
-            k_sort_scan_top<<<dim3(1, views), 256, 0, st>>>(w.scanBlocks, vsd);
-            k_sort_scatter<<<dim3((unsigned)nSort, views), 256, 0, st>>>(w.vs, kin, iin, shift, (int)nSort, w.sortHist, w.scanBlocks,
-                                                            kout, iout, vsd);
+            const dim3 grid((unsigned)nSort, views);
+            if (small) {
+                k_sort_hist<kSortTileSmall><<<grid, 256, 0, st>>>(w.vs, kin, shift, (int)nSort, w.sortHist, vsd);
+                k_sort_scatter<kSortTileSmall><<<grid, 256, 0, st>>>(w.vs, kin, iin, shift, (int)nSort, w.sortHist,
+                                                                     nullptr, kout, iout, vsd);
+            } else {
+                k_sort_hist<kSortTile><<<grid, 256, 0, st>>>(w.vs, kin, shift, (int)nSort, w.sortHist, vsd);
+                k_sort_scan_digits<<<dim3(256, views), 256, 0, st>>>(w.sortHist, (int)nSort, w.scanBlocks, vsd);
+                k_sort_scatter<kSortTile><<<grid, 256, 0, st>>>(w.vs, kin, iin, shift, (int)nSort, w.sortHist,
+                                                                w.scanBlocks, kout, iout, vsd);
+            }
             uint32_t* tk = kin; kin = kout; kout = tk;
             int32_t* ti = iin; iin = iout; iout = ti;
         }
