@@ -185,3 +185,29 @@ def test_host_indices_of_consecutive_frames(dev):
     with pytest.raises(ValueError):
         r.forward(*args, transformMatrix=t(sc.view)[None])
     assert torch.equal(r.indices, kept[0][0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("N,bd", [(0, 1), (1, 1), (5, 2), (4099, 1)])
+def test_forward_harmonics_formula(dev, N, bd, dtype):
+    """Per-splat shading against the quadratic forms written out in float64, with one set of
+    colours or several; sums of 16 products of numbers below 4."""
+    from splatting_amd.shading import ForwardSphericalHaromic
+    rng = np.random.default_rng(N)
+    m = ForwardSphericalHaromic().to(dev).to(dtype)
+    n = torch.tensor(rng.normal(size=(1, N, 3)), device=dev, dtype=dtype, requires_grad=True)
+    d = torch.tensor(rng.uniform(size=(bd, N, 3)), device=dev, dtype=dtype, requires_grad=True)
+    out = m(n, d)
+    M = m.buildShMatrix().detach().double()[0]
+    n4 = torch.cat([n.detach().double(), torch.ones((1, N, 1), device=dev, dtype=torch.float64)], -1)
+    n4.requires_grad_(True)
+    d64 = d.detach().double().requires_grad_(True)
+    ref = d64 * torch.stack([((n4 @ M[c]) * n4).sum(-1) for c in range(3)], -1) / np.pi
+    assert out.shape == (bd, N, 3) and out.is_contiguous()
+    tol = 256 * float(torch.finfo(dtype).eps)
+    assert torch.allclose(out.double(), ref, rtol=0.0, atol=tol)
+    g = torch.tensor(rng.normal(size=(bd, N, 3)), device=dev, dtype=dtype)
+    a = torch.autograd.grad(out, (n, d), g)
+    b = torch.autograd.grad(ref, (n4, d64), g.double())
+    assert torch.allclose(a[0].double(), b[0][..., :3], rtol=0.0, atol=4 * tol)
+    assert torch.allclose(a[1].double(), b[1], rtol=0.0, atol=4 * tol)
