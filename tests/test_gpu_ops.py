@@ -181,6 +181,30 @@ def test_filter_equal_depths(dev, k):
     assert np.abs(wrong - ref).max() > 1e-2
 
 
+@pytest.mark.parametrize("W,H,bn", [(5, 3, 2), (256, 86, 3), (181, 121, 3), (219, 200, 3)])
+@pytest.mark.parametrize("k", [1, 16, 31, 32, 33, 64])
+def test_filter_pixels_per_wave(dev, k, W, H, bn):
+    """One pixel per wavefront, several, and two at a time in halves, around their slot
+    counts: partial groups, groups that run into the next view, points per view, many equal
+    depths.  Bounds as for the wider kernels."""
+    from cudaExtensions import filtering
+    sc, p, n, nb, sd = scene_inputs(2, sd_scale=8.0)[:5]
+    rng = np.random.default_rng(277 + k)
+    P = np.stack([p * np.float32(1 + 0.1 * b) for b in range(bn)])
+    Nn = np.stack([n] * bn)
+    idx = rng.integers(0, 40, size=(bn, W, H, k)).astype(np.int32)
+    idx[rng.uniform(size=idx.shape) < 0.3] = -1
+    w = rng.uniform(0.0, 1.0, size=idx.shape).astype(np.float32)
+    g = rng.normal(size=idx.shape).astype(np.float32)
+    a = (W, H, sc.focal)
+    out = filtering.forward(t(idx, dev), t(w, dev), *a, t(P, dev), t(Nn, dev))
+    assert_close(out.cpu().numpy(), O.filter_forward(idx, w, *a, P, Nn), max(RTOL, 2 * k * 2.0 ** -24), "filter forward")
+    gw = filtering.backward(t(idx, dev), t(w, dev), t(g, dev), *a, t(P, dev), t(Nn, dev))
+    rg = O.filter_backward(idx, w, g, *a, P, Nn)
+    mg = magnitude(O.filter_backward, idx, w, g, *a, P, Nn)
+    assert_close(gw.cpu().numpy(), rg, RTOL, "filter backward", mag=mg, ops=max(64, 4 * k))
+
+
 @pytest.mark.parametrize("splats", [3, 400])
 @pytest.mark.parametrize("k", [65, 127, 128, 129, 250, 256, 257, 319, 1024])
 def test_filter_wide(dev, k, splats):

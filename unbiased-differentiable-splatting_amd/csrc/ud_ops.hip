@@ -9,6 +9,7 @@
 // Layouts follow the reference op surface: slot tensors are x-major
 // (bn, W, H, k) with pixel (i = x, j = y) at j + H (i + W b); point tensors
 // are (bn, N, 3) fp32, std-devs (1 | bn, N, 2).
+#include <type_traits>
 #include "ud_device.h"
 #include "../../include/udsplat.h"
 
@@ -677,7 +678,7 @@ __device__ __forceinline__ C dot3c(const C* a, const C* b)
 }
 
 template <class C>
-__device__ __forceinline__ C ray_depth(int i, int j, C Wf, C Hf, C ff, const C* p, const C* n)
+__device__ __forceinline__ void view_ray(int i, int j, C Wf, C Hf, C ff, C* dir)
 {
     C bx = (Wf - C(2) * (C)i) / (C(2) * ff);
     C by = -((Hf - C(2) * (C)j) / (C(2) * ff));
@@ -686,11 +687,22 @@ __device__ __forceinline__ C ray_depth(int i, int j, C Wf, C Hf, C ff, const C* 
     nn = nn + by * by;
     nn = nn + bz * bz;
     C inv = C(1) / sqrt(nn);
-    C dir[3] = { -(bx * inv), -(by * inv), -(bz * inv) };
+    dir[0] = -(bx * inv); dir[1] = -(by * inv); dir[2] = -(bz * inv);
+}
+template <class C>
+__device__ __forceinline__ C plane_depth(const C* dir, const C* p, const C* n)
+{
     C num = dot3c(p, n);
     C den = dot3c(dir, n);
     C d = num / den;
     return (d > C(0)) ? d : C(10000);
+}
+template <class C>
+__device__ __forceinline__ C ray_depth(int i, int j, C Wf, C Hf, C ff, const C* p, const C* n)
+{
+    C dir[3];
+    view_ray<C>(i, j, Wf, Hf, ff, dir);
+    return plane_depth<C>(dir, p, n);
 }
 
 // Cross-lane moves of the 64-lane wavefront through DPP (gfx9 controls:
@@ -716,7 +728,7 @@ __device__ __forceinline__ double dpp_from(double ident, double v)
 // rows, then the row broadcasts).
 template <int CTRL, int RM, class C>
 __device__ __forceinline__ void prod_step(C& v) { v = v * dpp_from<CTRL, RM>(C(1), v); }
-template <class C>
+template <int LANES = 64, class C>
 __device__ __forceinline__ C wave_prod_incl(C v)
 {
     prod_step<0x111, 0xf>(v);
@@ -724,7 +736,7 @@ __device__ __forceinline__ C wave_prod_incl(C v)
     prod_step<0x114, 0xf>(v);
     prod_step<0x118, 0xf>(v);
     prod_step<0x142, 0xa>(v);
-    prod_step<0x143, 0xc>(v);
+    if (LANES == 64) prod_step<0x143, 0xc>(v);
     return v;
 }
 
@@ -738,7 +750,7 @@ __device__ __forceinline__ void affine_step(C& A, C& B)
     A = A + B * tA;
     B = B * tB;
 }
-template <class C>
+template <int LANES = 64, class C>
 __device__ __forceinline__ void wave_affine_incl(C& A, C& B)
 {
     affine_step<0x111, 0xf>(A, B);
@@ -746,7 +758,19 @@ __device__ __forceinline__ void wave_affine_incl(C& A, C& B)
     affine_step<0x114, 0xf>(A, B);
     affine_step<0x118, 0xf>(A, B);
     affine_step<0x142, 0xa>(A, B);
-    affine_step<0x143, 0xc>(A, B);
+    if (LANES == 64) affine_step<0x143, 0xc>(A, B);
+}
+
+// v of a lane (its number uniform), the same in every lane
+__device__ __forceinline__ float lane_value(float v, int lane)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+    const long long a = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)a, lane), hi = __builtin_amdgcn_readlane((int)(a >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
 // Sum over the lanes, in lane 63 (zeros come in at the ends of the shifts).
@@ -779,7 +803,14 @@ __device__ __forceinline__ double quiet_nan(double) { return __longlong_as_doubl
 // get the same first term, so each ORs its bit into the mask at that index and
 // the second term is the count of mask bits below the lane.  Depths are never
 // NaN (ray_depth maps a non-positive or NaN quotient to 10000).
-template <bool BACKWARD, class S>
+// A wavefront takes one pixel, or TURNS of them one after another (two at a time, in
+// halves of 32 lanes, up to 32 slots), whose view rays its lanes work out first, a pixel
+// per lane.  Bound by instruction issue and, with more splats than an L2 holds, by the
+// reads of their planes.  Forward / backward against one pixel per wavefront: 640x480,
+// k = 24 in halves 99 / 111 -> 49 / 55 us (one pixel per half 67 / 73); four views of
+// 301x203, k = 40 under 60 003 splats 93 / 103 -> 82 / 93; 512x512 under 1M the same
+// 104 / 117; 128x128 pixels, too few for several each, 9.7 / 10.6 against 11.1 / 11.8.
+template <bool BACKWARD, int LANES, int TURNS, class S>
 __global__ __launch_bounds__(256) void k_filter_wave(long npix, int N, int W, int H, int k,
                                                      typename CompOf<S>::type ff, typename CompOf<S>::type gate,
                                                      const int32_t* __restrict__ idx, const S* __restrict__ wts,
@@ -788,88 +819,108 @@ __global__ __launch_bounds__(256) void k_filter_wave(long npix, int N, int W, in
                                                      S* __restrict__ out)
 {
     using C = typename CompOf<S>::type;
+    constexpr int AT = 64 / LANES;                      // pixels at a time
     __shared__ C sbuf[4][2][64];
     __shared__ C skey[4][64];
     __shared__ unsigned long long sgrp[4][64];
-    // the wavefront index is uniform: read it into a scalar so the pixel
-    // arithmetic below runs on the scalar unit
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), s = threadIdx.x & 63;
-    long pix = (long)blockIdx.x * 4 + wv;
-    if (pix >= npix) return;   // whole wave exits together
-    long b = pix / ((long)W * H);
-    int r = (int)(pix - b * (long)W * H);
-    int i = r / H, j = r - (r / H) * H;
-    long base = pix * k;
-    const bool act = s < k;
-    int id = act ? idx[base + s] : -1;
-    C w = act ? ld_c(wts, base + s) : C(0);
-    C gi = (BACKWARD && act) ? ld_c(gin, base + s) : C(0);
-    C d = C(10000);
-    if (id >= 0) {
-        long po = 3 * ((pb > 1 ? b * N : 0) + id);
-        C p[3] = { ld_c(pts, po), ld_c(pts, po + 1), ld_c(pts, po + 2) };
-        C n[3] = { ld_c(nrm, po), ld_c(nrm, po + 1), ld_c(nrm, po + 2) };
-        d = ray_depth<C>(i, j, (C)W, (C)H, ff, p, n);
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int s = lane & (LANES - 1), half = lane - s;  // slot; first lane of the pixel
+    const long first = ((long)blockIdx.x * 4 + wv) * (TURNS * AT);
+    if (first >= npix) return;                          // whole wave exits together
+    // lane q: the ray of pixel first + q (TURNS * AT <= 64); one pixel: every lane its ray
+    const uint32_t perView = (uint32_t)W * (uint32_t)H;
+    const long view0 = first / perView;                 // wave-uniform
+    const uint32_t at0 = (uint32_t)(first - view0 * perView);
+    C ray[3];
+    {
+        const uint32_t r = TURNS * AT == 1 ? at0 : (at0 + (uint32_t)lane) % perView;
+        const int i = (int)(r / (uint32_t)H), j = (int)(r - (uint32_t)i * (uint32_t)H);
+        view_ray<C>(i, j, (C)W, (C)H, ff, ray);
     }
     C* key = skey[wv];
-    key[s] = act ? d : quiet_nan(C(0));
-    sgrp[wv][s] = 0ull;
-    __builtin_amdgcn_wave_barrier();
-    int lt = 0;
-    const int k16 = (k + 15) & ~15;   // <= 64: the reads stay inside the row
-    for (int q0 = 0; q0 < k16; q0 += 16) {
-        C kq[16];
-#pragma unroll
-        for (int q = 0; q < 16; q++) kq[q] = key[q0 + q];
-#pragma unroll
-        for (int q = 0; q < 16; q++) lt += kq[q] < d;
-    }
-    if (act) atomicOr(&sgrp[wv][lt], 1ull << s);
-    __builtin_amdgcn_wave_barrier();
-    const unsigned long long grp = act ? sgrp[wv][lt] : 0ull;
-    const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(grp >> 32),
-                                                     __builtin_amdgcn_mbcnt_lo((unsigned)grp, lt));
-    // exclusive prefix product of (1 - w) in rank order
     C* sa = sbuf[wv][0];
     C* sb = sbuf[wv][1];
-    sb[s] = C(1);
-    if (BACKWARD) sa[s] = C(0);
-    __builtin_amdgcn_wave_barrier();
-    if (act) {
-        sb[rank] = C(1) - w;
-        if (BACKWARD) sa[rank] = gi * w;
+#pragma unroll 1
+    for (int turn = 0; turn < TURNS; turn++) {
+        const long pix0 = first + turn * AT;            // wave-uniform
+        if (pix0 >= npix) break;
+        const int sub = AT == 1 ? 0 : half >> 5;
+        const long pix = pix0 + sub;
+        const bool act = s < k && (AT == 1 || pix < npix);
+        C dir[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) dir[c] = TURNS * AT == 1 ? ray[c] : AT == 1 ? lane_value(ray[c], turn) : __shfl(ray[c], turn * AT + sub, 64);
+        const long base = pix * k;
+        const int id = act ? idx[base + s] : -1;
+        const C w = act ? ld_c(wts, base + s) : C(0);
+        const C gi = (BACKWARD && act) ? ld_c(gin, base + s) : C(0);
+        C d = C(10000);
+        if (id >= 0) {
+            const long po = 3 * ((pb > 1 ? (view0 + (at0 + (uint32_t)(turn * AT + sub)) / perView) * N : 0) + id);
+            C p[3] = { ld_c(pts, po), ld_c(pts, po + 1), ld_c(pts, po + 2) };
+            C n[3] = { ld_c(nrm, po), ld_c(nrm, po + 1), ld_c(nrm, po + 2) };
+            d = plane_depth<C>(dir, p, n);
+        }
+        key[lane] = act ? d : quiet_nan(C(0));
+        sgrp[wv][lane] = 0ull;
+        wave_order();
+        int lt = 0;
+        const int k16 = (k + 15) & ~15;                 // <= LANES: the reads stay inside the row
+        for (int q0 = 0; q0 < k16; q0 += 16) {
+            C kq[16];
+#pragma unroll
+            for (int q = 0; q < 16; q++) kq[q] = key[half + q0 + q];
+#pragma unroll
+            for (int q = 0; q < 16; q++) lt += kq[q] < d;
+        }
+        if (act) atomicOr(&sgrp[wv][half + lt], 1ull << s);
+        wave_order();
+        const unsigned long long grp = act ? sgrp[wv][half + lt] : 0ull;
+        const int rank = AT == 1 ? (int)__builtin_amdgcn_mbcnt_hi((unsigned)(grp >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)grp, lt))
+                                 : lt + __popc((unsigned)grp & ((1u << s) - 1u));
+        // exclusive prefix product of (1 - w) in rank order
+        sb[lane] = C(1);
+        if (BACKWARD) sa[lane] = C(0);
+        wave_order();
+        if (act) {
+            sb[half + rank] = C(1) - w;
+            if (BACKWARD) sa[half + rank] = gi * w;
+        }
+        wave_order();
+        const C incl = wave_prod_incl<LANES>(sb[lane]);
+        // transmittance in front of this slot: the inclusive product of the rank before it
+        C rem = __shfl(incl, half + (rank > 0 ? rank - 1 : 0), 64);
+        if (rank == 0) rem = C(1);
+        if (!BACKWARD) {
+            if (act) st_c(out, base + s, rem * w);
+            wave_order();
+            continue;
+        }
+        // backward (alphacompositingGrad.cuh:7-26).  In depth order, with T_r the
+        // transmittance in front of rank r, the reference's sum
+        //   g_r = [|w_r| > eps] gin_r out_r / w_r - [|1 - w_r| > eps] sum_{i>r} gin_i out_i / (1 - w_r)
+        // is [|w_r| > eps] gin_r T_r - [|1 - w_r| > eps] T_r S_r with
+        //   S_r = sum_{i>r} gin_i w_i prod_{r<t<i} (1 - w_t),
+        // the suffix recurrence S_r = a_{r+1} + b_{r+1} S_{r+1} (a = gin w, b = 1 - w).
+        // Nothing is divided, so a small w or 1 - w amplifies no rounding.
+        // Lane l of the pixel holds the affine map x -> A + B x of rank LANES - 1 - l
+        // (identity past the last slot); the inclusive scan composes ranks LANES - 1 ..
+        // LANES - 1 - l, outer (smaller rank) applied last.
+        C A = sa[half + LANES - 1 - s], B = sb[half + LANES - 1 - s];
+        wave_affine_incl<LANES>(A, B);
+        // S_r = U_{r+1}, held by lane LANES - 1 - (r + 1)
+        const int src = LANES - 2 - rank;
+        C after = __shfl(A, half + (src < 0 ? 0 : src), 64);
+        if (rank == LANES - 1) after = C(0);
+        // the reference's gates (|w| > 1e-4, |1 - w| > 1e-4); gate < 0 keeps every term
+        // (the exact derivative: nothing here is divided, so no term needs dropping)
+        C g = C(0);
+        if (fabs(w) > gate) g += gi * rem;
+        if (fabs(C(1) - w) > gate) g -= rem * after;
+        if (act) st_c(out, base + s, g);
+        wave_order();
     }
-    __builtin_amdgcn_wave_barrier();
-    const C incl = wave_prod_incl(sb[s]);
-    // transmittance in front of this slot: the inclusive product of the rank before it
-    C rem = __shfl(incl, rank > 0 ? rank - 1 : 0, 64);
-    if (rank == 0) rem = C(1);
-    if (!BACKWARD) {
-        if (act) st_c(out, base + s, rem * w);
-        return;
-    }
-    // backward (alphacompositingGrad.cuh:7-26).  In depth order, with T_r the
-    // transmittance in front of rank r, the reference's sum
-    //   g_r = [|w_r| > eps] gin_r out_r / w_r - [|1 - w_r| > eps] sum_{i>r} gin_i out_i / (1 - w_r)
-    // is [|w_r| > eps] gin_r T_r - [|1 - w_r| > eps] T_r S_r with
-    //   S_r = sum_{i>r} gin_i w_i prod_{r<t<i} (1 - w_t),
-    // the suffix recurrence S_r = a_{r+1} + b_{r+1} S_{r+1} (a = gin w, b = 1 - w).
-    // Nothing is divided, so a small w or 1 - w amplifies no rounding.
-    // Lane l holds the affine map x -> A + B x of rank 63 - l (identity past the
-    // last slot); the inclusive scan composes ranks 63 .. 63 - l, outer (smaller
-    // rank) applied last.
-    C A = sa[63 - s], B = sb[63 - s];
-    wave_affine_incl(A, B);
-    // S_r = U_{r+1}, held by lane 63 - (r + 1)
-    int src = 62 - rank;
-    C after = __shfl(A, src < 0 ? 0 : src, 64);
-    if (rank == 63) after = C(0);
-    // the reference's gates (|w| > 1e-4, |1 - w| > 1e-4); gate < 0 keeps every term
-    // (the exact derivative: nothing here is divided, so no term needs dropping)
-    C g = C(0);
-    if (fabs(w) > gate) g += gi * rem;
-    if (fabs(C(1) - w) > gate) g -= rem * after;
-    if (act) st_c(out, base + s, g);
 }
 
 // 64 < k <= 256: one wavefront per pixel, ROWS = 2 or 4 slots per lane (slot
@@ -1972,9 +2023,17 @@ int filter_t(int bn, int N, int W, int H, int k, double f, const int32_t* idx, c
     if (bn <= 0 || W <= 0 || H <= 0 || k <= 0 || k > 1024 || (pb != 1 && pb != bn)) return UDE_ERR_ARG;
     long npix = (long)bn * W * H;
     const C gate = exact ? C(-1) : C(1e-4);
-    if (k <= 64)
-        k_filter_wave<BWD, S><<<grid1(npix, 4), 256, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx, wts, gin, pts, nrm,
-                                                               pb, out);
+    // several pixels per wavefront where that still leaves each of the 1024 SIMDs eight wavefronts
+    // in halves, sixteen whole ones
+    auto wave = [&](auto lanes, auto turns) {
+        constexpr int L = decltype(lanes)::value, T = decltype(turns)::value;
+        k_filter_wave<BWD, L, T, S><<<grid1(npix, 4 * (64 / L) * T), 256, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx, wts,
+                                                                                   gin, pts, nrm, pb, out);
+    };
+    using std::integral_constant;
+    if (k <= 32 && npix >= 1024L * 8 * 8) wave(integral_constant<int, 32>{}, integral_constant<int, 4>{});
+    else if (k <= 64 && npix >= 1024L * 16 * 8) wave(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+    else if (k <= 64) wave(integral_constant<int, 64>{}, integral_constant<int, 1>{});
     else if (k <= 128)
         k_filter_rows<BWD, 2, S><<<grid1(npix, 4), 256, 0, st>>>(npix, N, W, H, k, (C)f, gate, idx, wts, gin, pts, nrm,
                                                                  pb, out);
