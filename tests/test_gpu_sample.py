@@ -300,3 +300,37 @@ def test_sort_and_cull_sizes(dev, N):
     for b in range(2):
         ref = O.fmm_weights_view(W, H, f, p[b], nb[b], sd[0], 0.0, 0.05)
         assert np.array_equal(got[b], ref), b
+
+
+@pytest.mark.parametrize("k", [2, 9, 16, 23, 24, 25])
+def test_sample_draws_in_halves(dev, k):
+    """Two pixels per wavefront up to k = 24: on an image whose sides are no multiples of the
+    tile, with more candidates than a half holds at most pixels and none at others."""
+    from cudaExtensions import sampling
+    sc, p, n, nb, sd = scene_inputs(0, sd_scale=4.0)
+    W, H, f = 45, 31, 0.5 * 45
+    got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), t(sd[None], dev), t(sd[None], dev), k, 0.0,
+                          0.01, seed=k)
+    sampling.check_errors()
+    ref = O.sample_view(W, H, f, p, nb, sd, k, 0.0, 0.01, seed=k)
+    assert (ref >= 0).any() and (ref < 0).any()
+    assert np.array_equal(got[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("seed,ties", [(1, 2), (2, 1), (0, 0)])
+def test_sample_equal_keys_in_halves(dev, seed, ties):
+    """Equal keys among a half's 24 slots: 24 copies of a splat at every pixel centre, whose
+    keys are the 24-bit uniforms themselves."""
+    from cudaExtensions import sampling
+    W = H = 96
+    f = 128.0
+    ii, jj = np.meshgrid(np.arange(W), np.arange(H), indexing="ij")
+    x = (ii - W / 2).ravel().astype(np.float32)
+    y = (H / 2 - jj).ravel().astype(np.float32)
+    P = np.repeat(np.stack([x, y, np.full_like(x, -f)], 1), 24, 0).astype(np.float32)
+    N = np.tile(np.float32([0.0, 0.0, 1.0]), (P.shape[0], 1))
+    S = np.full((P.shape[0], 2), 1.0, np.float32)
+    ref = O.sample_view(W, H, f, P, N, S, 24, 0.0, 0.01, seed=seed)
+    assert O.tie_pixels() == ties
+    got = sampling.sample(W, H, f, t(P[None], dev), t(N[None], dev), None, t(S[None], dev), 24, 0.0, 0.01, seed=seed)
+    assert np.array_equal(got[0].cpu().numpy(), ref)
