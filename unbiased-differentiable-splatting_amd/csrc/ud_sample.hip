@@ -2916,6 +2916,7 @@ __global__ __launch_bounds__(64) void k_sample_replay(int W, int H, int k, int L
                     // every shuffle runs on all 64 lanes; lane 0 then takes row r - 1's
                     // lane 63 (or nothing in row 0) as its predecessor
                     int start[kReplayRows];
+                    unsigned long long before[kReplayRows];               // the entry ahead of each
                     int carry = -1;
 #pragma unroll
                     for (int r = 0; r < kReplayRows; r++) {
@@ -2924,16 +2925,11 @@ __global__ __launch_bounds__(64) void k_sample_replay(int W, int H, int k, int L
                         const unsigned long long up = __shfl_up(v[r], 1, 64);
                         const unsigned long long wrap = __shfl(v[r > 0 ? r - 1 : 0], 63, 64);
                         const unsigned long long prev = lane > 0 ? up : r > 0 ? wrap : empty;
+                        before[r] = prev;
                         const bool st = pos >= s0 && pos < k && (pos == s0 || key_of(v[r]) != key_of(prev));
-                        int m = st ? pos : -1;
-#pragma unroll
-                        for (int o = 1; o < 64; o <<= 1) {
-                            const int u = __shfl_up(m, o, 64);
-                            if (lane >= o && u > m) m = u;
-                        }
-                        if (m < carry) m = carry;
-                        start[r] = m;
-                        carry = __shfl(m, 63, 64);
+                        const unsigned long long sm = __ballot(st), upto = sm & ((2ull << lane) - 1ull);
+                        start[r] = upto ? r * 64 + 63 - __clzll((long long)upto) : carry;
+                        if (sm) carry = r * 64 + 63 - __clzll((long long)sm);
                     }
                     // the first entry of the run ending at pos - 1: start of pos - 1, then its entry
                     unsigned long long nv[kReplayRows];
@@ -2951,12 +2947,9 @@ __global__ __launch_bounds__(64) void k_sample_replay(int W, int H, int k, int L
                             const unsigned long long g = __shfl(v[rr], sp & 63, 64);
                             if (sp >= 0 && (sp >> 6) == rr) from = g;
                         }
-                        const unsigned long long up = __shfl_up(v[r], 1, 64);
-                        const unsigned long long wrap = __shfl(v[r > 0 ? r - 1 : 0], 63, 64);
-                        const unsigned long long prev = lane > 0 ? up : r > 0 ? wrap : empty;
                         // inside a run (the empty slots, which end a list that is not full,
                         // are one run: a carried empty slot ends the insertion there)
-                        const bool inside = pos > s0 && key_of(v[r]) == key_of(prev);
+                        const bool inside = pos > s0 && key_of(v[r]) == key_of(before[r]);
                         nv[r] = pos >= k ? empty : pos < s0 ? v[r] : pos == s0 ? c : inside ? v[r] : from;
                     }
 #pragma unroll
