@@ -104,6 +104,12 @@ __device__ __forceinline__ float plog1mf(float u)
 // ---------------------------------------------------------------------------
 struct u32x4 { uint32_t x, y, z, w; };
 
+// a ^ b ^ c in one instruction (0x96: the truth table of three-input exclusive or)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+}
+
 __device__ __forceinline__ u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1)
 {
 #pragma unroll
@@ -115,9 +121,9 @@ __device__ __forceinline__ u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1
         const uint32_t lo0 = (uint32_t)p0, hi0 = (uint32_t)(p0 >> 32);
         const uint32_t lo1 = (uint32_t)p1, hi1 = (uint32_t)(p1 >> 32);
         u32x4 n;
-        n.x = hi1 ^ c.y ^ k0;
+        n.x = xor3(hi1, c.y, k0);
         n.y = lo1;
-        n.z = hi0 ^ c.w ^ k1;
+        n.z = xor3(hi0, c.w, k1);
         n.w = lo0;
         c = n;
     }
