@@ -3844,17 +3844,17 @@ __global__ void k_zero_f64(double* p, size_t stride, int views)
 // (tile maxima 130 and 75), but the pixels find their ranges at different nodes: thinned
 // on the spot, every visit waited for some lane's steps.  Bound by instruction issue (a
 // thinning step is a Philox block, a logarithm and a mixture).  16 views of 640x480 under
-// 2M splats: 5.85 -> 3.91 ms (512x512, 1M: 578 -> 368 us); queues of 2, 3, 6 ranges take
-// 4.37, 4.21, 4.21 against 4.15 ms here (before the branch-free exponential), walking
-// at twice as many thinning lanes 4.48, thinning at twice as many walking ones 4.47.  One
-// walk over the union of the tile's nodes with scalar loads visits 392 nodes: 7.24 ms.
+// 2M splats: 5.85 -> 3.47 ms (512x512, 1M: 578 -> 322 us); queues of 2, 4, 6 ranges take
+// 3.63, 3.49, 3.74 ms, walking only at 4/3 of the thinning lanes (or already at 3/4)
+// is 1 % slower.  One walk over the union of the tile's nodes with scalar loads visits
+// 392 nodes: 7.24 ms.
 // The first kPoissonStage samples of each lane are staged in LDS (slot-major,
 // [slot][lane], so the stores hit 64 distinct banks) and written out at
 // the end together with the empty slots, one tile row (2^lth contiguous pixels
 // x kcap slots) per coalesced pass of the wavefront; only samples past the
 // staged ones are stored directly.  A lane's scattered 4-byte stores would
 // otherwise leave partly written lines in L2 for the length of the walk.
-constexpr int kPoissonQueue = 4;
+constexpr int kPoissonQueue = 3;
 
 constexpr int kPoissonStage = 16;
 constexpr size_t kPoissonStageBytes = (size_t)kPoissonStage * 64 * 8;    // per wavefront
@@ -3946,68 +3946,77 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_poisson(TileCfg cfg,
         int nd = draws ? 0 : -1;
         int visits = 0;                               // a preorder walk visits each node at most once
         PNode pn = pnode[0];
+        // Both steps run in all lanes and select what a lane keeps: branches around the state
+        // (queue, node record) copied it at every join (3.78 ms).
         while (true) {
             const bool walks = nd >= 0 && cnt < kPoissonQueue, thins = cnt > 0;
             const unsigned long long mw = __ballot(walks), mt = __ballot(thins);
             if (!(mw | mt)) break;
             if (__popcll(mw) >= __popcll(mt)) {
-                if (!walks) continue;
                 float cx = fminf(fmaxf(qx, pn.lox), pn.hix);
                 float cy = fminf(fmaxf(qy, pn.loy), pn.hiy);
                 const float d2b = dist2(qx, qy, cx, cy);
                 // proposal bound over the node
                 float pB = fmode ? foot_mix(k1, a1, kf, d2b, foot_bound(a1, d2b)) : mix_d2(k0, a0, k1, a1, d2b);
-                float U = fminf(1.0f, lam * pB);
-                nd = pn.left;
-                if (!(pB >= kProposalPMin && U > 0.0f)) nd = pn.esc;      // past the subtree
-                else if (nd < 0 || !((float)(pn.last - pn.first + 1) * U > 1.0f)) {
-                    nd = pn.esc;
+                const float U = fminf(1.0f, lam * pB);
+                // outside the support: past the subtree; a leaf or few enough: thinned
+                const bool in = pB >= kProposalPMin && U > 0.0f;
+                const bool push = walks && in && (pn.left < 0 || !((float)(pn.last - pn.first + 1) * U > 1.0f));
+                const int to = in && !push ? pn.left : pn.esc;
 #pragma unroll
-                    for (int q = 0; q < kPoissonQueue; q++)
-                        if (cnt == q) { qpos[q] = pn.first - 1; qlast[q] = pn.last; qU[q] = U; }
-                    cnt++;
+                for (int q = 0; q < kPoissonQueue; q++) {
+                    const bool here = push && cnt == q;
+                    qpos[q] = here ? pn.first - 1 : qpos[q];
+                    qlast[q] = here ? pn.last : qlast[q];
+                    qU[q] = here ? U : qU[q];
                 }
-                if (++visits > 2 * n) { atomicOr(err, 8); nd = -1; }
-                if (nd >= 0) pn = pnode[nd];          // on its way while others thin
-            } else if (thins) {
+                cnt += push;
+                nd = walks ? to : nd;
+                visits += walks;
+                if (__ballot(visits > 2 * n)) {              // never
+                    if (visits > 2 * n) { atomicOr(err, 8); nd = -1; }
+                }
+                pn = pnode[nd >= 0 ? nd : 0];                // on its way while others thin
+            } else {
                 // one Philox block per step: word x draws the skip, word y the acceptance test
-                if (fresh) { il1 = 1.0f / plog1mf(qU[0]); fresh = false; }
+                if (thins && fresh) { il1 = 1.0f / plog1mf(qU[0]); fresh = false; }
                 const u32x4 blk = philox4x32_10(u32x4{ step, 0x80000000u, pixel, view }, seedLo, seedHi);
-                step++;
-                float u = u01(blk.x);
-                float r = plogf_normal(u) * il1;      // failures before the next candidate
-                if (!(r < (float)(qlast[0] - qpos[0]))) {
-#pragma unroll
-                    for (int q = 0; q + 1 < kPoissonQueue; q++) {
-                        qpos[q] = qpos[q + 1]; qlast[q] = qlast[q + 1]; qU[q] = qU[q + 1];
+                step += thins;
+                const float r = plogf_normal(u01(blk.x)) * il1;       // failures before the next candidate
+                const bool cand = thins && r < (float)(qlast[0] - qpos[0]), pop = thins && !cand;
+                const int pos = cand ? qpos[0] + (int)r + 1 : 0;
+                if (cand) {
+                    float pl;
+                    if (fmode) {
+                        const FootLeaf L = footLeaf[pos];
+                        const float d2 = dist2(qx, qy, L.x, L.y);
+                        pl = foot_mix(k1, a1, kf, d2, foot_leaf(L, a1, qx, qy, d2));
+                    } else {
+                        const float2 lp = leafXY[pos];
+                        pl = mix_d2(k0, a0, k1, a1, dist2(qx, qy, lp.x, lp.y));
                     }
-                    cnt--;
-                    fresh = true;
-                    continue;
+                    const float pi = fminf(1.0f, lam * pl);
+                    const float a = u01(blk.y);
+                    // in the support, and P = pi / U, exactly 1 when pi = U
+                    if (pl >= kProposalPMin && a * qU[0] <= pi) {
+                        if (ns < kcap) {
+                            const int32_t id = leafId[pos];
+                            const float ip = 1.0f / pi;
+                            if (ns < kPoissonStage) { sid[ns * 64 + lane] = id; sip[ns * 64 + lane] = ip; }
+                            else { oid[ns] = id; oip[ns] = ip; }
+                            ns++;
+                        } else over = true;
+                    }
                 }
-                const int pos = qpos[0] + (int)r + 1;
-                qpos[0] = pos;
-                float pl;
-                if (fmode) {
-                    const FootLeaf L = footLeaf[pos];
-                    const float d2 = dist2(qx, qy, L.x, L.y);
-                    pl = foot_mix(k1, a1, kf, d2, foot_leaf(L, a1, qx, qy, d2));
-                } else {
-                    const float2 lp = leafXY[pos];
-                    pl = mix_d2(k0, a0, k1, a1, dist2(qx, qy, lp.x, lp.y));
+                qpos[0] = cand ? pos : qpos[0];
+#pragma unroll
+                for (int q = 0; q + 1 < kPoissonQueue; q++) {
+                    qpos[q] = pop ? qpos[q + 1] : qpos[q];
+                    qlast[q] = pop ? qlast[q + 1] : qlast[q];
+                    qU[q] = pop ? qU[q + 1] : qU[q];
                 }
-                float pi = fminf(1.0f, lam * pl);
-                float a = u01(blk.y);
-                // in the support, and P = pi / U, exactly 1 when pi = U
-                if (pl >= kProposalPMin && a * qU[0] <= pi) {
-                    if (ns < kcap) {
-                        const int32_t id = leafId[pos];
-                        const float ip = 1.0f / pi;
-                        if (ns < kPoissonStage) { sid[ns * 64 + lane] = id; sip[ns * 64 + lane] = ip; }
-                        else { oid[ns] = id; oip[ns] = ip; }
-                        ns++;
-                    } else over = true;
-                }
+                cnt -= pop;
+                fresh = fresh || pop;
             }
         }
     }
