@@ -57,9 +57,8 @@ def test_tile_shapes_bit_exact(dev, restore_tiles):
                                         (60000, 1.0, 8), (60000, 0.25, 2), (60000, 0.0, 1)])
 def test_density_lists_of_any_length(dev, restore_tiles, N, cell, wpb):
     """Splats far smaller than a pixel, so that the density's terms are single leaves: tiles
-    whose term lists are empty, longer than the list (put off in segments) and longer than
-    the segments hold (walked with a stack), spread over the image (cell 1), over a quarter
-    of each side, and at one point.  Bit for bit the oracle's densities."""
+    whose term lists are empty, longer than the list (cut once) and many times longer,
+    spread over the image (cell 1), over a quarter of each side, and at one point.  Bit for bit the oracle's densities."""
     from cudaExtensions import sampling
     rng = np.random.default_rng(N)
     W, H, f = 40, 33, 48.0

@@ -3157,8 +3157,6 @@ __device__ __forceinline__ bool tile_lane(const TileCfg& c, int W, int H, int la
 }
 
 
-constexpr int kFmmStack = 136;
-
 // children record of internal node p for the density walk (after the expansions
 // of every band are selected)
 __device__ __forceinline__ FmmRec fmm_record(int p, int L0, const NodeGeo* __restrict__ geo,
@@ -3219,19 +3217,23 @@ __device__ __forceinline__ bool box4_meets_disc(const float* bx, float qx, float
 // parent's, and rounding keeps that order: a pixel that meets the child meets the parent).
 // A workgroup finds the terms of its tiles level by level: a list of nodes in walk order,
 // each node without a term replaced by its children that meet some pixel's disc, one
-// thread per node, so a level's record loads are in flight together.  A level that would
-// overflow the list is taken again for its first half, the rest waits in segments.  Then
+// thread per node, so a level's record loads are in flight together.  A level that runs
+// over the list is cut there; once the terms of what was kept are added, the walk starts
+// again from the root without the leaves up to the cut.  Then
 // kFmmTerms terms at a time come to LDS, each wavefront evaluates the (term, pixel) pairs
 // that meet, 64 at a time, and each pixel adds its values in order: bit for bit the
 // reference's sums.  (A term meets 9 of a tile's 64 pixels in the narrow band, 28 to 49 in
 // the wide one: a lane per pixel left most lanes idle.)
 // Bound by the latency of the levels' and terms' loads (62 % miss L2 in the larger case),
-// then by instruction issue.  Both bands of 512x512 under 1M splats 676 -> 490 us against
-// one wavefront's walk with a stack; 16 views of 640x480 under 2M splats 3.53 -> 3.24 ms.
-// Lists of 2048 take 555 us and 4.03 ms, two wavefronts per workgroup 554 us and 4.63 ms,
-// 32 terms at a time 672 us and 3.12 ms, one lane per pixel over its own terms 1023 us and
-// 3.34 ms.
-constexpr int kFmmTerms = 64, kFmmList = 1024, kFmmPairs = 384, kFmmSegments = 16;
+// then by instruction issue.  Both bands of 512x512 under 1M splats 676 -> 493 us against
+// one wavefront's walk with a stack; 16 views of 640x480 under 2M splats 3.53 -> 3.27 ms;
+// 8 views of 64x145 under 600K splats, up to ten thousand terms to a tile, 2.46 -> 1.89 ms
+// (putting the later half of a long level off in LDS, and a stack where that room ran out,
+// 3.78 ms).  Lists of 704 and 1024 take 516 us and 3.30 ms, two wavefronts per workgroup
+// 554 us and 4.63 ms, 32 terms at a time 672 us and 3.12 ms, one lane per pixel over its
+// own terms 1023 us and 3.34 ms.
+constexpr int kFmmTerms = 64, kFmmList = 1536, kFmmPairs = 384;
+
 
 // each active lane's word goes to LDS at the wavefront's base plus its lane's word
 __device__ __forceinline__ void load_to_lds(const float UD_GLOBAL* from, float* base)
@@ -3284,30 +3286,6 @@ __device__ __forceinline__ float fixed_series(const float4* co, float tx, float 
     return val;
 }
 
-// the same a row at a time from memory (few registers)
-template <int P>
-__device__ __forceinline__ float fixed_series_rows(const float UD_GLOBAL* co, float tx, float ty)
-{
-    const float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
-    float hy[P + 1];
-    hy[0] = ey;
-    hy[1] = (2.0f * ty) * ey;
-#pragma unroll
-    for (int q = 2; q <= P; q++) hy[q] = __builtin_fmaf(2.0f * ty, hy[q - 1], -((2.0f * (float)(q - 1)) * hy[q - 2]));
-    float val = 0.0f, h = ex, hm = 0.0f;
-#pragma unroll 1
-    for (int a = 0; a <= P; a++) {
-        float sa = 0.0f;
-#pragma unroll
-        for (int b = 0; b <= P; b++) sa = __builtin_fmaf(co[a * (P + 1) + b], hy[b], sa);
-        val = __builtin_fmaf(h, sa, val);
-        const float hn = a == 0 ? (2.0f * tx) * ex : __builtin_fmaf(2.0f * tx, h, -((2.0f * (float)a) * hm));
-        hm = h;
-        h = hn;
-    }
-    return val;
-}
-
 // words of an expansion's block in LDS: whole float4 words, an odd number of them, so
 // that lanes reading different blocks meet different banks
 constexpr int fmm_block(int p)
@@ -3316,15 +3294,10 @@ constexpr int fmm_block(int p)
     return 4 * (q | 1);
 }
 // LDS bytes of a workgroup of wpb wavefronts: the terms' blocks, boxes, centres, block
-// offsets and each wavefront's masks of them, two lists of nodes and the segments put
-// off; or the serial walk's stacks.  The list that is free while terms are added holds
-// the wavefronts' pairs.
+// offsets and each wavefront's masks of them, two lists of nodes, the wavefronts' pairs
 constexpr size_t fmm_lds(int p, int wpb)
 {
-    const size_t lists = (size_t)kFmmTerms * (4 * fmm_block(p) + 28 + 8 * wpb) + 3 * kFmmList * 4 +
-                         (size_t)kFmmPairs * 6 * wpb;
-    const size_t stacks = (size_t)kFmmStack * 24 * wpb;
-    return lists > stacks ? lists : stacks;
+    return (size_t)kFmmTerms * (4 * fmm_block(p) + 28 + 8 * wpb) + 2 * kFmmList * 4 + (size_t)kFmmPairs * 6 * wpb;
 }
 
 // |q - closest point of [lo, hi]| for the closest whole q in [a, b]
@@ -3345,71 +3318,11 @@ __device__ __forceinline__ bool box4_meets_tile(const float4& bx, const float4& 
     return d2 < rad * rad;
 }
 
-// The walk of one tile with an explicit stack, for tiles whose lists run over: the
-// wavefront runs it once for the union of its 64 pixels, each entry with the mask of the
-// lanes it was pushed for, so each lane sees its own nodes in its own order.  Karras trees
-// on 64-bit keys are at most 64 levels deep; a level keeps at most two entries pending, so
-// the stack stays within 2 * 64 + 4.
-template <int P>
-__device__ float fmm_serial(unsigned char* lds, int lane, bool valid, float qx, float qy, const Band& B, int L0, int b,
-                            const NodeGeo* geo, const FmmRec* frec, const int* fixOff, const float UD_GLOBAL* cf)
-{
-    unsigned long long* sM = (unsigned long long*)lds;
-    float2* sC = (float2*)(sM + kFmmStack);
-    int* sN = (int*)(sC + kFmmStack);
-    int* sF = sN + kFmmStack;
-    float w = 0.0f;
-    const unsigned long long all = __ballot(valid);
-    if (lane == 0) {
-        sN[0] = 0;
-        sF[0] = L0 > 0 ? fixOff[0] : -1;
-        sC[0] = make_float2(geo[0].cx, geo[0].cy);
-        sM[0] = all;
-    }
-    int sp = 1;
-    while (sp > 0) {
-        sp--;
-        wave_lds_fence();
-        const int nd = __builtin_amdgcn_readfirstlane(sN[sp]);
-        const int off = __builtin_amdgcn_readfirstlane(sF[sp]);
-        const float2 c = sC[sp];
-        const unsigned long long mask = sM[sp];
-        wave_lds_fence();
-        const bool act = (mask >> lane) & 1ull;
-        if (nd >= L0) {
-            if (act) w = w + band_point(B, qx, qy, c.x, c.y);
-            continue;
-        }
-        if (off >= 0) {
-            if (act) w = w + fixed_series_rows<P>(cf + off, (qx - c.x) * B.is2h, (qy - c.y) * B.is2h);
-            continue;
-        }
-        const FmmRec r = frec[nd];
-        const unsigned long long ml = __ballot(act && box4_meets_disc(r.lbox, qx, qy, B.radius));
-        const unsigned long long mr = __ballot(act && box4_meets_disc(r.rbox, qx, qy, B.radius));
-        if (sp + 2 > kFmmStack) break;                       // unreachable for trees of depth <= 64
-        if (ml) {
-            if (lane == 0) {
-                sN[sp] = r.left; sF[sp] = b ? r.lfix[1] : r.lfix[0];
-                sC[sp] = make_float2(r.lc[0], r.lc[1]); sM[sp] = ml;
-            }
-            sp++;
-        }
-        if (mr) {
-            if (lane == 0) {
-                sN[sp] = r.right; sF[sp] = b ? r.rfix[1] : r.rfix[0];
-                sC[sp] = make_float2(r.rc[0], r.rc[1]); sM[sp] = mr;
-            }
-            sp++;
-        }
-    }
-    return w;
-}
-
 template <int P>
 __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg, int W, int H,
                                                                     const ViewState* __restrict__ vs, size_t vstride,
                                                                     int nbands, const NodeGeo* geo,
+                                                                    const NodeAux* aux,
                                                                     const FmmRec* __restrict__ frec,
                                                                     const int* __restrict__ fixOff0,
                                                                     const int* __restrict__ fixOff1,
@@ -3424,11 +3337,11 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
     float2* tC = (float2*)(tBox + T);
     unsigned long long* tMask = (unsigned long long*)(tC + T);   // [wpb][T]
     int* tOff = (int*)(tMask + T * cfg.wpb);                 // -1: a leaf
-    int* list = tOff + T;                                    // three of kFmmList
+    int* list = tOff + T;                                    // two of kFmmList
     __shared__ float4 area[kMaxWavesPerBlock];               // the tiles, joined down a column
     __shared__ int areas;
     __shared__ int total[2][kMaxWavesPerBlock];
-    __shared__ int seg[kFmmSegments];
+    __shared__ int cutAt;
     const int tid = threadIdx.x, lane = tid & 63, wpb = cfg.wpb;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     int i = W, j = H;
@@ -3438,6 +3351,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
     const size_t v = blockIdx.y / nbands;                    // view
     vs = (const ViewState*)((const char*)vs + v * vstride);
     geo = (const NodeGeo*)((const char*)geo + v * vstride);
+    aux = (const NodeAux*)((const char*)aux + v * vstride);
     frec = (const FmmRec*)((const char*)frec + v * vstride);
     const int* fixOff = (const int*)((const char*)(b ? fixOff1 : fixOff0) + v * vstride);
     const float* coef = (const float*)((const char*)(b ? coef1 : coef0) + v * vstride);
@@ -3469,12 +3383,11 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
         const bool rootTerm = L0 == 0 || rootOff >= 0;
         int* A = list;
         int* O = list + kFmmList;
-        int* S = list + 2 * kFmmList;
-        float* val = (float*)(list + 3 * kFmmList) + kFmmPairs * wid;        // this wavefront's pairs
-        uint16_t* pair = (uint16_t*)((float*)(list + 3 * kFmmList) + kFmmPairs * wpb) + kFmmPairs * wid;
+        float* val = (float*)(list + 2 * kFmmList) + kFmmPairs * wid;        // this wavefront's pairs
+        uint16_t* pair = (uint16_t*)((float*)(list + 2 * kFmmList) + kFmmPairs * wpb) + kFmmPairs * wid;
         if (tid == 0) A[0] = 0;
-        int F = 1, put = 0, segs = 0;                        // entries, entries and segments put off
-        bool more = !rootTerm, serial = false;
+        int F = 1, end = n, cut = 0;                         // entries; leaves from end on are added, from cut on kept
+        bool more = !rootTerm;
         int turn = 1;
         __syncthreads();
         while (true) {
@@ -3496,6 +3409,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
                             f1 |= box4_meets_tile(rb, area[t], B.radius);
                             f2 |= box4_meets_tile(lb, area[t], B.radius);
                         }
+                        f1 &= (cl >= L0 ? cl - L0 : cl) + 1 < end;           // the right child's first leaf
                         o1 = cr >= L0 || fr >= 0 ? ~(2 * e + 1) : cr;
                         o2 = cl >= L0 || fl >= 0 ? ~(2 * e) : cl;
                     }
@@ -3511,28 +3425,27 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
                         kept += x & 0xffff;
                     }
                     turn ^= 1;
-                    if (kept > kFmmList) break;              // nothing of this chunk is written
-                    const int p = base + wave_rank(m1) + wave_rank(m2);
-                    if (f1) O[p] = o1;
-                    if (f2) O[p + (f1 ? 1 : 0)] = o2;
-                }
-                if (kept > kFmmList) {
-                    // put the later half of this level's list off and take the level again
-                    const int half = F / 2;
-                    if (put + F - half > kFmmList || segs == kFmmSegments) { serial = true; break; }
-                    for (int t = tid; t < F - half; t += 64 * wpb) S[put + t] = A[half + t];
-                    if (tid == 0) seg[segs] = F - half;
-                    put += F - half;
-                    segs++;
-                    F = half;
-                    more = true;
-                } else {
-                    F = kept;
-                    int* t = A; A = O; O = t;
+                    const int p = base + wave_rank(m1) + wave_rank(m2), p2 = p + (f1 ? 1 : 0);
+                    if (f1 && p < kFmmList) O[p] = o1;
+                    if (f2 && p2 < kFmmList) O[p2] = o2;
+                    if (kept > kFmmList) {
+                        // one past the last leaf of the first entry that is left out
+                        if ((f1 && p == kFmmList) || (f2 && p2 == kFmmList)) {
+                            const bool second = !(f1 && p == kFmmList);
+                            const int parent = e >= 0 ? e : ~e >> 1;
+                            if (second || (e < 0 && !(~e & 1))) {            // a left child
+                                const int cl = frec[parent].left;
+                                cutAt = (cl >= L0 ? cl - L0 : cl) + 1;
+                            } else cutAt = aux[parent].last + 1;
+                        }
+                        break;
+                    }
                 }
                 __syncthreads();
+                if (kept > kFmmList) cut = cutAt;
+                F = min(kept, kFmmList);
+                int* t = A; A = O; O = t;
             }
-            if (serial) break;
             for (int t0 = 0; t0 < F; t0 += T) {
                 const int nt = min(T, F - t0);
                 for (int t = tid; t < nt; t += 64 * wpb) {
@@ -3627,17 +3540,13 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
                 }
                 __syncthreads();
             }
-            if (segs == 0) break;
-            segs--;
-            F = seg[segs];
-            put -= F;
-            for (int t = tid; t < F; t += 64 * wpb) A[t] = S[put + t];
+            if (cut == 0) break;
+            end = cut;
+            cut = 0;
+            if (tid == 0) A[0] = 0;
+            F = 1;
             more = true;
             __syncthreads();
-        }
-        if (serial) {
-            __syncthreads();
-            w = fmm_serial<P>(fmmLds + (size_t)wid * (kFmmStack * 24), lane, valid, qx, qy, B, L0, b, geo, frec, fixOff, cf);
         }
     }
     if (valid) out[(long)j + (long)H * i] = w;
@@ -4367,7 +4276,7 @@ void fmm_eval(int W, int H, int views, int nbands, int p, const TreeWs& w, size_
     const dim3 grid = tile_grid(c, W, H, views * nbands);
     switch (p) {
 #define UD_EVAL(P) case P: k_fmm_eval<P><<<grid, 64 * c.wpb, fmm_lds(P, c.wpb), st>>>(                             \
-        c, W, H, w.vs, vstride, nbands, w.geo, w.frec, w.fixOff[0], nbands > 1 ? w.fixOff[1] : nullptr,            \
+        c, W, H, w.vs, vstride, nbands, w.geo, w.aux, w.frec, w.fixOff[0], nbands > 1 ? w.fixOff[1] : nullptr,            \
         w.fixCoef[0], nbands > 1 ? w.fixCoef[1] : nullptr, out, outStride, bandStride); break;
     UD_EVAL(4) UD_EVAL(5) UD_EVAL(6) UD_EVAL(7) UD_EVAL(8)
 #undef UD_EVAL
