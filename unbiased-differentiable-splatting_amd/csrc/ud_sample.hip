@@ -14,14 +14,16 @@
 //                     wavefront ballot ranking)
 //   5 k_hierarchy     Karras 2012 split on 64-bit keys (morton << 32 | pos)
 //   6 k_bottom_up     atomic fan-in: boxes, counts, centres, Hermite degree
-//   7 k_coef_*        coefficient slots (deg+1)^2 of the reachable expanded
-//                     nodes, device-wide exclusive scan
+//   7 k_coef_blocks   coefficient slots (deg+1)^2 of the reachable expanded
+//                     nodes, one reservation per workgroup
 //   8 k_moments       Hermite moments per node over its contiguous leaf range,
 //                     accumulated in FP64 in leaf order
 //   9 k_sample_walk   per pixel tile: union FGT walk (k_sample_descend: the capacity
 //                     descents)
 //  10 k_sample_draw   wavefront per pixel: sequential Poisson keys u/p from
-//                     Philox4x32-10, the k smallest in order
+//                     Philox4x32-10, the k smallest in order (k_sample_replay:
+//                     pixels with equal keys)
+// Views of at most 4096 splats take stages 1-6 in one workgroup (k_front_small).
 // The fixed-order and Poisson-rate paths share stages 1-6 and add expansion
 // selection and moments per band (k_fixed_*), walk records (k_fmm_records,
 // k_walk_records), the density walk (k_fmm_eval) and the thinning pass
