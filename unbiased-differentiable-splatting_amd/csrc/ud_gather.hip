@@ -215,13 +215,19 @@ inline int nearest_lanes(int k)
 }
 
 // `lanes` lanes per pixel, one candidate each (lanes strided by `lanes` when k > 64).
-// The distinct smaller words of the row as read and of the pixel's other candidates
-// bound a candidate's final slot from below, so its cascade starts there.  (Word j of the
-// final order then never leaves slot j once there: only smaller words could displace it,
-// and those settle before.)  A pixel that finds an empty row writes each word once, and
-// one that finds a full row writes only what enters.  Bound by the latency of reading the row and of the atomics.  One thread per
-// pixel, each candidate starting at slot 0, took 419 us at 2 x 256x256 pixels of 16
-// slots, 100 000 splats, K = 10 (now 60 us).
+// A candidate's cascade starts at a slot that its final one is not before: the number of
+// words known to be smaller, those of the row as read and those that the pixel's other
+// candidates bring.  (Word j of the final order then never leaves slot j once there: only
+// smaller words could displace it, and those settle before.)  The count holds only if no
+// word enters it twice, so all lanes of a pixel work on one copy of the row: lane q loads
+// words q, q + lanes, ... and hands them round in LDS.  Each candidate is then in that copy
+// for every lane (and dropped), or for none (and counted as a mate's); with a row read per
+// lane, one could find a mate's word in the row that the mate itself had read too early to
+// find.  Words that move on while the copy is made are seen once at most, since only a word
+// above all before it counts.  A pixel that finds an empty row writes each word once, and
+// one that finds a full row writes only what enters.  Bound by the latency of reading the
+// row and of the atomics.  One thread per pixel, each candidate starting at slot 0, took
+// 419 us at 2 x 256x256 pixels of 16 slots, 100 000 splats, K = 10 (now 48 us).
 template <class T>
 __global__ __launch_bounds__(256) void k_nearest_insert(long npix, int k, int lanes, int K, int N,
                                                         const int32_t* __restrict__ idx, const T* __restrict__ wts,
@@ -262,18 +268,25 @@ __global__ __launch_bounds__(256) void k_nearest_insert(long npix, int k, int la
             d2 = d2 + dz * dz;
             key = ((unsigned long long)__float_as_uint(d2) << 32) | (uint32_t)c;
         }
+        if (__ballot(key != kNearestEmpty) == 0ull) continue;   // the wavefront brings nothing
         int pos = 0;
-        if (live) {
-            bool there = false;
-            unsigned long long top = 0ull;              // a word that moves on while read counts once
-            for (int j = 0; j < K; j++) {
-                const unsigned long long v = __hip_atomic_load(row + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                pos += v < key && (j == 0 || v > top);
+        bool there = false;
+        unsigned long long top = 0ull;                  // the largest word seen
+        for (int j0 = 0; j0 < K; j0 += lanes) {
+            const int n = min(lanes, K - j0);
+            keys[threadIdx.x] = live && lane < n
+                                    ? __hip_atomic_load(row + j0 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                    : kNearestEmpty;
+            wave_order();
+            for (int t = 0; t < n; t++) {
+                const unsigned long long v = keys[grp + t];
+                pos += v < key && (j0 + t == 0 || v > top);
                 there |= v == key;
                 top = v > top ? v : top;
             }
-            if (there) key = kNearestEmpty;             // a copy is there, or was and was moved on
+            wave_order();
         }
+        if (there) key = kNearestEmpty;                 // a copy is there, or was and was moved on
         keys[threadIdx.x] = key;
         wave_order();
         bool copy = false;
