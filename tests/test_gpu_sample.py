@@ -334,3 +334,19 @@ def test_sample_equal_keys_in_halves(dev, seed, ties):
     assert O.tie_pixels() == ties
     got = sampling.sample(W, H, f, t(P[None], dev), t(N[None], dev), None, t(S[None], dev), 24, 0.0, 0.01, seed=seed)
     assert np.array_equal(got[0].cpu().numpy(), ref)
+
+
+def test_sample_most_tiles_beyond_the_lists(dev):
+    """Two views of 10x9 tiles of which about 80 each have up to 950 walked and 870
+    evaluated nodes, most of them more than a tile's lists hold."""
+    from cudaExtensions import sampling
+    sc, p, n, nb, sd = scene_inputs(0, 100_000, sd_scale=0.7)
+    W, H, f, k = 80, 72, 1.2 * 80, 16
+    P = np.stack([p, p * np.float32([-1.0, 1.0, 1.0])])
+    NB = np.stack([nb, nb * np.float32([-1.0, 1.0, 1.0])])
+    got = sampling.sample(W, H, f, t(P, dev), t(NB, dev), None, t(sd[None], dev), k, 0.0, 1e-7, seed=8)
+    sampling.check_errors()
+    for b in range(2):
+        ref = O.sample_view(W, H, f, P[b], NB[b], sd, k, 0.0, 1e-7, seed=8, view=b)
+        assert (ref >= 0).mean() > 0.5
+        assert np.array_equal(got[b].cpu().numpy(), ref)

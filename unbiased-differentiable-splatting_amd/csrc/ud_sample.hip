@@ -1854,8 +1854,11 @@ __device__ __forceinline__ int tile_descents(const TreeView& T, const SampRec UD
 }
 
 // k_sample_walk's pass for the tiles whose walk outgrows its LDS lists (queued
-// there): the same weights by one depth-first walk per wavefront, a persistent grid
-// over the queue.
+// there): the same weights by one depth-first walk per wavefront.  The grid has a
+// workgroup for every tile, since on a dense scene every tile may be here and each is one
+// long serial chain; those past the queue's end leave at once.  With 64 workgroups per view 4M
+// splats of an eighth of the usual size at 512x512, half of whose tiles are here, took 138 ms,
+// now 17.1.
 __global__ __launch_bounds__(64) void k_sample_walk_serial(int W, int H, int k, int L, int tiles,
                                                            const ViewState* __restrict__ vs, const NodeGeo* geo,
                                                            const NodeLnk* lnk, const NodeAux* aux, const float* coef,
@@ -1865,8 +1868,7 @@ __global__ __launch_bounds__(64) void k_sample_walk_serial(int W, int H, int k, 
                                                            int* __restrict__ errOut, VStride vsd)
 {
     walkQueue = vw(walkQueue, vsd.ws);
-    const int queued = walkQueue[0];
-    if ((int)blockIdx.x >= queued) return;
+    if ((int)blockIdx.x >= walkQueue[0]) return;
     vs = vw(vs, vsd.ws);
     srec = vw(srec, vsd.ws);
     trieWs = vw(trieWs, vsd.ws);
@@ -1884,139 +1886,137 @@ __global__ __launch_bounds__(64) void k_sample_walk_serial(int W, int H, int k, 
     const int L0 = vs->nc - 1;
     const float prec = vs->prec;
     const float unset = __builtin_nanf("");              // weight not computed yet
-    for (int qe = blockIdx.x; qe < queued; qe += gridDim.x) {
-        const int blk = walkQueue[1 + qe];
-        TrieRef tr;
-        tr.base = (float UD_GLOBAL*)trieWs + (long)blk * kTrieFields * tcap * 64 + lane;
-        const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
-        const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
-        const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
-        const bool valid = (i < W) && (j < H);
-        int2* rch = reach + (long)blk * L * 64 + lane;   // [launch][lane] of this tile
-        const float qx = (float)i, qy = (float)j;
-        int nt = 1;
-        bool bad = false;
-        float total = 0.0f;
-        tr.init(0, unset);                                // entry 0: the root
-        // ---- one depth-first pass over the union of the 64 lanes' FGT walks ----
-        // The wavefront visits nodes in the reference's left-to-right order; a lane
-        // is active inside a node exactly when its own walk enters that node, so
-        // each lane sees its own frontier in its own order.  A node's fields come
-        // with its parent's children record (SampRec): a descent loads one record,
-        // a truncated node or a right sibling popped from the stack loads nothing,
-        // an expanded node only its coefficients.  Trie entries are numbered for
-        // the wavefront (a big node any lane walks gets one; a lane that does not
-        // walk it finds unset weights there, as in an entry it would create), so
-        // the path's entries are wave-uniform and every trie store coalesces.
-        __shared__ SampChild s_rinfo[kMaxDepth];           // right siblings of the path
-        __shared__ unsigned long long s_walk[kMaxDepth];
-        __shared__ int s_pent[kMaxDepth];                  // trie entry of each path node, -1 none
-        __shared__ float s_coef[(kMaxDegree + 1) * (kMaxDegree + 1)];
-        __shared__ float s_pacc[kDepthLds * 64];
-        DepthF pacc;
-        pacc.lds = s_pacc + lane;
-        int big = 0;                 // leading path nodes with more than k sources
-        uint64_t rightBits = 0;      // bit d: node at depth d is its parent's right child
-        int d = 0;
-        bool act = valid;
-        bool overflow = false;
-        SampChild cur;               // the node at depth d (wave-uniform)
-        {
-            const NodeGeo g0 = ld_geo(T, 0);
-            cur.lox = g0.lox; cur.loy = g0.loy; cur.hix = g0.hix; cur.hiy = g0.hiy;
-            cur.cx = g0.cx; cur.cy = g0.cy; cur.r2 = g0.r2; cur.deg = g0.deg;
-            cur.off = T.aux[0].off; cur.count = T.lnk[0].count; cur.id = 0; cur.first = 0;
-        }
-        // a node's weight into its parent's entry (the root's: the total)
-        // a completed node's weight into its parent's entry, for every lane: the
-        // lanes that reached it store theirs, the others the unset marker (their
-        // descents evaluate it on demand); the root's weight is the total
-        auto report = [&](int dd, bool has, float w) {
-            if (dd == 0) { if (has) total = w; return; }
-            const int pe = s_pent[dd - 1];
-            if (pe >= 0) tr.set(pe, ((rightBits >> dd) & 1ull) ? 2 : 1, has ? w : unset);
-        };
-        auto uni = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
-        while (true) {
-            // cur is wave-uniform (the root's record, a children record, or the LDS
-            // stack); say so, so that it lives in scalar registers
-            cur.id = __builtin_amdgcn_readfirstlane(cur.id);
-            cur.deg = __builtin_amdgcn_readfirstlane(cur.deg);
-            cur.off = __builtin_amdgcn_readfirstlane(cur.off);
-            cur.count = __builtin_amdgcn_readfirstlane(cur.count);
-            NodeGeo g;
-            g.lox = uni(cur.lox); g.loy = uni(cur.loy); g.hix = uni(cur.hix); g.hiy = uni(cur.hiy);
-            g.cx = uni(cur.cx); g.cy = uni(cur.cy); g.r2 = uni(cur.r2); g.deg = cur.deg;
-            float wv = 0.0f;
-            bool walk = false;
-            if (g.deg >= 0) {
-                wv = eval_node_staged(T, g, cur.off, qx, qy, act, s_coef, lane);
-                if (act) {
-                    // ancestors whose weight a descent can compare: depth 0 and every
-                    // node whose parent has more than k sources (a prefix of the path,
-                    // since source counts shrink with depth)
-                    const int amax = d < big + 1 ? d : big + 1;
-                    for (int a = 0; a < amax; a++) pacc.set(a, pacc.get(a) + wv);
-                }
-            } else {
-                walk = act && !truncated(g, qx, qy);
-            }
-            unsigned long long wm = __ballot(walk);
-            if (wm != 0ull) {
-                if (d >= kMaxDepth - 1) { overflow = true; break; }
-                const SampRec R = srec[cur.id];           // the one load of a descent
-                __builtin_amdgcn_wave_barrier();
-                if (lane == 0) { s_rinfo[d] = R.r; s_walk[d] = wm; }
-                int e = -1;
-                if (d == 0) e = 0;
-                else if (cur.count > k && s_pent[d - 1] >= 0 && nt < DFSMAX) {
-                    e = nt++;
-                    tr.initCaps(e);
-                    tr.setKidHalf(s_pent[d - 1], (rightBits >> d) & 1ull, e + 1);
-                }
-                if (lane == 0) s_pent[d] = e;
-                __builtin_amdgcn_wave_barrier();
-                if (walk && d <= big) pacc.set(d, 0.0f);
-                if (big == d && cur.count > k) big = d + 1;
-                d++;
-                cur = R.l;
-                rightBits &= ~(1ull << d);
-                act = walk;
-                continue;
-            }
-            // the node is complete for every active lane (wv: its expansion, or 0
-            // where it is truncated); report and advance
-            report(d, act, wv);
-            bool done = false;
-            while (true) {
-                if (d == 0) { done = true; break; }
-                if (!((rightBits >> d) & 1ull)) {
-                    rightBits |= (1ull << d);
-                    __builtin_amdgcn_wave_barrier();
-                    cur = s_rinfo[d - 1];
-                    act = (s_walk[d - 1] >> lane) & 1ull;
-                    break;
-                }
-                d--;
-                if (big > d) big = d;
-                act = (s_walk[d] >> lane) & 1ull;
-                // its accumulator is kept exactly when its parent has an entry; the
-                // lanes that reached it without walking it (truncated) report 0
-                if (d == 0 || s_pent[d - 1] >= 0) {
-                    const bool reached = d == 0 ? act : ((s_walk[d - 1] >> lane) & 1ull) != 0;
-                    report(d, reached, act ? pacc.get(d) : 0.0f);
-                }
-            }
-            if (done) break;
-        }
-        if (overflow) bad = true;
-        total = fmaxf(0.0f, total);
-        int drawn = 0;
-        if (valid && !bad && total >= prec)
-            drawn = capacity_descents(T, tr, nt, tcap, k, L, L0, qx, qy, rch, bad);
-        if (valid && bad) atomicOr(errOut, 1);
-        for (int la = drawn; la < L; la++) rch[(long)la * 64] = make_int2(0, 0);
+    const int blk = walkQueue[1 + blockIdx.x];
+    TrieRef tr;
+    tr.base = (float UD_GLOBAL*)trieWs + (long)blk * kTrieFields * tcap * 64 + lane;
+    const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
+    const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
+    const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
+    const bool valid = (i < W) && (j < H);
+    int2* rch = reach + (long)blk * L * 64 + lane;   // [launch][lane] of this tile
+    const float qx = (float)i, qy = (float)j;
+    int nt = 1;
+    bool bad = false;
+    float total = 0.0f;
+    tr.init(0, unset);                                // entry 0: the root
+    // ---- one depth-first pass over the union of the 64 lanes' FGT walks ----
+    // The wavefront visits nodes in the reference's left-to-right order; a lane
+    // is active inside a node exactly when its own walk enters that node, so
+    // each lane sees its own frontier in its own order.  A node's fields come
+    // with its parent's children record (SampRec): a descent loads one record,
+    // a truncated node or a right sibling popped from the stack loads nothing,
+    // an expanded node only its coefficients.  Trie entries are numbered for
+    // the wavefront (a big node any lane walks gets one; a lane that does not
+    // walk it finds unset weights there, as in an entry it would create), so
+    // the path's entries are wave-uniform and every trie store coalesces.
+    __shared__ SampChild s_rinfo[kMaxDepth];           // right siblings of the path
+    __shared__ unsigned long long s_walk[kMaxDepth];
+    __shared__ int s_pent[kMaxDepth];                  // trie entry of each path node, -1 none
+    __shared__ float s_coef[(kMaxDegree + 1) * (kMaxDegree + 1)];
+    __shared__ float s_pacc[kDepthLds * 64];
+    DepthF pacc;
+    pacc.lds = s_pacc + lane;
+    int big = 0;                 // leading path nodes with more than k sources
+    uint64_t rightBits = 0;      // bit d: node at depth d is its parent's right child
+    int d = 0;
+    bool act = valid;
+    bool overflow = false;
+    SampChild cur;               // the node at depth d (wave-uniform)
+    {
+        const NodeGeo g0 = ld_geo(T, 0);
+        cur.lox = g0.lox; cur.loy = g0.loy; cur.hix = g0.hix; cur.hiy = g0.hiy;
+        cur.cx = g0.cx; cur.cy = g0.cy; cur.r2 = g0.r2; cur.deg = g0.deg;
+        cur.off = T.aux[0].off; cur.count = T.lnk[0].count; cur.id = 0; cur.first = 0;
     }
+    // a node's weight into its parent's entry (the root's: the total)
+    // a completed node's weight into its parent's entry, for every lane: the
+    // lanes that reached it store theirs, the others the unset marker (their
+    // descents evaluate it on demand); the root's weight is the total
+    auto report = [&](int dd, bool has, float w) {
+        if (dd == 0) { if (has) total = w; return; }
+        const int pe = s_pent[dd - 1];
+        if (pe >= 0) tr.set(pe, ((rightBits >> dd) & 1ull) ? 2 : 1, has ? w : unset);
+    };
+    auto uni = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
+    while (true) {
+        // cur is wave-uniform (the root's record, a children record, or the LDS
+        // stack); say so, so that it lives in scalar registers
+        cur.id = __builtin_amdgcn_readfirstlane(cur.id);
+        cur.deg = __builtin_amdgcn_readfirstlane(cur.deg);
+        cur.off = __builtin_amdgcn_readfirstlane(cur.off);
+        cur.count = __builtin_amdgcn_readfirstlane(cur.count);
+        NodeGeo g;
+        g.lox = uni(cur.lox); g.loy = uni(cur.loy); g.hix = uni(cur.hix); g.hiy = uni(cur.hiy);
+        g.cx = uni(cur.cx); g.cy = uni(cur.cy); g.r2 = uni(cur.r2); g.deg = cur.deg;
+        float wv = 0.0f;
+        bool walk = false;
+        if (g.deg >= 0) {
+            wv = eval_node_staged(T, g, cur.off, qx, qy, act, s_coef, lane);
+            if (act) {
+                // ancestors whose weight a descent can compare: depth 0 and every
+                // node whose parent has more than k sources (a prefix of the path,
+                // since source counts shrink with depth)
+                const int amax = d < big + 1 ? d : big + 1;
+                for (int a = 0; a < amax; a++) pacc.set(a, pacc.get(a) + wv);
+            }
+        } else {
+            walk = act && !truncated(g, qx, qy);
+        }
+        unsigned long long wm = __ballot(walk);
+        if (wm != 0ull) {
+            if (d >= kMaxDepth - 1) { overflow = true; break; }
+            const SampRec R = srec[cur.id];           // the one load of a descent
+            __builtin_amdgcn_wave_barrier();
+            if (lane == 0) { s_rinfo[d] = R.r; s_walk[d] = wm; }
+            int e = -1;
+            if (d == 0) e = 0;
+            else if (cur.count > k && s_pent[d - 1] >= 0 && nt < DFSMAX) {
+                e = nt++;
+                tr.initCaps(e);
+                tr.setKidHalf(s_pent[d - 1], (rightBits >> d) & 1ull, e + 1);
+            }
+            if (lane == 0) s_pent[d] = e;
+            __builtin_amdgcn_wave_barrier();
+            if (walk && d <= big) pacc.set(d, 0.0f);
+            if (big == d && cur.count > k) big = d + 1;
+            d++;
+            cur = R.l;
+            rightBits &= ~(1ull << d);
+            act = walk;
+            continue;
+        }
+        // the node is complete for every active lane (wv: its expansion, or 0
+        // where it is truncated); report and advance
+        report(d, act, wv);
+        bool done = false;
+        while (true) {
+            if (d == 0) { done = true; break; }
+            if (!((rightBits >> d) & 1ull)) {
+                rightBits |= (1ull << d);
+                __builtin_amdgcn_wave_barrier();
+                cur = s_rinfo[d - 1];
+                act = (s_walk[d - 1] >> lane) & 1ull;
+                break;
+            }
+            d--;
+            if (big > d) big = d;
+            act = (s_walk[d] >> lane) & 1ull;
+            // its accumulator is kept exactly when its parent has an entry; the
+            // lanes that reached it without walking it (truncated) report 0
+            if (d == 0 || s_pent[d - 1] >= 0) {
+                const bool reached = d == 0 ? act : ((s_walk[d - 1] >> lane) & 1ull) != 0;
+                report(d, reached, act ? pacc.get(d) : 0.0f);
+            }
+        }
+        if (done) break;
+    }
+    if (overflow) bad = true;
+    total = fmaxf(0.0f, total);
+    int drawn = 0;
+    if (valid && !bad && total >= prec)
+        drawn = capacity_descents(T, tr, nt, tcap, k, L, L0, qx, qy, rch, bad);
+    if (valid && bad) atomicOr(errOut, 1);
+    for (int la = drawn; la < L; la++) rch[(long)la * 64] = make_int2(0, 0);
 }
 
 // Sampler walk: one workgroup of four wavefronts per 8x8 pixel tile, one lane per
@@ -4212,7 +4212,7 @@ void launch_sample(int N, int W, int H, int k, uint32_t seedLo, uint32_t seedHi,
                                                                   vsd);
     k_sample_descend<<<dim3(tiles, views), 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
                                                         trie_entries(k), w.tileInfo, w.reach, err, vsd);
-    k_sample_walk_serial<<<dim3(tiles < 64u ? tiles : 64u, views), 64, 0, st>>>(
+    k_sample_walk_serial<<<dim3(tiles, views), 64, 0, st>>>(
         W, H, k, L, (int)tiles, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie, trie_entries(k), w.reach,
         w.walkQueue, err, vsd);
     const dim3 dg(tiles * (64 / kDrawWaves), views);
