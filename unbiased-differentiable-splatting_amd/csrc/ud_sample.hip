@@ -51,7 +51,7 @@ constexpr int kMaxDepth = 64;        // descent trace bound (reference STACKSIZE
 constexpr uint32_t kSampTileRun = 4;
 constexpr int kTrieFields = 5;       // 4-byte fields per descent-trie entry (TrieRef)
 constexpr int kWalkEntries = 320;    // trie entries the walk may create
-// per tile, for the descents: entries of the walk (-1: left to the serial form), error
+// per tile, for the descents: entries of the walk, error
 // flag; the pixels' totals from 64 on; the entries' info and node from 128 on
 constexpr int kTileInfo = 128 + 2 * kWalkEntries;
 // entries the descents may add: 32 per launch, and at least 96, since the walk keeps
@@ -156,7 +156,7 @@ struct TreeWs {
     SampRec* srec;        // per internal node: children records of the sampler's walk
     int2* reach;          // per launch and pixel lane: leaf range the capacity descent reached
     int* tileInfo;        // per sampler tile: what the descents need of its walk (kTileInfo words)
-    int* walkQueue;       // [0]: count, then the tiles k_sample_walk left to its serial form
+    int* walkQueue;       // [0]: count, then the tiles k_sample_walk left to its passes
     int* tieQueue;                    // [0]: count, then (sampler lane, final key bits) per lane that met equal keys
     float2* leafXY;       // sorted position -> screen position of the leaf
     float* coef;
@@ -1478,19 +1478,6 @@ __device__ __forceinline__ float hermite_at(const float* sc, int p, float tx, fl
     }
 }
 
-// eval_node for a wave-uniform node: the coefficient block is staged in LDS
-__device__ __forceinline__ float eval_node_staged(const TreeView& T, const NodeGeo& g, int off, float qx, float qy,
-                                                  bool act, float* sc, int lane)
-{
-    const int np = (g.deg + 1) * (g.deg + 1);
-    const float UD_GLOBAL* c = T.coef + off;
-    for (int q = lane; q < np; q += 64) sc[q] = c[q];
-    wave_lds_fence();
-    const float w = act ? hermite_at(sc, g.deg, (qx - g.cx) * T.is2h, (qy - g.cy) * T.is2h) : 0.0f;
-    wave_lds_fence();
-    return w;
-}
-
 __device__ __forceinline__ bool truncated(const NodeGeo& g, float qx, float qy)
 {
     float cx = fminf(fmaxf(qx, g.lox), g.hix);
@@ -1537,22 +1524,6 @@ __device__ __forceinline__ float key_of(unsigned long long v) { return __uint_as
 // weights (below clusters that were not walked) on demand.  The reference
 // keeps the k smallest keys in a sorted insertion list (ties keep insertion
 // order, sequentialPoissonRadixTree.cuh:15-41), which k_sample_draw selects.
-// Accumulators of k_sample_walk_serial's path, one per depth and lane, kept only for
-// the depths a descent compares (the leading nodes with more than k sources and
-// the first one below them): the first kDepthLds depths in LDS ([depth][lane],
-// indices are wave-uniform), deeper ones (rare: about 20 levels cover k = 40 at
-// 1M splats) in private memory.
-constexpr int kDepthLds = 20;
-struct DepthF {
-    float* lds;                     // this wavefront's [kDepthLds][64] slice, offset by the lane
-    float a[kMaxDepth - kDepthLds];
-    __device__ float get(int i) const { return i < kDepthLds ? lds[i * 64] : a[i - kDepthLds]; }
-    __device__ void set(int i, float v)
-    {
-        if (i < kDepthLds) lds[i * 64] = v;
-        else a[i - kDepthLds] = v;
-    }
-};
 
 // An entry holds the weights of its node's two children and their capacities, so
 // a descent step reads everything it compares in one round of loads:
@@ -1580,83 +1551,7 @@ struct TrieRef {
     {
         set(e, 0, 1.0f); set(e, 1, wUnset); set(e, 2, wUnset); setKids(e, 0); set(e, 4, 1.0f);
     }
-    // an entry of the union walk: both children's weights are stored for every
-    // lane when the walk leaves them, so only capacities and child links start here
-    __device__ void initCaps(int e) const { set(e, 0, 1.0f); setKids(e, 0); set(e, 4, 1.0f); }
 };
-
-// The ceil(sqrt(k)) capacity descents of one pixel over its trie (nt entries so
-// far), recording each launch's reached leaf range; returns the launches recorded
-// (bad: a path or the trie grew past its bound).
-__device__ __forceinline__ int capacity_descents(const TreeView& T, const TrieRef& tr, int nt, int TMAX, int k, int L,
-                                                 int L0, float qx, float qy, int2* rch, bool& bad)
-{
-    const float unset = __builtin_nanf("");              // weight not computed yet
-    int drawn = 0;
-    int pe[kMaxDepth];
-    float pp[kMaxDepth], pc[kMaxDepth];
-    for (int la = 0; la < L && !bad; la++) {
-        int e = 0, nd = 0, depth = 0;
-        uint64_t sideBits = 0;         // bit d: the step to depth d went right
-        pe[0] = 0;
-        NodeLnk lk = ld_lnk(T, nd);
-        while (lk.count > k) {
-            // one round of loads: the node's link (issued at the end of the last
-            // step) and the entry's weights, children and capacities
-            float wl = tr.get(e, 1), wr = tr.get(e, 2);
-            const int kids = tr.kids(e);
-            const float cl = tr.get(e, 0), cr = tr.get(e, 4);
-            if (wl != wl) {
-#pragma unroll 1
-                for (int c = 0; c < 2; c++) {              // one copy of the inlined walk
-                    const float w = tree_weight(T, c ? lk.right : lk.left, qx, qy);
-                    tr.set(e, 1 + c, w);
-                    if (c) wr = w; else wl = w;
-                }
-            }
-            wl = fmaxf(0.0f, wl); wr = fmaxf(0.0f, wr);
-            float sum = wl + wr;
-            wl = wl / sum; wr = wr / sum;
-            int el = (kids & 0xffff) - 1, er = (kids >> 16) - 1;
-            float sl = wl * cl, sr = wr * cr;
-            bool goRight = sl < sr;
-            int ce = goRight ? er : el;
-            int cnode = goRight ? lk.right : lk.left;
-            if (ce < 0) {
-                if (nt >= TMAX) { bad = true; break; }
-                ce = nt++;
-                tr.init(ce, unset);
-                tr.setKidHalf(e, goRight, ce + 1);
-            }
-            depth++;
-            if (depth >= kMaxDepth) { bad = true; break; }
-            pe[depth] = ce;
-            pp[depth] = goRight ? wr : wl;
-            pc[depth] = goRight ? cr : cl;     // its capacity, unchanged until the update below
-            if (goRight) sideBits |= 1ull << depth;
-            e = ce;
-            nd = cnode;
-            lk = ld_lnk(T, nd);
-        }
-        if (bad) break;
-        // capacities: an entry's lives in its parent's entry (field 4 if it is
-        // the right child, else 0); the path's were read on the way down
-        float prob = 1.0f;
-        for (int dd = depth; dd >= 1; dd--) {
-            const int par = pe[dd - 1];
-            const int fld = ((sideBits >> dd) & 1ull) ? 4 : 0;
-            tr.set(par, fld, fmaxf(0.0f, pc[dd] - prob));
-            prob = prob * pp[dd];
-        }
-        // the reached subtree's leaves are the contiguous sorted range
-        // [first, first + count); k_sample_draw keys them
-        const int cnt = lk.count;
-        const int first = (nd >= L0) ? nd - L0 : T.aux[nd].first;
-        rch[(long)la * 64] = make_int2(first, cnt);
-        drawn = la + 1;
-    }
-    return drawn;
-}
 
 // The path of a descent: entry << 1 | side (-1: no capacity to update), probability of
 // the step, capacity before it.  The first kPathLds steps in LDS ([step][lane]; a
@@ -1689,8 +1584,9 @@ struct DescentPath {
     }
 };
 
-// capacity_descents for a tile whose trie k_sample_walk built, with the tile's
-// entries described in LDS: info[e] holds the entries + 1 of its children (left |
+// The ceil(sqrt(k)) capacity descents of one pixel over its tile's trie (nt entries so
+// far), recording each launch's reached leaf range; returns the launches recorded (bad: a
+// path or the trie grew past its bound).  The tile's entries are described in LDS: info[e] holds the entries + 1 of its children (left |
 // right << 10) and which of them hold rows of the walk (bit 20 left, 21 right),
 // node[e] its tree node.
 //
@@ -1853,172 +1749,6 @@ __device__ __forceinline__ int tile_descents(const TreeView& T, const SampRec UD
     return drawn;
 }
 
-// k_sample_walk's pass for the tiles whose walk outgrows its LDS lists (queued
-// there): the same weights by one depth-first walk per wavefront.  The grid has a
-// workgroup for every tile, since on a dense scene every tile may be here and each is one
-// long serial chain; those past the queue's end leave at once.  With 64 workgroups per view 4M
-// splats of an eighth of the usual size at 512x512, half of whose tiles are here, took 138 ms,
-// now 17.1.
-__global__ __launch_bounds__(64) void k_sample_walk_serial(int W, int H, int k, int L, int tiles,
-                                                           const ViewState* __restrict__ vs, const NodeGeo* geo,
-                                                           const NodeLnk* lnk, const NodeAux* aux, const float* coef,
-                                                           const SampRec* __restrict__ srec, float* trieWs, int tcap,
-                                                           int2* __restrict__ reach,
-                                                           const int* __restrict__ walkQueue,
-                                                           int* __restrict__ errOut, VStride vsd)
-{
-    walkQueue = vw(walkQueue, vsd.ws);
-    if ((int)blockIdx.x >= walkQueue[0]) return;
-    vs = vw(vs, vsd.ws);
-    srec = vw(srec, vsd.ws);
-    trieWs = vw(trieWs, vsd.ws);
-    reach = vw(reach, vsd.ws);
-    TreeView T;
-    T.geo = (const NodeGeo UD_GLOBAL*)vw(geo, vsd.ws);
-    T.lnk = (const NodeLnk UD_GLOBAL*)vw(lnk, vsd.ws);
-    T.aux = (const NodeAux UD_GLOBAL*)vw(aux, vsd.ws);
-    T.coef = (const float UD_GLOBAL*)vw(coef, vsd.ws);
-    T.s2h = vs->s2h;
-    T.is2h = vs->is2h;
-    const int DFSMAX = tcap - walk_extra(L);             // entries the walk may create
-    const int lane = threadIdx.x;
-    const int tilesY = (H + 7) >> 3;
-    const int L0 = vs->nc - 1;
-    const float prec = vs->prec;
-    const float unset = __builtin_nanf("");              // weight not computed yet
-    const int blk = walkQueue[1 + blockIdx.x];
-    TrieRef tr;
-    tr.base = (float UD_GLOBAL*)trieWs + (long)blk * kTrieFields * tcap * 64 + lane;
-    const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
-    const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
-    const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
-    const bool valid = (i < W) && (j < H);
-    int2* rch = reach + (long)blk * L * 64 + lane;   // [launch][lane] of this tile
-    const float qx = (float)i, qy = (float)j;
-    int nt = 1;
-    bool bad = false;
-    float total = 0.0f;
-    tr.init(0, unset);                                // entry 0: the root
-    // ---- one depth-first pass over the union of the 64 lanes' FGT walks ----
-    // The wavefront visits nodes in the reference's left-to-right order; a lane
-    // is active inside a node exactly when its own walk enters that node, so
-    // each lane sees its own frontier in its own order.  A node's fields come
-    // with its parent's children record (SampRec): a descent loads one record,
-    // a truncated node or a right sibling popped from the stack loads nothing,
-    // an expanded node only its coefficients.  Trie entries are numbered for
-    // the wavefront (a big node any lane walks gets one; a lane that does not
-    // walk it finds unset weights there, as in an entry it would create), so
-    // the path's entries are wave-uniform and every trie store coalesces.
-    __shared__ SampChild s_rinfo[kMaxDepth];           // right siblings of the path
-    __shared__ unsigned long long s_walk[kMaxDepth];
-    __shared__ int s_pent[kMaxDepth];                  // trie entry of each path node, -1 none
-    __shared__ float s_coef[(kMaxDegree + 1) * (kMaxDegree + 1)];
-    __shared__ float s_pacc[kDepthLds * 64];
-    DepthF pacc;
-    pacc.lds = s_pacc + lane;
-    int big = 0;                 // leading path nodes with more than k sources
-    uint64_t rightBits = 0;      // bit d: node at depth d is its parent's right child
-    int d = 0;
-    bool act = valid;
-    bool overflow = false;
-    SampChild cur;               // the node at depth d (wave-uniform)
-    {
-        const NodeGeo g0 = ld_geo(T, 0);
-        cur.lox = g0.lox; cur.loy = g0.loy; cur.hix = g0.hix; cur.hiy = g0.hiy;
-        cur.cx = g0.cx; cur.cy = g0.cy; cur.r2 = g0.r2; cur.deg = g0.deg;
-        cur.off = T.aux[0].off; cur.count = T.lnk[0].count; cur.id = 0; cur.first = 0;
-    }
-    // a node's weight into its parent's entry (the root's: the total)
-    // a completed node's weight into its parent's entry, for every lane: the
-    // lanes that reached it store theirs, the others the unset marker (their
-    // descents evaluate it on demand); the root's weight is the total
-    auto report = [&](int dd, bool has, float w) {
-        if (dd == 0) { if (has) total = w; return; }
-        const int pe = s_pent[dd - 1];
-        if (pe >= 0) tr.set(pe, ((rightBits >> dd) & 1ull) ? 2 : 1, has ? w : unset);
-    };
-    auto uni = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
-    while (true) {
-        // cur is wave-uniform (the root's record, a children record, or the LDS
-        // stack); say so, so that it lives in scalar registers
-        cur.id = __builtin_amdgcn_readfirstlane(cur.id);
-        cur.deg = __builtin_amdgcn_readfirstlane(cur.deg);
-        cur.off = __builtin_amdgcn_readfirstlane(cur.off);
-        cur.count = __builtin_amdgcn_readfirstlane(cur.count);
-        NodeGeo g;
-        g.lox = uni(cur.lox); g.loy = uni(cur.loy); g.hix = uni(cur.hix); g.hiy = uni(cur.hiy);
-        g.cx = uni(cur.cx); g.cy = uni(cur.cy); g.r2 = uni(cur.r2); g.deg = cur.deg;
-        float wv = 0.0f;
-        bool walk = false;
-        if (g.deg >= 0) {
-            wv = eval_node_staged(T, g, cur.off, qx, qy, act, s_coef, lane);
-            if (act) {
-                // ancestors whose weight a descent can compare: depth 0 and every
-                // node whose parent has more than k sources (a prefix of the path,
-                // since source counts shrink with depth)
-                const int amax = d < big + 1 ? d : big + 1;
-                for (int a = 0; a < amax; a++) pacc.set(a, pacc.get(a) + wv);
-            }
-        } else {
-            walk = act && !truncated(g, qx, qy);
-        }
-        unsigned long long wm = __ballot(walk);
-        if (wm != 0ull) {
-            if (d >= kMaxDepth - 1) { overflow = true; break; }
-            const SampRec R = srec[cur.id];           // the one load of a descent
-            __builtin_amdgcn_wave_barrier();
-            if (lane == 0) { s_rinfo[d] = R.r; s_walk[d] = wm; }
-            int e = -1;
-            if (d == 0) e = 0;
-            else if (cur.count > k && s_pent[d - 1] >= 0 && nt < DFSMAX) {
-                e = nt++;
-                tr.initCaps(e);
-                tr.setKidHalf(s_pent[d - 1], (rightBits >> d) & 1ull, e + 1);
-            }
-            if (lane == 0) s_pent[d] = e;
-            __builtin_amdgcn_wave_barrier();
-            if (walk && d <= big) pacc.set(d, 0.0f);
-            if (big == d && cur.count > k) big = d + 1;
-            d++;
-            cur = R.l;
-            rightBits &= ~(1ull << d);
-            act = walk;
-            continue;
-        }
-        // the node is complete for every active lane (wv: its expansion, or 0
-        // where it is truncated); report and advance
-        report(d, act, wv);
-        bool done = false;
-        while (true) {
-            if (d == 0) { done = true; break; }
-            if (!((rightBits >> d) & 1ull)) {
-                rightBits |= (1ull << d);
-                __builtin_amdgcn_wave_barrier();
-                cur = s_rinfo[d - 1];
-                act = (s_walk[d - 1] >> lane) & 1ull;
-                break;
-            }
-            d--;
-            if (big > d) big = d;
-            act = (s_walk[d] >> lane) & 1ull;
-            // its accumulator is kept exactly when its parent has an entry; the
-            // lanes that reached it without walking it (truncated) report 0
-            if (d == 0 || s_pent[d - 1] >= 0) {
-                const bool reached = d == 0 ? act : ((s_walk[d - 1] >> lane) & 1ull) != 0;
-                report(d, reached, act ? pacc.get(d) : 0.0f);
-            }
-        }
-        if (done) break;
-    }
-    if (overflow) bad = true;
-    total = fmaxf(0.0f, total);
-    int drawn = 0;
-    if (valid && !bad && total >= prec)
-        drawn = capacity_descents(T, tr, nt, tcap, k, L, L0, qx, qy, rch, bad);
-    if (valid && bad) atomicOr(errOut, 1);
-    for (int la = drawn; la < L; la++) rch[(long)la * 64] = make_int2(0, 0);
-}
-
 // Sampler walk: one workgroup of four wavefronts per 8x8 pixel tile, one lane per
 // pixel for the weights and the descents.
 //
@@ -2037,18 +1767,31 @@ __global__ __launch_bounds__(64) void k_sample_walk_serial(int W, int H, int k, 
 // in order, from 0.  Walked nodes with more than k sources get a trie entry with
 // both children's weights, for the descents (k_sample_descend).
 //
-// The depth-first form of this pass (k_sample_walk_serial, still used where the
-// lists overflow) waits for a record or a coefficient block at nearly every one of
-// its steps, 250 of them per tile on average at 1M splats, 512x512 (555 in the densest
-// tile, which set the kernel's time), and its descents load every node of a path:
+// One depth-first walk per wavefront waits for a record or a coefficient block at nearly
+// every one of its steps, 250 of them per tile on average at 1M splats, 512x512 (555 in the
+// densest tile, which set the kernel's time), and its descents load every node of a path:
 // walk and descents 1912 us against 464 + 394 us (128x128, 4096 splats: 235 us against
 // 47 + 46 us).  Four wavefronts share a tile because a dense tile's own time ends the
 // kernel and a small image has fewer tiles than the chip has SIMDs (one wavefront per
 // tile, its descents in the same kernel: 1173 us and 118 us).
+//
+// A tile that outgrows the lists is queued, and the PASSES form, launched next with a
+// workgroup for every tile of which those past the queue's end leave at once, takes its
+// walk in passes over the leaves: each traverses the tree for the leaves [a, b) only,
+// b found by halving, with the walked nodes that reach into them and the evaluated ones
+// that begin in them.  In depth-first order a pass's rows follow those of the passes
+// before, so the sums go on where those left them: the total in registers, those of the
+// walked nodes that reach over a (one per level at most, sPath) in their trie entries.
+// Bit for bit the sums of one pass.  A kernel of its own, so that the single pass keeps its
+// registers.  Bound by the levels' latency, some 20 levels in each pass.  sampling.sample with
+// these tiles walked depth-first by one wavefront each against passes, at 512x512: 4M splats
+// a third of the usual size, a few tiles 7.76 -> 4.26 ms, an eighth, half of the tiles 17.1 ->
+// 7.5 ms (depth-first throughout 6.2 and 18.2).
 constexpr int kWalkWaves = 4;
 constexpr int kWalkNodes = 448;      // walked nodes a tile's lists hold (277 in that densest tile)
 constexpr int kWalkRows = 448;       // evaluated nodes (220); the trie has rows for as many (walk_extra)
 constexpr int kWalkTake = 8;         // evaluated nodes a wavefront takes at a time
+constexpr uint32_t kEntOpen = 1u << 22;   // sInfo: the entry's node reaches over an end of a pass
 
 // OR over the four lanes of a quad
 __device__ __forceinline__ uint32_t quad_or(uint32_t v)
@@ -2085,7 +1828,8 @@ struct CoefFetch {
     }
 };
 
-__global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H, int k, int L,
+template <bool PASSES>
+__global__ __launch_bounds__(64 * kWalkWaves, PASSES ? 4 : 6) void k_sample_walk(int W, int H, int k, int L,
                                                                  const ViewState* __restrict__ vs, const NodeGeo* geo,
                                                                  const NodeLnk* lnk, const NodeAux* aux,
                                                                  const float* coef, const SampRec* __restrict__ srec_,
@@ -2093,6 +1837,12 @@ __global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H
                                                                  int* __restrict__ tileInfo,
                                                                  int* __restrict__ walkQueue, VStride vsd)
 {
+    int blk = (int)blockIdx.x;
+    if constexpr (PASSES) {
+        const int* q = vw(walkQueue, vsd.ws);
+        if (blk >= q[0]) return;
+        blk = q[1 + blk];
+    }
     // walked nodes in level order: the pixels walking below it; its index; parent place
     // | side << 9 | (trie entry + 1) << 10 | first place in depth-first order << 19; its
     // evaluated nodes below the left | right << 16 child
@@ -2109,6 +1859,10 @@ __global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H
     __shared__ float sCoef[kWalkWaves][(kMaxDegree + 1) * (kMaxDegree + 1)];
     __shared__ unsigned long long sCount;                  // walked | evaluated << 20 | entries << 40
     __shared__ int sTicket;
+    // passes: trie entry + 1 (0: none) of the walked node of each level that reaches over
+    // the first leaf, and over the end; the last leaf at which a node begins
+    __shared__ int sPath[PASSES ? kMaxDepth : 1], sNext[PASSES ? kMaxDepth : 1];
+    __shared__ int sLast;
     vs = vw(vs, vsd.ws);
     trieWs = vw(trieWs, vsd.ws);
     const SampRec UD_GLOBAL* srec = (const SampRec UD_GLOBAL*)vw(srec_, vsd.ws);
@@ -2123,10 +1877,10 @@ __global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int entMax = tcap - walk_extra(L);              // entries the walk may create
     TrieRef tr;
-    tr.base = (float UD_GLOBAL*)trieWs + (long)blockIdx.x * kTrieFields * tcap * 64 + lane;
+    tr.base = (float UD_GLOBAL*)trieWs + (long)blk * kTrieFields * tcap * 64 + lane;
     float UD_GLOBAL* rows = tr.base + (long)kTrieFields * entMax * 64;     // entries only the descents create
     const int tilesY = (H + 7) >> 3;
-    const uint32_t tile = xcd_chunk_remap<kSampTileRun>(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, gridDim.x);
     const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
     const int i = ti * 8 + (lane >> 3), j = tj * 8 + (lane & 7);
     const bool valid = (i < W) && (j < H);
@@ -2150,252 +1904,327 @@ __global__ __launch_bounds__(64 * kWalkWaves, 6) void k_sample_walk(int W, int H
     const unsigned long long wm0 = __ballot(valid && g0.deg < 0 && !truncated(g0, qx, qy));
     if (threadIdx.x == 0) {
         sMask[0] = wm0; sNode[0] = 0; sLink[0] = 1u << 10;
-        sInfo[0] = 0u; sEntNode[0] = 0; sEntAt[0] = 0;
+        sInfo[0] = PASSES ? kEntOpen : 0u; sEntNode[0] = 0; sEntAt[0] = 0;
         sCount = (wm0 ? 1ull : 0ull) | (1ull << 40);
         sTicket = 0;
     }
+    if constexpr (PASSES)
+        if (threadIdx.x < kMaxDepth) sPath[threadIdx.x] = threadIdx.x == 0 ? 1 : 0;
     __syncthreads();
     int levels = 0, nodes = wm0 ? 1 : 0, evals = 0, nt = 1;
-    // ---- traversal ----
-    {
-        const int slot = lane >> 3, side = (lane >> 2) & 1, quad = lane & 3;
-        const float x0 = (float)(ti * 8), y0 = (float)(tj * 8 + 2 * quad);
-        int lo = 0, hi = nodes;                           // the level's walked nodes
-        while (lo < hi) {
-            if (levels >= kMaxDepth - 1) { bad = true; break; }       // a walk below the depth bound
-            if (threadIdx.x == 0) sLevel[levels] = (unsigned short)lo;
-            levels++;
-            for (int b0 = lo + 8 * wv; b0 < hi; b0 += 8 * kWalkWaves) {
-                const int at = b0 + slot;
-                const bool on = at < hi;
-                const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + (on ? sNode[at] : 0)) + 3 * side;
-                const f4v box = rec[0], mid = rec[1];
-                const i4v ref = *(const i4v UD_GLOBAL*)(rec + 2);
-                const unsigned long long act = on ? sMask[at] : 0ull;
-                const int parentEnt = on ? (int)((sLink[at] >> 10) & 511u) - 1 : -1;
-                const int deg = __float_as_int(mid.w);
-                // !truncated for the 8 x 2 pixels of this lane (same operations per pixel)
-                float dx2[8];
-#pragma unroll
-                for (int x = 0; x < 8; x++) {
-                    const float px = x0 + (float)x;
-                    const float dx = px - fminf(fmaxf(px, box.x), box.z);
-                    dx2[x] = dx * dx;
+    // passes: this one's leaves are [a, b); entries below nt0 are earlier passes'
+    const int leaves = vs->nc;
+    int a = 0, b = leaves, nt0 = 1;
+    while (true) {
+        // ---- traversal ----
+        {
+            if constexpr (PASSES) {
+                // the root again, no node over the end yet
+                if (threadIdx.x == 0) {
+                    sLink[0] = 1u << 10;
+                    sCount = 1ull | ((unsigned long long)nt0 << 40);
+                    sTicket = 0;
+                    sLast = a;
                 }
-                uint32_t in[2] = { 0u, 0u };
+                if (threadIdx.x < kMaxDepth) sNext[threadIdx.x] = 0;
+                __syncthreads();
+                levels = evals = 0;
+                nodes = 1;
+            }
+            bool over = false;                                // uniform over the workgroup
+            const int slot = lane >> 3, side = (lane >> 2) & 1, quad = lane & 3;
+            const float x0 = (float)(ti * 8), y0 = (float)(tj * 8 + 2 * quad);
+            int lo = 0, hi = nodes;                           // the level's walked nodes
+            while (lo < hi) {
+                if (levels >= kMaxDepth - 1) { bad = true; break; }       // a walk below the depth bound
+                if (threadIdx.x == 0) sLevel[levels] = (unsigned short)lo;
+                levels++;
+                for (int b0 = lo + 8 * wv; b0 < hi; b0 += 8 * kWalkWaves) {
+                    const int at = b0 + slot;
+                    const bool on = at < hi;
+                    const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + (on ? sNode[at] : 0)) + 3 * side;
+                    const f4v box = rec[0], mid = rec[1];
+                    const i4v ref = *(const i4v UD_GLOBAL*)(rec + 2);
+                    const unsigned long long act = on ? sMask[at] : 0ull;
+                    const int parentEnt = on ? (int)((sLink[at] >> 10) & 511u) - 1 : -1;
+                    const int deg = __float_as_int(mid.w);
+                    // !truncated for the 8 x 2 pixels of this lane (same operations per pixel)
+                    float dx2[8];
 #pragma unroll
-                for (int y = 0; y < 2; y++) {
-                    const float py = y0 + (float)y;
-                    const float dy = py - fminf(fmaxf(py, box.y), box.w);
-                    const float dy2 = dy * dy;
+                    for (int x = 0; x < 8; x++) {
+                        const float px = x0 + (float)x;
+                        const float dx = px - fminf(fmaxf(px, box.x), box.z);
+                        dx2[x] = dx * dx;
+                    }
+                    uint32_t in[2] = { 0u, 0u };
 #pragma unroll
-                    for (int x = 0; x < 8; x++) in[x >> 2] |= dx2[x] + dy2 < mid.z ? 1u << (8 * (x & 3) + y) : 0u;
+                    for (int y = 0; y < 2; y++) {
+                        const float py = y0 + (float)y;
+                        const float dy = py - fminf(fmaxf(py, box.y), box.w);
+                        const float dy2 = dy * dy;
+#pragma unroll
+                        for (int x = 0; x < 8; x++) in[x >> 2] |= dx2[x] + dy2 < mid.z ? 1u << (8 * (x & 3) + y) : 0u;
+                    }
+                    const uint32_t inLo = quad_or(in[0] << (2 * quad)), inHi = quad_or(in[1] << (2 * quad));
+                    const unsigned long long walk = act & (((unsigned long long)inHi << 32) | inLo);
+                    const bool lead = on && quad == 0;
+                    bool isEval = lead && deg >= 0;
+                    bool isWalk = lead && deg < 0 && walk != 0ull;
+                    bool wantEnt = isWalk && ref.y > k && parentEnt >= 0;
+                    const int from = ref.w, upto = ref.w + ref.y;             // the child's leaves
+                    if constexpr (PASSES) {
+                        isEval &= from >= a && from < b;
+                        isWalk &= from < b && upto > a;
+                        wantEnt &= isWalk && from >= a;
+                        if (isEval || isWalk) atomicMax(&sLast, from);
+                    }
+                    const unsigned long long bw = __ballot(isWalk), be = __ballot(isEval), bt = __ballot(wantEnt);
+                    unsigned long long base = 0;
+                    if (lane == 0)
+                        base = atomicAdd(&sCount, (unsigned long long)__popcll(bw) | ((unsigned long long)__popcll(be) << 20) |
+                                                      ((unsigned long long)__popcll(bt) << 40));
+                    base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(base >> 32)) << 32) |
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                    const int to = (int)(base & 0xfffffu) + __popcll(bw & lt);
+                    const int row = (int)((base >> 20) & 0xfffffu) + __popcll(be & lt);
+                    int ent = wantEnt ? (int)(base >> 40) + __popcll(bt & lt) : -1;
+                    if (ent >= entMax) ent = -1;
+                    const bool fresh = ent >= 0;
+                    if constexpr (PASSES)
+                        if (isWalk && from < a) ent = sPath[levels] - 1;
+                    if (isWalk && to < kWalkNodes) {
+                        sMask[to] = walk;
+                        sNode[to] = ref.z;
+                        sLink[to] = (uint32_t)at | ((uint32_t)side << 9) | ((uint32_t)(ent + 1) << 10);
+                        if (fresh) {
+                            sInfo[ent] = PASSES && upto > b ? kEntOpen : 0u;
+                            sEntNode[ent] = ref.z;
+                            sEntAt[ent] = (unsigned short)to;
+                            atomicOr(&sInfo[parentEnt], (uint32_t)(ent + 1) << (10 * side));
+                        }
+                        if constexpr (PASSES)
+                            if (upto > b) sNext[levels] = ent + 1;
+                    }
+                    if (isEval && row < kWalkRows) sRowLink[row] = (unsigned short)(at | (side << 9));
                 }
-                const uint32_t inLo = quad_or(in[0] << (2 * quad)), inHi = quad_or(in[1] << (2 * quad));
-                const unsigned long long walk = act & (((unsigned long long)inHi << 32) | inLo);
-                const bool lead = on && quad == 0;
-                const bool isEval = lead && deg >= 0;
-                const bool isWalk = lead && deg < 0 && walk != 0ull;
-                const bool wantEnt = isWalk && ref.y > k && parentEnt >= 0;
-                const unsigned long long bw = __ballot(isWalk), be = __ballot(isEval), bt = __ballot(wantEnt);
-                unsigned long long base = 0;
-                if (lane == 0)
-                    base = atomicAdd(&sCount, (unsigned long long)__popcll(bw) | ((unsigned long long)__popcll(be) << 20) |
-                                                  ((unsigned long long)__popcll(bt) << 40));
-                base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(base >> 32)) << 32) |
-                       (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-                const int to = (int)(base & 0xfffffu) + __popcll(bw & lt);
-                const int row = (int)((base >> 20) & 0xfffffu) + __popcll(be & lt);
-                int ent = wantEnt ? (int)(base >> 40) + __popcll(bt & lt) : -1;
-                if (ent >= entMax) ent = -1;
-                if (isWalk && to < kWalkNodes) {
-                    sMask[to] = walk;
-                    sNode[to] = ref.z;
-                    sLink[to] = (uint32_t)at | ((uint32_t)side << 9) | ((uint32_t)(ent + 1) << 10);
-                    if (ent >= 0) {
-                        sInfo[ent] = 0u;
-                        sEntNode[ent] = ref.z;
-                        sEntAt[ent] = (unsigned short)to;
-                        atomicOr(&sInfo[parentEnt], (uint32_t)(ent + 1) << (10 * side));
+                __syncthreads();
+                const unsigned long long c = sCount;
+                nodes = (int)(c & 0xfffffu);
+                evals = (int)((c >> 20) & 0xfffffu);
+                nt = (int)(c >> 40);
+                if (nodes > kWalkNodes || evals > kWalkRows) {
+                    if constexpr (!PASSES) {                              // left to the passes
+                        if (threadIdx.x == 0) {
+                            int* q = vw(walkQueue, vsd.ws);
+                            q[1 + atomicAdd(q, 1)] = blk;
+                        }
+                        return;
+                    }
+                    over = true;
+                    break;
+                }
+                lo = hi;
+                hi = nodes;
+                __syncthreads();                               // sCount is read before the next level adds to it
+            }
+            if constexpr (PASSES) {
+                if (over) {
+                    // half the leaves at which nodes begin.  A list of 448 overflows over at
+                    // least 7 of them, since at most 64 nodes begin at one: a < b < the old b
+                    b = a + (sLast - a + 1) / 2;
+                    if (b <= a) { bad = true; nt = nt0; break; }
+                    // the links to this traversal's entries go
+                    if (threadIdx.x < kMaxDepth && sPath[threadIdx.x] > 0) {
+                        uint32_t& x = sInfo[sPath[threadIdx.x] - 1];
+                        if ((int)(x & 1023u) > nt0) x &= ~1023u;
+                        if ((int)((x >> 10) & 1023u) > nt0) x &= ~(1023u << 10);
+                    }
+                    __syncthreads();
+                    continue;
+                }
+            }
+            if (nt > entMax) nt = entMax;
+        }
+        if (nodes > 0 && !bad) {
+            // the trie entries by number, in a pass those of its walked nodes
+            const int items = PASSES ? nodes : nt;
+            auto entry_of = [&](int it) { return PASSES ? (int)((sLink[it] >> 10) & 511u) - 1 : it; };
+            auto place_of = [&](int it) { return PASSES ? it : (int)sEntAt[it]; };
+            // ---- places (first wavefront) ----
+            if (wv == 0) {
+                if (lane == 0) sLevel[levels] = (unsigned short)nodes;
+                for (int x = lane; x < nodes; x += 64) sBelow[x] = 0u;
+                wave_lds_fence();
+                // evaluated nodes below each side, bottom-up
+                for (int e = lane; e < evals; e += 64) {
+                    const uint32_t l = sRowLink[e];
+                    atomicAdd(&sBelow[l & 511u], 1u << (16 * (l >> 9)));
+                }
+                wave_lds_fence();
+                for (int d = levels - 1; d > 0; d--) {
+                    for (int x = sLevel[d] + lane; x < sLevel[d + 1]; x += 64) {
+                        const uint32_t l = sLink[x], c = sBelow[x];
+                        atomicAdd(&sBelow[l & 511u], ((c & 0xffffu) + (c >> 16)) << (16 * ((l >> 9) & 1u)));
+                    }
+                    wave_lds_fence();
+                }
+                // first places in depth-first order, top-down (the root's is 0)
+                for (int d = 1; d < levels; d++) {
+                    for (int x = sLevel[d] + lane; x < sLevel[d + 1]; x += 64) {
+                        const uint32_t l = sLink[x], up = l & 511u;
+                        const uint32_t first = (sLink[up] >> 19) + (((l >> 9) & 1u) ? sBelow[up] & 0xffffu : 0u);
+                        sLink[x] = l | (first << 19);
+                    }
+                    wave_lds_fence();
+                }
+                for (int e = lane; e < evals; e += 64) {
+                    const uint32_t l = sRowLink[e], up = l & 511u;
+                    sRowAt[(sLink[up] >> 19) + ((l >> 9) ? sBelow[up] & 0xffffu : 0u)] = (unsigned short)e;
+                }
+                for (int t = lane; t < items; t += 64) {
+                    const int ent = entry_of(t);
+                    if (PASSES && ent < 0) continue;
+                    const uint32_t c = sBelow[place_of(t)];
+                    sInfo[ent] |= ((c & 0xffffu) ? 1u << 20 : 0u) | ((c >> 16) ? 1u << 21 : 0u);
+                }
+            }
+            // ---- values: kWalkTake nodes at a time, the next ones' records in flight ----
+            {
+                struct Take {
+                    f4v mid;
+                    int off, first, num;
+                    unsigned long long mask;
+                };
+                auto take = [&]() {
+                    Take t;
+                    int b = 0;
+                    if (lane == 0) b = atomicAdd(&sTicket, kWalkTake);
+                    t.first = __builtin_amdgcn_readfirstlane(b);
+                    t.num = evals - t.first < kWalkTake ? evals - t.first : kWalkTake;
+                    const uint32_t l = lane < t.num ? sRowLink[t.first + lane] : 0u;
+                    const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + sNode[l & 511u]) + 3 * (l >> 9);
+                    t.mid = rec[1];
+                    t.off = ((const i4v UD_GLOBAL*)(rec + 2))->x;
+                    t.mask = sMask[l & 511u];
+                    return t;
+                };
+                Take next = take();
+                while (next.num > 0) {                         // wave-uniform
+                    const Take t = next;
+                    next = take();
+                    auto coefs = [&](int q, CoefFetch& f) {
+                        const int p = __builtin_amdgcn_readlane(__float_as_int(t.mid.w), q);
+                        f.load(T.coef + __builtin_amdgcn_readlane(t.off, q), (p + 1) * (p + 1), lane);
+                    };
+                    CoefFetch f;
+                    coefs(0, f);
+                    for (int q = 0; q < t.num; q++) {
+                        const CoefFetch cur = f;
+                        if (q + 1 < t.num) coefs(q + 1, f);
+                        const unsigned long long m =
+                            ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(t.mask >> 32), q) << 32) |
+                            (uint32_t)__builtin_amdgcn_readlane((int)t.mask, q);
+                        rows[(long)(t.first + q) * 64] =
+                            eval(cur, __builtin_amdgcn_readlane(__float_as_int(t.mid.w), q),
+                                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.mid.x), q)),
+                                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.mid.y), q)), m);
                     }
                 }
-                if (isEval && row < kWalkRows) sRowLink[row] = (unsigned short)(at | (side << 9));
             }
             __syncthreads();
-            const unsigned long long c = sCount;
-            nodes = (int)(c & 0xfffffu);
-            evals = (int)((c >> 20) & 0xfffffu);
-            nt = (int)(c >> 40);
-            if (nodes > kWalkNodes || evals > kWalkRows) {            // left to the serial form
-                if (threadIdx.x == 0) {
-                    int* q = vw(walkQueue, vsd.ws);
-                    q[1 + atomicAdd(q, 1)] = (int)blockIdx.x;
-                    vw(tileInfo, vsd.ws)[(long)blockIdx.x * kTileInfo] = -1;
+            // ---- sums ----
+            // N sums of rows at once, num[q] of them from place at[q] on, each in order
+            auto sums = [&](auto count, const int* at, const int* num, float* out) {
+                constexpr int N = decltype(count)::value;
+                int m = 0;
+#pragma unroll
+                for (int q = 0; q < N; q++) m = num[q] > m ? num[q] : m;
+                for (int r = 0; r < m; r += 16 / N) {
+                    float v[N][16 / N];
+#pragma unroll
+                    for (int u = 0; u < 16 / N; u++)
+#pragma unroll
+                        for (int q = 0; q < N; q++)
+                            v[q][u] = r + u < num[q] ? rows[(long)sRowAt[at[q] + r + u] * 64] : 0.0f;
+#pragma unroll
+                    for (int u = 0; u < 16 / N; u++)           // adding 0 past the end changes nothing
+#pragma unroll
+                        for (int q = 0; q < N; q++) out[q] = out[q] + v[q][u];
                 }
-                return;
-            }
-            lo = hi;
-            hi = nodes;
-            __syncthreads();                               // sCount is read before the next level adds to it
-        }
-        if (nt > entMax) nt = entMax;
-    }
-    if (nodes > 0 && !bad) {
-        // ---- places (first wavefront) ----
-        if (wv == 0) {
-            if (lane == 0) sLevel[levels] = (unsigned short)nodes;
-            for (int x = lane; x < nodes; x += 64) sBelow[x] = 0u;
-            wave_lds_fence();
-            // evaluated nodes below each side, bottom-up
-            for (int e = lane; e < evals; e += 64) {
-                const uint32_t l = sRowLink[e];
-                atomicAdd(&sBelow[l & 511u], 1u << (16 * (l >> 9)));
-            }
-            wave_lds_fence();
-            for (int d = levels - 1; d > 0; d--) {
-                for (int x = sLevel[d] + lane; x < sLevel[d + 1]; x += 64) {
-                    const uint32_t l = sLink[x], c = sBelow[x];
-                    atomicAdd(&sBelow[l & 511u], ((c & 0xffffu) + (c >> 16)) << (16 * ((l >> 9) & 1u)));
-                }
-                wave_lds_fence();
-            }
-            // first places in depth-first order, top-down (the root's is 0)
-            for (int d = 1; d < levels; d++) {
-                for (int x = sLevel[d] + lane; x < sLevel[d + 1]; x += 64) {
-                    const uint32_t l = sLink[x], up = l & 511u;
-                    const uint32_t first = (sLink[up] >> 19) + (((l >> 9) & 1u) ? sBelow[up] & 0xffffu : 0u);
-                    sLink[x] = l | (first << 19);
-                }
-                wave_lds_fence();
-            }
-            for (int e = lane; e < evals; e += 64) {
-                const uint32_t l = sRowLink[e], up = l & 511u;
-                sRowAt[(sLink[up] >> 19) + ((l >> 9) ? sBelow[up] & 0xffffu : 0u)] = (unsigned short)e;
-            }
-            for (int t = lane; t < nt; t += 64) {
-                const uint32_t c = sBelow[sEntAt[t]];
-                sInfo[t] |= ((c & 0xffffu) ? 1u << 20 : 0u) | ((c >> 16) ? 1u << 21 : 0u);
-            }
-        }
-        // ---- values: kWalkTake nodes at a time, the next ones' records in flight ----
-        {
-            struct Take {
-                f4v mid;
-                int off, first, num;
-                unsigned long long mask;
             };
-            auto take = [&]() {
-                Take t;
-                int b = 0;
-                if (lane == 0) b = atomicAdd(&sTicket, kWalkTake);
-                t.first = __builtin_amdgcn_readfirstlane(b);
-                t.num = evals - t.first < kWalkTake ? evals - t.first : kWalkTake;
-                const uint32_t l = lane < t.num ? sRowLink[t.first + lane] : 0u;
-                const f4v UD_GLOBAL* rec = (const f4v UD_GLOBAL*)(srec + sNode[l & 511u]) + 3 * (l >> 9);
-                t.mid = rec[1];
-                t.off = ((const i4v UD_GLOBAL*)(rec + 2))->x;
-                t.mask = sMask[l & 511u];
-                return t;
-            };
-            Take next = take();
-            while (next.num > 0) {                         // wave-uniform
-                const Take t = next;
-                next = take();
-                auto coefs = [&](int q, CoefFetch& f) {
-                    const int p = __builtin_amdgcn_readlane(__float_as_int(t.mid.w), q);
-                    f.load(T.coef + __builtin_amdgcn_readlane(t.off, q), (p + 1) * (p + 1), lane);
+            if (wv == 0) {
+                const int at0 = 0;
+                sums(std::integral_constant<int, 1>{}, &at0, &evals, &total);
+            } else {
+                // trie entries.  Where one child holds all rows, only pixels of weight <= 0
+                // there read the weights (tile_descents): 0 and 0 for a pixel that reached it
+                auto put = [&](int ent, bool mine, float wl, float wr) {
+                    const uint32_t kids = sInfo[ent];
+                    tr.set(ent, 0, 1.0f);
+                    tr.set(ent, 1, mine ? wl : unset);
+                    tr.set(ent, 2, mine ? wr : unset);
+                    tr.setKids(ent, (int)((kids & 1023u) | (((kids >> 10) & 1023u) << 16)));
+                    tr.set(ent, 4, 1.0f);
                 };
-                CoefFetch f;
-                coefs(0, f);
-                for (int q = 0; q < t.num; q++) {
-                    const CoefFetch cur = f;
-                    if (q + 1 < t.num) coefs(q + 1, f);
-                    const unsigned long long m =
-                        ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(t.mask >> 32), q) << 32) |
-                        (uint32_t)__builtin_amdgcn_readlane((int)t.mask, q);
-                    rows[(long)(t.first + q) * 64] =
-                        eval(cur, __builtin_amdgcn_readlane(__float_as_int(t.mid.w), q),
-                             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.mid.x), q)),
-                             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.mid.y), q)), m);
-                }
-            }
-        }
-        __syncthreads();
-        // ---- sums ----
-        // N sums of rows at once, num[q] of them from place at[q] on, each in order
-        auto sums = [&](auto count, const int* at, const int* num, float* out) {
-            constexpr int N = decltype(count)::value;
-            int m = 0;
-#pragma unroll
-            for (int q = 0; q < N; q++) m = num[q] > m ? num[q] : m;
-            for (int r = 0; r < m; r += 16 / N) {
-                float v[N][16 / N];
-#pragma unroll
-                for (int u = 0; u < 16 / N; u++)
-#pragma unroll
-                    for (int q = 0; q < N; q++)
-                        v[q][u] = r + u < num[q] ? rows[(long)sRowAt[at[q] + r + u] * 64] : 0.0f;
-#pragma unroll
-                for (int u = 0; u < 16 / N; u++)           // adding 0 past the end changes nothing
-#pragma unroll
-                    for (int q = 0; q < N; q++) out[q] = out[q] + v[q][u];
-            }
-        };
-        if (wv == 0) {
-            const int at0 = 0;
-            sums(std::integral_constant<int, 1>{}, &at0, &evals, &total);
-        } else {
-            // trie entries.  Where one child holds all rows, only pixels of weight <= 0
-            // there read the weights (tile_descents): 0 and 0 for a pixel that reached it
-            auto put = [&](int ent, bool mine, float wl, float wr) {
-                const uint32_t kids = sInfo[ent];
-                tr.set(ent, 0, 1.0f);
-                tr.set(ent, 1, mine ? wl : unset);
-                tr.set(ent, 2, mine ? wr : unset);
-                tr.setKids(ent, (int)((kids & 1023u) | (((kids >> 10) & 1023u) << 16)));
-                tr.set(ent, 4, 1.0f);
-            };
-            for (int c0 = 0; c0 < nt; c0 += 64 * (kWalkWaves - 1)) {
-                const int mine = c0 + lane * (kWalkWaves - 1) + wv - 1;       // this lane's entry
-                const bool has = mine < nt;
-                const bool both = has && (sInfo[has ? mine : 0] >> 20) == 3u;
-                unsigned long long plain = __ballot(has && !both), branch = __ballot(both);
-                auto entry = [&](int q) { return c0 + q * (kWalkWaves - 1) + wv - 1; };
-                while (plain) {
-                    const int ent = entry(__builtin_ctzll(plain));
-                    plain &= plain - 1;
-                    put(ent, (sMask[sEntAt[ent]] >> lane) & 1ull, 0.0f, 0.0f);
-                }
-                while (branch) {                                // two at a time: 16 row loads in flight
-                    int ent[2], at[4], num[4];
-                    float w[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-                    ent[0] = entry(__builtin_ctzll(branch));
-                    branch &= branch - 1;
-                    const bool two = branch != 0ull;
-                    ent[1] = two ? entry(__builtin_ctzll(branch)) : ent[0];
-                    branch &= branch - 1;
-#pragma unroll
-                    for (int q = 0; q < 2; q++) {
-                        const int x = __builtin_amdgcn_readfirstlane((int)sEntAt[ent[q]]);
-                        const uint32_t below = __builtin_amdgcn_readfirstlane(sBelow[x]);
-                        at[2 * q] = (int)(__builtin_amdgcn_readfirstlane(sLink[x]) >> 19);
-                        num[2 * q] = q == 0 || two ? (int)(below & 0xffffu) : 0;
-                        at[2 * q + 1] = at[2 * q] + num[2 * q];
-                        num[2 * q + 1] = q == 0 || two ? (int)(below >> 16) : 0;
+                for (int c0 = 0; c0 < items; c0 += 64 * (kWalkWaves - 1)) {
+                    const int mine = c0 + lane * (kWalkWaves - 1) + wv - 1;       // this lane's entry
+                    const bool has = mine < items && (!PASSES || entry_of(mine) >= 0);
+                    const uint32_t type = sInfo[has ? entry_of(mine) : 0] >> 20;
+                    // one that reaches over an end of the pass keeps its sums
+                    const bool both = has && (PASSES ? (type & 3u) == 3u || type >= kEntOpen >> 20 : type == 3u);
+                    unsigned long long plain = __ballot(has && !both), branch = __ballot(both);
+                    auto item = [&](int q) { return c0 + q * (kWalkWaves - 1) + wv - 1; };
+                    while (plain) {
+                        const int it = item(__builtin_ctzll(plain));
+                        plain &= plain - 1;
+                        put(entry_of(it), (sMask[place_of(it)] >> lane) & 1ull, 0.0f, 0.0f);
                     }
-                    sums(std::integral_constant<int, 4>{}, at, num, w);
-                    put(ent[0], (sMask[sEntAt[ent[0]]] >> lane) & 1ull, w[0], w[1]);
-                    if (two) put(ent[1], (sMask[sEntAt[ent[1]]] >> lane) & 1ull, w[2], w[3]);
+                    while (branch) {                                // two at a time: 16 row loads in flight
+                        int it[2], ent[2], at[4], num[4];
+                        float w[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+                        it[0] = item(__builtin_ctzll(branch));
+                        branch &= branch - 1;
+                        const bool two = branch != 0ull;
+                        it[1] = two ? item(__builtin_ctzll(branch)) : it[0];
+                        branch &= branch - 1;
+#pragma unroll
+                        for (int q = 0; q < 2; q++) {
+                            ent[q] = __builtin_amdgcn_readfirstlane(entry_of(it[q]));
+                            const int x = __builtin_amdgcn_readfirstlane(place_of(it[q]));
+                            if (PASSES && a > 0 && ent[q] < nt0 && ((sMask[x] >> lane) & 1ull)) {
+                                w[2 * q] = tr.get(ent[q], 1);           // of the passes before
+                                w[2 * q + 1] = tr.get(ent[q], 2);
+                            }
+                            const uint32_t below = __builtin_amdgcn_readfirstlane(sBelow[x]);
+                            at[2 * q] = (int)(__builtin_amdgcn_readfirstlane(sLink[x]) >> 19);
+                            num[2 * q] = q == 0 || two ? (int)(below & 0xffffu) : 0;
+                            at[2 * q + 1] = at[2 * q] + num[2 * q];
+                            num[2 * q + 1] = q == 0 || two ? (int)(below >> 16) : 0;
+                        }
+                        sums(std::integral_constant<int, 4>{}, at, num, w);
+                        put(ent[0], (sMask[place_of(it[0])] >> lane) & 1ull, w[0], w[1]);
+                        if (two) put(ent[1], (sMask[place_of(it[1])] >> lane) & 1ull, w[2], w[3]);
+                    }
                 }
             }
+            __syncthreads();
         }
-        __syncthreads();
+        if (!PASSES || bad || b >= leaves) break;
+        if constexpr (PASSES) {
+            // as many leaves again, more after a pass that left room
+            const int span = b - a, used = nodes > evals ? nodes : evals;
+            const long more = (long)span * (used < kWalkNodes / 8 ? 16 : used < kWalkNodes / 2 ? 2 : 1);
+            a = b;
+            b = more < leaves - a ? a + (int)more : leaves;
+            nt0 = nt;
+            if (threadIdx.x < kMaxDepth) sPath[threadIdx.x] = threadIdx.x == 0 ? 1 : sNext[threadIdx.x];
+        }
     }
     // ---- for k_sample_descend: the pixels' totals, the entries of the trie ----
-    int* tileOut = vw(tileInfo, vsd.ws) + (long)blockIdx.x * kTileInfo;
+    int* tileOut = vw(tileInfo, vsd.ws) + (long)blk * kTileInfo;
     const int tileEnts = nodes > 0 ? nt : 0;
     for (int t = threadIdx.x; t < tileEnts; t += 64 * kWalkWaves) {
-        tileOut[128 + t] = (int)sInfo[t];
+        tileOut[128 + t] = (int)(sInfo[t] & ~kEntOpen);
         tileOut[128 + kWalkEntries + t] = sEntNode[t];
     }
     if (wv > 0) return;
@@ -2440,7 +2269,6 @@ __global__ __launch_bounds__(64, 4) void k_sample_descend(int W, int H, int k, i
     const int n = vs->nc;
     const bool runTree = n > 0;
     const int ents = runTree ? tile_[0] : 0;
-    if (ents < 0) return;                                // left to k_sample_walk_serial
     for (int t = lane; t < ents; t += 64) {
         sInfo[t] = (uint32_t)tile_[128 + t];
         sEntNode[t] = tile_[128 + kWalkEntries + t];
@@ -4207,14 +4035,13 @@ void launch_sample(int N, int W, int H, int k, uint32_t seedLo, uint32_t seedHi,
     hipEvent_t e0, e1;
     bool timed = timing_pair(0, &e0, &e1);
     if (timed) (void)hipEventRecord(e0, st);
-    k_sample_walk<<<dim3(tiles, views), 64 * kWalkWaves, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec,
-                                                                  w.trie, trie_entries(k), w.tileInfo, w.walkQueue,
-                                                                  vsd);
-    k_sample_descend<<<dim3(tiles, views), 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
-                                                        trie_entries(k), w.tileInfo, w.reach, err, vsd);
-    k_sample_walk_serial<<<dim3(tiles, views), 64, 0, st>>>(
-        W, H, k, L, (int)tiles, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie, trie_entries(k), w.reach,
-        w.walkQueue, err, vsd);
+    const dim3 wg(tiles, views);
+    k_sample_walk<false><<<wg, 64 * kWalkWaves, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
+                                                         trie_entries(k), w.tileInfo, w.walkQueue, vsd);
+    k_sample_walk<true><<<wg, 64 * kWalkWaves, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie,
+                                                        trie_entries(k), w.tileInfo, w.walkQueue, vsd);
+    k_sample_descend<<<wg, 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie, trie_entries(k),
+                                        w.tileInfo, w.reach, err, vsd);
     const dim3 dg(tiles * (64 / kDrawWaves), views);
     // a pixel has at most L ceil(k / 4) Philox blocks, 64 per iteration: 8 x 16, 12 x 32
     // and 16 x 64 at k = 64, 128 and 256
