@@ -81,6 +81,17 @@ def test_workspace_queries():
     assert L.ude_splat_workspace_bytes(1, 0) >= 256
 
 
+@pytest.mark.parametrize("k", [1, 4, 5, 9, 16, 40, 256])
+def test_sampler_trie_room(k):
+    """A pixel's descent trie holds 384 entries of the walk and 32 more for each of the
+    ceil(sqrt(k)) descents, of five 4 B fields; past them a call reports an error."""
+    from cudaExtensions import _lib
+    ws = _lib.lib().ude_sample_workspace_bytes
+    launches = next(n for n in range(1, 17) if n * n >= k)
+    per_tile = (ws(1000, 8 * 101, 8, k) - ws(1000, 8, 8, k)) // 100
+    assert per_tile >= 64 * 20 * (384 + 32 * launches)
+
+
 def test_missing_library_raises(monkeypatch, tmp_path):
     from cudaExtensions import _lib
     monkeypatch.setattr(_lib, "_lib", None)

@@ -50,9 +50,9 @@ constexpr int kMaxDepth = 64;        // descent trace bound (reference STACKSIZE
 // at 1M splats, 512x512, against one contiguous block of tiles per XCD)
 constexpr uint32_t kSampTileRun = 4;
 constexpr int kTrieFields = 5;       // 4-byte fields per descent-trie entry (TrieRef)
-constexpr int kWalkEntries = 320;    // trie entries the walk may create
-// per tile, for the descents: entries of the walk, error
-// flag; the pixels' totals from 64 on; the entries' info and node from 128 on
+constexpr int kWalkEntries = 384;    // trie entries the walk may create
+// per tile, for the descents: entries of the walk, error flag; the pixels' totals from 64
+// on; the entries' info and node from 128 on
 constexpr int kTileInfo = 128 + 2 * kWalkEntries;
 // entries the descents may add: 32 per launch, and at least 96, since the walk keeps
 // its up to 5 x 96 rows of values there
