@@ -316,3 +316,25 @@ def test_autotune_degree_picks_the_fastest_order():
             sampling.set_fixed_degree(9)
     finally:
         sampling.set_fixed_degree(6)
+
+
+@pytest.mark.parametrize("capturing", [False, True])
+@pytest.mark.parametrize("free,cached,views", [(640, 0, 8), (639, 0, 7), (100, 540, 8), (0, 160, 2), (127, 0, 1), (0, 0, 1)])
+def test_sampler_batch_leaves_memory(monkeypatch, free, cached, views, capturing):
+    """The trees of a batch take at most an eighth of the memory that is neither used nor
+    cached by this process, nor used by another: 8 trees of 10 bytes of 640, one of less
+    than 160.  The device is not asked while a graph is recorded."""
+    from cudaExtensions import _lib, sampling
+
+    def device(_):
+        assert not capturing
+        return free, 10 ** 6
+    held = {"reserved_bytes": 1000 + cached, "allocated_bytes": 1000}
+    monkeypatch.setattr(torch.cuda, "mem_get_info", device)
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict",
+                        lambda _: {k: {"all": {"current": v}} for k, v in held.items()})
+    monkeypatch.setattr(torch.cuda, "get_device_properties",
+                        lambda _: type("P", (), {"total_memory": 1000 + cached + free}))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    monkeypatch.setattr(_lib, "workspace", lambda nbytes, dev: nbytes)
+    assert sampling._view_workspace(10, 8, torch.device("cpu")) == 10 * views

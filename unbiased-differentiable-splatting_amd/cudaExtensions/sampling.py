@@ -69,10 +69,26 @@ def _views_at_once(bn, W, H):
     return max(1, min(bn, 8192 // max(tiles, 1)))
 
 
+def _spare_bytes(dev):
+    """Device memory that no tensor of this process and nothing else on the device holds."""
+    pool = torch.cuda.memory_stats_as_nested_dict(dev)
+    held = lambda kind: pool[kind]["all"]["current"] if pool else 0  # noqa: E731
+    cached = held("reserved_bytes") - held("allocated_bytes")
+    if torch.cuda.is_current_stream_capturing():         # the device is not asked then
+        free = torch.cuda.get_device_properties(dev).total_memory - held("reserved_bytes")
+    else:
+        free = torch.cuda.mem_get_info(dev)[0]
+    return free + cached
+
+
 def _view_workspace(nbytes, views, dev):
-    """The workspace of ``views`` trees of ``nbytes`` each: at most 8 GB, and one tree's
-    where the memory for more is not there."""
-    views = max(1, min(views, (8 << 30) // max(nbytes, 1)))
+    """The workspace of ``views`` trees of ``nbytes`` each: at most 8 GB, and an eighth of
+    the spare memory, so that the rest of the frame finds what it found beside one tree's.
+    One tree's where the memory for more is not there."""
+    nbytes = max(nbytes, 1)
+    views = min(views, (8 << 30) // nbytes)
+    if views > 1:
+        views = min(views, _spare_bytes(dev) // 8 // nbytes)
     if views > 1:
         try:
             return _lib.workspace(nbytes * views, dev)
