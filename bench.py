@@ -241,9 +241,14 @@ def cpu_baseline(sc, k=40, threads=None):
 
 def timed_steps(fn, steps, kernel=None):
     """Runs `steps` calls of fn between a device synchronisation on both sides;
-    returns (ms per step, summed ms and launches of the profiled sampling kernel)."""
+    returns (ms per step, summed ms and launches of the profiled sampling kernel).
+    The interpreter's garbage is collected before: its first full collection walks
+    every object of the imported modules, about 38 ms, and would fall into whichever
+    loop reaches it (the first 20 frames read 4.0 ms each instead of 2.2)."""
+    import gc
     import torch
     from cudaExtensions import sampling
+    gc.collect()
     torch.cuda.synchronize()
     if kernel:
         sampling.profile_sampler_begin(kernel)

@@ -224,6 +224,28 @@ def test_bench_refuses_multi_gpu():
     assert r.returncode == 2 and "one GPU" in r.stderr
 
 
+def test_bench_collects_garbage_before_it_times(monkeypatch):
+    """The interpreter's full collection falls before the timed steps, not among them."""
+    import gc
+    import bench
+    log = []
+
+    class Event:
+        def __init__(self, enable_timing):
+            pass
+
+        def record(self):
+            log.append("event")
+
+        def elapsed_time(self, other):
+            return 4.0
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: log.append("wait"))
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(gc, "collect", lambda *a: log.append("collect"))
+    ms, _, _ = bench.timed_steps(lambda: log.append("step"), 2)
+    assert log == ["collect", "wait", "event", "step", "step", "event", "wait"] and ms >= 2.0
+
+
 def test_bench_algorithmic_bytes():
     sys.path.insert(0, ROOT)
     import bench
