@@ -107,3 +107,46 @@ def test_tile_scale_formula(dev, shape):
     got = net.tile_scale(F, c)
     assert got.shape == c.shape
     assert rel(got.reshape(-1).cpu().numpy(), s.cpu().numpy()) < 2.0 ** -23
+
+
+def scale_case(dev, T, seed=5):
+    from splatting_amd.learned import RateNet
+    rng = np.random.default_rng(seed)
+    net = RateNet(t(rng.normal(size=M.N_PARAMS) * 0.3, dev), t(rng.normal(size=M.N_IN), dev),
+                  t(rng.uniform(0.5, 2.0, size=M.N_IN), dev))
+    return net, t(rng.normal(size=(T, M.N_IN)), dev), t(rng.uniform(0.0, 3000.0, size=T), dev)
+
+
+def scale_formula(net, F, c, lo, hi):
+    y = net.forward(F).double()
+    cd = c.double()
+    tot = cd.sum()
+    s = torch.exp((y - (y * cd).sum() / tot).clamp(-20.0, 20.0))
+    for _ in range(3):
+        s = (s * (tot / (s * cd).sum())).clamp(lo, hi)
+    return s
+
+
+@pytest.mark.parametrize("lo,hi", [(None, 4.0), (0.75, None), (torch.tensor(0.5), torch.tensor(2.0))])
+def test_tile_scale_open_and_tensor_bounds(dev, lo, hi):
+    """Bounds as torch.clamp takes them."""
+    lo, hi = (x.to(dev) if isinstance(x, torch.Tensor) else x for x in (lo, hi))
+    net, F, c = scale_case(dev, 40)
+    assert rel(net.tile_scale(F, c, lo, hi).cpu().numpy(), scale_formula(net, F, c, lo, hi).cpu().numpy()) < 2.0 ** -23
+
+
+def test_tile_scale_gradient_of_counts(dev):
+    """The multipliers are differentiable in the counts, in reverse and in forward mode."""
+    net, F, c = scale_case(dev, 60)
+    g = t(np.random.default_rng(2).normal(size=60), dev)
+    v = t(np.random.default_rng(3).normal(size=60), dev)
+    a, b = (c.double().requires_grad_(True) for _ in range(2))
+    ga, = torch.autograd.grad(net.tile_scale(F, a), a, g)
+    gb, = torch.autograd.grad(scale_formula(net, F, b, 0.75, 4.0), b, g.double())
+    assert torch.allclose(ga, gb, rtol=1e-6, atol=1e-9 * float(gb.abs().max()))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(c.double(), v.double())
+        tangent = torch.autograd.forward_ad.unpack_dual(net.tile_scale(F, dual)).tangent
+    assert abs(float((tangent.double() * g).sum()) - float((gb * v).sum())) < 1e-5 * float((gb * v).abs().sum())
+    with torch.no_grad():
+        assert not net.tile_scale(F, a).requires_grad

@@ -9,6 +9,7 @@ splats are drawn where: the inclusion weights stay 1/pi, so estimates stay
 unbiased whatever the network predicts.
 """
 import math
+import numbers
 
 import numpy as np
 import torch
@@ -92,11 +93,11 @@ class RateNet:
         """Rate multipliers for tiles with features (..., 32) and plain-rate sample
         counts (...): exp(prediction), rescaled so that the expected sample count
         sum(scale * counts) is unchanged, and kept within [lo, hi]."""
+        if not self._scale_in_kernels(feats, counts, lo, hi):
+            return self._scale_by_torch(feats, counts, lo, hi)
         F = _lib.f32(feats.reshape(-1, N_IN), "features")
         c = counts.reshape(-1).double().contiguous()
         T = F.shape[0]
-        if c.shape[0] != T:
-            raise ValueError("tile_scale: %d counts for %d tiles" % (c.shape[0], T))
         mean, std = (_lib.f32(torch.broadcast_to(x, (1, N_IN)), q) for x, q in ((self.mean, "mean"), (self.std, "std")))
         _lib.require_gpu(F, c, mean, std, self.params)
         out = torch.empty(T, dtype=torch.float32, device=F.device)
@@ -104,6 +105,29 @@ class RateNet:
         _call("ude_rate_scale", T, _lib.ptr(F), _lib.ptr(mean), _lib.ptr(std), _lib.ptr(self.params), _lib.ptr(c),
               float(lo), float(hi), _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream(F.device))
         return out.reshape(counts.shape)
+
+    def _scale_in_kernels(self, feats, counts, lo, hi):
+        """Whether ude_rate_scale takes the call: plain numbers as bounds, and counts that
+        nothing differentiates or batches."""
+        T = feats.numel() // N_IN
+        return (isinstance(lo, numbers.Real) and isinstance(hi, numbers.Real)
+                and counts.numel() == T and counts.device == feats.device
+                and not (counts.requires_grad and torch.is_grad_enabled())
+                and not torch._C._functorch.is_functorch_wrapped_tensor(counts)
+                and torch.autograd.forward_ad.unpack_dual(counts).tangent is None
+                and all(x.shape in ((), (1,), (N_IN,), (1, N_IN)) for x in (self.mean, self.std)))
+
+    def _scale_by_torch(self, feats, counts, lo, hi):
+        """The same for any bounds, differentiable in the counts."""
+        y = self.forward(feats.reshape(-1, N_IN)).reshape(counts.shape).double()
+        y = torch.nan_to_num(y, nan=0.0, posinf=20.0, neginf=-20.0)     # a non-finite feature: plain rate
+        c = counts.double()
+        tot = c.sum().clamp(min=1e-30)
+        y = y - (y * c).sum() / tot
+        s = torch.exp(y.clamp(-20.0, 20.0))
+        for _ in range(3):
+            s = (s * (tot / (s * c).sum().clamp(min=1e-30))).clamp(lo, hi)
+        return s.float().contiguous()
 
     def save(self, path):
         np.savez(path, params=self.params.cpu().numpy(), mean=self.mean.cpu().numpy(), std=self.std.cpu().numpy())
