@@ -127,6 +127,14 @@ def scale_formula(net, F, c, lo, hi):
     return s
 
 
+@pytest.mark.parametrize("T", [65535, 65536, 65537, 300_000])
+def test_tile_scale_of_many_tiles(dev, T):
+    """Around the count from which the sums over the tiles leave their one workgroup, to
+    float32 rounding of the formula in float64."""
+    net, F, c = scale_case(dev, T)
+    assert rel(net.tile_scale(F, c).cpu().numpy(), scale_formula(net, F, c, 0.75, 4.0).cpu().numpy()) < 2.0 ** -23
+
+
 @pytest.mark.parametrize("lo,hi", [(None, 4.0), (0.75, None), (torch.tensor(0.5), torch.tensor(2.0))])
 def test_tile_scale_open_and_tensor_bounds(dev, lo, hi):
     """Bounds as torch.clamp takes them."""
