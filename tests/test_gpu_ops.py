@@ -254,6 +254,24 @@ def test_transform_backward_shared_vectors(dev, bn, N, dtype):
             assert_close(a.cpu().numpy(), r, 8 * eps, "shared transform backward", mag=m, ops=max(64, bn), eps=eps)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("bn,N", [(2, 99_999), (2, 100_000), (3, 102_401), (65, 100_003), (200, 300)])
+def test_transform_backward_of_many_and_few_points(dev, bn, N, dtype):
+    """Both sides of the point count from which the views share their points' registers,
+    partial workgroups and more views than its sums hold; each sum has N or bn terms."""
+    from cudaExtensions import transform
+    rng = np.random.default_rng(bn + N)
+    M, v, g = rng.normal(size=(bn, 4, 4)), rng.normal(size=(1, N, 3)), rng.normal(size=(bn, N, 3))
+    if dtype == torch.float32:
+        M, v, g = (x.astype(np.float32) for x in (M, v, g))
+    eps = float(np.finfo(M.dtype).eps) / 2
+    got = transform.affineBackward(t(g, dev), t(M, dev), t(v, dev))
+    ref = O.transform_backward(True, g, M, v)
+    mag = magnitude(O.transform_backward, True, g, M, v)
+    for a, r, m in zip(got, ref, mag):
+        assert_close(a.cpu().numpy(), r, 8 * eps, "transform backward", mag=m, ops=max(64, bn), eps=eps)
+
+
 @pytest.mark.parametrize("affine", [True, False])
 @pytest.mark.parametrize("bn,vb", [(1, 1), (3, 1), (3, 3)])
 def test_transform(dev, affine, bn, vb):

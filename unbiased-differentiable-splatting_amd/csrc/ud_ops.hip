@@ -1322,7 +1322,7 @@ __device__ __forceinline__ double wave_sum_t(double v) { return wave_sum_d(v); }
 // atomics (1M points: 11.7 us, where 512 x 256 threads took 15.5 us and
 // 2048 x 256 33.5 us).
 template <class T>
-__global__ __launch_bounds__(1024) void k_transform_backward(int affine, int vb, int N, const T* __restrict__ g,
+__global__ __launch_bounds__(1024) void k_transform_backward(int affine, int bn, int vb, int N, const T* __restrict__ g,
                                                             const T* __restrict__ M, const T* __restrict__ v,
                                                             T* __restrict__ gM, T* __restrict__ gV)
 {
@@ -1345,7 +1345,8 @@ __global__ __launch_bounds__(1024) void k_transform_backward(int affine, int vb,
         }
         T gv[3];
         for (int c = 0; c < 3; c++) gv[c] = m[c] * g0 + m[4 + c] * g1 + m[8 + c] * g2;
-        for (int c = 0; c < 3; c++) gV[vo + c] = gv[c];
+        if (vb > 1 || bn == 1) { for (int c = 0; c < 3; c++) gV[vo + c] = gv[c]; }
+        else { for (int c = 0; c < 3; c++) atomicAdd(gV + vo + c, gv[c]); }
     }
     for (int q = 0; q < 12; q++) acc[q] = wave_sum_t(acc[q]);
     int wv = threadIdx.x >> 6;
@@ -1358,13 +1359,18 @@ __global__ __launch_bounds__(1024) void k_transform_backward(int affine, int vb,
     }
 }
 
-// The same with one vector set for all views (vb == 1 < bn).  A thread keeps its points
-// and their gradients in registers while it runs over the views, so the points' sums need
-// no atomics; the matrix sums of up to 64 views wait in LDS until the workgroup has seen
-// all its points.  Bound by reading g (the next view's values are loaded ahead): 2M points
-// and 16 views 124 us (81 at the rate of a copy), where a workgroup per view and a global atomic per point and
-// component took 890 us.
+// The same with one vector set for all views (vb == 1 < bn) and many points.  A thread keeps
+// its points and their gradients in registers while it runs over the views, so the points'
+// sums need no atomics; the matrix sums of up to 64 views wait in LDS until the workgroup has
+// seen all its points.  Bound by reading g (the next view's values are loaded ahead): 2M
+// points and 16 views 124 us (81 at the rate of a copy), where a workgroup per view and a
+// global atomic per point and component take 890 us.  With few points there are few
+// workgroups, and each runs over all views one after another: the line lies where both take
+// the same, at about 100 000 points for 8, 16, 64 and 200 views, in float and double (call
+// times of 16 views, atomics against this: 60 000 points 37 / 56 us, 200 000 108 / 58; of 200
+// views, 300 points 24 / 505).
 constexpr int kSharedViews = 64;
+constexpr int kSharedPoints = 100000;
 template <class T>
 constexpr int shared_points() { return sizeof(T) == 8 ? 2 : 4; }   // four doubles would not fit the registers
 
@@ -2062,14 +2068,14 @@ int transform_backward_t(int affine, int bn, int vb, int N, const T* g, const T*
 {
     if (bn <= 0 || bn > 65535 || N < 0 || (vb != 1 && vb != bn)) return UDE_ERR_ARG;
     if (N == 0) return UDE_OK;
-    if (vb == 1 && bn > 1) {
+    if (vb == 1 && bn > 1 && N >= kSharedPoints) {
         const unsigned blocks = grid1(N, 1024 * shared_points<T>());
         k_transform_backward_shared<T><<<blocks < 256u ? blocks : 256u, 1024, 0, st>>>(affine, bn, N, g, M, v, gM, gV);
         return launch_status();
     }
     const unsigned blocks = grid1(N, 1024) < 256u ? grid1(N, 1024) : 256u;
     dim3 grid(blocks, bn);
-    k_transform_backward<T><<<grid, 1024, 0, st>>>(affine, vb, N, g, M, v, gM, gV);
+    k_transform_backward<T><<<grid, 1024, 0, st>>>(affine, bn, vb, N, g, M, v, gM, gV);
     return launch_status();
 }
 
