@@ -60,6 +60,30 @@ def test_gather_tiles(dev, W, H, k, N, C):
     assert_close(g64.cpu().numpy(), ref, 1e-12, "gather f64", mag=mag, ops=256, eps=EPS64)
 
 
+@pytest.mark.parametrize("C", [1, 3, 4, 7, 8, 15])
+@pytest.mark.parametrize("bn,W,H,k,N", [(2, 129, 97, 29, 40), (1, 153, 151, 31, 3000), (1, 153, 151, 31, 100_000),
+                                        (3, 217, 213, 6, 700), (1, 340, 300, 2, 90), (1, 500, 450, 1, 90)])
+def test_gather_of_many_slots(dev, bn, W, H, k, N, C):
+    """Calls large enough for the tiles' tables, and on both sides of the counts and row
+    widths from which they are used: partial tiles of both sizes, fewer and more splats than a
+    table holds.  Bounds as above."""
+    from cudaExtensions import pixelgather
+    rng = np.random.default_rng(W + C)
+    idx = random_slots(rng, bn, W, H, k, N)
+    if N > 1000:                                        # neighbouring pixels share most of theirs
+        idx[:, : W // 2] = np.where(idx[:, : W // 2] < 0, -1, idx[:, : W // 2] % 150)
+    u = rng.normal(size=idx.shape + (C,)).astype(np.float32)
+    u[rng.uniform(size=u.shape) < 0.1] = 0.0
+    mag = O.pixel_gather(idx, np.abs(u.astype(np.float64)), N)
+    ref = O.pixel_gather(idx, u.astype(np.float64), N)
+    most = int(np.bincount(idx[idx >= 0].ravel()).max())
+    g32 = pixelgather.gather(t(idx, dev), t(u, dev), N)
+    assert_close(g32.cpu().numpy(), ref, 1e-5, "gather f32", mag=mag, ops=max(64, most))
+    if C > 1:
+        g64 = pixelgather.gather(t(idx, dev), t(u, dev, torch.float64), N)
+        assert_close(g64.cpu().numpy(), ref, 1e-12, "gather f64", mag=mag, ops=max(256, most), eps=EPS64)
+
+
 def test_autograd_adjoint(dev):
     from splatting_amd.extensions import PixelScatterGather
     rng = np.random.default_rng(5)

@@ -89,6 +89,26 @@ inline int gather_entries(size_t rowBytes)
     return e;
 }
 
+// Where a tile's sums gain.  Setting up and writing out the tables takes some 6 us more than
+// the atomics of a small call, the more the wider the rows.  Atomics against tiles, us:
+//   float, one channel:   200x150 of 8 slots 21 / 10, 40x30 of 40 5 / 11
+//   three:                200x150 of 8 23 / 17, 2 x 100x100 of 16 20 / 24, 64x64 of 24 15 / 17
+//   six:                  200x150 of 24 54 / 37, 100x80 of 40 23 / 33
+//   eight:                512x512 of 40 473 / 477, 300x300 of 40 142 / 168 (rows of 32 bytes
+//                         reach memory as whole sectors, which sums by element do not beat)
+//   twelve:               400x300 of 24 233 / 194, 2 x 250x250 of 16 122 / 151
+//   double, three:        200x150 of 8 18 / 16, 40x30 of 40 16 / 17
+//   six:                  512x512 of 2 37 / 25, 8 x 40x30 of 40 16 / 19
+// One slot per pixel has nothing to share within it (512x512, three channels, 18 / 22).
+template <class T>
+inline bool gather_by_tiles(long nslots, int k, int C)
+{
+    if (k < 2) return false;
+    if (sizeof(T) == 8) return nslots >= (C <= 3 ? 200000 : 500000);
+    if (C >= 8) return C >= 12 && nslots >= 2500000;
+    return nslots >= (C <= 3 ? 200000 : 700000);
+}
+
 template <class T>
 __global__ __launch_bounds__(kGatherThreads) void k_pixel_gather_tile(int W, int H, int k, int N, int C, int side,
                                                                      int entries, const int32_t* __restrict__ idx,
@@ -171,11 +191,13 @@ int gather_t(int bn, int W, int H, int k, int N, int C, const int32_t* idx, cons
     if (bn <= 0 || W <= 0 || H <= 0 || k <= 0 || N < 0 || C <= 0) return UDE_ERR_ARG;
     if (N == 0) return UDE_OK;
     const long nslots = (long)bn * W * H * k;
-    // tiles of 16x16 where that gives the chip's 256 CUs a workgroup each, else of 8x8
+    // tiles of 16x16 where they keep most of the 256 CUs at two workgroups, else of 8x8 (three
+    // channels: 280x290 pixels, 342 tiles, 101 us against 69; 400x300, 475 tiles, 72 against 77)
     auto tiles = [&](int side) { return (long)((W + side - 1) / side) * ((H + side - 1) / side); };
-    const int side = tiles(16) * bn >= 256 ? 16 : 8;
+    const int side = tiles(16) * bn >= 400 ? 16 : 8;
     const int entries = gather_entries((size_t)C * sizeof(T));
-    if (entries >= kGatherMinEntries && k <= 1024 && tiles(side) <= INT_MAX && bn <= 65535)
+    if (gather_by_tiles<T>(nslots, k, C) && entries >= kGatherMinEntries && k <= 1024 && tiles(side) <= INT_MAX &&
+        bn <= 65535)
         k_pixel_gather_tile<T><<<dim3((unsigned)tiles(side), bn), kGatherThreads,
                                  entries * (C * sizeof(T) + sizeof(int32_t)), st>>>(W, H, k, N, C, side, entries, idx,
                                                                                     values, out);
