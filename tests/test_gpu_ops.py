@@ -348,6 +348,19 @@ def test_interpolation_tiles(dev, W, H, k, N, ab, dtype):
     assert_close(gA.cpu().numpy(), rA, 8 * eps, "interp grad attr", mag=mA, ops=max(64, most), eps=eps)
 
 
+@pytest.mark.parametrize("k", [1, 2, 7, 8, 9])
+def test_interpolation_double_few_slots(dev, k):
+    """Both sides of the slot count from which a pixel has several lanes; sums of k terms."""
+    from cudaExtensions import interpolation
+    rng = np.random.default_rng(k)
+    idx = random_slots(rng, 2, 37, 21, k, 90)
+    w, a = rng.uniform(size=idx.shape), rng.normal(size=(2, 90, 3))
+    eps = float(np.finfo(np.float64).eps) / 2
+    out = interpolation.forward(t(idx, dev), t(w, dev), t(a, dev))
+    assert_close(out.cpu().numpy(), O.interp_forward(idx, w, a), 8 * eps, "interp forward",
+                 mag=magnitude(O.interp_forward, idx, w, a), eps=eps)
+
+
 @pytest.mark.parametrize("cb", [1, 2])
 def test_sh_shading(dev, cb):
     from cudaExtensions import shading

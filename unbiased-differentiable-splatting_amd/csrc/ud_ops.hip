@@ -1486,9 +1486,10 @@ __global__ void k_interp_forward(long npix, int W, int H, int k, int ab, int N, 
     }
 }
 
-// interpolation.forward for double, C = 3: sixteen lanes per pixel read its slots side by
-// side and add their sums (151x97 pixels, k = 40: 23.9 -> 6.0 us against a lane per pixel,
-// whose reads lie 8 k bytes apart and follow one another).
+// interpolation.forward for double, C = 3, k >= 8: sixteen lanes per pixel read its slots side
+// by side and add their sums (151x97 pixels, k = 40: 23.9 -> 6.0 us against a lane per pixel,
+// whose reads lie 8 k bytes apart and follow one another).  With fewer slots most lanes have
+// none (512x512 of 1, 2 and 4 slots 19 us, a lane per pixel 14; 1024x768 of 8 53, and 86).
 template <class T>
 __global__ __launch_bounds__(256) void k_interp_forward_lanes(long npix, int W, int H, int k, int ab, int N,
                                                               const int32_t* __restrict__ idx,
@@ -2095,7 +2096,7 @@ int interp_forward_t(int bn, int W, int H, int k, int ab, int N, int C, const in
         }
     }
     if constexpr (sizeof(T) == 8) {
-        if (C == 3) {
+        if (C == 3 && k >= 8) {
             k_interp_forward_lanes<T><<<grid1(npix, 16), 256, 0, st>>>(npix, W, H, k, ab, N, idx, wts, attr, out);
             return launch_status();
         }
