@@ -116,3 +116,35 @@ def test_fmm_other_orders_bit_exact(dev, p):
         O.set_fixed_degree(6)
     assert sampling.get_fixed_degree() == 6
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("degree", [4, 5, 6, 7, 8])
+@pytest.mark.parametrize("N,spread", [(2, 1.0), (90, 1.0), (700, 1.0), (3000, 1.0), (3000, 0.05), (6000, 0.2), (2500, 0.0)])
+def test_densities_of_few_and_clustered_splats(dev, N, spread, degree):
+    """Both forms of the density walk and both list lengths, in the narrow band, the wide one
+    or both: images whose tiles reach few splats, many, and few outside a cluster (at one
+    point: a tree as deep as equal keys make it), under every order of the expansions."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng(N)
+    W, H, f = 136, 120, 150.0
+    z = -np.float32(2.0) - rng.uniform(size=N).astype(np.float32)
+    x, y = ((0.55 + (rng.uniform(size=N) - 0.5) * spread) * s - s / 2 for s in (W, H))
+    x[: N // 40], y[: N // 40] = ((rng.uniform(size=N // 40) - 0.5) * s for s in (W, H))
+    p = np.stack([-x * z / f, y * z / f, z], -1).astype(np.float32)
+    nb = np.tile(np.float32([0.0, 0.0, -1.0]), (N, 1))
+    sd = np.full((N, 2), 4e-3, np.float32)
+    dens = torch.zeros((1, 2, W, H), dtype=torch.float32, device=dev)
+    O.set_fixed_degree(degree)
+    sampling.set_fixed_degree(degree)
+    try:
+        sampling.samplePoisson(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), 8, 0.0, 0.01, seed=5,
+                               rate=0.5, densities=dens)
+        got = run_gpu(dev, W, H, f, p, nb, sd)
+        rdens = O.poisson_view(W, H, f, p, nb, sd, 8, 0.5, 0.0, 0.01, seed=5)[2]
+        ref = O.fmm_weights_view(W, H, f, p, nb, sd)
+    finally:
+        O.set_fixed_degree(6)
+        sampling.set_fixed_degree(6)
+    assert (rdens > 0).any()
+    assert np.array_equal(dens[0].cpu().numpy(), rdens)
+    assert np.array_equal(got, ref)

@@ -3063,6 +3063,17 @@ __device__ __forceinline__ bool box4_meets_disc(const float* bx, float qx, float
 // 554 us and 4.63 ms, 32 terms at a time 672 us and 3.12 ms, one lane per pixel over its
 // own terms 1023 us and 3.34 ms.
 constexpr int kFmmTerms = 64, kFmmList = 1536, kFmmPairs = 384;
+// Where a tile reaches few leaves each wavefront walks for itself (fmm_stack): the level form's
+// barriers then cost more than the walk's waits, which other wavefronts hide.  The line is the
+// number of leaves in reach if they lie evenly in the root's box, 6 to 16 with the band's
+// wavefronts.  Level form against stack, us: 4096x2160 under 64 / 6400 / 256 000 / 1M / 3M
+// splats 214 / 484 / 844 / 1149 / 1788 and 117 / 249 / 470 / 820 / 1850 (of the last 22 leaves
+// per tile); 16 views of 640x480 under 6400, two bands, 700 and 430; 512x512 under 20 000, both
+// ways 109; 256x256 under 6400, 49 and 63.  The lists are short where splats are few, so that
+// five workgroups of four wavefronts fit a CU's LDS instead of four (4096x2160 under 64 000,
+// stack, 409 us with long lists, 358).
+constexpr float kFmmReachLow = 6.0f, kFmmReachHigh = 16.0f, kFmmReachPerWave = 1.0f / 512.0f;
+constexpr int kFmmListShort = 512, kFmmListShortSplats = 14;     // splats per 64 pixels
 
 
 // each active lane's word goes to LDS at the wavefront's base plus its lane's word
@@ -3125,9 +3136,9 @@ constexpr int fmm_block(int p)
 }
 // LDS bytes of a workgroup of wpb wavefronts: the terms' blocks, boxes, centres, block
 // offsets and each wavefront's masks of them, two lists of nodes, the wavefronts' pairs
-constexpr size_t fmm_lds(int p, int wpb)
+constexpr size_t fmm_lds(int p, int wpb, int list)
 {
-    return (size_t)kFmmTerms * (4 * fmm_block(p) + 28 + 8 * wpb) + 2 * kFmmList * 4 + (size_t)kFmmPairs * 6 * wpb;
+    return (size_t)kFmmTerms * (4 * fmm_block(p) + 28 + 8 * wpb) + 2 * (size_t)list * 4 + (size_t)kFmmPairs * 6 * wpb;
 }
 
 // |q - closest point of [lo, hi]| for the closest whole q in [a, b]
@@ -3148,8 +3159,92 @@ __device__ __forceinline__ bool box4_meets_tile(const float4& bx, const float4& 
     return d2 < rad * rad;
 }
 
+// The reference's walk by one wavefront for the union of its 64 pixels: stack entries carry
+// the mask of pixels for which the node was pushed, so each pixel sees its own nodes in its
+// own order (the shared stack is its stack with other pixels' entries interleaved, in the same
+// last-in-first-out order).  A pushed entry also carries the child's centre and expansion
+// offset from its parent's FmmRec, so leaves and expansions need no node load and a descent
+// needs one wave-uniform record load.  An internal entry just below the top is handled in the
+// same step as the top entry, its children pushed in the order that popping one after the
+// other leaves.  Karras trees on 64-bit keys are at most 64 levels deep; a level keeps at most
+// two entries pending, so the stack stays within 2 * 64 + 4.
+constexpr int kFmmStack = 136;
+struct FmmEntry {
+    int node, off;                   // its expansion's offset, -1 for none / a leaf
+    float2 c;
+    unsigned long long mask;
+};
+
 template <int P>
-__global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg, int W, int H,
+__device__ __forceinline__ float fmm_stack(const Band& B, int L0, int b, const FmmRec* __restrict__ frec,
+                                           const int* __restrict__ fixOff, const NodeGeo* __restrict__ geo,
+                                           const float UD_GLOBAL* cf, float qx, float qy, bool valid, FmmEntry* stack,
+                                           int lane)
+{
+    constexpr int NC = (P + 1) * (P + 1), Q = (NC + 3) / 4;
+    float w = 0.0f;
+    const unsigned long long all = __ballot(valid);
+    if (lane == 0) stack[0] = FmmEntry{ 0, L0 > 0 ? fixOff[0] : -1, make_float2(geo[0].cx, geo[0].cy), all };
+    int sp = 1;
+    while (sp > 0) {
+        sp--;
+        wave_lds_fence();
+        const FmmEntry top = stack[sp], low = stack[sp > 0 ? sp - 1 : 0];
+        wave_lds_fence();
+        const int nd = __builtin_amdgcn_readfirstlane(top.node), off = __builtin_amdgcn_readfirstlane(top.off);
+        const int nd2 = __builtin_amdgcn_readfirstlane(low.node), off2 = __builtin_amdgcn_readfirstlane(low.off);
+        const bool act = (top.mask >> lane) & 1ull;
+        // the term of a leaf or an expansion on top of the stack
+        auto add_top = [&]() {
+            const float tx = (qx - top.c.x) * B.is2h, ty = (qy - top.c.y) * B.is2h;
+            const float ex = pexpf(-(tx * tx)), ey = pexpf(-(ty * ty));
+            if (nd >= L0) {
+                if (act) w = w + (0.0f + (B.c * ex) * ey);
+                return;
+            }
+            // wave-uniform block, fetched by broadcast vector loads issued together
+            const float UD_GLOBAL* cc = cf + off;
+            float4 co[Q];
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                co[q] = make_float4(cc[4 * q], 4 * q + 1 < NC ? cc[4 * q + 1] : 0.0f, 4 * q + 2 < NC ? cc[4 * q + 2] : 0.0f,
+                                    4 * q + 3 < NC ? cc[4 * q + 3] : 0.0f);
+            if (act) w = w + fixed_series<P>(co, tx, ty, ex, ey);
+        };
+        const bool topInt = nd < L0 && off < 0;
+        const bool lowInt = sp > 0 && nd2 < L0 && off2 < 0;
+        if (!topInt && !lowInt) {
+            add_top();
+            continue;
+        }
+        if (lowInt) sp--;
+        const bool two = topInt && lowInt;
+        const int ndA = topInt ? nd : nd2;                   // the upper internal entry
+        const FmmRec r = frec[ndA];
+        const FmmRec r2 = frec[two ? nd2 : ndA];
+        if (!topInt) add_top();
+        const bool actA = topInt ? act : (bool)((low.mask >> lane) & 1ull);
+        const bool act2 = two && ((low.mask >> lane) & 1ull);
+        const unsigned long long ml = __ballot(actA && box4_meets_disc(r.lbox, qx, qy, B.radius));
+        const unsigned long long mr = __ballot(actA && box4_meets_disc(r.rbox, qx, qy, B.radius));
+        const unsigned long long ml2 = __ballot(act2 && box4_meets_disc(r2.lbox, qx, qy, B.radius));
+        const unsigned long long mr2 = __ballot(act2 && box4_meets_disc(r2.rbox, qx, qy, B.radius));
+        if (sp + 4 > kFmmStack) break;                       // unreachable for trees of depth <= 64
+        auto push = [&](unsigned long long m, int node, int fix, float cx, float cy) {
+            if (!m) return;
+            if (lane == 0) stack[sp] = FmmEntry{ node, fix, make_float2(cx, cy), m };
+            sp++;
+        };
+        push(ml2, r2.left, b ? r2.lfix[1] : r2.lfix[0], r2.lc[0], r2.lc[1]);
+        push(mr2, r2.right, b ? r2.rfix[1] : r2.rfix[0], r2.rc[0], r2.rc[1]);
+        push(ml, r.left, b ? r.lfix[1] : r.lfix[0], r.lc[0], r.lc[1]);
+        push(mr, r.right, b ? r.rfix[1] : r.rfix[0], r.rc[0], r.rc[1]);
+    }
+    return w;
+}
+
+template <int P>
+__global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg, int W, int H, int listLen,
                                                                     const ViewState* __restrict__ vs, size_t vstride,
                                                                     int nbands, const NodeGeo* geo,
                                                                     const NodeAux* aux,
@@ -3167,7 +3262,7 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
     float2* tC = (float2*)(tBox + T);
     unsigned long long* tMask = (unsigned long long*)(tC + T);   // [wpb][T]
     int* tOff = (int*)(tMask + T * cfg.wpb);                 // -1: a leaf
-    int* list = tOff + T;                                    // two of kFmmList
+    int* list = tOff + T;                                    // two of listLen
     __shared__ float4 area[kMaxWavesPerBlock];               // the tiles, joined down a column
     __shared__ int areas;
     __shared__ int total[2][kMaxWavesPerBlock];
@@ -3188,11 +3283,21 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
     out = (float*)((char*)out + v * outStride + (size_t)b * bandStride);
     const int n = vs->nc;
     float w = 0.0f;
-    if (n > 0) {
-        const float UD_GLOBAL* cf = (const float UD_GLOBAL*)coef;
-        const Band B = vs->band[b];
-        const int L0 = n - 1;
-        const float qx = (float)i, qy = (float)j;
+    const Band B = vs->band[b];
+    const float UD_GLOBAL* cf = (const float UD_GLOBAL*)coef;
+    const float qx = (float)i, qy = (float)j;
+    const int L0 = n - 1;
+    // the leaves that a tile reaches if they lie evenly in the root's box (uniform over the
+    // band's workgroups)
+    const float4 root = *(const float4*)&geo[0].lox;
+    const float reach = (float)n * ((float)cfg.tw + 2.0f * B.radius) * ((float)(1 << cfg.lth) + 2.0f * B.radius) /
+                        ((fminf(root.z, (float)W) - fmaxf(root.x, 0.0f) + 2.0f * B.radius) *
+                         (fminf(root.w, (float)H) - fmaxf(root.y, 0.0f) + 2.0f * B.radius));
+    const float waves = (float)gridDim.x * (float)gridDim.y * (float)wpb;
+    if (n > 0 && reach < fminf(fmaxf(waves * kFmmReachPerWave, kFmmReachLow), kFmmReachHigh)) {
+        if (has)
+            w = fmm_stack<P>(B, L0, b, frec, fixOff, geo, cf, qx, qy, valid, (FmmEntry*)fmmLds + kFmmStack * wid, lane);
+    } else if (n > 0) {
         const int i0 = __builtin_amdgcn_readfirstlane(i), j0 = __builtin_amdgcn_readfirstlane(j);
         const int i1 = min(i0 + cfg.tw, W) - 1, j1 = min(j0 + (1 << cfg.lth), H) - 1;
         const float4 own = make_float4((float)i0, (float)i1, (float)j0, (float)j1);   // if has
@@ -3212,9 +3317,9 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
         const int rootOff = L0 > 0 ? fixOff[0] : -1;
         const bool rootTerm = L0 == 0 || rootOff >= 0;
         int* A = list;
-        int* O = list + kFmmList;
-        float* val = (float*)(list + 2 * kFmmList) + kFmmPairs * wid;        // this wavefront's pairs
-        uint16_t* pair = (uint16_t*)((float*)(list + 2 * kFmmList) + kFmmPairs * wpb) + kFmmPairs * wid;
+        int* O = list + listLen;
+        float* val = (float*)(list + 2 * listLen) + kFmmPairs * wid;        // this wavefront's pairs
+        uint16_t* pair = (uint16_t*)((float*)(list + 2 * listLen) + kFmmPairs * wpb) + kFmmPairs * wid;
         if (tid == 0) A[0] = 0;
         int F = 1, end = n, cut = 0;                         // entries; leaves from end on are added, from cut on kept
         bool more = !rootTerm;
@@ -3256,12 +3361,12 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
                     }
                     turn ^= 1;
                     const int p = base + wave_rank(m1) + wave_rank(m2), p2 = p + (f1 ? 1 : 0);
-                    if (f1 && p < kFmmList) O[p] = o1;
-                    if (f2 && p2 < kFmmList) O[p2] = o2;
-                    if (kept > kFmmList) {
+                    if (f1 && p < listLen) O[p] = o1;
+                    if (f2 && p2 < listLen) O[p2] = o2;
+                    if (kept > listLen) {
                         // one past the last leaf of the first entry that is left out
-                        if ((f1 && p == kFmmList) || (f2 && p2 == kFmmList)) {
-                            const bool second = !(f1 && p == kFmmList);
+                        if ((f1 && p == listLen) || (f2 && p2 == listLen)) {
+                            const bool second = !(f1 && p == listLen);
                             const int parent = e >= 0 ? e : ~e >> 1;
                             if (second || (e < 0 && !(~e & 1))) {            // a left child
                                 const int cl = frec[parent].left;
@@ -3272,8 +3377,8 @@ __global__ __launch_bounds__(64 * kMaxWavesPerBlock) void k_fmm_eval(TileCfg cfg
                     }
                 }
                 __syncthreads();
-                if (kept > kFmmList) cut = cutAt;
-                F = min(kept, kFmmList);
+                if (kept > listLen) cut = cutAt;
+                F = min(kept, listLen);
                 int* t = A; A = O; O = t;
             }
             for (int t0 = 0; t0 < F; t0 += T) {
@@ -4095,7 +4200,7 @@ void fixed_expansions(int N, int nbands, int p, const TreeWs& w, hipStream_t st,
 // densities of bands 0 .. nbands-1 of `views` views in one launch: w is the
 // first view's workspace, the others follow vstride bytes apart; view v writes
 // band b to out + v outStride + b bandStride bytes
-void fmm_eval(int W, int H, int views, int nbands, int p, const TreeWs& w, size_t vstride, float* out,
+void fmm_eval(int N, int W, int H, int views, int nbands, int p, const TreeWs& w, size_t vstride, float* out,
               size_t outStride, size_t bandStride, hipStream_t st)
 {
     const TileCfg c = g_tile[0];
@@ -4103,9 +4208,10 @@ void fmm_eval(int W, int H, int views, int nbands, int p, const TreeWs& w, size_
     bool timed = timing_pair(1, &e0, &e1);
     if (timed) (void)hipEventRecord(e0, st);
     const dim3 grid = tile_grid(c, W, H, views * nbands);
+    const int list = N < kFmmListShortSplats * (((long)W * H + 63) / 64) ? kFmmListShort : kFmmList;
     switch (p) {
-#define UD_EVAL(P) case P: k_fmm_eval<P><<<grid, 64 * c.wpb, fmm_lds(P, c.wpb), st>>>(                             \
-        c, W, H, w.vs, vstride, nbands, w.geo, w.aux, w.frec, w.fixOff[0], nbands > 1 ? w.fixOff[1] : nullptr,            \
+#define UD_EVAL(P) case P: k_fmm_eval<P><<<grid, 64 * c.wpb, fmm_lds(P, c.wpb, list), st>>>(                       \
+        c, W, H, list, w.vs, vstride, nbands, w.geo, w.aux, w.frec, w.fixOff[0], nbands > 1 ? w.fixOff[1] : nullptr,            \
         w.fixCoef[0], nbands > 1 ? w.fixCoef[1] : nullptr, out, outStride, bandStride); break;
     UD_EVAL(4) UD_EVAL(5) UD_EVAL(6) UD_EVAL(7) UD_EVAL(8)
 #undef UD_EVAL
@@ -4187,7 +4293,7 @@ int ude_fmm_weights(int bn, int N, int W, int H, double f, double smoothing, dou
         if (rc != UDE_OK) return rc;
         fixed_expansions(N, 1, p, w, st);
         k_fmm_records<<<grid1(N, 256), 256, 0, st>>>(w.vs, w.geo, w.lnk, w.fixOff[0], nullptr, w.frec, VStride{});
-        fmm_eval(W, H, 1, 1, p, w, 0, out + perView * b, 0, 0, st);
+        fmm_eval(N, W, H, 1, 1, p, w, 0, out + perView * b, 0, 0, st);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? UDE_OK : UDE_ERR_LAUNCH;
@@ -4250,7 +4356,7 @@ int ude_sample_poisson(int bn, int N, int W, int H, int kcap, double f, double s
         float* d0 = densOut ? densOut + perView * 2 * g : w.dens[0];
         float* d1 = densOut ? d0 + perView : w.dens[1];
         const size_t dstride = densOut ? sizeof(float) * 2 * perView : per;
-        fmm_eval(W, H, span, 2, p, w, per, d0, dstride, (size_t)((char*)d1 - (char*)d0), st);
+        fmm_eval(N, W, H, span, 2, p, w, per, d0, dstride, (size_t)((char*)d1 - (char*)d0), st);
         const float* ts = tileScale ? tileScale + (long)tsW * tsH * g : nullptr;
         hipEvent_t e0, e1;
         bool timed = timing_pair(2, &e0, &e1);
