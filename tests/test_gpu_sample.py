@@ -350,3 +350,23 @@ def test_sample_most_tiles_beyond_the_lists(dev):
         ref = O.sample_view(W, H, f, P[b], NB[b], sd, k, 0.0, 1e-7, seed=8, view=b)
         assert (ref >= 0).mean() > 0.5
         assert np.array_equal(got[b].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("k", [1, 9, 24, 25, 64, 128, 129])
+@pytest.mark.parametrize("W,H", [(725, 724), (1025, 516)])
+def test_sample_large_images(dev, W, H, k):
+    """Images of more than 8192 tiles, on which a wavefront draws for 16 pixels: tiles without
+    splats, with a few pixels that have some, and dense ones, partial tiles at both edges."""
+    from cudaExtensions import sampling
+    rng = np.random.default_rng(k)
+    N, f = 700, 700.0
+    p = rng.uniform([-1.0, -0.8, -3.0], [1.0, 0.8, -2.0], size=(N, 3)).astype(np.float32)
+    p[: N // 2, :2] = p[: N // 2, :2] * 0.05 + 0.2
+    p[0, :2] = (W / 2 - 1) / f * -p[0, 2], (H / 2 - 1) / f * p[0, 2]
+    nb = np.tile(np.float32([0.0, 0.0, -1.0]), (N, 1))
+    sd = rng.uniform(0.002, 0.02, size=(N, 2)).astype(np.float32)
+    got = sampling.sample(W, H, f, t(p[None], dev), t(nb[None], dev), None, t(sd[None], dev), k, 0.0, 0.01, seed=k)
+    sampling.check_errors()
+    ref = O.sample_view(W, H, f, p, nb, sd, k, 0.0, 0.01, seed=k)
+    assert 0.01 < (ref[..., 0] >= 0).mean() < 0.9
+    assert np.array_equal(got[0].cpu().numpy(), ref)

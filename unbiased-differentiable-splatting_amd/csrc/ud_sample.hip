@@ -1902,6 +1902,16 @@ __global__ __launch_bounds__(64 * kWalkWaves, PASSES ? 4 : 6) void k_sample_walk
     // ---- the root ----
     const NodeGeo g0 = ld_geo(T, 0);
     const unsigned long long wm0 = __ballot(valid && g0.deg < 0 && !truncated(g0, qx, qy));
+    int* tileOut = vw(tileInfo, vsd.ws) + (long)blk * kTileInfo;
+    // a tile that evaluates nothing: its weights, 0, start no descent, so that it needs no trie
+    auto nothing = [&]() {
+        if (wv == 0) {
+            if (lane < 2) tileOut[lane] = 0;
+            tileOut[64 + lane] = __float_as_int(0.0f);
+        }
+    };
+    const bool skips = !PASSES && g0.deg < 0 && vs->prec > 0.0f;          // uniform
+    if (skips && wm0 == 0ull) { nothing(); return; }
     if (threadIdx.x == 0) {
         sMask[0] = wm0; sNode[0] = 0; sLink[0] = 1u << 10;
         sInfo[0] = PASSES ? kEntOpen : 0u; sEntNode[0] = 0; sEntAt[0] = 0;
@@ -2045,6 +2055,7 @@ __global__ __launch_bounds__(64 * kWalkWaves, PASSES ? 4 : 6) void k_sample_walk
             }
             if (nt > entMax) nt = entMax;
         }
+        if (skips && evals == 0 && !bad) { nothing(); return; }
         if (nodes > 0 && !bad) {
             // the trie entries by number, in a pass those of its walked nodes
             const int items = PASSES ? nodes : nt;
@@ -2221,7 +2232,6 @@ __global__ __launch_bounds__(64 * kWalkWaves, PASSES ? 4 : 6) void k_sample_walk
         }
     }
     // ---- for k_sample_descend: the pixels' totals, the entries of the trie ----
-    int* tileOut = vw(tileInfo, vsd.ws) + (long)blk * kTileInfo;
     const int tileEnts = nodes > 0 ? nt : 0;
     for (int t = threadIdx.x; t < tileEnts; t += 64 * kWalkWaves) {
         tileOut[128 + t] = (int)(sInfo[t] & ~kEntOpen);
@@ -2351,8 +2361,35 @@ __device__ __forceinline__ bool draw_word(float qx, float qy, float2 xy, float i
 // threshold queues itself (tieQueue: its sampler lane and its k-th smallest key,
 // infinite with fewer than k keys), and k_sample_replay redraws it through the
 // reference's insertion.
+//
+// A pixel that no launch drew for gets its empty slots at once.  From kDrawManyTiles tiles on a
+// wavefront takes 16 pixels of a tile one after another, the empty ones found for all of them
+// with one load (up to two rows of keys; with four the loop's registers cost more).  2048x1024
+// under 6400 splats, k = 40, 4 % of the pixels not empty: 1420 -> 190 us; under 16, k = 8: 641
+// -> 52.  At 512x512, half the line's tiles, turns save nothing under 100 000 splats at k = 40
+// and cost 7 % at k = 64.
 constexpr int kDrawWaves = 4;
-template <int ROWS, int IT>
+constexpr int kDrawTurns = 16;
+constexpr long kDrawManyTiles = 8192;
+
+// pixels of the tile that some launch drew for: where one did, the first did
+__device__ __forceinline__ unsigned long long drawn_pixels(const int2* __restrict__ reach, int blk, int L, int lane)
+{
+    return __ballot(reach[(long)blk * L * 64 + lane].y > 0);
+}
+
+// empty slots for the 16 pixels from pl on of a tile: two of its columns, each contiguous
+__device__ __forceinline__ void empty_columns(int W, int H, int k, int ti, int tj, int pl, int lane, int32_t* out)
+{
+    const int j = tj * 8, n = min(8, H - j) * k;
+    for (int c = 0; c < 2; c++) {
+        const int i = ti * 8 + (pl >> 3) + c;
+        if (i >= W) break;
+        for (int x = lane; x < n; x += 64) out[((long)j + (long)H * i) * k + x] = -1;
+    }
+}
+
+template <int ROWS, int IT, int TURNS>
 __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw(int W, int H, int k, int L, int tiles,
                                                                  uint32_t seedLo, uint32_t seedHi, uint32_t view,
                                                                  const ViewState* __restrict__ vs,
@@ -2377,151 +2414,163 @@ __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw(int W, int H, i
     // the blocks of a sampler tile run on the XCD its walk ran on (tile t was
     // workgroup t of the walk: XCD t mod 8), whose L2 holds its reached ranges and
     // most of its leaves
-    constexpr int per = 64 / kDrawWaves;                // workgroups per tile
+    constexpr int per = 64 / (kDrawWaves * TURNS);      // workgroups per tile
     const int full = tiles & ~7, d = blockIdx.x;
     const int blk = d < full * per ? (d >> 3) / per * 8 + (d & 7) : d / per;
-    const int pl = (d < full * per ? (d >> 3) % per : d % per) * kDrawWaves + wv;
+    const int pl0 = ((d < full * per ? (d >> 3) % per : d % per) * kDrawWaves + wv) * TURNS;
     const int tilesY = (H + 7) >> 3;
     const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
     const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
-    const int i = ti * 8 + (pl >> 3), j = tj * 8 + (pl & 7);
-    if (i >= W || j >= H) return;                       // wave-uniform
     const float is2h = vs->is2h;
-    const float qx = (float)i, qy = (float)j;
-    const uint32_t pixel = (uint32_t)(j + H * i);
-    const int2 fc = lane < L ? reach[((long)blk * L + lane) * 64 + pl] : make_int2(0, 0);
-    uint32_t key[4 * IT];
-    int pos[IT];
-    int blocks = 0;                                     // Philox blocks of the pixel
-#pragma unroll
-    for (int it = 0; it < IT; it++) {
-        if (it > 0 && blocks <= 64 * it) {              // wave-uniform
-#pragma unroll
-            for (int q = 0; q < 4; q++) key[4 * it + q] = kNoKey;
-            pos[it] = 0;
+    const unsigned long long some = TURNS > 1 ? drawn_pixels(reach, blk, L, lane) : ~0ull;
+    if (TURNS > 1 && some == 0ull) { empty_columns(W, H, k, ti, tj, pl0, lane, out); return; }
+#pragma unroll 1
+    for (int turn = 0; turn < TURNS; turn++) {
+        const int pl = pl0 + turn;
+        const int i = ti * 8 + (pl >> 3), j = tj * 8 + (pl & 7);
+        if (i >= W || j >= H) continue;                     // wave-uniform
+        const float qx = (float)i, qy = (float)j;
+        const uint32_t pixel = (uint32_t)(j + H * i);
+        int2 fc = make_int2(0, 0);
+        if (((some >> pl) & 1ull) && lane < L) fc = reach[((long)blk * L + lane) * 64 + pl];
+        if (__ballot(fc.y > 0) == 0ull) {
+            for (int s = lane; s < k; s += 64) out[(long)pixel * k + s] = -1;
             continue;
         }
-        const int t = it * 64 + lane;
-        int la = 0, kk0 = 0, first = 0, cnt = 0;
-        blocks = 0;
-        for (int l = 0; l < L; l++) {
-            const int f = __builtin_amdgcn_readlane(fc.x, l), c = __builtin_amdgcn_readlane(fc.y, l);
-            const int nb = (c + 3) >> 2;
-            if (t >= blocks && t < blocks + nb) { la = l; kk0 = 4 * (t - blocks); first = f; cnt = c; }
-            blocks += nb;
-        }
-        const u32x4 rnd = philox4x32_10(u32x4{ (uint32_t)(kk0 >> 2), (uint32_t)la, pixel, view }, seedLo, seedHi);
-        pos[it] = first + kk0;
-        float2 xy[4];
+        uint32_t key[4 * IT];
+        int pos[IT];
+        int blocks = 0;                                     // Philox blocks of the pixel
 #pragma unroll
-        for (int q = 0; q < 4; q++) xy[q] = kk0 + q < cnt ? leafXY[pos[it] + q] : make_float2(0.0f, 0.0f);
+        for (int it = 0; it < IT; it++) {
+            if (it > 0 && blocks <= 64 * it) {              // wave-uniform
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t kb = draw_key(qx, qy, xy[q], is2h,
-                                         (q == 0) ? rnd.x : (q == 1) ? rnd.y : (q == 2) ? rnd.z : rnd.w);
-            key[4 * it + q] = kk0 + q < cnt ? kb : kNoKey;
-        }
-    }
-    auto count = [&](uint32_t x) {
-        int c = 0;
-#pragma unroll
-        for (int e = 0; e < 4 * IT; e++) c += __popcll(__ballot(key[e] <= x));
-        return c;
-    };
-    // threshold: every finite key if at most CAP, else one that k .. CAP keys meet
-    uint32_t thr = kInfKey - 1;
-    int m = count(thr);
-    bool tie = false;
-    uint32_t kth = kInfKey;                             // the k-th smallest key
-    if (m > CAP) {
-        uint32_t lo = 0, hi = kInfKey - 1, step = 1u << 23;   // count(lo) < k, count(hi) > CAP
-        uint32_t mid = 0x3f800000u;                     // keys lie around 1: gallop by octaves from there
-        while (true) {
-            m = count(mid);
-            if (m >= k && m <= CAP) { thr = mid; break; }
-            const bool up = m < k;
-            if (up) lo = mid; else hi = mid;
-            if (hi - lo <= 1) { tie = true; kth = hi; break; }    // more than CAP - k keys equal hi
-            if (up && hi == kInfKey - 1) mid = hi - mid > step ? mid + step : lo + ((hi - lo) >> 1);
-            else if (!up && lo == 0) mid = mid > step ? mid - step : hi >> 1;
-            else mid = lo + ((hi - lo) >> 1);
-            if (step < 1u << 30) step <<= 1;            // 2^30 spans the keys above 1; past that, halve
-        }
-    }
-    if (!tie) {
-        uint32_t* sk = sKey[wv];
-        int base = 0;
-#pragma unroll
-        for (int e = 0; e < 4 * IT; e++) {
-            const bool in = key[e] <= thr;
-            const unsigned long long mk = __ballot(in);
-            const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0));
-            if (in) { sk[at] = key[e]; sPos[wv][at] = pos[e >> 2] + (e & 3); }
-            base += __popcll(mk);
-        }
-#pragma unroll
-        for (int r = 0; r < ROWS; r++)
-            if (r * 64 + lane >= m) sk[r * 64 + lane] = kNoKey;
-        wave_lds_fence();
-        uint32_t mine[ROWS];
-        int id[ROWS], rank[ROWS];
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            const int e = r * 64 + lane;
-            mine[r] = sk[e];
-            id[r] = e < m ? leafId[sPos[wv][e]] : -1;
-            rank[r] = 0;
-        }
-        for (int q0 = 0; q0 < CAP; q0 += 16) {
-            if (q0 >= m) break;                         // wave-uniform
-            uint32_t o[16];
-#pragma unroll
-            for (int q = 0; q < 16; q += 4) {
-                const uint4 v = *(const uint4*)(sk + q0 + q);
-                o[q] = v.x; o[q + 1] = v.y; o[q + 2] = v.z; o[q + 3] = v.w;
+                for (int q = 0; q < 4; q++) key[4 * it + q] = kNoKey;
+                pos[it] = 0;
+                continue;
             }
-#pragma unroll
-            for (int q = 0; q < 16; q++)
-#pragma unroll
-                for (int r = 0; r < ROWS; r++) rank[r] += o[q] < mine[r];
-        }
-        // equal keys share a rank: of the lanes writing one place, one reads its own entry back
-#pragma unroll
-        for (int r = 0; r < ROWS; r++)
-            if (r * 64 + lane < m) sOwner[wv][rank[r]] = r * 64 + lane;
-        wave_lds_fence();
-        bool dup = false;
-        uint32_t top = 0;
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            if (r * 64 + lane >= m) continue;
-            dup |= sOwner[wv][rank[r]] != r * 64 + lane;
-            if (rank[r] < k && mine[r] > top) top = mine[r];
-        }
-        tie = __ballot(dup) != 0ull;
-        if (tie && m >= k) {
-            for (int o = 32; o > 0; o >>= 1) {
-                const uint32_t x = (uint32_t)__shfl_xor((int)top, o, 64);
-                top = x > top ? x : top;
+            const int t = it * 64 + lane;
+            int la = 0, kk0 = 0, first = 0, cnt = 0;
+            blocks = 0;
+            for (int l = 0; l < L; l++) {
+                const int f = __builtin_amdgcn_readlane(fc.x, l), c = __builtin_amdgcn_readlane(fc.y, l);
+                const int nb = (c + 3) >> 2;
+                if (t >= blocks && t < blocks + nb) { la = l; kk0 = 4 * (t - blocks); first = f; cnt = c; }
+                blocks += nb;
             }
-            kth = top;
+            const u32x4 rnd = philox4x32_10(u32x4{ (uint32_t)(kk0 >> 2), (uint32_t)la, pixel, view }, seedLo, seedHi);
+            pos[it] = first + kk0;
+            float2 xy[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) xy[q] = kk0 + q < cnt ? leafXY[pos[it] + q] : make_float2(0.0f, 0.0f);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t kb = draw_key(qx, qy, xy[q], is2h,
+                                             (q == 0) ? rnd.x : (q == 1) ? rnd.y : (q == 2) ? rnd.z : rnd.w);
+                key[4 * it + q] = kk0 + q < cnt ? kb : kNoKey;
+            }
         }
-        wave_lds_fence();
-        int32_t* o = out + (long)pixel * k;
+        auto count = [&](uint32_t x) {
+            int c = 0;
+#pragma unroll
+            for (int e = 0; e < 4 * IT; e++) c += __popcll(__ballot(key[e] <= x));
+            return c;
+        };
+        // threshold: every finite key if at most CAP, else one that k .. CAP keys meet
+        uint32_t thr = kInfKey - 1;
+        int m = count(thr);
+        bool tie = false;
+        uint32_t kth = kInfKey;                             // the k-th smallest key
+        if (m > CAP) {
+            uint32_t lo = 0, hi = kInfKey - 1, step = 1u << 23;   // count(lo) < k, count(hi) > CAP
+            uint32_t mid = 0x3f800000u;                     // keys lie around 1: gallop by octaves from there
+            while (true) {
+                m = count(mid);
+                if (m >= k && m <= CAP) { thr = mid; break; }
+                const bool up = m < k;
+                if (up) lo = mid; else hi = mid;
+                if (hi - lo <= 1) { tie = true; kth = hi; break; }    // more than CAP - k keys equal hi
+                if (up && hi == kInfKey - 1) mid = hi - mid > step ? mid + step : lo + ((hi - lo) >> 1);
+                else if (!up && lo == 0) mid = mid > step ? mid - step : hi >> 1;
+                else mid = lo + ((hi - lo) >> 1);
+                if (step < 1u << 30) step <<= 1;            // 2^30 spans the keys above 1; past that, halve
+            }
+        }
         if (!tie) {
-            int* so = sOwner[wv];                       // ids in rank order
+            uint32_t* sk = sKey[wv];
+            int base = 0;
+#pragma unroll
+            for (int e = 0; e < 4 * IT; e++) {
+                const bool in = key[e] <= thr;
+                const unsigned long long mk = __ballot(in);
+                const int at = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0));
+                if (in) { sk[at] = key[e]; sPos[wv][at] = pos[e >> 2] + (e & 3); }
+                base += __popcll(mk);
+            }
 #pragma unroll
             for (int r = 0; r < ROWS; r++)
-                if (r * 64 + lane < m) so[rank[r]] = id[r];
+                if (r * 64 + lane >= m) sk[r * 64 + lane] = kNoKey;
             wave_lds_fence();
-            for (int s = lane; s < k; s += 64) o[s] = s < m ? so[s] : -1;
+            uint32_t mine[ROWS];
+            int id[ROWS], rank[ROWS];
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                const int e = r * 64 + lane;
+                mine[r] = sk[e];
+                id[r] = e < m ? leafId[sPos[wv][e]] : -1;
+                rank[r] = 0;
+            }
+            for (int q0 = 0; q0 < CAP; q0 += 16) {
+                if (q0 >= m) break;                         // wave-uniform
+                uint32_t o[16];
+#pragma unroll
+                for (int q = 0; q < 16; q += 4) {
+                    const uint4 v = *(const uint4*)(sk + q0 + q);
+                    o[q] = v.x; o[q + 1] = v.y; o[q + 2] = v.z; o[q + 3] = v.w;
+                }
+#pragma unroll
+                for (int q = 0; q < 16; q++)
+#pragma unroll
+                    for (int r = 0; r < ROWS; r++) rank[r] += o[q] < mine[r];
+            }
+            // equal keys share a rank: of the lanes writing one place, one reads its own entry back
+#pragma unroll
+            for (int r = 0; r < ROWS; r++)
+                if (r * 64 + lane < m) sOwner[wv][rank[r]] = r * 64 + lane;
+            wave_lds_fence();
+            bool dup = false;
+            uint32_t top = 0;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                if (r * 64 + lane >= m) continue;
+                dup |= sOwner[wv][rank[r]] != r * 64 + lane;
+                if (rank[r] < k && mine[r] > top) top = mine[r];
+            }
+            tie = __ballot(dup) != 0ull;
+            if (tie && m >= k) {
+                for (int o = 32; o > 0; o >>= 1) {
+                    const uint32_t x = (uint32_t)__shfl_xor((int)top, o, 64);
+                    top = x > top ? x : top;
+                }
+                kth = top;
+            }
+            wave_lds_fence();
+            int32_t* o = out + (long)pixel * k;
+            if (!tie) {
+                int* so = sOwner[wv];                       // ids in rank order
+#pragma unroll
+                for (int r = 0; r < ROWS; r++)
+                    if (r * 64 + lane < m) so[rank[r]] = id[r];
+                wave_lds_fence();
+                for (int s = lane; s < k; s += 64) o[s] = s < m ? so[s] : -1;
+            }
         }
-    }
-    if (tie && lane == 0) {
-        const int e = atomicAdd(tieQueue, 1);
-        tieQueue[1 + 2 * e] = blk * 64 + pl;
-        tieQueue[2 + 2 * e] = (int)kth;
+        if (tie && lane == 0) {
+            const int e = atomicAdd(tieQueue, 1);
+            tieQueue[1 + 2 * e] = blk * 64 + pl;
+            tieQueue[2 + 2 * e] = (int)kth;
+        }
+        wave_lds_fence();
     }
 }
 
@@ -2531,6 +2580,7 @@ __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw(int W, int H, i
 // k = 24: 271 -> 166 us.
 inline bool draw_halves(int k, int L) { return k <= 32 && L * ((k + 3) / 4) <= 32; }
 
+template <int TURNS>
 __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw_halves(int W, int H, int k, int L, int tiles,
                                                                         uint32_t seedLo, uint32_t seedHi,
                                                                         uint32_t view, const ViewState* __restrict__ vs,
@@ -2552,118 +2602,130 @@ __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw_halves(int W, i
     __shared__ int sOwner[kDrawWaves][64];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int s = lane & 31, h0 = lane & 32;            // lane of the pixel, its first lane
-    constexpr int per = 32 / kDrawWaves;                // workgroups per tile, as above
+    constexpr int per = 32 / (kDrawWaves * TURNS);      // workgroups per tile, as above
     const int full = tiles & ~7, d = blockIdx.x;
     const int blk = d < full * per ? (d >> 3) / per * 8 + (d & 7) : d / per;
-    const int pl = 2 * ((d < full * per ? (d >> 3) % per : d % per) * kDrawWaves + wv) + (h0 >> 5);
+    const int pl0 = 2 * TURNS * ((d < full * per ? (d >> 3) % per : d % per) * kDrawWaves + wv) + (h0 >> 5);
     const int tilesY = (H + 7) >> 3;
     const uint32_t tile = xcd_chunk_remap<kSampTileRun>((uint32_t)blk, (uint32_t)tiles);
     const int ti = tile / tilesY, tj = tile - (tile / tilesY) * tilesY;
-    const int i = ti * 8 + (pl >> 3), j = tj * 8 + (pl & 7);
-    const bool in = i < W && j < H;
-    if (!__ballot(in)) return;                          // wave-uniform
     const float is2h = vs->is2h;
-    const float qx = (float)i, qy = (float)j;
-    const uint32_t pixel = in ? (uint32_t)(j + H * i) : 0u;
-    const int2 fc = in && s < L ? reach[((long)blk * L + s) * 64 + pl] : make_int2(0, 0);
-    auto half_of = [&](unsigned long long m) { return h0 ? (uint32_t)(m >> 32) : (uint32_t)m; };
-    int la = 0, kk0 = 0, first = 0, cnt = 0, blocks = 0;
-    for (int l = 0; l < L; l++) {
-        const int f = __shfl(fc.x, h0 + l, 64), c = __shfl(fc.y, h0 + l, 64);
-        const int nb = (c + 3) >> 2;
-        if (s >= blocks && s < blocks + nb) { la = l; kk0 = 4 * (s - blocks); first = f; cnt = c; }
-        blocks += nb;
-    }
-    const u32x4 rnd = philox4x32_10(u32x4{ (uint32_t)(kk0 >> 2), (uint32_t)la, pixel, view }, seedLo, seedHi);
-    const int pos = first + kk0;
-    uint32_t key[4];
-    {
-        float2 xy[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) xy[q] = kk0 + q < cnt ? leafXY[pos + q] : make_float2(0.0f, 0.0f);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t kb = draw_key(qx, qy, xy[q], is2h,
-                                         (q == 0) ? rnd.x : (q == 1) ? rnd.y : (q == 2) ? rnd.z : rnd.w);
-            key[q] = kk0 + q < cnt ? kb : kNoKey;
+    const unsigned long long some = TURNS > 1 ? drawn_pixels(reach, blk, L, lane) : ~0ull;
+    if (TURNS > 1 && some == 0ull) { empty_columns(W, H, k, ti, tj, pl0 - (h0 >> 5), lane, out); return; }
+#pragma unroll 1
+    for (int turn = 0; turn < TURNS; turn++) {
+        const int pl = pl0 + 2 * turn;
+        const int i = ti * 8 + (pl >> 3), j = tj * 8 + (pl & 7);
+        const bool in = i < W && j < H;
+        if (!__ballot(in)) continue;                        // wave-uniform
+        const float qx = (float)i, qy = (float)j;
+        const uint32_t pixel = in ? (uint32_t)(j + H * i) : 0u;
+        int2 fc = make_int2(0, 0);
+        if (in && ((some >> pl) & 1ull) && s < L) fc = reach[((long)blk * L + s) * 64 + pl];
+        if (__ballot(fc.y > 0) == 0ull) {                   // both pixels are empty
+            if (in && s < k) out[(long)pixel * k + s] = -1;
+            continue;
         }
-    }
-    auto count = [&](uint32_t x) {
-        int c = 0;
-#pragma unroll
-        for (int e = 0; e < 4; e++) c += __popc(half_of(__ballot(key[e] <= x)));
-        return c;
-    };
-    // threshold: every finite key if at most 32, else one that k .. 32 keys meet; the search
-    // of k_sample_draw, each half with its own interval
-    uint32_t thr = kInfKey - 1;
-    int m = count(thr);
-    bool tie = false, search = m > 32;
-    uint32_t kth = kInfKey;                             // the k-th smallest key
-    uint32_t lo = 0, hi = kInfKey - 1, step = 1u << 23, mid = 0x3f800000u;
-    while (__ballot(search)) {
-        const int c = count(mid);
-        if (!search) continue;
-        if (c >= k && c <= 32) { thr = mid; m = c; search = false; continue; }
-        const bool up = c < k;
-        if (up) lo = mid; else hi = mid;
-        if (hi - lo <= 1) { tie = true; kth = hi; search = false; continue; }
-        if (up && hi == kInfKey - 1) mid = hi - mid > step ? mid + step : lo + ((hi - lo) >> 1);
-        else if (!up && lo == 0) mid = mid > step ? mid - step : hi >> 1;
-        else mid = lo + ((hi - lo) >> 1);
-        if (step < 1u << 30) step <<= 1;
-    }
-    uint32_t* sk = sKey[wv] + h0;
-    int* so = sOwner[wv] + h0;
-    sKey[wv][lane] = kNoKey;
-    wave_lds_fence();
-    int base = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const bool take = !tie && key[e] <= thr;
-        const uint32_t mk = half_of(__ballot(take));
-        const int at = base + __popc(mk & ((1u << s) - 1u));
-        if (take) { sk[at] = key[e]; sPos[wv][h0 + at] = pos + e; }
-        base += __popc(mk);
-    }
-    wave_lds_fence();
-    const bool held = !tie && s < m;
-    const uint32_t mine = sk[s];
-    const int id = held ? leafId[sPos[wv][lane]] : -1;
-    int rank = 0;
-    for (int q0 = 0; q0 < 32; q0 += 16) {
-        if (!__ballot(held && q0 < m)) break;
-        uint32_t o[16];
-#pragma unroll
-        for (int q = 0; q < 16; q += 4) {
-            const uint4 v = *(const uint4*)(sk + q0 + q);
-            o[q] = v.x; o[q + 1] = v.y; o[q + 2] = v.z; o[q + 3] = v.w;
+        auto half_of = [&](unsigned long long m) { return h0 ? (uint32_t)(m >> 32) : (uint32_t)m; };
+        int la = 0, kk0 = 0, first = 0, cnt = 0, blocks = 0;
+        for (int l = 0; l < L; l++) {
+            const int f = __shfl(fc.x, h0 + l, 64), c = __shfl(fc.y, h0 + l, 64);
+            const int nb = (c + 3) >> 2;
+            if (s >= blocks && s < blocks + nb) { la = l; kk0 = 4 * (s - blocks); first = f; cnt = c; }
+            blocks += nb;
         }
+        const u32x4 rnd = philox4x32_10(u32x4{ (uint32_t)(kk0 >> 2), (uint32_t)la, pixel, view }, seedLo, seedHi);
+        const int pos = first + kk0;
+        uint32_t key[4];
+        {
+            float2 xy[4];
 #pragma unroll
-        for (int q = 0; q < 16; q++) rank += o[q] < mine;
-    }
-    // equal keys share a rank: of the lanes writing one place, one reads its own entry back
-    if (held) so[rank] = s;
-    wave_lds_fence();
-    const bool dup = held && so[rank] != s;
-    uint32_t top = held && rank < k ? mine : 0u;
-    if (half_of(__ballot(dup))) {
-        tie = true;
-        kth = kInfKey;
-    }
-    for (int o = 16; o > 0; o >>= 1) {
-        const uint32_t x = (uint32_t)__shfl_xor((int)top, o, 64);
-        top = x > top ? x : top;
-    }
-    if (tie && m >= k && top > 0u) kth = top;           // equal keys among those held
-    wave_lds_fence();
-    if (held && !tie) so[rank] = id;                    // ids in rank order
-    wave_lds_fence();
-    if (in && !tie && s < k) out[(long)pixel * k + s] = s < m ? so[s] : -1;
-    if (in && tie && s == 0) {
-        const int e = atomicAdd(tieQueue, 1);
-        tieQueue[1 + 2 * e] = blk * 64 + pl;
-        tieQueue[2 + 2 * e] = (int)kth;
+            for (int q = 0; q < 4; q++) xy[q] = kk0 + q < cnt ? leafXY[pos + q] : make_float2(0.0f, 0.0f);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t kb = draw_key(qx, qy, xy[q], is2h,
+                                             (q == 0) ? rnd.x : (q == 1) ? rnd.y : (q == 2) ? rnd.z : rnd.w);
+                key[q] = kk0 + q < cnt ? kb : kNoKey;
+            }
+        }
+        auto count = [&](uint32_t x) {
+            int c = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) c += __popc(half_of(__ballot(key[e] <= x)));
+            return c;
+        };
+        // threshold: every finite key if at most 32, else one that k .. 32 keys meet; the search
+        // of k_sample_draw, each half with its own interval
+        uint32_t thr = kInfKey - 1;
+        int m = count(thr);
+        bool tie = false, search = m > 32;
+        uint32_t kth = kInfKey;                             // the k-th smallest key
+        uint32_t lo = 0, hi = kInfKey - 1, step = 1u << 23, mid = 0x3f800000u;
+        while (__ballot(search)) {
+            const int c = count(mid);
+            if (!search) continue;
+            if (c >= k && c <= 32) { thr = mid; m = c; search = false; continue; }
+            const bool up = c < k;
+            if (up) lo = mid; else hi = mid;
+            if (hi - lo <= 1) { tie = true; kth = hi; search = false; continue; }
+            if (up && hi == kInfKey - 1) mid = hi - mid > step ? mid + step : lo + ((hi - lo) >> 1);
+            else if (!up && lo == 0) mid = mid > step ? mid - step : hi >> 1;
+            else mid = lo + ((hi - lo) >> 1);
+            if (step < 1u << 30) step <<= 1;
+        }
+        uint32_t* sk = sKey[wv] + h0;
+        int* so = sOwner[wv] + h0;
+        sKey[wv][lane] = kNoKey;
+        wave_lds_fence();
+        int base = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const bool take = !tie && key[e] <= thr;
+            const uint32_t mk = half_of(__ballot(take));
+            const int at = base + __popc(mk & ((1u << s) - 1u));
+            if (take) { sk[at] = key[e]; sPos[wv][h0 + at] = pos + e; }
+            base += __popc(mk);
+        }
+        wave_lds_fence();
+        const bool held = !tie && s < m;
+        const uint32_t mine = sk[s];
+        const int id = held ? leafId[sPos[wv][lane]] : -1;
+        int rank = 0;
+        for (int q0 = 0; q0 < 32; q0 += 16) {
+            if (!__ballot(held && q0 < m)) break;
+            uint32_t o[16];
+#pragma unroll
+            for (int q = 0; q < 16; q += 4) {
+                const uint4 v = *(const uint4*)(sk + q0 + q);
+                o[q] = v.x; o[q + 1] = v.y; o[q + 2] = v.z; o[q + 3] = v.w;
+            }
+#pragma unroll
+            for (int q = 0; q < 16; q++) rank += o[q] < mine;
+        }
+        // equal keys share a rank: of the lanes writing one place, one reads its own entry back
+        if (held) so[rank] = s;
+        wave_lds_fence();
+        const bool dup = held && so[rank] != s;
+        uint32_t top = held && rank < k ? mine : 0u;
+        if (half_of(__ballot(dup))) {
+            tie = true;
+            kth = kInfKey;
+        }
+        for (int o = 16; o > 0; o >>= 1) {
+            const uint32_t x = (uint32_t)__shfl_xor((int)top, o, 64);
+            top = x > top ? x : top;
+        }
+        if (tie && m >= k && top > 0u) kth = top;           // equal keys among those held
+        wave_lds_fence();
+        if (held && !tie) so[rank] = id;                    // ids in rank order
+        wave_lds_fence();
+        if (in && !tie && s < k) out[(long)pixel * k + s] = s < m ? so[s] : -1;
+        if (in && tie && s == 0) {
+            const int e = atomicAdd(tieQueue, 1);
+            tieQueue[1 + 2 * e] = blk * 64 + pl;
+            tieQueue[2 + 2 * e] = (int)kth;
+        }
+        wave_lds_fence();
     }
 }
 
@@ -4147,17 +4209,23 @@ void launch_sample(int N, int W, int H, int k, uint32_t seedLo, uint32_t seedHi,
                                                         trie_entries(k), w.tileInfo, w.walkQueue, vsd);
     k_sample_descend<<<wg, 64, 0, st>>>(W, H, k, L, w.vs, w.geo, w.lnk, w.aux, w.coef, w.srec, w.trie, trie_entries(k),
                                         w.tileInfo, w.reach, err, vsd);
-    const dim3 dg(tiles * (64 / kDrawWaves), views);
     // a pixel has at most L ceil(k / 4) Philox blocks, 64 per iteration: 8 x 16, 12 x 32
     // and 16 x 64 at k = 64, 128 and 256
-#define UD_DRAW(R, I) k_sample_draw<R, I><<<dg, 64 * kDrawWaves, 0, st>>>(                                            \
+    auto draw = [&](auto turns) {
+        constexpr int T = decltype(turns)::value;
+        const dim3 dg(tiles * (64 / (kDrawWaves * T)), views);
+#define UD_DRAW(R, I) k_sample_draw<R, I, T><<<dg, 64 * kDrawWaves, 0, st>>>(                                         \
         W, H, k, L, (int)tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out, w.tieQueue, vsd)
-    if (draw_halves(k, L))
-        k_sample_draw_halves<<<dim3(tiles * (32 / kDrawWaves), views), 64 * kDrawWaves, 0, st>>>(
-            W, H, k, L, (int)tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out, w.tieQueue, vsd);
-    else if (k <= 64) UD_DRAW(1, 2);
-    else if (k <= 128) UD_DRAW(2, 6);
-    else UD_DRAW(4, 16);
+        if (draw_halves(k, L)) {
+            constexpr int TH = T > 8 ? 8 : T;
+            k_sample_draw_halves<TH><<<dim3(tiles * (32 / (kDrawWaves * TH)), views), 64 * kDrawWaves, 0, st>>>(
+                W, H, k, L, (int)tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA, w.reach, out, w.tieQueue, vsd);
+        } else if (k <= 64) UD_DRAW(1, 2);
+        else if (k <= 128) UD_DRAW(2, 6);
+        else UD_DRAW(4, 16);
+    };
+    if ((long)tiles * views >= kDrawManyTiles && k <= 128) draw(std::integral_constant<int, kDrawTurns>{});
+    else draw(std::integral_constant<int, 1>{});
 #undef UD_DRAW
     k_sample_replay<<<dim3(64, views), 64, 0, st>>>(W, H, k, L, tiles, seedLo, seedHi, view, w.vs, w.leafXY, w.idsA,
                                                     w.reach, w.tieQueue, out, vsd);
