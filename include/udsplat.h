@@ -154,7 +154,9 @@ int ude_tile_features(int bn, int N, int W, int H, double f, double smoothing, d
 int ude_mlp_param_count(void);
 size_t ude_mlp_workspace_bytes(int T);
 
-/* y[t] = network(X[t]) for T rows of 32 features. */
+/* y[t] = network(X[t]) for T rows of 32 features.  The kernel keeps everything in
+ * registers and LDS and leaves ws alone; less than ude_mlp_workspace_bytes(T) is
+ * refused all the same. */
 int ude_mlp_forward(int T, const float* X, const float* params, float* y, void* ws, size_t wsBytes,
                     ude_stream_t stream);
 

@@ -23,7 +23,7 @@
 //  10 k_sample_draw   wavefront per pixel: sequential Poisson keys u/p from
 //                     Philox4x32-10, the k smallest in order (k_sample_replay:
 //                     pixels with equal keys)
-// Views of at most 4096 splats take stages 1-6 in one workgroup (k_front_small).
+// Views of at most 4096 splats take stages 1-4 in one workgroup (k_front_small).
 // The fixed-order and Poisson-rate paths share stages 1-6 and add expansion
 // selection and moments per band (k_fixed_*), walk records (k_fmm_records,
 // k_walk_records), the density walk (k_fmm_eval) and the thinning pass
@@ -724,9 +724,12 @@ __global__ __launch_bounds__(256) void k_sort_scatter(const ViewState* __restric
 
 // ---------------------------------------------------------------------------
 // State, bandwidth, cull and sort of up to kFrontSplats splats in one workgroup and one
-// launch: at these sizes the 18 kernels above take 2 to 9 us each, most of it their own
-// start and end (4096 splats: 71 us in all, here 47; 256: 47, here 12).  The line lies
-// where a 20-bit key and a position fill a 32-bit word, which a bitonic network in LDS
+// launch: at these sizes the 11 kernels above are mostly their own starts and ends, while
+// the network's steps grow with the splats.  sampling.sample of one 64x64 view, k = 8, on the
+// device / until the call has ended, those kernels -> this one: 64 splats 71 -> 54 / 129 ->
+// 95 us, 1024 146 -> 132 / 187 -> 161, 3072 218 -> 220 / 257 -> 249, 4096 248 -> 253 / 287 ->
+// 283; 16 views of 4096 306 both / 362 -> 358.  The line lies where the device's time is even,
+// and where a 20-bit key and a position fill a 32-bit word, which a bitonic network in LDS
 // sorts; the order is the stable radix sort's.
 // ---------------------------------------------------------------------------
 constexpr int kFrontSplats = 4096;
@@ -2333,7 +2336,7 @@ __device__ __forceinline__ bool draw_word(float qx, float qy, float2 xy, float i
 
 // Sequential Poisson keys over the leaves each launch reached (the walk's
 // capacity descents do not depend on the keys, so they run first, in
-// k_sample_walk): in a Karras tree the leaves of a subtree are the contiguous
+// k_sample_descend): in a Karras tree the leaves of a subtree are the contiguous
 // sorted range [first, first + count), in the left-to-right order nextLeaf visits
 // (sequentialPoissonDynamicTree.cuh:16-53), and every leaf carries the single
 // Hermite coefficient 1, so E(leaf) = e^{-tx^2} e^{-ty^2}.  Key u / E with u the
@@ -2740,8 +2743,8 @@ __global__ __launch_bounds__(64 * kDrawWaves) void k_sample_draw_halves(int W, i
 // position s > s0 keeps its entry inside a run and otherwise takes the first
 // entry of the run ending at s - 1; s0 takes c.  Candidates are keyed 64 at a
 // time, one per lane, and inserted in the reference's order; one whose key is
-// above the final list's largest (queued by k_sample_draw: the heap ends with the
-// same largest key) is skipped, as it only ever joins runs the list drops whole.
+// above the final list's largest (k_sample_draw queued the pixel's k-th smallest
+// key) is skipped, as it only ever joins runs the list drops whole.
 // A persistent grid drains the queue.
 constexpr int kReplayRows = 4;
 __global__ __launch_bounds__(64) void k_sample_replay(int W, int H, int k, int L, unsigned drawBlocks, uint32_t seedLo,
