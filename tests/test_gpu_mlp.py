@@ -158,3 +158,50 @@ def test_tile_scale_gradient_of_counts(dev):
     assert abs(float((tangent.double() * g).sum()) - float((gb * v).sum())) < 1e-5 * float((gb * v).abs().sum())
     with torch.no_grad():
         assert not net.tile_scale(F, a).requires_grad
+
+
+def ordered_case(T, seed):
+    """Hidden units that are exact: H1 = relu of the features and of their negatives, H2 = H1."""
+    rng = np.random.default_rng(seed)
+    X = M.bf16(rng.normal(size=(T, M.N_IN))).astype(np.float32)
+    P = np.zeros(M.N_PARAMS, np.float32)
+    P[:M.OFF_B1] = np.hstack([np.eye(M.N_IN), -np.eye(M.N_IN)]).ravel()
+    P[M.OFF_W2:M.OFF_B2] = np.eye(M.N_HID).ravel()
+    P[M.OFF_W3:M.OFF_B3] = M.bf16(rng.normal(size=M.N_HID))
+    P[M.OFF_B3] = rng.normal()
+    tgt, w = rng.normal(size=T).astype(np.float32), rng.uniform(0.5, 2.0, size=T).astype(np.float32)
+    H = np.maximum(np.hstack([X, -X]), 0.0).astype(np.float32)
+    y = np.zeros(T, np.float32)
+    for k in range(M.N_HID):                    # exact products (16 bits), float32 sums in order
+        y = y + H[:, k] * P[M.OFF_W3 + k]
+    return X, P, tgt, w, H, y + P[M.OFF_B3]
+
+
+@pytest.mark.parametrize("T", [1, 15, 64, 333, 20011])
+def test_output_layer_sums_in_order(dev, T):
+    from splatting_amd.learned import RateNet
+    X, P, _, _, _, y = ordered_case(T, T)
+    net = RateNet(t(P, dev), t(np.zeros(M.N_IN), dev), t(np.ones(M.N_IN), dev))
+    assert np.array_equal(net.forward(t(X, dev)).cpu().numpy(), y)
+
+
+@pytest.mark.parametrize("T", [1, 33, 320, 1025])
+def test_output_gradient_rounds_the_ordered_sums(dev, T):
+    """dZ2 = bf16(dy W3) of dy in float32 from the sums in order.  dW2 sums at most T exact
+    products per element in float32, within T 2^-23 of their magnitudes; a term rounded the
+    other way is 2^-8 of itself off."""
+    from splatting_amd.learned import RateNet
+    f = np.float32
+    for seed in range(12):
+        X, P, tgt, w, H, y = ordered_case(T, 1000 * T + seed)
+        s = np.zeros(1024, f)
+        for a in range(0, T, 1024):
+            s[:min(1024, T - a)] += w[a:a + 1024]
+        while len(s) > 1:
+            s = s[:len(s) // 2] + s[len(s) // 2:]
+        dy = (f(2.0) * w) * (y - tgt) * (f(1.0) / s[0])
+        z = M.bf16(dy[:, None] * P[M.OFF_W3:M.OFF_B3]) * (H > 0)
+        ref, mag = H.T.astype(np.float64) @ z, H.T.astype(np.float64) @ np.abs(z)
+        net = RateNet(t(P, dev), t(np.zeros(M.N_IN), dev), t(np.ones(M.N_IN), dev))
+        g = net.loss_grad(t(X, dev), t(tgt, dev), t(w, dev))[1].cpu().numpy()
+        assert np.all(np.abs(g[M.OFF_W2:M.OFF_B2].reshape(ref.shape) - ref) <= T * 2.0 ** -23 * mag)

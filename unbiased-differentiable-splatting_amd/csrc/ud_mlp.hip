@@ -13,7 +13,7 @@
 // rows accumulate in registers (the accumulator layout of H1 and dZ2 is the operand
 // layout of H1^T dZ2).  One kernel per layer and direction took 15 launches per
 // training evaluation, and its weight-gradient products walked all T rows in one
-// wavefront per 16x16 weights: 1310 us at T = 20480 (now 48 us).
+// wavefront per 16x16 weights: 1310 us at T = 20480 (now 51 us).
 //
 // Parameter block (FP32, 6337 floats): W1 [32][64], b1 [64], W2 [64][64],
 // b2 [64], W3 [64], b3 [1] (row-major, input index first).
@@ -53,7 +53,9 @@ struct Weights {
     uint16_t w1t[kHid * kPad1];              // W1 transposed: [out][in]
     uint16_t w2t[kHid * kPad2];              // W2 transposed: [out][in]
     uint16_t w2[kHid * kPad2];               // W2: [in][out]
-    float b1[kHid], b2[kHid], w3[kHid], b3;  // w3 rounded to bfloat16
+    float b1[kHid], b2[kHid];
+    __align__(16) float w3[kHid];            // rounded to bfloat16
+    float b3;
 };
 
 __device__ __forceinline__ void load_weights(const float* __restrict__ P, Weights& w, bool back)
@@ -102,7 +104,10 @@ __device__ __forceinline__ void to_rows(uint16_t* buf, const bf16x4 (&x)[4], bf1
 }
 
 // H1, H2 (bfloat16, accumulator layout) and y (rows 4g + v, in every lane of a row
-// group) of the 16 rows from t0 on; feature k is (X[k] - mean[k]) / std[k], or X[k]
+// group) of the 16 rows from t0 on; feature k is (X[k] - mean[k]) / std[k], or X[k].
+// y is summed in the order of the hidden units: dZ2 = dy W3 rounds to bfloat16, where a
+// last bit of y that depends on the split moves a term by 2^-9 (one of 317 x 64 changed
+// the gradient by 1.7e-5).  Sixteen lanes side by side cost k_mlp_train 39 -> 42 us at T = 20480.
 __device__ __forceinline__ void forward16(int T, const float* __restrict__ X, const float* __restrict__ mean,
                                           const float* __restrict__ std, long t0, const Weights& w, uint16_t* buf,
                                           int r, int g, bf16x4 (&h1)[4], bf16x4 (&h2)[4], float (&y)[4])
@@ -129,8 +134,6 @@ __device__ __forceinline__ void forward16(int T, const float* __restrict__ X, co
     bf16x4 rows[4];
     to_rows(buf, h1, rows, r, g);
 #pragma unroll
-    for (int v = 0; v < 4; v++) y[v] = 0.0f;
-#pragma unroll
     for (int c = 0; c < 4; c++) {
         f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
@@ -139,14 +142,22 @@ __device__ __forceinline__ void forward16(int T, const float* __restrict__ X, co
         for (int v = 0; v < 4; v++) {
             const uint16_t h = f2bf(fmaxf(z[v] + w.b2[16 * c + r], 0.0f));
             h2[c][v] = (short)h;
-            y[v] += bf2f(h) * w.w3[16 * c + r];
+            buf[(4 * g + v) * kPad2 + 16 * c + r] = h;
         }
     }
+    lds_fence();
+    float s = 0.0f;                          // row r
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        for (int o = 1; o < 16; o <<= 1) y[v] += __shfl_xor(y[v], o, 64);
-        y[v] += w.b3;
+    for (int k = 0; k < kHid; k += 4) {
+        const bf16x4 h = frag(buf + r * kPad2 + k);
+        const f32x4 q = *(const f32x4*)(w.w3 + k);
+#pragma unroll
+        for (int v = 0; v < 4; v++) s = s + bf2f((uint16_t)h[v]) * q[v];
     }
+    s = s + w.b3;
+    lds_fence();
+#pragma unroll
+    for (int v = 0; v < 4; v++) y[v] = __shfl(s, 4 * g + v, 64);
 }
 
 __global__ __launch_bounds__(64 * kWaves) void k_mlp_forward(int T, const float* __restrict__ X,
@@ -169,20 +180,25 @@ __global__ __launch_bounds__(64 * kWaves) void k_mlp_forward(int T, const float*
     }
 }
 
-// sum of the loss weights (T without weights), fixed order; its inverse, 0 for no weight
+// sum of the loss weights (T without weights): 1024 strided sums, added pairwise from the
+// furthest apart on (dy takes its order from here, see forward16); its inverse, 0 for no weight
 __global__ __launch_bounds__(1024) void k_weight_sum(int T, const float* __restrict__ weight, float* __restrict__ inv)
 {
-    __shared__ float sw[16];
+    __shared__ float sw[1024];
     float s = 0.0f;
     for (int t = threadIdx.x; t < T; t += 1024) s = s + (weight ? weight[t] : 1.0f);
-    s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = s;
+    sw[threadIdx.x] = s;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        float W = sw[0];
-        for (int q = 1; q < 16; q++) W = W + sw[q];
-        inv[0] = W > 0.0f ? 1.0f / W : 0.0f;
-    }
+    if (threadIdx.x >= 64) return;
+    float p[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) p[q] = sw[threadIdx.x + 64 * q];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < o; q++) p[q] = p[q] + p[q + o];
+    for (int o = 32; o > 0; o >>= 1) p[0] = p[0] + __shfl_down(p[0], o, 64);
+    if (threadIdx.x == 0) inv[0] = p[0] > 0.0f ? 1.0f / p[0] : 0.0f;
 }
 
 // Forward and backward of the weighted mean-square loss, dy = 2 w (y - target) / sum(w):
