@@ -360,3 +360,17 @@ def test_sampler_batch_leaves_memory(monkeypatch, free, cached, views, capturing
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
     monkeypatch.setattr(_lib, "workspace", lambda nbytes, dev: nbytes)
     assert sampling._view_workspace(10, 8, torch.device("cpu")) == 10 * views
+
+
+@pytest.mark.parametrize("capturing,views", [(False, 4), (True, 1)])
+def test_sampler_batch_without_allocator_statistics(monkeypatch, capturing, views):
+    """Pluggable allocators refuse to be asked what they hold."""
+    from cudaExtensions import _lib, sampling
+
+    def refuses(_):
+        raise RuntimeError("no statistics")
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda _: (320, 10 ** 6))
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", refuses)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    monkeypatch.setattr(_lib, "workspace", lambda nbytes, dev: nbytes)
+    assert sampling._view_workspace(10, 8, torch.device("cpu")) == 10 * views

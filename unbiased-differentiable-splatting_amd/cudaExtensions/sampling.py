@@ -70,11 +70,17 @@ def _views_at_once(bn, W, H):
 
 
 def _spare_bytes(dev):
-    """Device memory that no tensor of this process and nothing else on the device holds."""
-    pool = torch.cuda.memory_stats_as_nested_dict(dev)
+    """Device memory that no tensor of this process and nothing else on the device holds.
+    A pluggable allocator reports no statistics: then what the device itself calls free, and
+    none while a graph is recorded."""
+    capturing = torch.cuda.is_current_stream_capturing()         # the device is not asked then
+    try:
+        pool = torch.cuda.memory_stats_as_nested_dict(dev)
+    except RuntimeError:
+        return 0 if capturing else torch.cuda.mem_get_info(dev)[0]
     held = lambda kind: pool[kind]["all"]["current"] if pool else 0  # noqa: E731
     cached = held("reserved_bytes") - held("allocated_bytes")
-    if torch.cuda.is_current_stream_capturing():         # the device is not asked then
+    if capturing:
         free = torch.cuda.get_device_properties(dev).total_memory - held("reserved_bytes")
     else:
         free = torch.cuda.mem_get_info(dev)[0]
